@@ -133,18 +133,19 @@ int tri_validate_ffn_swiglu(const tri_tensor* x, const tri_tensor* w_gate, const
                             const tri_tensor* w_down, const tri_tensor* hidden, const tri_tensor* out,
                             const tri_tensor* workspace);
 
-/* Workspace of the few-row path.  With at most 64 rows (the reference's own
- * regime: M = 16 new tokens, convert_eval_rms.py:61-107; up to 128 rows when w
- * is at most 64 MB) a product x.w is bound
- * by streaming w from HBM once; the library then splits the K axis over many
- * workgroups, which needs room for fp32 partial sums.  Every FFN entry point
- * takes that room as `workspace`, a 1-D byte buffer (TRI_U8, 16-byte aligned)
- * or NULL; without it, or when it is too small, the large-tile kernels run
- * (same results to rounding, slower for few rows).  tri_gemm_workspace_bytes
- * sizes it for one product [M, K] x [K, ncols] (ncols = 2 F for the gate/up
- * pair); tri_ffn_workspace_bytes for a whole FFN (x [M, N], hidden width F,
- * including the N x N output projection of tri_ffn_block).  Both return 0 when
- * the shape never takes the few-row path.  The attention entry points carry
+/* Workspace of products with few or middling rows (1 to about 1100; the
+ * reference's own regime is M = 16 new tokens, convert_eval_rms.py:61-107).
+ * Such a product is bound by streaming w from HBM once; where whole tiles
+ * would leave part of the chip idle the library cuts the K axis into parts,
+ * which needs room for fp32 partial sums.  Every FFN entry point takes that
+ * room as `workspace`, a 1-D byte buffer (TRI_U8, 16-byte aligned) or NULL;
+ * without it, or when it is too small, a plan that does without runs (same
+ * results to rounding, slower).  tri_gemm_workspace_bytes sizes it for one
+ * product [M, K] x [K, ncols] (ncols = 2 F for the gate/up pair);
+ * tri_ffn_workspace_bytes for a whole FFN (x [M, N], hidden width F, including
+ * the N x N output projection of tri_ffn_block).  Both return 0 when no
+ * product of the shape is cut into parts, except that up to 64 rows at least
+ * the size of one part is returned.  The attention entry points carry
  * the same room inside their scratch buffer (tri_qkv_scratch_bytes), next to
  * the partial results of their key-split attention kernels (few new tokens,
  * or a chunk of tokens against thousands of cached keys). */

@@ -1,0 +1,106 @@
+"""The GEMMs of ring.hip / ring_qkv.hip (few and middling rows) at the sizes where their tiles, remainders and parts can
+go wrong, against fp32 products on the GPU.
+
+Tolerance: both sides sum in fp32, so a result differs by its one rounding to fp16 (half an ulp, 2^-11 of the value;
+two ulps allowed) and by the order of the sums (a few 2^-24 of the summed magnitudes, which are of order one here)."""
+import pytest
+import torch
+
+from trinity_amd import ext
+
+pytestmark = pytest.mark.gpu
+REL, ABS = 2.0 ** -9, 1e-4
+
+
+@pytest.fixture
+def rn():
+    g = torch.Generator(device="cuda:0")
+    g.manual_seed(5)
+    return lambda *s, std=1.0: torch.empty(*s, dtype=torch.float16, device="cuda:0").normal_(0.0, std, generator=g)
+
+
+def check(got, want, what):
+    torch.cuda.synchronize()
+    bad = (got.float() - want).abs() > REL * want.abs() + ABS
+    assert torch.isfinite(got).all() and not bad.any(), "%s: %d of %d, first at %s" % (
+        what, int(bad.sum()), bad.numel(), bad.nonzero()[:1].tolist())
+
+
+@pytest.mark.parametrize("M,K,N", [
+    (1, 64, 8), (1, 96, 136), (32, 4096, 4096), (33, 96, 1000),      # one row; half a k tile at the end; tile edges
+    (64, 14336, 4096), (65, 4544, 4544), (97, 4544, 4672),           # parts of K, ragged columns
+    (129, 4096, 6144), (160, 4544, 18176), (161, 1056, 5000),        # row blocks with a remainder; K = 16.5 k tiles
+    (300, 14336, 4096), (333, 18176, 4544), (700, 4096, 6144),
+    (1100, 4096, 4096), (1101, 512, 1024),                           # the largest rows of the family, and one more
+])
+@pytest.mark.parametrize("kcontig", [False, True])
+@pytest.mark.parametrize("with_ws", [False, True])
+def test_plain_and_residual(rn, M, K, N, kcontig, with_ws):
+    x, r = rn(M, K), rn(M, N)
+    w = rn(N, K, std=K ** -0.5).t() if kcontig else rn(K, N, std=K ** -0.5)
+    ws = torch.empty(ext.gemm_workspace_bytes(M, K, N), dtype=torch.uint8, device="cuda:0") if with_ws else None
+    out = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda:0")
+    ext.matmul(x, w, r, out, workspace=ws)
+    check(out, x.float() @ w.float() + r.float(), "x.w + r")
+
+
+@pytest.mark.parametrize("M,K,F", [
+    (1, 4096, 14336), (16, 96, 72), (48, 4096, 14336), (90, 4096, 14336), (130, 4096, 14336), (300, 4096, 14336),
+    (100, 4544, 4544), (256, 4544, 4544), (500, 1024, 4000),
+])
+@pytest.mark.parametrize("kcontig", [False, True])
+def test_gated_with_row_scale(rn, M, K, F, kcontig):
+    x, rs = rn(M, K), torch.rand(M, device="cuda:0") + 0.5
+    wg, wu = ((rn(F, K, std=K ** -0.5).t() if kcontig else rn(K, F, std=K ** -0.5)) for _ in range(2))
+    ws = torch.empty(ext.gemm_workspace_bytes(M, K, 2 * F), dtype=torch.uint8, device="cuda:0")
+    a, b = (x.float() @ wg.float()) * rs[:, None], (x.float() @ wu.float()) * rs[:, None]
+    for workspace in (ws, None):
+        out = torch.full((M, F), float("nan"), dtype=torch.float16, device="cuda:0")
+        ext.gateup_swiglu(x, wg, wu, rs, out, workspace=workspace)
+        check(out, a * torch.sigmoid(a) * b, "gated")
+
+
+@pytest.mark.parametrize("S,N,Hq,Hkv,D", [
+    (1, 64, 4, 4, 64), (33, 96, 5, 1, 128), (100, 4096, 32, 8, 128), (260, 4096, 32, 8, 128), (200, 4544, 71, 1, 64),
+    (700, 128, 32, 8, 128), (1000, 128, 71, 1, 64), (1100, 160, 32, 4, 128),  # a tile across two weight matrices
+])
+@pytest.mark.parametrize("qknorm", [False, True])
+@pytest.mark.parametrize("kcontig", [False, True])
+def test_qkv_projection(rn, S, N, Hq, Hkv, D, qknorm, kcontig):
+    """The appended K / V rows and the q rows the projection leaves at the start of the scratch buffer."""
+    x = rn(S, N)
+    wq, wk, wv = ((rn(h * D, N, std=N ** -0.5).t() if kcontig else rn(N, h * D, std=N ** -0.5)) for h in (Hq, Hkv, Hkv))
+    P = 5
+    kc, vc = rn(Hkv, P + S, D), rn(Hkv, P + S, D)
+    kept = kc[:, :P].clone(), vc[:, :P].clone()
+    p = ext.attn_params(Hq, Hkv, D, S, kv_prefix=P, qknorm=qknorm, rms_eps=1e-5)
+    scratch = torch.empty(ext.qkv_scratch_bytes(p, N), dtype=torch.uint8, device="cuda:0")
+    # (a log-sum-exp pass keeps nothing fused away: q is stored by every path)
+    s1, s2 = (torch.empty(Hq, P + S, dtype=torch.float32, device="cuda:0") for _ in range(2))
+    ext.roco(x, None, wq, wk, wv, kc, vc, scratch, torch.empty(S, Hq * D, dtype=torch.float16, device="cuda:0"), s1, s2, p)
+
+    def proj(w, heads, norm):
+        t = (x.float() @ w.float()).view(S, heads, D)
+        if norm:
+            t = t.half().float()
+            t = t * torch.rsqrt((t * t).mean(-1, keepdim=True) + 1e-5)
+        return t
+
+    check(scratch[: S * Hq * D * 2].view(torch.float16).view(S, Hq, D), proj(wq, Hq, qknorm), "q")
+    check(kc[:, P:], proj(wk, Hkv, qknorm).transpose(0, 1), "k")
+    check(vc[:, P:], proj(wv, Hkv, False).transpose(0, 1), "v")
+    assert torch.equal(kc[:, :P], kept[0]) and torch.equal(vc[:, :P], kept[1])
+
+
+@pytest.mark.parametrize("M,N,F", [(1, 64, 64), (16, 4096, 1024), (100, 4544, 512), (1200, 512, 256)])
+def test_ffn_block_row_statistic(rn, M, N, F):
+    """rsqrt(mean(attn_O2^2)) from the merge of the output projection, and from the kernel of its own."""
+    o2, x, wo = rn(M, N), rn(M, N), rn(N, N, std=N ** -0.5)
+    wa, wb, w2 = rn(N, F, std=N ** -0.5), rn(N, F, std=N ** -0.5), rn(F, N, std=F ** -0.5)
+    attn, rows = torch.empty_like(x), torch.zeros(M, dtype=torch.float32, device="cuda:0")
+    ws = torch.empty(max(16, ext.ffn_workspace_bytes(M, N, F)), dtype=torch.uint8, device="cuda:0")
+    ext.ffn_block(o2, wo, x, wa, wb, w2, attn, rows, torch.empty(M, F, dtype=torch.float16, device="cuda:0"),
+                  torch.empty_like(x), None, workspace=ws)
+    check(attn, o2.float() @ wo.float() + x.float(), "attn_O2")
+    want = torch.rsqrt((attn.double() ** 2).mean(1)).float()
+    assert ((rows - want).abs() <= 1e-5 * want).all()  # fp32 sums of N squares

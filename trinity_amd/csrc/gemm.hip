@@ -386,29 +386,14 @@ static TilePlan best_plan(int M, int N, int& which) {
   return best;
 }
 
-// Split factor for an [M, K] x [K, N] product with many rows, 1 = a tile plan is at least as good.  Split-K
-// runs all of N as 256 x 128 tiles in `s` parts each and pays for writing and reading the fp32 partials
-// (taken at 4 TB/s against 3.9 TFLOP/s per CU); it wins only when even the best tile plan leaves most of the
-// chip idle and K is deep.
-static int plan_large_split(int M, int K, int N) {
-  if (M <= kSkinnyMaxRows || skinny_workspace_bytes(M, K, N) > 0 || K % 32 != 0 || K < 2048 || N % 8 != 0) return 1;
-  int which;
-  const double base = best_plan(M, N, which).cost;
-  const int mid_all = ((M + 255) / 256) * ((N + 127) / 128);
-  const double t_big = 2.0 * 65536.0 * K / 3.9e12;
-  int best = 1;
-  double best_cost = base * 0.8;  // worth it only for a clear gain
-  for (int s = 2; s <= 16; ++s) {  // (Llama-3-8B FFN at 128 rows: 149.5 us with at most 4 parts, 133.2 us with up to 16)
-    if (K / 32 / s < 16) break;
-    const double cost = 0.65 / s * ((mid_all * s + kCUs - 1) / kCUs) + (2.0 * s * M * (double)N * 4 / 4e12) / t_big;
-    if (cost < best_cost) { best_cost = cost; best = s; }
-  }
-  return best;
-}
+// What a tile plan should take, in us: 6 us of launch, first loads and epilogue, and 27 ns per unit of K for a round
+// of 256 x 256 tiles (Llama-3-8B and Falcon-7B products, 256 to 1536 rows: within 12 %).
+static float plan_us(const TilePlan& p, int K) { return 6.0f + 0.0272f * (float)K * (float)p.cost; }
 
-int64_t large_split_workspace_bytes(int M, int K, int N) {
-  const int s = plan_large_split(M, K, N);
-  return s > 1 ? (int64_t)s * M * N * 4 : 0;
+// The ring kernels' plan for a product, if it beats a tile plan of big_us.
+static bool ring_wins(float big_us, int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes, RingPlan& plan) {
+  plan = ring_plan(M, K, ncols, unit, min_bn, ws_bytes);
+  return plan.tile >= 0 && plan.us < big_us;
 }
 
 // plain and GELU epilogues on the direct-to-LDS path: pick the cheapest plan
@@ -426,13 +411,35 @@ static int launch_gemm_fast(const GemmArgs& a, hipStream_t stream) {
   }
 }
 
-int launch_gemm(const GemmArgs& a, hipStream_t stream) {
-  if (a.M <= 0 || a.N <= 0) return 0;
+// the tile plan a product gets when the ring kernels do not take it: plain and GELU products over row-major weights
+// choose from the whole family, the others keep the two-shape plan
+static TilePlan big_plan(int M, int N, int epi, bool kcontig) {
+  int which;
+  if (epi == EPI_SWIGLU) return make_plan(M, N, 128, 256, 64, kCostMidN, true);
+  return kcontig ? make_plan(M, N, 256, 256, 128, kCostMidN, true) : best_plan(M, N, which);
+}
+
+// A tile over row-major gate and up weights reads half its width from each: 32 columns, 64 bytes of a row, are too little
+// (1 row x [4096, 14336 x 2] with 64 x 64 tiles 82 us, with 128 columns 43 us).
+constexpr int kGatedMinBn = 128;
+
+// Up to 64 rows the size of one part is returned even where the best plan has no parts: callers take a size of zero
+// to mean "not a few-row shape".
+static int64_t plan_workspace_bytes(int M, int K, int ncols, int unit, int min_bn) {
+  const RingPlan plan = ring_plan(M, K, ncols, unit, min_bn, INT64_MAX);
+  return plan.tile < 0 || (plan.ksplit == 1 && M > 64) ? 0 : (int64_t)plan.ksplit * M * ncols * 4;
+}
+
+int64_t gemm_workspace_bytes(int M, int K, int ncols) {
+  const int64_t any = plan_workspace_bytes(M, K, ncols, 1, 0), gated = plan_workspace_bytes(M, K, ncols, 1, kGatedMinBn);
+  return any > gated ? any : gated;
+}
+
+static int launch_gemm_big(const GemmArgs& a, hipStream_t stream) {
+  const TilePlan two = make_plan(a.M, a.N, a.epi == EPI_SWIGLU ? 128 : 256, 256, a.epi == EPI_SWIGLU ? 64 : 128, kCostMidN, true);
   if (a.w_kcontig) {
     // K-contiguous weights: the two-shape plan (256 x 256 rounds, then 256 x 128 tiles) on the direct-to-LDS loop
     if (a.K % 32 != 0 || a.K < 32) return -1;  // (refused by the entry points before any launch)
-    const TilePlan two = make_plan(a.M, a.N, a.epi == EPI_SWIGLU ? 128 : 256, 256, a.epi == EPI_SWIGLU ? 64 : 128,
-                                   kCostMidN, true);
     switch (a.epi) {
       case EPI_NONE: return launch_gemm_plan<FastBig, FastMidN, EPI_NONE, true>(a, two, stream);
       case EPI_GELU: return launch_gemm_plan<FastBig, FastMidN, EPI_GELU, true>(a, two, stream);
@@ -440,17 +447,7 @@ int launch_gemm(const GemmArgs& a, hipStream_t stream) {
     }
     return -1;
   }
-  if (a.M <= kSkinnyWideMaxRows) {  // few rows: stream the weights with the split-K kernels when shape and workspace allow
-    const int r = launch_skinny_gemm(a, stream);
-    if (r <= 0) return r;
-  }
-  if (a.M > kSkinnyMaxRows && a.ws != nullptr && a.epi != EPI_SWIGLU) {
-    const int s = plan_large_split(a.M, a.K, a.N);
-    if (s > 1 && a.ws_bytes >= (int64_t)s * a.M * a.N * 4) return launch_gemm_splitk(a, s, stream);
-  }
   const bool fast = (a.K % 32 == 0) && a.K >= 32;
-  const int out_mid = a.epi == EPI_SWIGLU ? 64 : 128;
-  const TilePlan two = make_plan(a.M, a.N, a.epi == EPI_SWIGLU ? 128 : 256, 256, out_mid, kCostMidN, true);
   switch (a.epi) {
     case EPI_NONE:
       return fast ? launch_gemm_fast<EPI_NONE>(a, stream) : launch_gemm_plan<SlowBig, SlowMidN, EPI_NONE>(a, two, stream);
@@ -461,6 +458,17 @@ int launch_gemm(const GemmArgs& a, hipStream_t stream) {
                   : launch_gemm_plan<SlowBig, SlowMidN, EPI_SWIGLU>(a, two, stream);
   }
   return -1;
+}
+
+int launch_gemm(const GemmArgs& a, hipStream_t stream) {
+  if (a.M <= 0 || a.N <= 0) return 0;
+  RingPlan plan;
+  if (ring_wins(plan_us(big_plan(a.M, a.N, a.epi, a.w_kcontig != 0), a.K), a.M, a.K, a.epi == EPI_SWIGLU ? 2 * a.N : a.N, 1,
+                a.epi == EPI_SWIGLU && !a.w_kcontig ? kGatedMinBn : 0, a.ws != nullptr ? a.ws_bytes : 0, plan))
+    return launch_ring_gemm(a, plan, stream);
+  const int rc = launch_gemm_big(a, stream);
+  if (rc != 0 || a.rowstat_out == nullptr) return rc;
+  return launch_rmsnorm(a.out, a.ldo, nullptr, nullptr, 0, a.rowstat_out, a.M, a.N, 0.f, stream);
 }
 
 // Tile plan of the projection: as for the GEMMs, full rounds of 256 x 256 tiles plus a second shape for the
@@ -476,23 +484,14 @@ static int launch_qkv_t(QkvProjArgs a, const TilePlan& p, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-template <int D>
-static int launch_qkv_d(const QkvProjArgs& a, hipStream_t stream) {
-  const int ntot = (a.Hq + 2 * a.Hkv) * D;
-  const bool fast = (a.K % 32 == 0) && a.K >= 32;
-  TilePlan best = make_plan(a.S, ntot, 256, 128, 256, kCostMidM, true);
-  if (a.w_kcontig) {
-    // K-contiguous weights (K % 32 == 0, checked at the boundary): 256 x 256 rounds and / or 128 x 256 tiles, whose
-    // wave tiles are 128 columns - whole heads - so QKNorm needs no other shape
-    if (!fast) return -1;
-    const TilePlan all_mid = make_plan(a.S, ntot, 256, 128, 256, kCostMidM, false);
-    return launch_qkv_t<FastBig, FastMidM, D, true>(a, all_mid.cost < best.cost - 1e-9 ? all_mid : best, stream);
-  }
-  if (!fast) return launch_qkv_t<SlowBig, SlowMidM, D>(a, best, stream);
-  int which = 0;
+// row-major weights; `head`: the wave tile (all columns of the narrow shapes) must hold whole heads of that width
+// (0: any).  which = 2 * shape + (no big segment).
+static TilePlan qkv_plan(int S, int ntot, int head, int& which) {
+  TilePlan best = make_plan(S, ntot, 256, 128, 256, kCostMidM, true);
+  which = 0;
   auto consider = [&](int id, int mid_bm, int out_mid, double c, bool use_big) {
-    if (a.qknorm && out_mid % D != 0) return;  // the wave tile (all columns of the shape) must hold whole heads
-    const TilePlan p = make_plan(a.S, ntot, 256, mid_bm, out_mid, c, use_big);
+    if (head != 0 && out_mid % head != 0) return;
+    const TilePlan p = make_plan(S, ntot, 256, mid_bm, out_mid, c, use_big);
     if (p.cost < best.cost - 1e-9) { best = p; which = id; }
   };
   consider(1, 128, 256, kCostMidM, false);
@@ -502,6 +501,25 @@ static int launch_qkv_d(const QkvProjArgs& a, hipStream_t stream) {
   consider(5, 256, 160, kCostFit160, false);
   consider(6, 256, 192, kCostFit192, true);
   consider(7, 256, 192, kCostFit192, false);
+  return best;
+}
+
+// K-contiguous weights (K % 32 == 0, checked at the boundary): 256 x 256 rounds and / or 128 x 256 tiles, whose wave
+// tiles are 128 columns - whole heads - so QKNorm needs no other shape
+static TilePlan qkv_plan_kcontig(int S, int ntot) {
+  const TilePlan two = make_plan(S, ntot, 256, 128, 256, kCostMidM, true);
+  const TilePlan all_mid = make_plan(S, ntot, 256, 128, 256, kCostMidM, false);
+  return all_mid.cost < two.cost - 1e-9 ? all_mid : two;
+}
+
+template <int D>
+static int launch_qkv_d(const QkvProjArgs& a, hipStream_t stream) {
+  const int ntot = (a.Hq + 2 * a.Hkv) * D;
+  const bool fast = (a.K % 32 == 0) && a.K >= 32;
+  if (a.w_kcontig) return fast ? launch_qkv_t<FastBig, FastMidM, D, true>(a, qkv_plan_kcontig(a.S, ntot), stream) : -1;
+  if (!fast) return launch_qkv_t<SlowBig, SlowMidM, D>(a, make_plan(a.S, ntot, 256, 128, 256, kCostMidM, true), stream);
+  int which;
+  const TilePlan best = qkv_plan(a.S, ntot, a.qknorm ? D : 0, which);
   switch (which >> 1) {
     case 0: return launch_qkv_t<FastBig, FastMidM, D>(a, best, stream);
     case 1: return launch_qkv_t<FastBig, Fit96, D>(a, best, stream);
@@ -510,16 +528,21 @@ static int launch_qkv_d(const QkvProjArgs& a, hipStream_t stream) {
   }
 }
 
+int64_t qkv_workspace_bytes(int S, int K, int ncols, int unit) { return plan_workspace_bytes(S, K, ncols, unit, 0); }
+
 int launch_qkv_proj(const QkvProjArgs& a, hipStream_t stream, int* deferred_ksplit) {
   if (deferred_ksplit != nullptr) *deferred_ksplit = 0;
   if (a.S <= 0) return 0;
-  if (a.S <= kSkinnyWideMaxRowsQkv && !a.w_kcontig) {  // (the few-row split-K kernels read row-major weights)
-    const int r = launch_skinny_qkv(a, stream, deferred_ksplit);
-    if (r <= 0) return r;
-  }
-  if (a.D == 128) return launch_qkv_d<128>(a, stream);
-  if (a.D == 64) return launch_qkv_d<64>(a, stream);
-  return -1;
+  if (a.D != 64 && a.D != 128) return -1;
+  const int ncols = (a.Hq + 2 * a.Hkv) * a.D;
+  int which;
+  RingPlan plan;
+  const TilePlan big = a.w_kcontig ? qkv_plan_kcontig(a.S, ncols) : qkv_plan(a.S, ncols, a.qknorm ? a.D : 0, which);
+  // (its weights are small enough to come from the Infinity Cache when the caller uses them again: the large tiles
+  // are then a tenth faster than over weights from HBM, the ring kernels hardly - 658 to 1000 rows, both within 2 %)
+  if (ring_wins(0.9f * plan_us(big, a.K), a.S, a.K, ncols, a.qknorm ? a.D : 1, 0, a.ws != nullptr ? a.ws_bytes : 0, plan))
+    return launch_ring_qkv(a, plan, stream, deferred_ksplit);
+  return a.D == 128 ? launch_qkv_d<128>(a, stream) : launch_qkv_d<64>(a, stream);
 }
 
 }  // namespace tri

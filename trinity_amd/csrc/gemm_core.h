@@ -219,9 +219,10 @@ struct DmaTile {
   static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
 };
 
+template <bool NT = false>  // NT: non-temporal
 __device__ __forceinline__ void load_to_lds16(const half_t* g, half_t* l) {
   __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)g,
-                                   (__attribute__((address_space(3))) void*)l, 16, 0, 0);
+                                   (__attribute__((address_space(3))) void*)l, 16, 0, NT ? 2 : 0);
 }
 
 // s_waitcnt vmcnt(n) leaving the other counters unconstrained (gfx9 encoding)

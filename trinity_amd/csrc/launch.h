@@ -67,7 +67,7 @@ struct GemmArgs {
   const half_t* w2;
   int64_t ldw2;
   // weights stored K-contiguous (W^T [N][K]): ldw / ldw2 are then the strides between weight columns.  Needs
-  // K % 32 == 0; takes the large-tile kernels whatever M (the few-row and split-K paths read row-major weights).
+  // K % 32 == 0.
   int w_kcontig;
   const float* rowscale;   // nullable, [M]
   const half_t* residual;  // nullable
@@ -77,38 +77,29 @@ struct GemmArgs {
   int M, N, K;
   int epi;
   int n_big, big_cols;  // tile plan (filled in by launch_gemm): workgroups and columns covered by big tiles
-  float* ws;            // nullable: fp32 workspace for the split-K path taken when M <= kSkinnyMaxRows
+  float* ws;            // nullable: fp32 workspace for plans that cut K into parts (gemm_workspace_bytes)
   int64_t ws_bytes;
-  // Few-row path only (set when skinny_gemm_applies(args)): the merge kernel computes the row scale itself,
-  // rowscale[m] = rsqrt(mean(rownorm_src[m, 0..rownorm_n)^2)), and also stores it to rownorm_out[m] - the
-  // RMSNorm statistic of the FFN block without a kernel of its own.
-  const half_t* rownorm_src;
-  int64_t rownorm_ld;
-  int rownorm_n;
-  float* rownorm_out;
+  // nullable: also leave rsqrt(mean(out[m, :]^2)) - the RMSNorm statistic of the finished rows - in rowstat_out[m]
+  // (plain epilogue only)
+  float* rowstat_out;
 };
 int launch_gemm(const GemmArgs& a, hipStream_t stream);
 
-// Few-row GEMMs (M <= kSkinnyMaxRows) are bound by streaming the weights once from HBM.  They run as a
-// split-K kernel (many workgroups, each a [k range] x [128 columns] slab, fp32 partial sums into the
-// workspace) followed by a finalize kernel that adds the partials and applies the epilogue.
-constexpr int kSkinnyMaxRows = 64;
-// ... and more rows when the weights are small enough to stay in the 256 MB Infinity Cache while the workgroups of
-// the different 64-row blocks stream them (each block reads every slab again): up to 128 rows for plain products
-// (beyond that the large tiles' split-K plan is ahead: 4544 x 4544 at 256 rows 34.5 against 45.9 us), up to 256 for
-// the Q/K/V projection, which has no such plan (Llama-3-8B heads, 50 MB of weights: 128 rows 59.3 -> 35.9 us, 256
-// rows 65.3 -> 54.3 us; with 100 MB of weights the gain is gone at 256 rows, hence the limit on the bytes)
-constexpr int kSkinnyWideMaxRows = 128, kSkinnyWideMaxRowsQkv = 256;
-constexpr int64_t kSkinnyWideMaxBytes = (int64_t)64 << 20;
-// bytes of workspace that guarantee the split-K path for an [M, K] x [K, ncols] product (ncols counts gate and
-// up columns separately for SwiGLU); 0 when the shape never takes that path
-int64_t skinny_workspace_bytes(int M, int K, int ncols, bool qkv = false);  // qkv: the Q/K/V projection's row limit
-int launch_skinny_gemm(const GemmArgs& a, hipStream_t stream);
-bool skinny_gemm_applies(const GemmArgs& a);  // launch_gemm(a) will take the few-row path
-// Many rows, but a tile count that fills the chip badly and a deep K: split-K over half-size tiles with the
-// same workspace and finalize kernels (plain and GELU epilogues).  0 bytes = never taken for this shape.
-int64_t large_split_workspace_bytes(int M, int K, int N);
-int launch_gemm_splitk(const GemmArgs& a, int s, hipStream_t stream);  // s parts per 256 x 128 tile
+// Few and middling rows (ring.hip): which tile of its family, and in how many parts of K, an [M, K] x [K, ncols]
+// product runs, and what it should take (us, with the merge of its parts).  tile < 0: not for these kernels.
+struct RingPlan {
+  int tile, ksplit;
+  float us;
+};
+constexpr int kRingMaxRows = 1100;  // beyond this the large tiles fill the chip (and the cost model was not fitted)
+// ncols: weight columns (gate and up, or q, k and v, together).  Tiles must be a multiple of `unit` wide (whole heads; 1
+// otherwise) and at least min_bn.  ws_bytes: fp32 workspace for partial results, ksplit * M * ncols * 4 bytes (1: none).
+RingPlan ring_plan(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes);
+int launch_ring_gemm(const GemmArgs& a, const RingPlan& plan, hipStream_t stream);
+// workspace that lets launch_gemm take its best plan for [M, K] x [K, ncols] (0: no plan in parts)
+int64_t gemm_workspace_bytes(int M, int K, int ncols);
+// the same for the Q/K/V projection; unit as in ring_plan
+int64_t qkv_workspace_bytes(int S, int K, int ncols, int unit);
 
 // [Q | K | V] = X . [Wq | Wk | Wv], optional per-head RMSNorm of Q and K,
 // scattered to q [S, Hq*D] and the head-major k/v buffers.
@@ -124,15 +115,15 @@ struct QkvProjArgs {
   int S, K, Hq, Hkv, D, P;
   int qknorm;
   float eps;
-  float* ws;  // nullable: split-K workspace (see skinny_workspace_bytes), used when S <= kSkinnyMaxRows
+  float* ws;  // nullable: fp32 workspace for plans that cut K into parts (qkv_workspace_bytes)
   int64_t ws_bytes;
   int n_big, big_cols;  // tile plan (filled in by launch_qkv_proj)
   int w_kcontig;        // the three weight matrices are K-contiguous (ldwq / ldwk / ldwv: strides between columns)
 };
-// deferred_ksplit (nullable): when given and the few-row path runs, its merge kernel is left out - q, k and v stay
-// fp32 partial results ws [ksplit][S][(Hq + 2 Hkv) * D] for the attention kernel to merge - and the number of
-// splits is stored there; 0 is stored when the projection finished the job itself.
-int launch_skinny_qkv(const QkvProjArgs& a, hipStream_t stream, int* deferred_ksplit = nullptr);
+// deferred_ksplit (nullable): when given and the projection runs in parts, its merge kernel is left out - q, k and v
+// stay fp32 partial results ws [ksplit][S][(Hq + 2 Hkv) * D] for the attention kernel to merge - and the number of
+// parts is stored there; 0 is stored when the projection finished the job itself.
+int launch_ring_qkv(const QkvProjArgs& a, const RingPlan& plan, hipStream_t stream, int* deferred_ksplit);
 int launch_qkv_proj(const QkvProjArgs& a, hipStream_t stream, int* deferred_ksplit = nullptr);
 
 struct AttnArgs {

@@ -1,0 +1,271 @@
+// Main loop and tile family of the GEMMs with few and middling rows (1 to about 1000 tokens), shared by ring.hip
+// (FFN products) and ring_qkv.hip (Q/K/V projection).
+//
+// What bounds them: streaming the weights once.  To keep 5 TB/s coming from HBM a CU needs some 60 KB of weights in
+// flight at any time, whatever else it does, so the LDS is one ring of NST stages, each holding a 64-deep k tile of
+// both operands, and a stage is requested again as soon as the barrier has freed it: NST - 1 tiles are always on
+// their way.  (The large-tile loop of gemm_core.h keeps its activations in two buffers and loads complete in order,
+// so its weights are never more than about one tile ahead: 64 rows x [4096, 28672] 59 us there and in the split-K
+// kernel, 44 us here = 5.3 TB/s; 128 rows 64 -> 51 us.)
+//
+// 64-deep k tiles: an activation row, and a K-contiguous weight column, is then read in whole 128-byte lines.
+// Both operands go global -> LDS without passing through registers (1 KB per wave instruction), XOR-swizzled by the
+// choice of the chunk each lane fetches:
+//   activations [BM][64], K-contiguous weights [BN][64]: chunk c (8 per row) of row r at slot c ^ ((r >> 1) & 7)
+//   row-major weights [64][BN]: chunk c of row k at slot c ^ ((k & 3) << 2), or c ^ (((k >> 1) & 1) << 2) where a
+//   row is not a multiple of 256 bytes - the four rows of a transpose read then fall on different banks.
+// One barrier per k tile, in front of its last k16 step, when the next tile must have landed; the loads of a tile are
+// spread one by one between the MFMAs of the four steps after the barrier that freed their stage.
+#if (defined(TRI_BF16) && !defined(TRI_RING_H_BF16)) || (!defined(TRI_BF16) && !defined(TRI_RING_H_F16))
+#ifdef TRI_BF16
+#define TRI_RING_H_BF16
+#else
+#define TRI_RING_H_F16
+#endif
+#include "gemm_core.h"
+#include "launch.h"
+
+namespace tri {
+
+// NTW: the weights are requested non-temporally (each line is wanted once: a single row block).
+template <int BM_, int BN_, int WM_, int WN_, int NST_, bool NTW_ = false>
+struct RingTile {
+  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, NST = NST_, BK = 64;
+  static constexpr bool NTW = NTW_;
+  static constexpr int NW = WM * WN, NT = NW * 64;
+  static constexpr int TM = BM / WM, TN = BN / WN, MI = TM / 32, NI = TN / 32;
+  static constexpr int X_HALFS = BM * BK, STAGE = (BM + BN) * BK;
+  static constexpr int LDS_BYTES = NST * STAGE * 2;
+  static constexpr int XI = BM / 8 / NW, WI = BN / 8 / NW, L = XI + WI;  // 1 KB load instructions per wave and k tile
+  static constexpr int CPR = BN / 8;                                     // 16-byte chunks per row-major weight row
+  static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0 && TM % 32 == 0 && TN % 32 == 0, "tile split");
+  static_assert(NST >= 3 && LDS_BYTES <= 160 * 1024, "LDS budget");
+  static_assert((NST - 2) * L + L / 4 < 64, "loads in flight fit vmcnt");
+};
+
+// The family (planned by ring_plan below).  Waves are arranged so that every tile has at least one wave per SIMD
+// and an accumulator of at most 160 registers; eight waves where the tile is large enough to share (they hide each
+// other's LDS reads: 128 x 256 at 512 rows 138 -> 136 us, 64 x 128 at 64 rows of [4096, 14336 x 2] 44.7 -> 44.2 us).
+// Non-temporal weights where one block of at most 32 rows sees them: 16 rows x [18176, 4544] in 7 parts 29.6 -> 27.1 us
+// (6.1 TB/s), x [14336, 4096] in 8 parts 22.6 -> 21.2 us; at 64 rows the gain is gone (42.7 -> 43.6, 25.1 -> 23.6 us).
+#define TRI_RING_TILES(X)        \
+  X(0, 32, 128, 1, 4, 4, false)  \
+  X(1, 64, 64, 2, 2, 5, false)   \
+  X(2, 64, 128, 2, 4, 3, false)  \
+  X(3, 96, 128, 1, 4, 5, false)  \
+  X(4, 128, 128, 2, 4, 5, false) \
+  X(5, 128, 192, 2, 2, 4, false) \
+  X(6, 128, 256, 2, 4, 3, false) \
+  X(7, 160, 256, 1, 4, 3, false) \
+  X(8, 32, 128, 1, 4, 4, true)
+constexpr int kRingTiles = 9;
+
+// Workgroup id -> (row block, column tile, split): row blocks fastest, so that the workgroups that stream the same
+// weights for different rows run together, then columns.  With several row blocks, or tiles of 96 rows and more, the
+// round robin of workgroups over the XCDs is undone first: an XCD's L2 then sees the weights once for all its row
+// blocks and one run of the activations (100 rows, K = 18176: 42.5 -> 37.7 us).  A single block of few rows has
+// nothing to share, and neighbouring columns on different XCDs consume whole DRAM pages together (16 rows,
+// K = 4096, 28672 columns: 42.0 -> 40.3 us).
+__device__ __forceinline__ void ring_coords(int pid, int nrb, int ntn, int ksplit, bool chunked, int& rb, int& tn, int& split) {
+  if (chunked) {
+    const int total = nrb * ntn * ksplit, per = total >> 3, rem = total & 7, xcd = pid & 7;
+    pid = xcd * per + (xcd < rem ? xcd : rem) + (pid >> 3);
+  }
+  rb = pid % nrb;
+  pid /= nrb;
+  tn = pid % ntn;
+  split = pid / ntn;
+}
+
+// acc[ni][mi] = W-tile^T x X-tile over k in [0, K) of the given pointers (K % 32 == 0, K >= 64).
+//   wmap(c, ldw): NTL (K-contiguous weights): c = LDS row of the weight tile -> start of that column's k run;
+//   otherwise c = column chunk of the tile -> its first element at k = 0, ldw = distance between k rows.
+// SWAP exchanges the MFMA operands (rows = tokens in the registers, columns across the lanes).
+// K % 64 == 32: the last k tile starts at K - 64 and its first two k16 steps, already done, are left out.
+template <class T, bool NTL, bool SWAP, class WMap>
+__device__ __forceinline__ void gemm_mainloop_ring(const half_t* __restrict__ x, int64_t ldx, int m0, int M, int K,
+                                                   WMap wmap, half_t* lds, float16v (&acc)[T::NI][T::MI]) {
+  constexpr int NW = T::NW, BK = T::BK, BN = T::BN, NST = T::NST, XI = T::XI, WI = T::WI, L = T::L, CPR = T::CPR;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int wm = wave % T::WM, wn = wave / T::WM;
+  const int l32 = lane & 31, g = lane >> 5;
+  const int KT = (K + BK - 1) / BK;
+
+  const half_t* xsrc[XI];
+  const half_t* wsrc[WI];
+  // a lane keeps its column chunk, and with it the distance between k rows, over all instructions - unless a row is not
+  // a divisor of 64 chunks (BN = 192), where a tile across two weight matrices needs the distance per instruction
+  constexpr int NLD = (!NTL && 64 % CPR != 0) ? WI : 1;
+  int64_t ldw[NLD];
+#pragma unroll
+  for (int i = 0; i < XI; ++i) {
+    const int rloc = (i * NW + wave) * 8 + (lane >> 3);
+    int row = m0 + rloc;
+    row = row < M ? row : M - 1;
+    xsrc[i] = x + (int64_t)row * ldx + ((lane & 7) ^ ((rloc >> 1) & 7)) * 8;
+  }
+#pragma unroll
+  for (int i = 0; i < WI; ++i) {
+    if constexpr (NTL) {
+      const int nloc = (i * NW + wave) * 8 + (lane >> 3);
+      wsrc[i] = wmap(nloc, ldw[0]) + ((lane & 7) ^ ((nloc >> 1) & 7)) * 8;
+    } else {
+      const int p = (i * NW + wave) * 64 + lane;
+      const int krow = p / CPR, slot = p % CPR;
+      const int chunk = CPR % 16 == 0 ? slot ^ ((krow & 3) << 2) : slot ^ (((krow >> 1) & 1) << 2);
+      wsrc[i] = wmap(chunk, ldw[i % NLD]) + (int64_t)krow * ldw[i % NLD];
+    }
+  }
+  // first k of tile kt; past the end the loop keeps its load count (the waits assume it): the last tile again
+  auto koff = [&](int kt) { return min(kt * BK, K - BK); };
+  // position of a k tile in both operands, carried from tile to tile (a product per lane and tile would cost as many
+  // instructions as the loads themselves where a tile crosses two weight matrices)
+  struct KPos {
+    int k;
+    int64_t w[NLD];
+  };
+  int64_t wstep[NLD];  // 64 rows on
+#pragma unroll
+  for (int j = 0; j < NLD; ++j) wstep[j] = NTL ? BK : BK * ldw[j];
+  auto advance = [&](KPos& o, int kt) {  // to tile kt, from the tile before
+    const int k = koff(kt), d = k - o.k;  // uniform: 64, then 32 at an odd end, then 0
+    o.k = k;
+    if (d == BK) {
+#pragma unroll
+      for (int j = 0; j < NLD; ++j) o.w[j] += wstep[j];
+    } else if (d != 0) {
+#pragma unroll
+      for (int j = 0; j < NLD; ++j) o.w[j] += wstep[j] / 2;
+    }
+  };
+  auto load_one = [&](const KPos& o, int st, int i) {
+    half_t* b = lds + st * T::STAGE;
+    if (i < XI) load_to_lds16(xsrc[i] + o.k, b + (i * NW + wave) * 512);
+    else load_to_lds16<T::NTW>(wsrc[i - XI] + o.w[(i - XI) % NLD], b + T::X_HALFS + ((i - XI) * NW + wave) * 512);
+  };
+
+  // ---- fragment read offsets (halfs)
+  const int sx = (l32 >> 1) & 7;
+  int xoff[4], woff_t[4], woff_n[T::NI];
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk) {
+    xoff[kk] = (wm * T::TM + l32) * BK + (((kk * 2 + g) ^ sx) << 3);
+    woff_t[kk] = T::X_HALFS + (wn * T::TN + l32) * BK + (((kk * 2 + g) ^ sx) << 3);
+  }
+  const int j4 = (lane & 15) >> 2;
+#pragma unroll
+  for (int ni = 0; ni < T::NI; ++ni) {
+    const int chunk = (wn * T::TN + ni * 32) / 8 + ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1);
+    const int slot = CPR % 16 == 0 ? chunk ^ (j4 << 2) : chunk ^ (((j4 >> 1) & 1) << 2);
+    woff_n[ni] = T::X_HALFS + (g * 8 + j4) * BN + (slot << 3) + (lane & 1) * 4;
+  }
+  half8v wf[2][T::NI], xf[2][T::MI];
+  auto read_one = [&](int st, int kk, int buf, int i) {
+    const half_t* b = lds + st * T::STAGE;
+    if (i < T::NI) {
+      if constexpr (NTL) {
+        wf[buf][i] = lds_read8(b + woff_t[kk] + i * 32 * BK);
+      } else {
+        const half_t* p = b + woff_n[i] + kk * 16 * BN;
+        wf[buf][i] = cat8(lds_read_tr16(p), lds_read_tr16(p + 4 * BN));
+      }
+    } else {
+      xf[buf][i - T::NI] = lds_read8(b + xoff[kk] + (i - T::NI) * 32 * BK);
+    }
+  };
+  constexpr int NM = T::NI * T::MI, NF = T::NI + T::MI;
+  auto mfma_one = [&](int buf, int i) {
+    const int ni = i / T::MI, mq = i % T::MI;
+    const int mi = (ni & 1) ? T::MI - 1 - mq : mq;  // serpentine: consecutive MFMAs share a source operand
+    acc[ni][mi] = SWAP ? mfma32(xf[buf][mi], wf[buf][ni], acc[ni][mi]) : mfma32(wf[buf][ni], xf[buf][mi], acc[ni][mi]);
+  };
+  // one k16 step, slot by slot (a schedule fence after each): MFMA i on set `buf`, its share of the loads [lo, hi) of
+  // the tile at `o` into stage st and of the fragment reads of step rkk of stage rst into the other set (rkk < 0: none)
+  auto step = [&](int buf, const KPos& o, int st, int lo, int hi, int rst, int rkk) {
+    const int n = hi - lo;
+#pragma unroll
+    for (int i = 0; i < NM; ++i) {
+      mfma_one(buf, i);
+#pragma unroll
+      for (int j = lo + i * n / NM; j < lo + (i + 1) * n / NM; ++j) load_one(o, st, j);
+      if (rkk >= 0) {
+#pragma unroll
+        for (int j = i * NF / NM; j < (i + 1) * NF / NM; ++j) read_one(rst, rkk, buf ^ 1, j);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+#pragma unroll
+  for (int ni = 0; ni < T::NI; ++ni)
+#pragma unroll
+    for (int mi = 0; mi < T::MI; ++mi)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[ni][mi][r] = 0.f;
+
+  // a quarter of tile kt + NST's loads is issued in the last step of tile kt, the rest in the first three of kt + 1
+  constexpr int L0 = L / 4, L1 = L / 2, L2 = 3 * L / 4;
+  KPos pos;
+  pos.k = 0;
+#pragma unroll
+  for (int j = 0; j < NLD; ++j) pos.w[j] = 0;
+#pragma unroll
+  for (int s = 0; s < NST - 1; ++s) {
+#pragma unroll
+    for (int i = 0; i < L; ++i) load_one(pos, s, i);
+    advance(pos, s + 1);
+  }
+#pragma unroll
+  for (int i = 0; i < L0; ++i) load_one(pos, NST - 1, i);
+  TRI_WAIT_VMCNT((NST - 2) * L + L0);
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int i = 0; i < NF; ++i) read_one(0, 0, 0, i);
+  int st = 0;
+  for (int kt = 0; kt < KT - 1; ++kt) {
+    const int sn = st == NST - 1 ? 0 : st + 1;
+    const int sp = st == 0 ? NST - 1 : st - 1;  // the stage of tile kt - 1, taken by tile kt + NST - 1
+    __builtin_amdgcn_sched_barrier(0);
+    step(0, pos, sp, L0, L1, st, 1);
+    step(1, pos, sp, L1, L2, st, 2);
+    step(0, pos, sp, L2, L, st, 3);
+    // this wave's reads of tile kt are over and its share of tile kt + 1 has landed; kt + 2 .. kt + NST - 1 in flight
+    constexpr int V = (NST - 2) * L;
+    __builtin_amdgcn_s_waitcnt((V & 15) | ((V >> 4) << 14) | 0x0070);  // vmcnt(V) lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    advance(pos, kt + NST);
+    __builtin_amdgcn_sched_barrier(0);
+    step(1, pos, st, 0, L0, sn, 0);
+    st = sn;
+  }
+  if (K % BK == 0) {
+    step(0, pos, 0, 0, 0, st, 1);
+    step(1, pos, 0, 0, 0, st, 2);
+  } else {
+#pragma unroll
+    for (int i = 0; i < NF; ++i) read_one(st, 2, 0, i);
+  }
+  step(0, pos, 0, 0, 0, st, 3);
+  step(1, pos, 0, 0, 0, st, -1);
+  TRI_WAIT_VMCNT(0);
+}
+
+// k tiles per part of a plan (the last part takes what is left, and the odd 32 of a K that is not a multiple of 64)
+inline int ring_kt_per_part(int K, int ksplit) { return (K / 64 + ksplit - 1) / ksplit; }
+
+struct RingArgs {
+  const half_t* x;
+  int64_t ldx;
+  const half_t* w[3];  // column segments, concatenated logically
+  int64_t ldw[3];      // distance between k rows (row-major) or between columns (K-contiguous)
+  int seg_begin[3];    // first logical column of each segment (unused segments start at ncols)
+  int M, K, ncols, ksplit;
+  float* partial;      // [ksplit][M][ncols]
+};
+// fp32 partial results of the plan's parts
+int launch_ring_partial(const RingArgs& a, int tile, bool kcontig, hipStream_t stream);
+
+}  // namespace tri
+
+#endif  // once per element type

@@ -1,0 +1,369 @@
+// GEMMs with few and middling rows (see ring.h for the main loop and what bounds it): the products of the FFNs and of
+// the FFN block from 1 to about 1000 tokens, and fp32 partial products for the Q/K/V projection.
+//
+//   ring_epi_kernel       one workgroup per tile over the whole of K; row scale, activation, residual, one rounding and
+//                         whole-row stores in its epilogue
+//   ring_partial_kernel   the same tile over a part of K, fp32 partial products [split][row][column] to the workspace
+//   ring_finalize_*       sum over the parts in a fixed order (results do not depend on scheduling) and the epilogue
+//
+// Parts are taken only where whole tiles leave CUs without work: they cost 8 bytes of traffic per output and part
+// and a second launch.  ring_plan chooses tile and parts by cost.
+#include "ring.h"
+
+#include <math.h>
+
+namespace tri {
+
+template <class T, bool WT>
+__global__ __launch_bounds__(T::NT) void ring_partial_kernel(RingArgs a) {
+  extern __shared__ __attribute__((aligned(16))) half_t lds[];
+  const int nrb = (a.M + T::BM - 1) / T::BM, ntn = (a.ncols + T::BN - 1) / T::BN;
+  int rb, tn, split;
+  ring_coords(blockIdx.x, nrb, ntn, a.ksplit, nrb > 1 || T::BM >= 96, rb, tn, split);
+  const int m0 = rb * T::BM, n0 = tn * T::BN;
+  const int per = (a.K / 64 + a.ksplit - 1) / a.ksplit;  // as ring_kt_per_part
+  const int k0 = split * per * 64;
+  const int kr = split == a.ksplit - 1 ? a.K - k0 : per * 64;
+  auto wmap = [&](int c, int64_t& ldw) -> const half_t* {
+    int col = n0 + (WT ? c : c * 8);
+    col = col < a.ncols ? col : 0;
+    const int seg = col >= a.seg_begin[2] ? 2 : (col >= a.seg_begin[1] ? 1 : 0);
+    const int64_t ld = seg == 2 ? a.ldw[2] : (seg == 1 ? a.ldw[1] : a.ldw[0]);
+    const half_t* w = seg == 2 ? a.w[2] : (seg == 1 ? a.w[1] : a.w[0]);
+    col -= seg == 2 ? a.seg_begin[2] : (seg == 1 ? a.seg_begin[1] : a.seg_begin[0]);
+    ldw = ld;
+    return WT ? w + (int64_t)col * ld + k0 : w + col + (int64_t)k0 * ld;
+  };
+  float16v acc[T::NI][T::MI];
+  gemm_mainloop_ring<T, WT, true>(a.x + k0, a.ldx, m0, a.M, kr, wmap, lds, acc);
+
+  // lanes run along the columns: 128 bytes of a row per half wave and store
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wm = wave % T::WM, wn = wave / T::WM;
+  const int l32 = lane & 31, g = lane >> 5;
+  float* base = a.partial + (int64_t)split * a.M * a.ncols;
+#pragma unroll
+  for (int ni = 0; ni < T::NI; ++ni) {
+    const int n = n0 + wn * T::TN + ni * 32 + l32;
+    if (n >= a.ncols) continue;
+#pragma unroll
+    for (int mi = 0; mi < T::MI; ++mi)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int m = m0 + wm * T::TM + mi * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
+        if (m < a.M) base[(int64_t)m * a.ncols + n] = acc[ni][mi][r];
+      }
+  }
+}
+
+// out = act(rowscale * X.W) [+ residual].  EPI_SWIGLU: the left half of a tile's columns are gate columns, the right
+// half the matching up columns, so the two halves of an output sit in different waves: the up halves pass through LDS
+// as fp32 (interleaving gate and up in steps of 16 columns keeps them in one lane, but row-major weights are then read
+// in pieces of 32 bytes: 16 rows x [4096, 14336 x 2] 46.0 -> 47.1 us, 128 rows 56.8 -> 60.7 us).
+template <class T, int EPI, bool WT>
+__global__ __launch_bounds__(T::NT) void ring_epi_kernel(GemmArgs a) {
+  extern __shared__ __attribute__((aligned(16))) half_t lds[];
+  constexpr bool GATED = EPI == EPI_SWIGLU;
+  constexpr int OUT_BN = GATED ? T::BN / 2 : T::BN;
+  const int nrb = (a.M + T::BM - 1) / T::BM, ntn = (a.N + OUT_BN - 1) / OUT_BN;
+  int rb, tn, split;
+  ring_coords(blockIdx.x, nrb, ntn, 1, nrb > 1 || T::BM >= 96, rb, tn, split);
+  const int m0 = rb * T::BM, n0 = tn * OUT_BN;
+  auto wmap = [&](int c, int64_t& ldw) -> const half_t* {
+    const int nloc = WT ? c : c * 8;
+    int col;
+    const half_t* w = a.w;
+    ldw = a.ldw;
+    if (GATED) {
+      col = n0 + nloc % OUT_BN;
+      if (nloc >= OUT_BN) { w = a.w2; ldw = a.ldw2; }
+    } else {
+      col = n0 + nloc;
+    }
+    col = col < a.N ? col : n0;
+    return WT ? w + (int64_t)col * ldw : w + col;
+  };
+  float16v acc[T::NI][T::MI];
+  gemm_mainloop_ring<T, WT, false>(a.x, a.ldx, m0, a.M, a.K, wmap, lds, acc);
+
+  // A lane owns one token and four consecutive columns per register quad: the tile turns around in LDS (free now) and
+  // leaves as rows, 16 bytes per lane.
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wm = wave % T::WM, wn = wave / T::WM;
+  const int l32 = lane & 31, g = lane >> 5;
+  constexpr int RS = OUT_BN + 8;  // halfs per staged row
+  constexpr int US = OUT_BN + 4;  // floats per row of the up half
+  static_assert(T::BM * RS * 2 <= T::LDS_BYTES && (!GATED || (T::BM * US * 4 <= T::LDS_BYTES && T::WN % 2 == 0)), "the staged tile fits the ring");
+  float* up = reinterpret_cast<float*>(lds);
+  const bool up_wave = GATED && wn >= T::WN / 2;
+  __syncthreads();  // every wave is done with the ring (and every load into it has landed)
+  if (up_wave) {
+#pragma unroll
+    for (int mi = 0; mi < T::MI; ++mi)
+#pragma unroll
+      for (int ni = 0; ni < T::NI; ++ni)
+#pragma unroll
+        for (int rq = 0; rq < 4; ++rq) {
+          const float4v v = {acc[ni][mi][rq * 4], acc[ni][mi][rq * 4 + 1], acc[ni][mi][rq * 4 + 2], acc[ni][mi][rq * 4 + 3]};
+          *reinterpret_cast<float4v*>(up + (wm * T::TM + mi * 32 + l32) * US + (wn - T::WN / 2) * T::TN + ni * 32 + rq * 8 + g * 4) = v;
+        }
+  }
+  if (GATED) __syncthreads();
+  if (!up_wave) {
+#pragma unroll
+    for (int mi = 0; mi < T::MI; ++mi) {
+      const int mloc = wm * T::TM + mi * 32 + l32, m = m0 + mloc;
+      const bool mok = m < a.M;
+      const float rs = (a.rowscale != nullptr && mok) ? a.rowscale[m] : 1.0f;
+#pragma unroll
+      for (int ni = 0; ni < T::NI; ++ni)
+#pragma unroll
+        for (int rq = 0; rq < 4; ++rq) {
+          const int nloc = wn * T::TN + ni * 32 + rq * 8 + g * 4, n = n0 + nloc;
+          float4v u = {0.f, 0.f, 0.f, 0.f};
+          if (GATED) u = *reinterpret_cast<const float4v*>(up + mloc * US + nloc);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            float c = acc[ni][mi][rq * 4 + e] * rs;
+            if (EPI == EPI_GELU) c = gelu_erf(c);
+            if (GATED) c = silu(c) * (u[e] * rs);
+            acc[ni][mi][rq * 4 + e] = c;
+          }
+          if (a.residual != nullptr && mok && n < a.N) {
+            const half4v rr = *reinterpret_cast<const half4v*>(a.residual + (int64_t)m * a.ldr + n);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[ni][mi][rq * 4 + e] += (float)rr[e];
+          }
+        }
+    }
+  }
+  if (GATED) __syncthreads();  // the up half has been read
+  if (!up_wave) {
+#pragma unroll
+    for (int mi = 0; mi < T::MI; ++mi)
+#pragma unroll
+      for (int ni = 0; ni < T::NI; ++ni)
+#pragma unroll
+        for (int rq = 0; rq < 4; ++rq) {
+          const half4v h = {(half_t)acc[ni][mi][rq * 4], (half_t)acc[ni][mi][rq * 4 + 1], (half_t)acc[ni][mi][rq * 4 + 2], (half_t)acc[ni][mi][rq * 4 + 3]};
+          *reinterpret_cast<half4v*>(lds + (wm * T::TM + mi * 32 + l32) * RS + wn * T::TN + ni * 32 + rq * 8 + g * 4) = h;
+        }
+  }
+  __syncthreads();
+  constexpr int CH = OUT_BN / 8;  // 16-byte chunks per staged row
+#pragma unroll 4
+  for (int idx = threadIdx.x; idx < T::BM * CH; idx += T::NT) {
+    const int row = idx / CH, ch = idx % CH;
+    const int m = m0 + row, n = n0 + ch * 8;
+    // (column counts are multiples of eight: a chunk lies wholly inside or wholly outside)
+    if (m < a.M && n < a.N) *reinterpret_cast<half8v*>(a.out + (int64_t)m * a.ldo + n) = *reinterpret_cast<const half8v*>(lds + row * RS + ch * 8);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// merge of the parts
+// ---------------------------------------------------------------------------
+// out[m, n..n+3] for one thread; the arithmetic mirrors the epilogues above
+template <int EPI>
+__device__ __forceinline__ half4v finalize_group(const GemmArgs& a, const float* partial, int ksplit, int m, int n, float rs) {
+  const int ntot = EPI == EPI_SWIGLU ? 2 * a.N : a.N;
+  const int64_t stride = (int64_t)a.M * ntot, off = (int64_t)m * ntot + n;
+  float4v v = sum_splits(partial, ksplit, stride, off);
+  float4v u = {0.f, 0.f, 0.f, 0.f};
+  if (EPI == EPI_SWIGLU) u = sum_splits(partial, ksplit, stride, off + a.N);
+  float o[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float c = v[e] * rs;
+    if (EPI == EPI_GELU) c = gelu_erf(c);
+    if (EPI == EPI_SWIGLU) c = silu(c) * (u[e] * rs);
+    o[e] = c;
+  }
+  if (a.residual != nullptr) {
+    const half4v rr = *reinterpret_cast<const half4v*>(a.residual + (int64_t)m * a.ldr + n);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] += (float)rr[e];
+  }
+  const half4v h = {(half_t)o[0], (half_t)o[1], (half_t)o[2], (half_t)o[3]};
+  *reinterpret_cast<half4v*>(a.out + (int64_t)m * a.ldo + n) = h;
+  return h;
+}
+
+template <int EPI>
+__global__ __launch_bounds__(256) void ring_finalize_kernel(GemmArgs a, const float* partial, int ksplit) {
+  const int groups = a.N / 4;
+  const int idx = blockIdx.x * 256 + threadIdx.x;
+  if (idx >= a.M * groups) return;
+  const int m = idx / groups, n = (idx % groups) * 4;
+  finalize_group<EPI>(a, partial, ksplit, m, n, a.rowscale != nullptr ? a.rowscale[m] : 1.0f);
+}
+
+// Plain epilogue, one workgroup per row: also leaves the RMSNorm statistic of the finished row in rowstat_out[m].
+__global__ __launch_bounds__(1024) void ring_finalize_rowstat_kernel(GemmArgs a, const float* partial, int ksplit) {
+  __shared__ float part[16];
+  const int m = blockIdx.x, t = threadIdx.x;
+  const float rs = a.rowscale != nullptr ? a.rowscale[m] : 1.0f;
+  float ss = 0.f;
+  for (int g = t; g < a.N / 4; g += 1024) {
+    const half4v h = finalize_group<EPI_NONE>(a, partial, ksplit, m, g * 4, rs);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ss = fmaf((float)h[e], (float)h[e], ss);
+  }
+  ss = wave_sum(ss);
+  if ((t & 63) == 0) part[t >> 6] = ss;
+  __syncthreads();
+  if (t == 0) {
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s += part[i];
+    a.rowstat_out[m] = rsqrtf(s / (float)a.N);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// host side
+// ---------------------------------------------------------------------------
+template <class T, bool WT>
+static int launch_partial_t(const RingArgs& a, hipStream_t stream) {
+  constexpr auto kern = ring_partial_kernel<T, WT>;
+  if (set_max_lds<kern, T::LDS_BYTES>() != 0) return -1;
+  const int nrb = (a.M + T::BM - 1) / T::BM, ntn = (a.ncols + T::BN - 1) / T::BN;
+  hipLaunchKernelGGL(kern, dim3(nrb * ntn * a.ksplit), dim3(T::NT), T::LDS_BYTES, stream, a);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+int launch_ring_partial(const RingArgs& a, int tile, bool kcontig, hipStream_t stream) {
+  switch (tile) {
+#define TRI_RING_CASE(id, bm, bn, wm, wn, nst, nt)                                                  \
+  case id:                                                                                      \
+    return kcontig ? launch_partial_t<RingTile<bm, bn, wm, wn, nst, nt>, true>(a, stream) \
+                   : launch_partial_t<RingTile<bm, bn, wm, wn, nst, nt>, false>(a, stream);
+    TRI_RING_TILES(TRI_RING_CASE)
+#undef TRI_RING_CASE
+  }
+  return -1;
+}
+
+template <class T, int EPI, bool WT>
+static int launch_epi_t(const GemmArgs& a, hipStream_t stream) {
+  constexpr auto kern = ring_epi_kernel<T, EPI, WT>;
+  if (set_max_lds<kern, T::LDS_BYTES>() != 0) return -1;
+  constexpr int OUT_BN = EPI == EPI_SWIGLU ? T::BN / 2 : T::BN;
+  const int nrb = (a.M + T::BM - 1) / T::BM, ntn = (a.N + OUT_BN - 1) / OUT_BN;
+  hipLaunchKernelGGL(kern, dim3(nrb * ntn), dim3(T::NT), T::LDS_BYTES, stream, a);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+template <int EPI>
+static int launch_epi(const GemmArgs& a, int tile, hipStream_t stream) {
+  switch (tile) {
+#define TRI_RING_CASE(id, bm, bn, wm, wn, nst, nt)                                                       \
+  case id:                                                                                           \
+    return a.w_kcontig ? launch_epi_t<RingTile<bm, bn, wm, wn, nst, nt>, EPI, true>(a, stream) \
+                       : launch_epi_t<RingTile<bm, bn, wm, wn, nst, nt>, EPI, false>(a, stream);
+    TRI_RING_TILES(TRI_RING_CASE)
+#undef TRI_RING_CASE
+  }
+  return -1;
+}
+
+// Cost of a plan in us, fitted to 4100 timings on the card (the Q/K/V, output, FFN up and FFN down products of
+// Llama-3-8B and Falcon-7B sizes, 16 to 1024 rows, both weight layouts, up to 16 parts): 4 % rms, and the plan it picks
+// is 1.3 % slower on average than the best plan of the family.  Three times add up in part (as a 3/2-norm):
+//   memory    the weights once at 8 TB/s - less when the workgroups do not divide evenly over the CUs and some CUs have
+//             one more to stream - and what is written;
+//   compute   k tiles in a row on the busiest CU, by tile and by whether workgroups share a CU;
+//   loads     every byte that passes from L2 to LDS, at 37 TB/s over the chip;
+// and per wave of workgroups 2 us of first loads and epilogue.  Parts cost a merge: 3.5 us and their bytes at 6 TB/s.
+struct RingCost {
+  int bm, bn, per_cu;   // per_cu: workgroups that fit a CU's LDS
+  float alone, shared;  // us per k tile of a workgroup with a CU to itself / of each of several
+};
+#define TRI_RING_PER_CU(bm, bn, nst) ((160 * 1024) / (((bm) + (bn)) * 128 * (nst)))
+static const RingCost kRingCost[kRingTiles] = {
+    {32, 128, TRI_RING_PER_CU(32, 128, 4), 0.264f, 0.222f},  {64, 64, TRI_RING_PER_CU(64, 64, 5), 0.215f, 0.181f},
+    {64, 128, TRI_RING_PER_CU(64, 128, 3), 0.354f, 0.272f},  {96, 128, TRI_RING_PER_CU(96, 128, 5), 0.429f, 0.431f},
+    {128, 128, TRI_RING_PER_CU(128, 128, 5), 0.480f, 0.490f}, {128, 192, TRI_RING_PER_CU(128, 192, 4), 0.660f, 0.691f},
+    {128, 256, TRI_RING_PER_CU(128, 256, 3), 0.743f, 0.755f}, {160, 256, TRI_RING_PER_CU(160, 256, 3), 0.914f, 1.006f},
+    {32, 128, TRI_RING_PER_CU(32, 128, 4), 0.264f, 0.222f}};
+constexpr int kRingTileOneBlock = 8;  // the non-temporal tile, for a single row block
+
+static RingPlan ring_plan_search(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes) {
+  RingPlan best = {-1, 1, 1e30f};
+  const int KT = K / 64;
+  const float wbytes = 2.0f * (float)K * (float)ncols, obytes = 4.0f * (float)M * (float)ncols;
+  for (int tile = 0; tile < kRingTiles; ++tile) {
+    const RingCost& c = kRingCost[tile];
+    if (c.bn % unit != 0 || c.bn < min_bn) continue;
+    if (tile == kRingTileOneBlock && M > c.bm) continue;
+    if (tile == 0 && M <= c.bm) continue;  // (the non-temporal twin serves these)
+    const int tiles = ((M + c.bm - 1) / c.bm) * ((ncols + c.bn - 1) / c.bn);
+    int last_per = 0;
+    for (int s = 1; s <= 16; ++s) {
+      const int per = ring_kt_per_part(K, s);
+      if (s > 1 && (per < 4 || s * tiles > 1024 || s * (int64_t)obytes > ws_bytes)) break;
+      const int ks = (KT + per - 1) / per;
+      if (per == last_per || ks != s) continue;  // (no more parts than before)
+      last_per = per;
+      const int wg = tiles * ks, share = (wg + 255) / 256;
+      const float even = share == 1 ? 1.0f : sqrtf((float)wg / (256.0f * share));
+      const float mem = wbytes / (8e6f * even) + (ks > 1 ? ks * obytes : 0.5f * obytes) / 3e6f;
+      const float it = share == 1 ? c.alone : (c.alone > c.shared * share ? c.alone : c.shared * share);
+      const float comp = per * it;
+      const float loads = (float)wg * per * (c.bm + c.bn) * 128.0f / 37e6f;
+      const float sum = cbrtf(mem * sqrtf(mem) + comp * sqrtf(comp) + loads * sqrtf(loads));
+      const float us = 1.1f + 1.9f * ((share + c.per_cu - 1) / c.per_cu) + sum * sum +
+                       (ks > 1 ? 3.5f + ks * obytes / 6e6f : 0.f);
+      if (us < best.us) { best.tile = tile; best.ksplit = ks; best.us = us; }
+    }
+  }
+  return best;
+}
+
+// The search is a pure function of its arguments and takes a microsecond or two, as long as a launch; each thread
+// keeps the last few answers.
+RingPlan ring_plan(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes) {
+  if (M < 1 || M > kRingMaxRows || K % 32 != 0 || K < 64 || ncols < 8) return RingPlan{-1, 1, 1e30f};
+  struct Entry { int M, K, ncols, unit, min_bn; int64_t ws_bytes; RingPlan plan; };
+  static thread_local Entry memo[64] = {};
+  Entry& e = memo[((unsigned)M * 31u + (unsigned)K * 17u + (unsigned)ncols * 7u + (unsigned)unit + (unsigned)min_bn / 128u + (unsigned)(ws_bytes >> 8) * 3u) % 64u];
+  if (e.M != M || e.K != K || e.ncols != ncols || e.unit != unit || e.min_bn != min_bn || e.ws_bytes != ws_bytes)
+    e = Entry{M, K, ncols, unit, min_bn, ws_bytes, ring_plan_search(M, K, ncols, unit, min_bn, ws_bytes)};
+  return e.plan;
+}
+
+int launch_ring_gemm(const GemmArgs& a, const RingPlan& plan, hipStream_t stream) {
+  const bool gated = a.epi == EPI_SWIGLU;
+  if (plan.ksplit == 1) {
+    int rc = -1;
+    switch (a.epi) {
+      case EPI_NONE: rc = launch_epi<EPI_NONE>(a, plan.tile, stream); break;
+      case EPI_GELU: rc = launch_epi<EPI_GELU>(a, plan.tile, stream); break;
+      case EPI_SWIGLU: rc = launch_epi<EPI_SWIGLU>(a, plan.tile, stream); break;
+    }
+    if (rc != 0 || a.rowstat_out == nullptr) return rc;
+    return launch_rmsnorm(a.out, a.ldo, nullptr, nullptr, 0, a.rowstat_out, a.M, a.N, 0.f, stream);
+  }
+  RingArgs r = {};
+  r.x = a.x; r.ldx = a.ldx; r.M = a.M; r.K = a.K; r.ncols = gated ? 2 * a.N : a.N; r.ksplit = plan.ksplit; r.partial = a.ws;
+  r.w[0] = a.w; r.ldw[0] = a.ldw; r.seg_begin[0] = 0;
+  r.w[1] = r.w[2] = gated ? a.w2 : a.w;
+  r.ldw[1] = r.ldw[2] = gated ? a.ldw2 : a.ldw;
+  r.seg_begin[1] = gated ? a.N : r.ncols;
+  r.seg_begin[2] = r.ncols;
+  if (launch_ring_partial(r, plan.tile, a.w_kcontig != 0, stream) != 0) return -1;
+  if (a.rowstat_out != nullptr && a.epi == EPI_NONE) {
+    hipLaunchKernelGGL(ring_finalize_rowstat_kernel, dim3(a.M), dim3(1024), 0, stream, a, a.ws, plan.ksplit);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+  }
+  const dim3 grid((a.M * (a.N / 4) + 255) / 256), block(256);
+  switch (a.epi) {
+    case EPI_NONE: hipLaunchKernelGGL(ring_finalize_kernel<EPI_NONE>, grid, block, 0, stream, a, a.ws, plan.ksplit); break;
+    case EPI_GELU: hipLaunchKernelGGL(ring_finalize_kernel<EPI_GELU>, grid, block, 0, stream, a, a.ws, plan.ksplit); break;
+    case EPI_SWIGLU: hipLaunchKernelGGL(ring_finalize_kernel<EPI_SWIGLU>, grid, block, 0, stream, a, a.ws, plan.ksplit); break;
+    default: return -1;
+  }
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+}  // namespace tri
