@@ -334,6 +334,9 @@ static TilePlan make_plan(int M, int N, int out_big, int mid_bm, int out_mid, do
   const int tiles_m = (M + 255) / 256;
   const int ct_big = (N + out_big - 1) / out_big;  // column tiles if everything were big
   const int total_big = tiles_m * ct_big;
+  // everything big, the last round part empty, where the second shape would not end sooner: 512 rows x
+  // [4096, 14336 x 2] is 224 tiles in one round, 114 us, and was two rounds of 448 half tiles, 141 us
+  const int rounds_big = (total_big + kCUs - 1) / kCUs;
   int full_ct = 0;                                 // column tiles that make whole rounds of big tiles
   if (use_big && total_big >= kCUs) {
     full_ct = ((total_big / kCUs) * kCUs) / tiles_m;
@@ -344,6 +347,7 @@ static TilePlan make_plan(int M, int N, int out_big, int mid_bm, int out_mid, do
   const int rest = N - p.big_cols;
   p.n_mid = ((M + mid_bm - 1) / mid_bm) * ((rest + out_mid - 1) / out_mid);
   p.cost = (p.n_big + kCUs - 1) / kCUs + mid_cost * ((p.n_mid + kCUs - 1) / kCUs);
+  if (use_big && rounds_big < p.cost) p = TilePlan{total_big, N, 0, (double)rounds_big};
   return p;
 }
 
