@@ -41,30 +41,38 @@ class AttentionPlan:
         self.scale, self.causal, self.n_kv_heads, self.eps = scale, causal, n_kv_heads, eps
         self.noise_seed, self.as_mean_var = noise_seed, as_mean_var
         self._cache = {}
+        self._last = None
 
     def _params(self, X, WK):
+        """Parameters and scratch size of a call; the last ones are kept, since most callers repeat a shape (filling the
+        structure and asking for the size take 8 us, as long as a kernel of a decode step)."""
         S, N = X.shape
         if self.M is not None and S != self.M:
             raise ValueError("X has %d rows, the plan was built for M = %d" % (S, self.M))
-        D = self.D
-        H = self.H if self.H is not None else N // D
-        Hkv = self.n_kv_heads if self.n_kv_heads is not None else WK.shape[1] // D
-        return ext.attn_params(H, Hkv, D, S, kv_prefix=self.P, scale=self.scale, causal=self.causal,
-                               rms_eps=self.eps, prenorm=self.prenorm, qknorm=self.qknorm, tau=self.tau,
-                               noise_seed=self.noise_seed), S, N, H
+        kv_cols = WK.shape[1]
+        key = (S, N, kv_cols, self.D, self.H, self.n_kv_heads, self.P, self.scale, self.causal, self.eps, self.prenorm,
+               self.qknorm, self.tau, self.noise_seed)
+        last = self._last
+        if last is None or last[0] != key:
+            H = self.H if self.H is not None else N // self.D
+            Hkv = self.n_kv_heads if self.n_kv_heads is not None else kv_cols // self.D
+            p = ext.attn_params(H, Hkv, self.D, S, kv_prefix=self.P, scale=self.scale, causal=self.causal,
+                                rms_eps=self.eps, prenorm=self.prenorm, qknorm=self.qknorm, tau=self.tau,
+                                noise_seed=self.noise_seed)
+            self._last = last = (key, p, ext.qkv_scratch_bytes(p, N), H)
+        return last[1], last[2], S, last[3]
 
-    def _scratch(self, p, N, dev):
-        need = ext.qkv_scratch_bytes(p, N)
+    def _scratch(self, need, X):
         buf = self._cache.get("scratch")
-        if buf is None or buf.numel() < need or buf.device != dev:
-            buf = torch.empty(need, dtype=torch.uint8, device=dev)
+        if buf is None or buf.numel() < need or buf.device != X.device:
+            buf = torch.empty(need, dtype=torch.uint8, device=X.device)
             self._cache["scratch"] = buf
         return buf
 
     def run(self, X, WQ, WK, WV, O2, K_cache=None, V_cache=None, noise=None, C_out=None, C_out1=None, C_out2=None,
             norm_w=None, lse=None):
-        p, S, N, H = self._params(X, WK)
-        scratch = self._scratch(p, N, X.device)
+        p, need, S, H = self._params(X, WK)
+        scratch = self._scratch(need, X)
         L = self.P + S
         if self.variant == "vanilla":
             ext.qkv_attention(X, norm_w, WQ, WK, WV, K_cache, V_cache, scratch, lse, O2, p)

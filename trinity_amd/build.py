@@ -10,6 +10,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libtrinity_amd.so")
+NATIVE = os.path.join(HERE, "_native.so")  # CPython binding of LIB for torch tensors (csrc/bind.cpp)
 KERNEL_SOURCES = ["rmsnorm.hip", "ring.hip", "ring_qkv.hip", "gemm.hip", "attn.hip", "attn_few.hip", "scores.hip", "kvfp8.hip"]
 # every kernel translation unit is compiled twice: for fp16 elements (namespace tri) and, with these defines, for
 # bf16 elements (the same text in namespace tri_bf16); abi.hip dispatches on the element type of a call
@@ -44,6 +45,33 @@ def hipcc():
     return exe
 
 
+def cxx():
+    exe = shutil.which("g++")
+    if exe is None:
+        raise RuntimeError("g++ not found; the Python binding cannot be built")
+    return exe
+
+
+def torch_libs():
+    from torch.utils import cpp_extension
+
+    return ["-L" + p for p in cpp_extension.library_paths()] + ["-ltorch_python", "-ltorch_cpu", "-lc10"]
+
+
+def compile_binding(obj):
+    """csrc/bind.cpp: host code against the torch and Python headers."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    inc = ["-I" + p for p in cpp_extension.include_paths() + [sysconfig.get_paths()["include"]]]
+    cmd = [cxx(), "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI]
+    r = subprocess.run(cmd + inc + ["-c", os.path.join(CSRC, "bind.cpp"), "-o", obj], capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed on bind.cpp:\n%s\n%s" % (r.stdout, r.stderr))
+
+
 def build(verbose=True, jobs=7):
     """Compile every translation unit and link the shared library."""
     from concurrent.futures import ThreadPoolExecutor
@@ -64,7 +92,9 @@ def build(verbose=True, jobs=7):
             sys.stderr.write(err + "\n")
         return obj
 
+    bind_obj = os.path.join(objdir, "bind.o")
     with ThreadPoolExecutor(max_workers=jobs) as ex:
+        binding = ex.submit(compile_binding, bind_obj)
         objs = list(ex.map(compile_one, UNITS))
     cmd = [cc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs
     r = subprocess.run(cmd, capture_output=True, text=True)
@@ -74,8 +104,13 @@ def build(verbose=True, jobs=7):
     import ctypes
 
     ctypes.CDLL(LIB)
+    binding.result()
+    cmd = [cxx(), "-shared", "-o", NATIVE, bind_obj, "-L" + HERE, "-ltrinity_amd", "-Wl,-rpath,$ORIGIN"] + torch_libs()
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("link of the binding failed:\n%s\n%s" % (r.stdout, r.stderr))
     if verbose:
-        print("built", LIB)
+        print("built", LIB, NATIVE)
     return LIB
 
 

@@ -320,13 +320,15 @@ static RingPlan ring_plan_search(int M, int K, int ncols, int unit, int min_bn, 
   return best;
 }
 
-// The search is a pure function of its arguments and takes a microsecond or two, as long as a launch; each thread
-// keeps the last few answers.
+// The search is a pure function of its arguments and takes 5 to 10 us, longer than a launch; each thread keeps the
+// answers it was last given.
 RingPlan ring_plan(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes) {
   if (M < 1 || M > kRingMaxRows || K % 32 != 0 || K < 64 || ncols < 8) return RingPlan{-1, 1, 1e30f};
   struct Entry { int M, K, ncols, unit, min_bn; int64_t ws_bytes; RingPlan plan; };
-  static thread_local Entry memo[64] = {};
-  Entry& e = memo[((unsigned)M * 31u + (unsigned)K * 17u + (unsigned)ncols * 7u + (unsigned)unit + (unsigned)min_bn / 128u + (unsigned)(ws_bytes >> 8) * 3u) % 64u];
+  static thread_local Entry memo[256] = {};
+  uint64_t h = (uint64_t)M;
+  for (const uint64_t v : {(uint64_t)K, (uint64_t)ncols, (uint64_t)unit, (uint64_t)min_bn, (uint64_t)ws_bytes}) h = (h ^ v) * 0x9E3779B97F4A7C15ull;
+  Entry& e = memo[h >> 56];
   if (e.M != M || e.K != K || e.ncols != ncols || e.unit != unit || e.min_bn != min_bn || e.ws_bytes != ws_bytes)
     e = Entry{M, K, ncols, unit, min_bn, ws_bytes, ring_plan_search(M, K, ncols, unit, min_bn, ws_bytes)};
   return e.plan;

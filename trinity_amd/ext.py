@@ -1,9 +1,10 @@
-"""ctypes binding of libtrinity_amd.so for torch tensors.
+"""Binding of libtrinity_amd.so for torch tensors.
 
 PyTorch is used for device memory and streams only: every function below
-marshals `tensor.data_ptr()` / shape / strides into the C structs of
-include/trinity_amd.h and calls the matching `tri_*` entry point on torch's
-current HIP stream.  There is no CPU or eager fallback: a missing library or a
+hands `tensor.data_ptr()` / shape / strides to the matching `tri_*` entry point
+of include/trinity_amd.h on torch's current HIP stream.  Calls that launch work
+go through the compiled binding (csrc/bind.cpp), validation and measurement
+through ctypes.  There is no CPU or eager fallback: a missing library or a
 non-zero status raises.
 """
 import ctypes
@@ -93,6 +94,23 @@ def lib():
     return _lib
 
 
+_native = None
+
+
+def native():
+    """The compiled binding (built in-tree by trinity_amd.build, next to the library)."""
+    global _native
+    if _native is None:
+        lib()
+        try:
+            from . import _native as mod
+        except ImportError as e:
+            raise RuntimeError("the compiled binding cannot be loaded (%s); run `python -m trinity_amd.build` - there is"
+                               " no fallback path" % e) from e
+        _native = mod
+    return _native
+
+
 def as_tri(t):
     """torch tensor (or None) -> TriTensor (or None).  No copies are made."""
     if t is None:
@@ -117,6 +135,16 @@ def _ref(s):
 
 def _stream(t):
     return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+
+
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # (absent in CPU-only builds of torch)
+
+
+def _stream_ptr(t):
+    """torch's current stream on the tensor's GPU as an integer, without a Stream object in between."""
+    if _raw_stream is not None and t.is_cuda:
+        return _raw_stream(t.get_device())
+    return torch.cuda.current_stream(t.device).cuda_stream
 
 
 def _check(fn, status):
@@ -152,10 +180,10 @@ def attn_params(n_q_heads, n_kv_heads, head_dim, seq, kv_prefix=0, scale=None, c
 
 
 def qkv_scratch_bytes(params, n_model=0):
-    n = lib().tri_qkv_scratch_bytes(ctypes.byref(params), ctypes.c_int64(n_model))
+    n = native().qkv_scratch_bytes(params, n_model)
     if n < 0:
-        _check("tri_qkv_scratch_bytes", int(n))
-    return int(n)
+        _check("tri_qkv_scratch_bytes", n)
+    return n
 
 
 # --------------------------------------------------------------------------- entry points
@@ -168,61 +196,76 @@ def prepare():
 
 
 def rmsnorm(x, w, y, eps=0.0, validate_only=False):
-    args = [x, w, y, ctypes.c_float(eps)]
     if validate_only:
-        return _call("tri_validate_rmsnorm", args, True)
-    return _call("tri_rmsnorm", args + [_stream(x)], False)
+        return _call("tri_validate_rmsnorm", [x, w, y, ctypes.c_float(eps)], True)
+    st = native().rmsnorm(x, w, y, eps, _stream_ptr(x))
+    if st:
+        _check("tri_rmsnorm", st)
+    return st
 
 
 def gemm_workspace_bytes(m, k, ncols):
-    """Bytes of split-K workspace for one [m, k] x [k, ncols] product (0: the few-row path is never taken)."""
-    fn = lib().tri_gemm_workspace_bytes
-    fn.restype = ctypes.c_int64
-    return int(fn(ctypes.c_int64(m), ctypes.c_int64(k), ctypes.c_int64(ncols)))
+    """Bytes of workspace that let one [m, k] x [k, ncols] product take its best plan (0: it needs none)."""
+    return native().gemm_workspace_bytes(m, k, ncols)
 
 
 def ffn_workspace_bytes(m, n, f):
-    """Bytes of split-K workspace that serve every product of an FFN on x [m, n] with hidden width f."""
-    fn = lib().tri_ffn_workspace_bytes
-    fn.restype = ctypes.c_int64
-    return int(fn(ctypes.c_int64(m), ctypes.c_int64(n), ctypes.c_int64(f)))
+    """Bytes of workspace that serve every product of an FFN on x [m, n] with hidden width f."""
+    return native().ffn_workspace_bytes(m, n, f)
 
 
 def ffn_swiglu(x, w_gate, w_up, w_down, hidden, out, workspace=None, validate_only=False):
-    args = [x, w_gate, w_up, w_down, hidden, out, workspace]
     if validate_only:
-        return _call("tri_validate_ffn_swiglu", args, True)
-    return _call("tri_ffn_swiglu", args + [_stream(x)], False)
+        return _call("tri_validate_ffn_swiglu", [x, w_gate, w_up, w_down, hidden, out, workspace], True)
+    st = native().ffn_swiglu(x, w_gate, w_up, w_down, hidden, out, workspace, _stream_ptr(x))
+    if st:
+        _check("tri_ffn_swiglu", st)
+    return st
 
 
 def gateup_swiglu(x, w_gate, w_up, row_scale, hidden, workspace=None):
-    return _call("tri_gateup_swiglu", [x, w_gate, w_up, row_scale, hidden, workspace, _stream(x)], False)
+    st = native().gateup_swiglu(x, w_gate, w_up, row_scale, hidden, workspace, _stream_ptr(x))
+    if st:
+        _check("tri_gateup_swiglu", st)
+    return st
 
 
 def matmul(x, w, residual, out, workspace=None):
-    return _call("tri_matmul", [x, w, residual, out, workspace, _stream(x)], False)
+    st = native().matmul(x, w, residual, out, workspace, _stream_ptr(x))
+    if st:
+        _check("tri_matmul", st)
+    return st
 
 
 def ffn_gelu(x, w1, w2, hidden, out, workspace=None, validate_only=False):
-    args = [x, w1, w2, hidden, out, workspace]
     if validate_only:
-        return _call("tri_validate_ffn_gelu", args, True)
-    return _call("tri_ffn_gelu", args + [_stream(x)], False)
+        return _call("tri_validate_ffn_gelu", [x, w1, w2, hidden, out, workspace], True)
+    st = native().ffn_gelu(x, w1, w2, hidden, out, workspace, _stream_ptr(x))
+    if st:
+        _check("tri_ffn_gelu", st)
+    return st
 
 
 def ffn_block(o2, wo, x, wff1a, wff1b, wff2, attn_o2, row_scratch, ff1, ff2, o_ff_norm=None, workspace=None,
               validate_only=False):
-    args = [o2, wo, x, wff1a, wff1b, wff2, attn_o2, row_scratch, ff1, ff2, o_ff_norm, workspace]
     if validate_only:
-        return _call("tri_validate_ffn_block", args, True)
-    return _call("tri_ffn_block", args + [_stream(x)], False)
+        return _call("tri_validate_ffn_block", [o2, wo, x, wff1a, wff1b, wff2, attn_o2, row_scratch, ff1, ff2, o_ff_norm,
+                                                workspace], True)
+    st = native().ffn_block(o2, wo, x, wff1a, wff1b, wff2, attn_o2, row_scratch, ff1, ff2, o_ff_norm, workspace,
+                            _stream_ptr(x))
+    if st:
+        _check("tri_ffn_block", st)
+    return st
 
 
 def qkv_attention(x, norm_w, wq, wk, wv, k_cache, v_cache, scratch, lse, out, params, validate_only=False):
-    args = [x, norm_w, wq, wk, wv, k_cache, v_cache, scratch, lse, out, ctypes.byref(params)]
     if validate_only:
-        return _call("tri_validate_qkv_attention", args, True)
-    return _call("tri_qkv_attention", args + [_stream(x)], False)
+        return _call("tri_validate_qkv_attention", [x, norm_w, wq, wk, wv, k_cache, v_cache, scratch, lse, out,
+                                                    ctypes.byref(params)], True)
+    st = native().qkv_attention(x, norm_w, wq, wk, wv, k_cache, v_cache, scratch, lse, out, params, _stream_ptr(x))
+    if st:
+        _check("tri_qkv_attention", st)
+    return st
 
 
 STATIC_SCRATCH_BYTES = 64 * 1024 * 1024  # TRI_STATIC_SCRATCH_BYTES
@@ -231,25 +274,33 @@ STATIC_SCRATCH_BYTES = 64 * 1024 * 1024  # TRI_STATIC_SCRATCH_BYTES
 def qkv_attention_static(x, norm_w, wq, wk, wv, k_cache, v_cache, lse, out, params, status_only=False):
     """tri_qkv_attention with the library's own per-GPU scratch array (nothing is allocated); with `status_only`
     the status is returned instead of raised."""
-    stream = _stream(x) if x.is_cuda else None  # (host tensors: only to read the status of a call that is refused)
-    args = [x, norm_w, wq, wk, wv, k_cache, v_cache, lse, out, ctypes.byref(params), stream]
-    return _call("tri_qkv_attention_static", args, status_only)
+    stream = _stream_ptr(x) if x.is_cuda else 0  # (host tensors: only to read the status of a call that is refused)
+    st = native().qkv_attention_static(x, norm_w, wq, wk, wv, k_cache, v_cache, lse, out, params, stream)
+    if st and not status_only:
+        _check("tri_qkv_attention_static", st)
+    return st
 
 
 def keyformer(x, norm_w, wq, wk, wv, k_cache, v_cache, scratch, noise, out, score, params, validate_only=False):
-    args = [x, norm_w, wq, wk, wv, k_cache, v_cache, scratch, noise, out, score, ctypes.byref(params)]
     if validate_only:
-        return _call("tri_validate_keyformer", args, True)
-    return _call("tri_keyformer", args + [_stream(x)], False)
+        return _call("tri_validate_keyformer", [x, norm_w, wq, wk, wv, k_cache, v_cache, scratch, noise, out, score,
+                                                ctypes.byref(params)], True)
+    st = native().keyformer(x, norm_w, wq, wk, wv, k_cache, v_cache, scratch, noise, out, score, params, _stream_ptr(x))
+    if st:
+        _check("tri_keyformer", st)
+    return st
 
 
 def roco(x, norm_w, wq, wk, wv, k_cache, v_cache, scratch, out, sum_out, sumsq_out, params, as_mean_var=False,
          validate_only=False):
-    args = [x, norm_w, wq, wk, wv, k_cache, v_cache, scratch, out, sum_out, sumsq_out,
-            ctypes.c_int32(int(bool(as_mean_var))), ctypes.byref(params)]
     if validate_only:
-        return _call("tri_validate_roco", args, True)
-    return _call("tri_roco", args + [_stream(x)], False)
+        return _call("tri_validate_roco", [x, norm_w, wq, wk, wv, k_cache, v_cache, scratch, out, sum_out, sumsq_out,
+                                           ctypes.c_int32(int(bool(as_mean_var))), ctypes.byref(params)], True)
+    st = native().roco(x, norm_w, wq, wk, wv, k_cache, v_cache, scratch, out, sum_out, sumsq_out, int(bool(as_mean_var)),
+                       params, _stream_ptr(x))
+    if st:
+        _check("tri_roco", st)
+    return st
 
 
 def issue_probe(with_mfma, n_valu, n_trans, waves_per_simd, iters=4096, workgroups=256, device="cuda:0"):
