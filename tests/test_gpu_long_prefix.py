@@ -1,0 +1,31 @@
+"""Few and middling tokens against a long cached prefix at the sizes where the split of the key axis and the merge of
+its parts can go wrong, against the CPU oracle.
+
+Tolerance: both sides hold q, k, v and the output in fp16 and sum in fp32; the kernels also round the probabilities to
+fp16.  With values of order one that is a few 2^-11 of the sum of |p v| <= 4 in O2 (2^-7 allowed), and in the
+log-sum-exp the rounding of q and k in a dot product of D terms, 2^-11 * sqrt(D) * scale (2e-3 allowed)."""
+import math
+
+import pytest
+
+import oracle
+from gpu_util import run_qkv
+from util import assert_close, attn_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("S,Hq,Hkv,D,P", [
+    (1, 4, 1, 128, 2047), (1, 4, 1, 128, 2048),   # the last key count with eight parts, and the first with nine
+    (3, 2, 2, 64, 8189), (7, 5, 1, 64, 2400),     # 32 parts; a merge whose last workgroup is part empty
+    (255, 8, 4, 128, 2100), (256, 8, 4, 128, 2100),  # either side of the row count that one-way merging takes
+])
+def test_parts_of_the_key_axis(dev, S, Hq, Hkv, D, P):
+    t = attn_inputs(S, 64, Hq, Hkv, D, P=P, w_std=0.1)
+    scale = 1.0 / math.sqrt(D)
+    want = oracle.qkv_attention(t["x"], t["wq"], t["wk"], t["wv"], n_q_heads=Hq, n_kv_heads=Hkv, head_dim=D,
+                                scale=scale, causal=True, kv_prefix=P, k_cache=t["k_cache"], v_cache=t["v_cache"],
+                                want_lse=True)
+    got = run_qkv(t, dev, Hq=Hq, Hkv=Hkv, D=D, P=P, scale=scale, causal=True, want_lse=True)
+    assert_close(got["O2"], want["O2"], 2.0 ** -7, 2.0 ** -7, "O2")
+    assert_close(got["lse"], want["lse"], 1e-3, 2e-3, "lse")

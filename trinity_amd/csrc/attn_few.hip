@@ -415,13 +415,21 @@ __global__ __launch_bounds__(NW * 64) void attn_few_kernel(AttnArgs a) {
   attn_few_body<D, KEYFORMER, FP8, FUSED, NW>(a, lds);
 }
 
-// One thread per (head, query, four output columns): merge the splits.
-template <int D>
+// Merge of the splits: one lane per (head, query, four output columns).  WAYS = 1: a lane merges them all.  WAYS = 4:
+// the four waves of a workgroup take every fourth split of the same lanes' columns and merge through LDS.  What
+// bounds the kernel is the chain of round trips to the other XCDs' partial results, eight splits each, so four ways
+// are the kernel for more than eight splits (16 tokens x 32 heads, 32 splits 7.5 -> 4.6 us; 1 token x 32 heads, 16
+// splits 4.8 -> 3.9) - up to the point where one way fills the chip (33 tokens x 71 heads, 147 workgroups 6.6 -> 5.4 us;
+// 112 x 32 heads, 448 workgroups 7.2 -> 7.6; 200 x 32 heads, 800 workgroups 8.4 -> 10.1).
+constexpr int kCombineGroup = 8;             // splits per round trip
+constexpr int kCombineFullWorkgroups = 256;  // one-way workgroups that fill the chip
+template <int D, int WAYS>
 __global__ __launch_bounds__(256) void attn_few_combine_kernel(AttnArgs a, int nsplit) {
   constexpr int LPQ = D / 4;
-  const int idx = blockIdx.x * 256 + threadIdx.x;
-  const int pair = idx / LPQ, d4 = idx % LPQ;
-  if (pair >= a.Hq * a.S) return;
+  const int t = threadIdx.x;
+  const int way = WAYS == 1 ? 0 : t / 64, lane = WAYS == 1 ? t : t % 64;
+  const int idx = blockIdx.x * (256 / WAYS) + lane;
+  const int pair = min(idx / LPQ, a.Hq * a.S - 1), d4 = idx % LPQ;  // (lanes past the end repeat the last row and store nothing)
   const int h = pair / a.S, q = pair % a.S;
   const float* stats = a.ws + (int64_t)a.Hq * nsplit * a.S * D;
   // splits are taken eight at a time with all their loads (statistics and O rows) in flight together (past the
@@ -429,18 +437,18 @@ __global__ __launch_bounds__(256) void attn_few_combine_kernel(AttnArgs a, int n
   // groups of eight, so up to eight splits cost one round trip
   float M = kNegBig, Mp = kNegBig, L = 0.f, Lp = 0.f;
   float4v acc = {0.f, 0.f, 0.f, 0.f};
-  for (int s0 = 0; s0 < nsplit; s0 += 8) {
-    float4v v[8], ov[8];
+  for (int s0 = way; s0 < nsplit; s0 += kCombineGroup * WAYS) {
+    float4v v[kCombineGroup], ov[kCombineGroup];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int s = s0 + j < nsplit ? s0 + j : nsplit - 1;
+    for (int j = 0; j < kCombineGroup; ++j) {
+      const int s = min(s0 + j * WAYS, nsplit - 1);
       const int64_t row = ((int64_t)h * nsplit + s) * a.S + q;
       v[j] = *reinterpret_cast<const float4v*>(stats + row * 4);
       ov[j] = *reinterpret_cast<const float4v*>(a.ws + row * D + d4 * 4);
     }
     float Mn = M, Mpn = Mp;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < kCombineGroup; ++j) {
       Mn = fmaxf(Mn, v[j][0]);
       Mpn = fmaxf(Mpn, v[j][2]);
     }
@@ -452,8 +460,8 @@ __global__ __launch_bounds__(256) void attn_few_combine_kernel(AttnArgs a, int n
     M = Mn;
     Mp = Mpn;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (s0 + j < nsplit) {
+    for (int j = 0; j < kCombineGroup; ++j) {
+      if (s0 + j * WAYS < nsplit) {
         const float w = fast_exp2(v[j][0] - M);
         L = fmaf(v[j][1], w, L);
         Lp = fmaf(v[j][3], fast_exp2(v[j][2] - Mp), Lp);
@@ -462,6 +470,31 @@ __global__ __launch_bounds__(256) void attn_few_combine_kernel(AttnArgs a, int n
       }
     }
   }
+  if (WAYS > 1) {
+    __shared__ float4v part[WAYS > 1 ? 2 * 256 : 1];
+    part[t] = float4v{M, L, Mp, Lp};
+    part[256 + t] = acc;
+    __syncthreads();
+    if (way != 0) return;
+#pragma unroll
+    for (int w = 1; w < WAYS; ++w) {
+      M = fmaxf(M, part[w * 64 + lane][0]);
+      Mp = fmaxf(Mp, part[w * 64 + lane][2]);
+    }
+    L = 0.f;
+    Lp = 0.f;
+    acc = float4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < WAYS; ++w) {
+      const float4v s4 = part[w * 64 + lane], o4 = part[256 + w * 64 + lane];
+      const float sc = fast_exp2(s4[0] - M);
+      L = fmaf(s4[1], sc, L);
+      Lp = fmaf(s4[3], fast_exp2(s4[2] - Mp), Lp);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] = fmaf(o4[e], sc, acc[e]);
+    }
+  }
+  if (idx / LPQ >= a.Hq * a.S) return;
   const float inv = a.out_scale / L;
   half4v hv;
 #pragma unroll
@@ -471,6 +504,16 @@ __global__ __launch_bounds__(256) void attn_few_combine_kernel(AttnArgs a, int n
     if (a.lse != nullptr) a.lse[(int64_t)h * a.S + q] = (M + fast_log2(L)) * kLn2;
     if (a.lse_pert != nullptr) a.lse_pert[(int64_t)h * a.S + q] = (Mp + fast_log2(Lp)) * kLn2;
   }
+}
+
+template <int D>
+static int launch_combine_t(const AttnArgs& a, int nsplit, hipStream_t stream) {
+  const int64_t lanes = (int64_t)a.Hq * a.S * (D / 4);
+  if (nsplit > kCombineGroup && lanes < 256 * kCombineFullWorkgroups)
+    hipLaunchKernelGGL((attn_few_combine_kernel<D, 4>), dim3((unsigned)((lanes + 63) / 64)), dim3(256), 0, stream, a, nsplit);
+  else
+    hipLaunchKernelGGL((attn_few_combine_kernel<D, 1>), dim3((unsigned)((lanes + 255) / 256)), dim3(256), 0, stream, a, nsplit);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 // Per-key accumulators over few queries (RoCo sum p / sum p^2, KeyFormer sum of perturbed probabilities).
@@ -655,16 +698,11 @@ static int launch_few_t(const AttnArgs& a, hipStream_t stream) {
   if (set_max_lds<kern, LDS>() != 0) return -1;
   hipLaunchKernelGGL(kern, dim3(nsplit, a.Hq), dim3(NW * 64), LDS, stream, a);
   if (hipGetLastError() != hipSuccess) return -1;
-  const int threads = a.Hq * a.S * (D / 4);
-  hipLaunchKernelGGL(attn_few_combine_kernel<D>, dim3((threads + 255) / 256), dim3(256), 0, stream, a, nsplit);
-  return hipGetLastError() == hipSuccess ? 0 : -1;
+  return launch_combine_t<D>(a, nsplit, stream);
 }
 
 int launch_attention_few_combine(const AttnArgs& a, int nsplit, hipStream_t stream) {
-  const int threads = a.Hq * a.S * (a.D / 4);
-  if (a.D == 128) hipLaunchKernelGGL(attn_few_combine_kernel<128>, dim3((threads + 255) / 256), dim3(256), 0, stream, a, nsplit);
-  else hipLaunchKernelGGL(attn_few_combine_kernel<64>, dim3((threads + 255) / 256), dim3(256), 0, stream, a, nsplit);
-  return hipGetLastError() == hipSuccess ? 0 : -1;
+  return a.D == 128 ? launch_combine_t<128>(a, nsplit, stream) : launch_combine_t<64>(a, nsplit, stream);
 }
 
 // returns 1 when the shape / workspace does not allow this path (the caller then uses the general kernel)
