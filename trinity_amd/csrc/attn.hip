@@ -83,24 +83,33 @@ __device__ __forceinline__ void attn_wg_map(int id, int Hq, int nqb, int& qb, in
 //
 // SPLIT: few new tokens against a long cached prefix (16-bit caches: every variant; fp8 caches: plain attention).  The query heads that share a KV head
 // are stacked along the query axis - row j of a KV head is (head hk * group + j / S, token j % S) - so K / V are read
-// once per 128 rows instead of once per head, and the key axis is cut into runs of a.split_tiles tiles per
-// workgroup; the unnormalised (O, max, sum) of every run go to the workspace in the layout of the few-query kernel
-// and are merged by its combine kernel.
-// With FP8 (SPLIT only) K and V come from fp8 (e4m3) caches: a tile travels global -> registers while the tile
-// before it is worked on, and is converted to the 16-bit element type on its way into the same swizzled LDS places
-// (exact; the scales ride on a.scale and a.out_scale).
-template <int D, int QT, int KF, int KW, bool SPLIT = false, bool FP8 = false>
+// once per 128 rows instead of once per head, and the tiles of the key axis are dealt out in turn to a.split_runs
+// workgroups (all of them then sweep one region of the cache together: 32 KV heads, 30000 fp8 keys 79 -> 77.5 us against
+// runs of neighbouring tiles); the unnormalised (O, max, sum) of every run go to the workspace in the layout of the
+// few-query kernel and are merged by its combine kernel.  KW = 2 here: pairs of tiles, dealt out as pairs.
+//
+// HALVES = 2 (SPLIT): at most 64 rows, two query groups; the waves of a group take 32 of a tile's 64 keys each and
+// merge as the key ways do.  With a group per wave half the waves or more had no rows at all, and what bounds the
+// kernel there is not HBM but the chain of LDS reads, MFMAs and exponentials of a tile step (64 rows, 32768 fp8 keys,
+// 8 KV heads: 27.8 -> 22.2 us = 3.0 TB/s; two tiles per step for eight waves are level with this).
+//
+// With FP8 (SPLIT only) K and V come from fp8 (e4m3) caches: a tile travels global -> registers while the tile (HALVES:
+// the two tiles) before it is worked on, and is converted to the 16-bit element type on its way into the same swizzled
+// LDS places (exact; the scales ride on a.scale and a.out_scale).
+template <int D, int QT, int KF, int KW, bool SPLIT = false, bool FP8 = false, int HALVES = 1>
 __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, const half_t* __restrict__ qglob) {
   // (qglob = a.q; the qualifier is what keeps the compiler from waiting for the loads in flight before the
   // first LDS transpose read of a tile - see attn_fwd_pipe_body)
-  static_assert(!SPLIT || (QT == 1 && KW == 1), "the split variant is the four-wave kernel");
+  static_assert(!SPLIT || QT == 1, "the split variant: 32 rows per wave");
   static_assert(!FP8 || SPLIT, "fp8 caches are read by the split variant only");
+  static_assert(HALVES == 1 || SPLIT, "half tiles per wave: the split variant only");
   constexpr bool KEYFORMER = KF != 0;
   constexpr bool kf_fast = KF == 2;
   // a wave may meet tiles without a visible key before it has met one (its state is then still -inf / 0)
   constexpr bool GUARD = KW > 1 || SPLIT;
   using L = AttnLds<D>;
-  constexpr int BQ = 4 * 32 * QT;
+  constexpr int BQ = 4 * 32 * QT / HALVES;
+  constexpr int MT = 2 / HALVES;  // blocks of 32 keys a wave takes of a tile
   constexpr int NWAVE = 4 * KW;
   constexpr int KSTEPS = D / 16, DT = D / 32;
   const int t = threadIdx.x, lane = t & 63;
@@ -108,7 +117,9 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, co
   // query group; which of the stage's tiles.  (Eight waves: the two key ways of a query group sit on SIMDs
   // 2 w and 2 w + 1, so that every SIMD holds one of the groups 0, 1 and one of the groups 2, 3 - see FOLD.)
   static_assert(KW == 1 || QT == 1, "eight waves: 32 queries per wave");
-  const int wave = KW == 2 ? wave_all / 2 : wave_all % 4, kway = KW == 2 ? wave_all % 2 : wave_all / 4;
+  const int wave = SPLIT ? wave_all % (4 / HALVES) : (KW == 2 ? wave_all / 2 : wave_all % 4);
+  const int kway = SPLIT ? wave_all / (4 / HALVES) : (KW == 2 ? wave_all % 2 : wave_all / 4);
+  const int ktile = kway / HALVES, khalf = kway % HALVES;  // tile of the stage; block of 32 keys of it (HALVES)
   const int l32 = lane & 31, g = lane >> 5;
   const int group = a.Hq / a.Hkv;
   const int rows = SPLIT ? group * a.S : a.S;  // length of the query axis
@@ -126,7 +137,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, co
   const int Ltot = a.P + a.S;
   int qw0 = qb * BQ + wave * 32 * QT;  // first query of this wave
   int qend = qb * BQ + BQ;              // the workgroup's key range is that of query qend - 1
-  if (KW == 2 && a.causal) {
+  if (!SPLIT && KW == 2 && a.causal) {
     // FOLD: under the causal mask the late query blocks have many key tiles and the early ones few, and this
     // variant runs where there is one workgroup per CU at most - nothing evens that out.  So a workgroup takes
     // two 64-query half blocks that add up to the same work everywhere: groups 0, 1 the half block nhb - 1 - qb
@@ -158,9 +169,9 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, co
   // ---- key range of this workgroup
   const int qlast = min(qend, a.S) - 1;
   const int kend = (a.causal && !SPLIT) ? min(Ltot, a.P + qlast + 1) : Ltot;  // keys [0, kend)
-  const int nkt_all = (kend + kKeyTile - 1) / kKeyTile;
-  const int kt_begin = SPLIT ? split * a.split_tiles : 0;                      // tiles [kt_begin, nkt)
-  const int nkt = SPLIT ? min(nkt_all, kt_begin + a.split_tiles) : nkt_all;
+  const int nkt = (kend + kKeyTile - 1) / kKeyTile;
+  // first tile of a step: the runs take the tiles (pairs of tiles, KW = 2) of the key axis in turn
+  auto step_tile = [&](int step) { return (SPLIT ? split + step * a.split_runs : step) * KW; };
   const int wave_qmax = min(qw0 + 32 * QT, a.S) - 1;  // last real query of this wave (may be < qw0)
 
   // ---- global -> LDS loads of K/V tiles through buffer descriptors: the per-thread byte offset is fixed
@@ -188,7 +199,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, co
     for (int i = 0; i < L::INSTR; ++i) {
       const int ti = (i * NWAVE + wave_all) / kInstrPerTile;         // tile within the stage (wave-uniform)
       const int wi = (i * NWAVE + wave_all) % kInstrPerTile;         // 1 KB slice within the tile
-      const int kt = kt_begin + step * KW + ti;
+      const int kt = step_tile(step) + ti;
       half_t* ks = st + ti * L::STAGE_HALFS;
       half_t* vs = ks + L::K_HALFS;
       // the tile advance goes into the per-lane offset: the scalar offset of a buffer load is not range-checked
@@ -201,33 +212,33 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, co
 
   // ---- fp8 caches: 16-byte pieces (sixteen values: two chunks) of a tile, D / 64 per thread for K and V each
   constexpr int PIECES = D / 64, PPR = D / 16;  // pieces per thread; per row
-  uint4v kraw[PIECES], vraw[PIECES];
-  auto fetch8 = [&](int step) {
-    const int kt = kt_begin + step;
+  struct Raw8 {
+    uint4v k[PIECES], v[PIECES];
+  };
+  Raw8 raw_even, raw_odd;  // (HALVES) tiles of even and of odd steps: two tiles are on their way at any time
+  auto fetch8 = [&](int step, Raw8& raw) {
+    const int kt = step_tile(step);
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
-      const int piece = i * 256 + t;
-      const int key = kt * kKeyTile + piece / PPR, j = piece % PPR;
-      kraw[i] = uint4v{0u, 0u, 0u, 0u};  // fp8 zeros past the last key
-      vraw[i] = uint4v{0u, 0u, 0u, 0u};
-      if (key < Ltot) {
-        kraw[i] = *reinterpret_cast<const uint4v*>(a.k8 + (int64_t)hk * a.k8_sh + (int64_t)key * a.k8_sr + j * 16);
-        vraw[i] = *reinterpret_cast<const uint4v*>(a.v8 + (int64_t)hk * a.v8_sh + (int64_t)key * a.v8_sr + j * 16);
-      }
+      const int piece = i * NWAVE * 64 + t;
+      // (past the last key: the last one again - its scores are masked, and an unconditional load lets the waits count)
+      const int key = min(kt * kKeyTile + piece / PPR, Ltot - 1), j = piece % PPR;
+      raw.k[i] = *reinterpret_cast<const uint4v*>(a.k8 + (int64_t)hk * a.k8_sh + (int64_t)key * a.k8_sr + j * 16);
+      raw.v[i] = *reinterpret_cast<const uint4v*>(a.v8 + (int64_t)hk * a.v8_sh + (int64_t)key * a.v8_sr + j * 16);
     }
   };
-  auto commit8 = [&](int step) {
-    half_t* ks = lds + (step & 1) * L::STAGE_HALFS;
-    half_t* vs = ks + L::K_HALFS;
+  auto commit8 = [&](int step, const Raw8& raw) {
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
-      const int piece = i * 256 + t;
-      const int row = piece / PPR, j = piece % PPR;
+      const int piece = i * NWAVE * 64 + t;
+      const int row = piece / PPR % kKeyTile, j = piece % PPR;
+      half_t* ks = lds + (step & 1) * (KW * L::STAGE_HALFS) + piece / PPR / kKeyTile * L::STAGE_HALFS;
+      half_t* vs = ks + L::K_HALFS;
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
         const int chunk = 2 * j + c;
-        *reinterpret_cast<half8v*>(ks + row * D + ((chunk ^ L::fk(row)) << 3)) = fp8x8_to_half8(uint2v{kraw[i][2 * c], kraw[i][2 * c + 1]});
-        *reinterpret_cast<half8v*>(vs + row * D + ((chunk ^ L::fv(row)) << 3)) = fp8x8_to_half8(uint2v{vraw[i][2 * c], vraw[i][2 * c + 1]});
+        *reinterpret_cast<half8v*>(ks + row * D + ((chunk ^ L::fk(row)) << 3)) = fp8x8_to_half8(uint2v{raw.k[i][2 * c], raw.k[i][2 * c + 1]});
+        *reinterpret_cast<half8v*>(vs + row * D + ((chunk ^ L::fv(row)) << 3)) = fp8x8_to_half8(uint2v{raw.v[i][2 * c], raw.v[i][2 * c + 1]});
       }
     }
   };
@@ -264,40 +275,41 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, co
 
   // One key tile.  The body is inlined once per value of MASK, so that full (unmasked) tiles carry no
   // masking arithmetic at all.
-  auto tile = [&](int kt, const bool MASK) __attribute__((always_inline)) {
+  auto tile = [&](int step, int kt, const bool MASK) __attribute__((always_inline)) {
     // MASK is wave-uniform; the empty asm statements keep the masking code behind real branches (left alone,
     // the compiler turns it into per-element selects that every full tile would pay for)
-    const half_t* ks_ = lds + (((kt - kt_begin) / KW) & 1) * (KW * L::STAGE_HALFS) + kway * L::STAGE_HALFS;
-    const int key0 = kt * kKeyTile;
+    // (HALVES: the wave's block of 32 keys; the swizzles of a row depend on its low five bits only)
+    const half_t* ks_ = lds + (step & 1) * (KW * L::STAGE_HALFS) + ktile * L::STAGE_HALFS + khalf * 32 * D;
+    const int key0 = kt * kKeyTile + khalf * 32;
     // ---- S^T = K . Q^T
-    float16v st[2][QT];
+    float16v st[MT][QT];
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int nt = 0; nt < QT; ++nt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) st[mt][nt][r] = 0.f;
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) {
-      half8v kf[2];
+      half8v kf[MT];
 #pragma unroll
-      for (int mt = 0; mt < 2; ++mt) kf[mt] = lds_read8(ks_ + koff[ks] + mt * 32 * D);
+      for (int mt = 0; mt < MT; ++mt) kf[mt] = lds_read8(ks_ + koff[ks] + mt * 32 * D);
 #pragma unroll
-      for (int mt = 0; mt < 2; ++mt)
+      for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int nt = 0; nt < QT; ++nt) st[mt][nt] = mfma32(kf[mt], qf[nt][ks], st[mt][nt]);
     }
-    half8v pf[QT][2][2];
+    half8v pf[QT][MT][2];
 #pragma unroll
     for (int nt = 0; nt < QT; ++nt) {
       const int qlim = a.causal ? a.P + qtok[nt] : Ltot;  // last visible key
       if (KEYFORMER && !kf_fast) {
         // perturbed logits feed only their own running max / sum
-        float sp[2][16];
+        float sp[MT][16];
         float mx = -INFINITY;
         const int qq = qtok[nt];
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
+        for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
           for (int rq = 0; rq < 4; ++rq) {
             const int key = key0 + mt * 32 + rq * 8 + g * 4;
@@ -325,7 +337,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, co
         const float mref = (GUARD && mnew == -INFINITY) ? 0.f : mnew;
         float sum = 0.f;
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
+        for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
           for (int r = 0; r < 16; ++r) sum += fast_exp2(sp[mt][r] - mref);
         lp_i[nt] = lp_i[nt] * fast_exp2(mp_i[nt] - mref) + sum;
@@ -335,7 +347,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, co
       if (MASK) {
         asm volatile("");
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
+        for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             const int key = key0 + mt * 32 + (r >> 2) * 8 + g * 4 + (r & 3);
@@ -344,7 +356,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, co
       }
       float mx = -INFINITY;
 #pragma unroll
-      for (int mt = 0; mt < 2; ++mt)
+      for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) mx = fmaxf(mx, st[mt][nt][r]);
       mx = pair_max(mx) * c2;  // scale > 0
@@ -360,7 +372,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, co
       const float nm = (GUARD && m_i[nt] == -INFINITY) ? 0.f : -m_i[nt];
       float sum = 0.f, sump = 0.f;
 #pragma unroll
-      for (int mt = 0; mt < 2; ++mt)
+      for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {
           float wgt[8];
@@ -394,7 +406,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, co
     }
     // ---- O^T += V^T . P^T
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh)
 #pragma unroll
@@ -406,36 +418,62 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, co
         }
   };
 
-  const int nsteps = (nkt - kt_begin + KW - 1) / KW;  // (> 0: the launcher starts no workgroup without tiles)
-  if (FP8) fetch8(0);
-  else issue(0);
-  for (int step = 0; step < nsteps; ++step) {
-    if (FP8) {
-      commit8(step);  // (waits for its loads; the stage was last read two steps ago, before the previous barrier)
-      __syncthreads();
-      if (step + 1 < nsteps) fetch8(step + 1);
-    } else {
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's share of the stage has landed
-      __builtin_amdgcn_s_barrier();        // ... and everybody's; the stage before is retired
-      if (step + 1 < nsteps) issue(step + 1);
-    }
-    const int kt = kt_begin + step * KW + kway;
+  // (> 0: the launcher starts no workgroup without tiles)
+  const int nsteps = SPLIT ? ((nkt + KW - 1) / KW - split + a.split_runs - 1) / a.split_runs : (nkt + KW - 1) / KW;
+  auto work = [&](int step) __attribute__((always_inline)) {
+    const int kt = step_tile(step) + ktile;
     const int key0 = kt * kKeyTile;
     // a wave whose queries all precede this tile has nothing to add (nor has one past the last tile); with
     // stacked heads every wave that has rows at all holds every token
-    const bool active = SPLIT ? qw0 < rows
+    const bool active = SPLIT ? qw0 < rows && kt < nkt
                               : (kt < nkt && !(a.causal && key0 > a.P + wave_qmax) && !(KW == 2 && qw0 >= a.S));
     const bool need_mask = (key0 + kKeyTile > Ltot) || (a.causal && key0 + kKeyTile - 1 > a.P + (SPLIT ? 0 : qw0));
-    if (active) tile(kt, need_mask);
+    if (active) tile(step, kt, need_mask);
+  };
+  if (FP8 && HALVES == 1) {
+    fetch8(0, raw_even);
+    for (int step = 0; step < nsteps; ++step) {
+      commit8(step, raw_even);
+      __syncthreads();
+      fetch8(step + 1, raw_even);
+      work(step);
+    }
+  } else if (FP8) {
+    auto step8 = [&](int step, Raw8& raw) __attribute__((always_inline)) {
+      commit8(step, raw);  // (waits for its loads; the stage was last read two steps ago, before the previous barrier)
+      __syncthreads();
+      fetch8(step + 2, raw);
+      work(step);
+    };
+    fetch8(0, raw_even);
+    fetch8(1, raw_odd);
+    // (left from the middle: were the second half skipped instead, the wait at the loop's head would have to assume
+    // that the tile it needs is the one requested last)
+    for (int step = 0;; step += 2) {
+      step8(step, raw_even);
+      if (step + 1 >= nsteps) break;
+      step8(step + 1, raw_odd);
+      if (step + 2 >= nsteps) break;
+    }
+  } else {
+    issue(0);
+    for (int step = 0; step < nsteps; ++step) {
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's share of the stage has landed
+      __builtin_amdgcn_s_barrier();        // ... and everybody's; the stage before is retired
+      if (step + 1 < nsteps) issue(step + 1);
+      work(step);
+    }
   }
 
-  // ---- KW > 1: the waves of the second key way hand their state over through LDS (lane for lane); those of
-  // the first merge it into theirs and go on to the epilogue
-  if (KW > 1) {
+  // ---- several key ways: the waves of the upper half of them hand their state over through LDS (lane for lane) and
+  // leave, those of the lower half merge it into theirs; the last ones go on to the epilogue
+  constexpr int GROUPS = NWAVE / (KW * HALVES);
+#pragma unroll
+  for (int ways = KW * HALVES / 2; ways >= 1; ways /= 2) {
     constexpr int REG = QT * (DT * 16 + 4);  // floats per lane
-    float* mg = reinterpret_cast<float*>(lds) + wave * REG * 64 + lane;
-    __syncthreads();  // every wave is done with the K/V stages
-    if (kway == 1) {
+    float* mg = reinterpret_cast<float*>(lds) + (wave + kway % ways * GROUPS) * REG * 64 + lane;
+    __syncthreads();  // every wave is done with the K/V stages (with the states handed over before)
+    if (kway >= ways && kway < 2 * ways) {
 #pragma unroll
       for (int nt = 0; nt < QT; ++nt) {
         float* r = mg + nt * (DT * 16 + 4) * 64;
@@ -447,7 +485,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, co
       }
     }
     __syncthreads();
-    if (kway == 1) return;
+    if (kway >= ways) continue;
 #pragma unroll
     for (int nt = 0; nt < QT; ++nt) {
       const float* r = mg + nt * (DT * 16 + 4) * 64;
@@ -473,11 +511,12 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, co
         for (int e = 0; e < 16; ++e) o[dt][nt][e] = o[dt][nt][e] * a0 + r[(4 + dt * 16 + e) * 64] * a1;
     }
   }
+  if (KW * HALVES > 1 && kway != 0) return;
 
   if (SPLIT) {
     // ---- this run's unnormalised result: O [Hq][runs][S][D], then (max, sum, perturbed max, perturbed sum)
     // [Hq][runs][S][4]
-    const int nsplit = (nkt_all + a.split_tiles - 1) / a.split_tiles;
+    const int nsplit = a.split_runs;
 #pragma unroll
     for (int nt = 0; nt < QT; ++nt) {
       const float l = pair_sum(l_i[nt]);
@@ -1009,10 +1048,10 @@ __global__ __launch_bounds__(256 * KW * QW) __attribute__((amdgpu_waves_per_eu(2
   else attn_fwd_body<D, QT, KF, KW>(a, lds, a.q);
 }
 
-template <int D, int KF, bool FP8>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_split_kernel(AttnArgs a) {
+template <int D, int KF, bool FP8, int HALVES, int KW>
+__global__ __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_split_kernel(AttnArgs a) {
   extern __shared__ __attribute__((aligned(16))) half_t lds[];
-  attn_fwd_body<D, 1, KF, 1, true, FP8>(a, lds, a.q);
+  attn_fwd_body<D, 1, KF, KW, true, FP8, HALVES>(a, lds, a.q);
 }
 
 template <int D, int QT, int KF, int KW, int QW = 1>
@@ -1036,47 +1075,63 @@ static int launch_attn_kf(const AttnArgs& a, int kf, hipStream_t stream) {
 }
 
 // Few new tokens against a long prefix; returns 1 when the call is not of that kind.
-// Workgroups aimed at (two per CU) and the most runs the key axis is cut into: every run adds a partial result per
-// (head, token) that the merge kernel reads, eight runs per round trip.  16 tokens, 32768 keys: Llama-3-8B's 8 KV
-// heads 57.8 us with 64 runs, 52.8 us with 32; 32 KV heads want the 512 workgroups (134 us; 148 us with 256)
+// Workgroups aimed at (eight waves per CU) and the most runs the key axis is cut into: every run adds a partial result
+// per (head, token) that the merge kernel reads, eight runs per round trip.  16 tokens, 32768 keys: Llama-3-8B's 8 KV
+// heads 55.1 us for the whole block with 64 runs, 51.3 with 32; 32 KV heads want the 512 workgroups (9000 keys 54.0 us,
+// 55.3 with 256).  One or two workgroups per run leave the chip so idle that 64 runs pay (71 heads on one KV head, one
+// token, 30000 fp8 keys 33.4 -> 29.2 us).  A run has at least four tiles, or two where its partial result is small
+// (one token: 2500 keys, 71 heads 21.5 -> 20.2 us, 4096 keys, 32 heads 23.5 -> 23.0; 16 tokens, 4000 keys 26.3 -> 27.0).
 constexpr int kSplitTargetWorkgroups = 512;
-constexpr int kSplitMaxRuns = 32;
-constexpr int kSplitMinTiles = 4;            // key tiles per workgroup, at least
-template <int D, int KF, bool FP8>
-static int launch_attn_split_t(const AttnArgs& a, int nwg, hipStream_t stream) {
-  using L = AttnLds<D>;
-  constexpr auto kern = attn_split_kernel<D, KF, FP8>;
-  if (set_max_lds<kern, L::BYTES>() != 0) return -1;
-  hipLaunchKernelGGL(kern, dim3(nwg), dim3(256), L::BYTES, stream, a);
+constexpr int kSplitMaxRuns = 32, kSplitMaxRunsFew = 64, kSplitFewBase = 2;
+constexpr int kSplitMinTiles = 4, kSplitMinTilesDecode = 2, kSplitDecodeTokens = 4;
+constexpr int kSplitHalvesRows = 64;  // two query groups of 32
+template <int D, int KF, bool FP8, int HALVES, int KW>
+static int launch_attn_split_h(const AttnArgs& a, int nwg, hipStream_t stream) {
+  constexpr int LDS = KW * AttnLds<D>::BYTES;
+  static_assert(KW * 2 * (D / 2 + 4) * 64 * 4 <= LDS, "the merge area fits the K/V stages");
+  constexpr auto kern = attn_split_kernel<D, KF, FP8, HALVES, KW>;
+  if (set_max_lds<kern, LDS>() != 0) return -1;
+  hipLaunchKernelGGL(kern, dim3(nwg), dim3(256 * KW), LDS, stream, a);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-// Key tiles per workgroup and number of runs for a call, 0 = the call is not of this kind: at least kSplitMinKeys
+template <int D, int KF, bool FP8>
+static int launch_attn_split_t(const AttnArgs& a, int nwg, hipStream_t stream) {
+  // chunks: eight waves on two tiles at a time, half the runs and with them half the partial results (300 tokens against
+  // 6000 keys 83.8 -> 77.7 us for the whole block, 48 against 6000 39.6 -> 35.7, 100 x 71 heads against 9000 51 -> 46)
+  if constexpr (!FP8)
+    if (a.S > kFewMaxQueries) return launch_attn_split_h<D, KF, FP8, 1, 2>(a, nwg, stream);
+  return (a.Hq / a.Hkv) * a.S <= kSplitHalvesRows ? launch_attn_split_h<D, KF, FP8, 2, 1>(a, nwg, stream)
+                                                  : launch_attn_split_h<D, KF, FP8, 1, 1>(a, nwg, stream);
+}
+
+// Number of runs for a call; false: the call is not of this kind, which takes at least kSplitMinKeys
 // keys and either few new tokens or so few that the prefill kernel would start at most kSplitMaxPrefillWorkgroups
 // workgroups, each walking the whole key axis alone (chunks of a long prompt, speculative tokens).
 // (Llama-3-8B heads: 64 tokens against 4096 keys 81.5 -> 41.8 us for the whole block, 128 against 8192 166 -> 87 us,
 // 512 against 32768 506 -> 364 us; 512 against 2048 level)
 constexpr int kSplitMaxPrefillWorkgroups = 128;
-static int split_plan(int S, int Hq, int Hkv, int Ltot, int* nsplit) {
+static bool split_plan(int S, int Hq, int Hkv, int Ltot, int* nsplit) {
   *nsplit = 0;
-  if (S < 1 || Ltot < kSplitMinKeys) return 0;
+  if (S < 1 || Ltot < kSplitMinKeys) return false;
   const bool few = S <= kFewMaxQueries;
-  if (!few && (int64_t)((S + 127) / 128) * Hq > kSplitMaxPrefillWorkgroups) return 0;
+  if (!few && (int64_t)((S + 127) / 128) * Hq > kSplitMaxPrefillWorkgroups) return false;
   const int rows = (Hq / Hkv) * S;
   const int base = ((rows + 127) / 128) * Hkv;  // workgroups per run of keys
   const int nkt = (Ltot + kKeyTile - 1) / kKeyTile;
-  int runs = kSplitTargetWorkgroups / base;
-  runs = runs < 1 ? 1 : (runs > kSplitMaxRuns ? kSplitMaxRuns : runs);
-  if (!few && runs < 2) return 0;
-  int tiles = (nkt + runs - 1) / runs;
-  tiles = tiles < kSplitMinTiles ? kSplitMinTiles : tiles;
-  *nsplit = (nkt + tiles - 1) / tiles;
-  return tiles;
+  const int max_runs = base <= kSplitFewBase ? kSplitMaxRunsFew : kSplitMaxRuns;
+  int runs = (few ? kSplitTargetWorkgroups : kSplitTargetWorkgroups / 2) / base;
+  runs = runs < 1 ? 1 : (runs > max_runs ? max_runs : runs);
+  if (!few && runs < 2) return false;
+  const int min_tiles = S <= kSplitDecodeTokens ? kSplitMinTilesDecode : kSplitMinTiles;
+  const int most = (nkt + min_tiles - 1) / min_tiles;
+  *nsplit = runs < most ? runs : most;
+  return true;
 }
 
 int64_t split_attn_workspace_bytes(int S, int Hq, int Hkv, int D, int Ltot) {
   int nsplit;
-  if ((D != 64 && D != 128) || Hkv < 1 || split_plan(S, Hq, Hkv, Ltot, &nsplit) == 0) return 0;
+  if ((D != 64 && D != 128) || Hkv < 1 || !split_plan(S, Hq, Hkv, Ltot, &nsplit)) return 0;
   return (int64_t)Hq * nsplit * S * (D + 4) * 4;
 }
 
@@ -1086,12 +1141,11 @@ static int launch_attn_split(const AttnArgs& a, hipStream_t stream) {
   if (a.pj != nullptr || a.ws == nullptr || (a.D != 64 && a.D != 128) || (a.k8 != nullptr && (a.v8 == nullptr || kf != 0)))
     return 1;
   int nsplit;
-  const int tiles = split_plan(a.S, a.Hq, a.Hkv, Ltot, &nsplit);
-  if (tiles == 0) return 1;
+  if (!split_plan(a.S, a.Hq, a.Hkv, Ltot, &nsplit)) return 1;
   const int base = (((a.Hq / a.Hkv) * a.S + 127) / 128) * a.Hkv;
   if (a.ws_bytes < (int64_t)a.Hq * nsplit * a.S * (a.D + 4) * 4) return 1;
   AttnArgs b = a;
-  b.split_tiles = tiles;
+  b.split_runs = nsplit;
   const int nwg = nsplit * base;
   int rc;
   if (a.D == 128) {

@@ -150,7 +150,7 @@ struct AttnArgs {
   // the S new rows of k / v are not read from memory but summed from the projection's partial results
   // pj [pj_ksplit][S][pj_ntot] (columns [q heads | k heads | v heads]), rounded, RMS-normalised per head when
   // qknorm (q and k), and stored to q_w and to rows [P, P+S) of k_w / v_w (the buffers k / v point to) on the way.
-  int split_tiles;  // set by launch_attention for its long-prefix variant: key tiles (64 keys) per workgroup
+  int split_runs;  // set by launch_attention for its long-prefix variant: runs the key tiles are dealt out to
   const float* pj;
   int pj_ksplit, pj_ntot, qknorm;
   float eps;
