@@ -223,8 +223,9 @@ int tri_validate_qkv_attention(const tri_tensor* x, const tri_tensor* norm_w, co
  * graph capture, tight serving loops, harnesses that forbid hipMalloc.  No counterpart in the reference (its
  * callers allocate every buffer, convert_eval_rms.py:141-176).  Same arguments and results as tri_qkv_attention
  * without `scratch`: the library keeps that memory itself, TRI_STATIC_SCRATCH_BYTES of device memory per GPU,
- * held from the moment the library is loaded on that GPU until the process ends.  A call whose
- * tri_qkv_scratch_bytes exceeds it returns TRI_ERR_SCRATCH and launches nothing (64 MiB hold e.g. the Llama-3-8B
+ * held from the moment the library is loaded on that GPU until the process ends.  Where
+ * tri_qkv_scratch_bytes exceeds it, the workspaces among that memory (which only let faster plans run) shrink; a call
+ * that does not fit even so returns TRI_ERR_SCRATCH and launches nothing (64 MiB hold e.g. the Llama-3-8B
  * block up to 4096 new tokens and every reference-shaped call).  The call allocates nothing; its first use on a
  * device looks the array's address up (tri_prepare does the same ahead of time).  All calls on one GPU share
  * the one array: calls that may overlap in time (different streams, different threads) race - serialise them. */

@@ -138,3 +138,29 @@ def test_static_scratch_refuses_what_does_not_fit(dev):
     assert ext.qkv_attention_static(x, None, w, wkv, wkv, None, None, None, out, p, status_only=True) == -7
     torch.cuda.synchronize()
     assert (out == 7).all()
+
+
+@pytest.mark.parametrize("S,Hq,Hkv,D,P,fp8", [
+    (700, 32, 8, 128, 4000, True),   # room for part of the projection's partial sums
+    (3, 32, 32, 128, 4000, True),    # ... and for the fewest runs of the key-split attention only
+])
+def test_static_scratch_holds_calls_without_full_workspaces(dev, S, Hq, Hkv, D, P, fp8):
+    """Calls whose whole scratch layout exceeds the array still run, on smaller workspaces: against the same call with
+    caller-provided scratch.  The two differ in the order of fp32 sums; a new row's fp8 code may then land one step away,
+    2^-3 of one of thousands of values (2^-7 allowed)."""
+    N = 4096
+    g = torch.Generator().manual_seed(5)
+    rn = lambda *shape, std=1.0: (torch.randn(*shape, generator=g) * std).half().to(dev)
+    x, wq, wk, wv = rn(S, N), rn(N, Hq * D, std=0.02), rn(N, Hkv * D, std=0.02), rn(N, Hkv * D, std=0.02)
+    kc, vc = rn(Hkv, P + S, D), rn(Hkv, P + S, D)
+    if fp8:
+        kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
+    p = ext.attn_params(Hq, Hkv, D, S, kv_prefix=P, causal=True, prenorm=S > 64, qknorm=S > 64, kv_fp8=fp8, k_scale=1.0,
+                        v_scale=1.0)
+    assert ext.qkv_scratch_bytes(p, N) > ext.STATIC_SCRATCH_BYTES
+    want, got = (torch.zeros(S, Hq * D, dtype=torch.float16, device=dev) for _ in range(2))
+    scratch = torch.empty(ext.qkv_scratch_bytes(p, N), dtype=torch.uint8, device=dev)
+    ext.qkv_attention(x, None, wq, wk, wv, kc.clone(), vc.clone(), scratch, None, want, p)
+    ext.qkv_attention_static(x, None, wq, wk, wv, kc, vc, None, got, p)
+    torch.cuda.synchronize()
+    assert (got.float() - want.float()).abs().max().item() <= 2.0 ** -7 * max(1.0, want.float().abs().max().item())

@@ -69,7 +69,10 @@ struct Scratch {
 
 inline int64_t align256(int64_t x) { return (x + 255) & ~(int64_t)255; }
 
-Scratch scratch_layout(const tri_attn_params* p, int64_t n_model) {
+// Layout in at most `budget` bytes.  The two workspaces (partial sums of the projection, partial results of the
+// key-split attention) only let faster plans run: where the whole layout does not fit, the second shrinks to the size
+// that every plan accepts and the first to what is left.  The total may exceed the budget all the same.
+Scratch scratch_layout(const tri_attn_params* p, int64_t n_model, int64_t budget = INT64_MAX) {
   Scratch s{};
   const int64_t S = p->seq, Hq = p->n_q_heads, Hkv = p->n_kv_heads, D = p->head_dim;
   int64_t off = 0;
@@ -82,15 +85,22 @@ Scratch scratch_layout(const tri_attn_params* p, int64_t n_model) {
   // few or middling tokens: room for the partial sums of the projection and for the partial results of the
   // key-split attention (separate: the attention kernel merges the former while it writes the latter)
   s.ws_bytes = qkv_workspace_bytes((int)S, (int)n_model, (int)((Hq + 2 * Hkv) * D), p->qknorm ? (int)D : 1);
-  s.ws_off = off; off = align256(off + s.ws_bytes);
-  s.aws_bytes = few_attn_workspace_bytes((int)S, (int)Hq, (int)D, (int)(p->kv_prefix + S));
-  {
-    const int64_t split = split_attn_workspace_bytes((int)S, (int)Hq, (int)Hkv, (int)D, (int)(p->kv_prefix + S));
-    s.aws_bytes = s.aws_bytes > split ? s.aws_bytes : split;
-  }
-  s.aws_off = off; off = align256(off + s.aws_bytes);
+  const int64_t few = few_attn_workspace_bytes((int)S, (int)Hq, (int)D, (int)(p->kv_prefix + S));
+  auto attn_bytes = [&](bool least) {
+    const int64_t split = split_attn_workspace_bytes((int)S, (int)Hq, (int)Hkv, (int)D, (int)(p->kv_prefix + S), least);
+    return few > split ? few : split;
+  };
+  s.aws_bytes = attn_bytes(false);
   // fp8 caches: 16-bit copies of all P + S rows for the kernels that read 16-bit K / V tiles
   const int64_t copy = p->kv_fp8 ? Hkv * ((int64_t)p->kv_prefix + S) * D * 2 : 0;
+  const int64_t rest = off + 2 * align256(copy);
+  if (rest + align256(s.ws_bytes) + align256(s.aws_bytes) > budget) {
+    s.aws_bytes = attn_bytes(true);
+    const int64_t left = (budget - rest - align256(s.aws_bytes)) & ~(int64_t)255;
+    s.ws_bytes = left <= 0 ? 0 : (s.ws_bytes < left ? s.ws_bytes : left);
+  }
+  s.ws_off = off; off = align256(off + s.ws_bytes);
+  s.aws_off = off; off = align256(off + s.aws_bytes);
   s.kd_off = off; off = align256(off + copy);
   s.vd_off = off; off = align256(off + copy);
   s.total = off;
@@ -462,12 +472,13 @@ int tri_qkv_attention_static(const tri_tensor* x, const tri_tensor* norm_w, cons
   // the size first: a call that does not fit the array is refused before anything else is looked at
   const int64_t need = tri_qkv_scratch_bytes(p, x->shape[1]);
   if (need < 0) return (int)need;
-  if (need > kStaticScratchBytes) return TRI_ERR_SCRATCH;
+  if (need > kStaticScratchBytes && scratch_layout(p, x->shape[1], kStaticScratchBytes).total > kStaticScratchBytes)
+    return TRI_ERR_SCRATCH;
   // every other argument is checked against a stand-in for the array (right size and alignment, never
   // dereferenced), so that a bad call fails without touching the GPU
   tri_tensor scratch{};
   scratch.ptr = reinterpret_cast<void*>(static_cast<uintptr_t>(256));
-  scratch.shape[0] = kStaticScratchBytes;
+  scratch.shape[0] = need > kStaticScratchBytes ? need : kStaticScratchBytes;
   scratch.stride[0] = 1;
   scratch.ndim = 1;
   scratch.dtype = TRI_U8;
@@ -475,6 +486,7 @@ int tri_qkv_attention_static(const tri_tensor* x, const tri_tensor* norm_w, cons
   unsigned char* ptr = nullptr;
   TRI_TRY(static_scratch_ptr(&ptr));
   scratch.ptr = ptr;
+  scratch.shape[0] = kStaticScratchBytes;
   return TRI_DISPATCH(x, impl_qkv_attention(x, norm_w, wq, wk, wv, k_cache, v_cache, &scratch, lse, out, p, hip_stream));
 }
 

@@ -1111,8 +1111,8 @@ static int launch_attn_split_t(const AttnArgs& a, int nwg, hipStream_t stream) {
 // (Llama-3-8B heads: 64 tokens against 4096 keys 81.5 -> 41.8 us for the whole block, 128 against 8192 166 -> 87 us,
 // 512 against 32768 506 -> 364 us; 512 against 2048 level)
 constexpr int kSplitMaxPrefillWorkgroups = 128;
-static bool split_plan(int S, int Hq, int Hkv, int Ltot, int* nsplit) {
-  *nsplit = 0;
+static bool split_plan(int S, int Hq, int Hkv, int Ltot, int* nsplit, int* least) {
+  *nsplit = *least = 0;
   if (S < 1 || Ltot < kSplitMinKeys) return false;
   const bool few = S <= kFewMaxQueries;
   if (!few && (int64_t)((S + 127) / 128) * Hq > kSplitMaxPrefillWorkgroups) return false;
@@ -1126,13 +1126,17 @@ static bool split_plan(int S, int Hq, int Hkv, int Ltot, int* nsplit) {
   const int min_tiles = S <= kSplitDecodeTokens ? kSplitMinTilesDecode : kSplitMinTiles;
   const int most = (nkt + min_tiles - 1) / min_tiles;
   *nsplit = runs < most ? runs : most;
+  // the fewest runs: of at least four tiles, all of one length, at most 32
+  const int cap = runs < kSplitMaxRuns ? runs : kSplitMaxRuns;
+  const int tiles = (nkt + cap - 1) / cap < kSplitMinTiles ? kSplitMinTiles : (nkt + cap - 1) / cap;
+  *least = (nkt + tiles - 1) / tiles;
   return true;
 }
 
-int64_t split_attn_workspace_bytes(int S, int Hq, int Hkv, int D, int Ltot) {
-  int nsplit;
-  if ((D != 64 && D != 128) || Hkv < 1 || !split_plan(S, Hq, Hkv, Ltot, &nsplit)) return 0;
-  return (int64_t)Hq * nsplit * S * (D + 4) * 4;
+int64_t split_attn_workspace_bytes(int S, int Hq, int Hkv, int D, int Ltot, bool least) {
+  int nsplit, fewest;
+  if ((D != 64 && D != 128) || Hkv < 1 || !split_plan(S, Hq, Hkv, Ltot, &nsplit, &fewest)) return 0;
+  return (int64_t)Hq * (least ? fewest : nsplit) * S * (D + 4) * 4;
 }
 
 static int launch_attn_split(const AttnArgs& a, hipStream_t stream) {
@@ -1140,10 +1144,12 @@ static int launch_attn_split(const AttnArgs& a, hipStream_t stream) {
   const int kf = a.lse_pert == nullptr ? 0 : ((a.noise == nullptr && a.tau == 1.0f) ? 2 : 1);
   if (a.pj != nullptr || a.ws == nullptr || (a.D != 64 && a.D != 128) || (a.k8 != nullptr && (a.v8 == nullptr || kf != 0)))
     return 1;
-  int nsplit;
-  if (!split_plan(a.S, a.Hq, a.Hkv, Ltot, &nsplit)) return 1;
+  int nsplit, fewest;
+  if (!split_plan(a.S, a.Hq, a.Hkv, Ltot, &nsplit, &fewest)) return 1;
   const int base = (((a.Hq / a.Hkv) * a.S + 127) / 128) * a.Hkv;
-  if (a.ws_bytes < (int64_t)a.Hq * nsplit * a.S * (a.D + 4) * 4) return 1;
+  const int64_t run_bytes = (int64_t)a.Hq * a.S * (a.D + 4) * 4;
+  if (a.ws_bytes < fewest * run_bytes) return 1;
+  if (a.ws_bytes < nsplit * run_bytes) nsplit = (int)(a.ws_bytes / run_bytes);
   AttnArgs b = a;
   b.split_runs = nsplit;
   const int nwg = nsplit * base;
