@@ -71,6 +71,17 @@ __device__ __forceinline__ half8v fp8x8_to_half8(uint2v w) {
   return h;
 }
 
+// four values / scale to OCP fp8 (e4m3): round to nearest even, saturating at +-448
+__device__ __forceinline__ uint32_t half4_to_fp8x4(half4v x, float scale) {
+  float f[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) f[e] = fminf(fmaxf((float)x[e] / scale, -448.0f), 448.0f);
+  int w = 0;
+  w = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], w, false);
+  w = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], w, true);
+  return (uint32_t)w;
+}
+
 // LDS transpose read: a 16-lane block reads a [4 rows][16 columns] patch of
 // 16-bit elements, lane j of the block addressing row j/4, columns 4*(j%4)..+3;
 // lane j receives column j of the patch, rows 0..3.

@@ -534,8 +534,9 @@ static int launch_qkv_d(const QkvProjArgs& a, hipStream_t stream) {
 
 int64_t qkv_workspace_bytes(int S, int K, int ncols, int unit) { return plan_workspace_bytes(S, K, ncols, unit, 0); }
 
-int launch_qkv_proj(const QkvProjArgs& a, hipStream_t stream, int* deferred_ksplit) {
+int launch_qkv_proj(const QkvProjArgs& a, hipStream_t stream, int* deferred_ksplit, bool* appended) {
   if (deferred_ksplit != nullptr) *deferred_ksplit = 0;
+  if (appended != nullptr) *appended = false;
   if (a.S <= 0) return 0;
   if (a.D != 64 && a.D != 128) return -1;
   const int ncols = (a.Hq + 2 * a.Hkv) * a.D;
@@ -545,7 +546,7 @@ int launch_qkv_proj(const QkvProjArgs& a, hipStream_t stream, int* deferred_kspl
   // (its weights are small enough to come from the Infinity Cache when the caller uses them again: the large tiles
   // are then a tenth faster than over weights from HBM, the ring kernels hardly - 658 to 1000 rows, both within 2 %)
   if (ring_wins(0.9f * plan_us(big, a.K), a.S, a.K, ncols, a.qknorm ? a.D : 1, 0, a.ws != nullptr ? a.ws_bytes : 0, plan))
-    return launch_ring_qkv(a, plan, stream, deferred_ksplit);
+    return launch_ring_qkv(a, plan, stream, deferred_ksplit, appended);
   return a.D == 128 ? launch_qkv_d<128>(a, stream) : launch_qkv_d<64>(a, stream);
 }
 

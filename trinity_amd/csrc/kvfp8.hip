@@ -2,7 +2,8 @@
 //
 //   kv_quant_append_kernel   rows [P, P+S) of the caches = fp8(new k / k_scale), fp8(new v / v_scale), read from
 //                            the fp16 rows the projection has just written (round to nearest even, saturating
-//                            at +-448)
+//                            at +-448); a projection that runs in parts appends the rows in the merge of its parts
+//                            instead (ring_qkv.hip: 16 tokens against 32752 keys 41.2 -> 39.2 us for the whole block)
 //   kv_dequant_kernel        rows [0, rows) of the caches as 16-bit elements WITHOUT the scale (every e4m3 value
 //                            is exact in fp16 and bf16): the attention kernels fold k_scale into the softmax
 //                            scale and v_scale into the final normalisation, so nothing is rounded twice
@@ -26,18 +27,8 @@ __global__ __launch_bounds__(256) void kv_quant_append_kernel(KvQuantArgs a) {
                      : a.kc + (int64_t)hk * a.kc_sh + (int64_t)(a.P + m) * a.kc_sr;
   const float scale = isv ? a.v_scale : a.k_scale;
   const half8v x = *reinterpret_cast<const half8v*>(src + c * 8);
-  float f[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) f[e] = fminf(fmaxf((float)x[e] / scale, -448.0f), 448.0f);
-  uint2v out;
-  int w = 0;
-  w = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], w, false);
-  w = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], w, true);
-  out[0] = (uint32_t)w;
-  w = 0;
-  w = __builtin_amdgcn_cvt_pk_fp8_f32(f[4], f[5], w, false);
-  w = __builtin_amdgcn_cvt_pk_fp8_f32(f[6], f[7], w, true);
-  out[1] = (uint32_t)w;
+  const half4v lo = {x[0], x[1], x[2], x[3]}, hi = {x[4], x[5], x[6], x[7]};
+  const uint2v out = {half4_to_fp8x4(lo, scale), half4_to_fp8x4(hi, scale)};
   *reinterpret_cast<uint2v*>(dst + c * 8) = out;
 }
 

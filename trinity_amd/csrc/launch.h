@@ -119,12 +119,19 @@ struct QkvProjArgs {
   int64_t ws_bytes;
   int n_big, big_cols;  // tile plan (filled in by launch_qkv_proj)
   int w_kcontig;        // the three weight matrices are K-contiguous (ldwq / ldwk / ldwv: strides between columns)
+  // nullable: fp8 caches that the merge of partial results appends the new k / v rows to (rows [append_row,
+  // append_row + S)) in place of k / v, as launch_kv_quant_append would from there
+  uint8_t *k8, *v8;
+  int64_t k8_sh, k8_sr, v8_sh, v8_sr;
+  int append_row;
+  float k_scale, v_scale;
 };
 // deferred_ksplit (nullable): when given and the projection runs in parts, its merge kernel is left out - q, k and v
 // stay fp32 partial results ws [ksplit][S][(Hq + 2 Hkv) * D] for the attention kernel to merge - and the number of
 // parts is stored there; 0 is stored when the projection finished the job itself.
-int launch_ring_qkv(const QkvProjArgs& a, const RingPlan& plan, hipStream_t stream, int* deferred_ksplit);
-int launch_qkv_proj(const QkvProjArgs& a, hipStream_t stream, int* deferred_ksplit = nullptr);
+// appended (nullable): whether the new rows went to k8 / v8 instead of k / v.
+int launch_ring_qkv(const QkvProjArgs& a, const RingPlan& plan, hipStream_t stream, int* deferred_ksplit, bool* appended);
+int launch_qkv_proj(const QkvProjArgs& a, hipStream_t stream, int* deferred_ksplit = nullptr, bool* appended = nullptr);
 
 struct AttnArgs {
   const half_t* q;  // [S, Hq*D]

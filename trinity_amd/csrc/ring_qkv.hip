@@ -78,7 +78,7 @@ __global__ __launch_bounds__(T::NT) void ring_qkv_kernel(QkvProjArgs a) {
 }
 
 // Merge of partial products: one group of D/4 consecutive lanes per (row, head): sum the parts, round, optionally
-// RMS-normalise the head (q and k only), scatter to q / the cache rows.
+// RMS-normalise the head (q and k only), scatter to q / the cache rows (rows of an fp8 cache: converted on the way).
 template <int D>
 __global__ __launch_bounds__(256) void ring_finalize_qkv_kernel(QkvProjArgs a, const float* partial, int ksplit) {
   constexpr int LPH = D / 4;  // lanes per head
@@ -108,7 +108,14 @@ __global__ __launch_bounds__(256) void ring_finalize_qkv_kernel(QkvProjArgs a, c
       for (int e = 0; e < 4; ++e) h[e] = (half_t)((float)h[e] * nrm);
     }
   }
-  if (live) *reinterpret_cast<half4v*>(dst + li * 4) = h;
+  if (!live) return;
+  if (a.k8 != nullptr && seg != 0) {
+    uint8_t* d8 = seg == 1 ? a.k8 + (int64_t)((col0 - nq) / D) * a.k8_sh + (int64_t)(a.append_row + m) * a.k8_sr
+                           : a.v8 + (int64_t)((col0 - nq - nkv) / D) * a.v8_sh + (int64_t)(a.append_row + m) * a.v8_sr;
+    *reinterpret_cast<uint32_t*>(d8 + li * 4) = half4_to_fp8x4(h, seg == 1 ? a.k_scale : a.v_scale);
+  } else {
+    *reinterpret_cast<half4v*>(dst + li * 4) = h;
+  }
 }
 
 template <class T, int D, bool WT>
@@ -133,7 +140,7 @@ static int launch_qkv_tile(const QkvProjArgs& a, int tile, hipStream_t stream) {
   return -1;
 }
 
-int launch_ring_qkv(const QkvProjArgs& a, const RingPlan& plan, hipStream_t stream, int* deferred_ksplit) {
+int launch_ring_qkv(const QkvProjArgs& a, const RingPlan& plan, hipStream_t stream, int* deferred_ksplit, bool* appended) {
   if (plan.ksplit == 1)
     return a.D == 128 ? launch_qkv_tile<128>(a, plan.tile, stream) : launch_qkv_tile<64>(a, plan.tile, stream);
   const int nq = a.Hq * a.D, nkv = a.Hkv * a.D;
@@ -147,6 +154,7 @@ int launch_ring_qkv(const QkvProjArgs& a, const RingPlan& plan, hipStream_t stre
     *deferred_ksplit = plan.ksplit;
     return 0;
   }
+  if (appended != nullptr) *appended = a.k8 != nullptr;
   const int threads = a.S * (a.Hq + 2 * a.Hkv) * (a.D / 4);
   const dim3 grid((threads + 255) / 256), block(256);
   if (a.D == 128) hipLaunchKernelGGL(ring_finalize_qkv_kernel<128>, grid, block, 0, stream, a, a.ws, plan.ksplit);
