@@ -1167,14 +1167,15 @@ static int launch_attn_split(const AttnArgs& a, hipStream_t stream) {
   return launch_attention_few_combine(b, nsplit, stream);
 }
 
-int launch_attention(const AttnArgs& a, hipStream_t stream) {
+int launch_attention(const AttnArgs& a, hipStream_t stream, int* merge_parts) {
+  if (merge_parts != nullptr) *merge_parts = 0;
   if (a.S <= 0) return 0;
   {
     const int r = launch_attn_split(a, stream);
     if (r <= 0) return r;
   }
   if (a.S <= kFewMaxQueries) {
-    const int r = launch_attention_few(a, stream);
+    const int r = launch_attention_few(a, stream, merge_parts);
     if (r <= 0) return r;
   }
   if (a.k == nullptr || a.v == nullptr) return -1;  // (fp8 caches are read by the two variants above only)

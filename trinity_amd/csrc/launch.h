@@ -163,13 +163,15 @@ struct AttnArgs {
   float eps;
   half_t *q_w, *k_w, *v_w;
 };
-int launch_attention(const AttnArgs& a, hipStream_t stream);
+// merge_parts (nullable): when given, the few-query kernel may leave its partial results in a.ws for the score kernel to
+// merge (ScoreArgs::part); their number, or 0 when out and the log-sum-exp are finished, is stored there.
+int launch_attention(const AttnArgs& a, hipStream_t stream, int* merge_parts = nullptr);
 
 // With at most kFewMaxQueries queries attention is bound by reading the K/V cache once; it then runs split
 // over the key axis (partial results in the workspace) followed by a merge kernel.
 constexpr int kFewMaxQueries = 32;
 int64_t few_attn_workspace_bytes(int S, int Hq, int D, int Ltot);
-int launch_attention_few(const AttnArgs& a, hipStream_t stream);
+int launch_attention_few(const AttnArgs& a, hipStream_t stream, int* merge_parts = nullptr);
 int launch_attention_few_combine(const AttnArgs& a, int nsplit, hipStream_t stream);  // the merge kernel alone
 // workspace of launch_attention's long-prefix variant for a call (0 when it does not take it): for all the runs it would
 // cut the key axis into, or (least) for the fewest it works with - given less than the former it takes fewer runs
@@ -214,6 +216,13 @@ struct ScoreArgs {
   float scale, tau;
   int causal, mode, mean_var;
   uint64_t seed;
+  // few queries: attention left part_n (at most eight) partial results in `part`, in the few-query kernel's layout; lse
+  // is then not read, and the scores' kernel also writes out = the merged rows * out_scale
+  const float* part;
+  int part_n;
+  half_t* out;
+  int64_t ldo;
+  float out_scale;
 };
 int launch_scores(const ScoreArgs& a, hipStream_t stream);
 int launch_scores_few(const ScoreArgs& a, hipStream_t stream);  // S <= kFewMaxQueries; 1 = not applicable
