@@ -78,6 +78,19 @@ struct Params {
 
 void* stream_of(PyObject* o) { return PyLong_AsVoidPtr(o); }
 
+// Other Python threads run while the library works (a launch may wait for room in a stream's queue, and what that queue
+// waits for may need the interpreter: a host callback in Python, a thread that feeds another stream).
+struct NoGil {
+  PyThreadState* state = PyEval_SaveThread();
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
+template <class F>
+int call(F f) {
+  if (PyErr_Occurred() != nullptr) return 0;
+  const NoGil nogil;
+  return f();
+}
+
 template <class F>
 PyObject* run(F f) {
   try {
@@ -97,7 +110,7 @@ TRI_BIND(rmsnorm) {
     if (!marshal(a, n, 3, 1, t)) return 0;
     const double eps = PyFloat_AsDouble(a[3]);
     void* s = stream_of(a[4]);
-    return PyErr_Occurred() != nullptr ? 0 : tri_rmsnorm(t.p[0], t.p[1], t.p[2], (float)eps, s);
+    return call([&] { return tri_rmsnorm(t.p[0], t.p[1], t.p[2], (float)eps, s); });
   });
 }
 TRI_BIND(ffn_swiglu) {
@@ -105,7 +118,7 @@ TRI_BIND(ffn_swiglu) {
     Tensors t;
     if (!marshal(a, n, 7, 0, t)) return 0;
     void* s = stream_of(a[7]);
-    return PyErr_Occurred() != nullptr ? 0 : tri_ffn_swiglu(t.p[0], t.p[1], t.p[2], t.p[3], t.p[4], t.p[5], t.p[6], s);
+    return call([&] { return tri_ffn_swiglu(t.p[0], t.p[1], t.p[2], t.p[3], t.p[4], t.p[5], t.p[6], s); });
   });
 }
 TRI_BIND(gateup_swiglu) {
@@ -113,7 +126,7 @@ TRI_BIND(gateup_swiglu) {
     Tensors t;
     if (!marshal(a, n, 6, 0, t)) return 0;
     void* s = stream_of(a[6]);
-    return PyErr_Occurred() != nullptr ? 0 : tri_gateup_swiglu(t.p[0], t.p[1], t.p[2], t.p[3], t.p[4], t.p[5], s);
+    return call([&] { return tri_gateup_swiglu(t.p[0], t.p[1], t.p[2], t.p[3], t.p[4], t.p[5], s); });
   });
 }
 TRI_BIND(matmul) {
@@ -121,7 +134,7 @@ TRI_BIND(matmul) {
     Tensors t;
     if (!marshal(a, n, 5, 0, t)) return 0;
     void* s = stream_of(a[5]);
-    return PyErr_Occurred() != nullptr ? 0 : tri_matmul(t.p[0], t.p[1], t.p[2], t.p[3], t.p[4], s);
+    return call([&] { return tri_matmul(t.p[0], t.p[1], t.p[2], t.p[3], t.p[4], s); });
   });
 }
 TRI_BIND(ffn_gelu) {
@@ -129,7 +142,7 @@ TRI_BIND(ffn_gelu) {
     Tensors t;
     if (!marshal(a, n, 6, 0, t)) return 0;
     void* s = stream_of(a[6]);
-    return PyErr_Occurred() != nullptr ? 0 : tri_ffn_gelu(t.p[0], t.p[1], t.p[2], t.p[3], t.p[4], t.p[5], s);
+    return call([&] { return tri_ffn_gelu(t.p[0], t.p[1], t.p[2], t.p[3], t.p[4], t.p[5], s); });
   });
 }
 TRI_BIND(ffn_block) {
@@ -137,8 +150,9 @@ TRI_BIND(ffn_block) {
     Tensors t;
     if (!marshal(a, n, 12, 0, t)) return 0;
     void* s = stream_of(a[12]);
-    return PyErr_Occurred() != nullptr ? 0
-        : tri_ffn_block(t.p[0], t.p[1], t.p[2], t.p[3], t.p[4], t.p[5], t.p[6], t.p[7], t.p[8], t.p[9], t.p[10], t.p[11], s);
+    return call([&] {
+      return tri_ffn_block(t.p[0], t.p[1], t.p[2], t.p[3], t.p[4], t.p[5], t.p[6], t.p[7], t.p[8], t.p[9], t.p[10], t.p[11], s);
+    });
   });
 }
 TRI_BIND(qkv_attention) {
@@ -147,8 +161,9 @@ TRI_BIND(qkv_attention) {
     if (!marshal(a, n, 10, 1, t)) return 0;
     const Params p(a[10]);
     void* s = stream_of(a[11]);
-    return PyErr_Occurred() != nullptr ? 0
-        : tri_qkv_attention(t.p[0], t.p[1], t.p[2], t.p[3], t.p[4], t.p[5], t.p[6], t.p[7], t.p[8], t.p[9], p.p, s);
+    return call([&] {
+      return tri_qkv_attention(t.p[0], t.p[1], t.p[2], t.p[3], t.p[4], t.p[5], t.p[6], t.p[7], t.p[8], t.p[9], p.p, s);
+    });
   });
 }
 TRI_BIND(qkv_attention_static) {
@@ -157,8 +172,9 @@ TRI_BIND(qkv_attention_static) {
     if (!marshal(a, n, 9, 1, t)) return 0;
     const Params p(a[9]);
     void* s = stream_of(a[10]);
-    return PyErr_Occurred() != nullptr ? 0
-        : tri_qkv_attention_static(t.p[0], t.p[1], t.p[2], t.p[3], t.p[4], t.p[5], t.p[6], t.p[7], t.p[8], p.p, s);
+    return call([&] {
+      return tri_qkv_attention_static(t.p[0], t.p[1], t.p[2], t.p[3], t.p[4], t.p[5], t.p[6], t.p[7], t.p[8], p.p, s);
+    });
   });
 }
 TRI_BIND(keyformer) {
@@ -167,8 +183,9 @@ TRI_BIND(keyformer) {
     if (!marshal(a, n, 11, 1, t)) return 0;
     const Params p(a[11]);
     void* s = stream_of(a[12]);
-    return PyErr_Occurred() != nullptr ? 0
-        : tri_keyformer(t.p[0], t.p[1], t.p[2], t.p[3], t.p[4], t.p[5], t.p[6], t.p[7], t.p[8], t.p[9], t.p[10], p.p, s);
+    return call([&] {
+      return tri_keyformer(t.p[0], t.p[1], t.p[2], t.p[3], t.p[4], t.p[5], t.p[6], t.p[7], t.p[8], t.p[9], t.p[10], p.p, s);
+    });
   });
 }
 TRI_BIND(roco) {  // (as_mean_var comes before the parameters, as in the C entry point)
@@ -178,9 +195,10 @@ TRI_BIND(roco) {  // (as_mean_var comes before the parameters, as in the C entry
     const long mean_var = PyLong_AsLong(a[11]);
     const Params p(a[12]);
     void* s = stream_of(a[13]);
-    return PyErr_Occurred() != nullptr ? 0
-        : tri_roco(t.p[0], t.p[1], t.p[2], t.p[3], t.p[4], t.p[5], t.p[6], t.p[7], t.p[8], t.p[9], t.p[10],
-                   (int32_t)mean_var, p.p, s);
+    return call([&] {
+      return tri_roco(t.p[0], t.p[1], t.p[2], t.p[3], t.p[4], t.p[5], t.p[6], t.p[7], t.p[8], t.p[9], t.p[10],
+                      (int32_t)mean_var, p.p, s);
+    });
   });
 }
 #undef TRI_BIND
