@@ -18,6 +18,7 @@ RTOL = ATOL = 1e-2
     (16, 4544, False, 0.0),        # the reference's point (M = 16, Falcon width, no weight, no eps)
     (37, 4544, True, 1e-5),
     (1, 8, True, 1e-5),
+    (5, 2056, True, 1e-5), (5, 3072, False, 1e-5), (5, 3080, True, 1e-5),   # either side of what three waves cover
     (5, 8192, True, 1e-6),
     (3, 10240, True, 1e-5),        # longer than the register-resident path
     (7, 100, False, 1e-5),         # not a multiple of 8

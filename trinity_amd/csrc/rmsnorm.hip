@@ -130,61 +130,72 @@ __global__ __launch_bounds__(256) void rmsnorm_row_kernel(const half_t* __restri
   }
 }
 
-// Few rows (fewer than there are waves on the chip): one 256-thread workgroup per row, the row read once with
-// 16-byte loads (up to 4 chunks per thread: n <= 8192) and kept in registers.  With `b` the row is
-// a[m] + b[m] * bscale[m] (the trailing residual of the Falcon-shaped FFN block,
-// baseline/ffn_ref.py:114-121 in the reference) before it is normalised.
-template <int CH, bool ADD>
-__global__ __launch_bounds__(256) void rmsnorm_block_kernel(const half_t* __restrict__ x, int64_t ldx,
-                                                            const half_t* __restrict__ b, int64_t ldb,
-                                                            const float* __restrict__ bscale,
-                                                            const half_t* __restrict__ w, half_t* __restrict__ y,
-                                                            int64_t ldy, float* __restrict__ rstd_out, int n, float eps) {
-  __shared__ float part[4];
+// Few rows, and rows that a wave cannot hold: one workgroup of NT threads per row, the row read once with 16-byte loads
+// (up to 4 chunks per thread: n <= 8192) and kept in registers.  With `b` the row is a[m] + b[m] * bscale[m] (the
+// trailing residual of the Falcon-shaped FFN block, baseline/ffn_ref.py:114-121 in the reference) before it is
+// normalised.  What bounds it is one trip to memory and back per row, so all its loads, those of the weights among them,
+// are on their way before anything waits (chunks past the end re-read the last one and are zeroed by a select: a branch
+// around a load makes the compiler wait for it).
+template <int CH, int NT, bool ADD, bool HAS_W>
+__global__ __launch_bounds__(NT) void rmsnorm_block_kernel(const half_t* __restrict__ x, int64_t ldx,
+                                                           const half_t* __restrict__ b, int64_t ldb,
+                                                           const float* __restrict__ bscale,
+                                                           const half_t* __restrict__ w, half_t* __restrict__ y,
+                                                           int64_t ldy, float* __restrict__ rstd_out, int n, float eps) {
+  __shared__ float part[NT / 64];
   const int row = blockIdx.x, t = threadIdx.x;
   const int nch = n >> 3;
   const uint4v* xr = reinterpret_cast<const uint4v*>(x + (int64_t)row * ldx);
   const uint4v* br = ADD ? reinterpret_cast<const uint4v*>(b + (int64_t)row * ldb) : nullptr;
   const float bs = ADD ? bscale[row] : 0.f;
+  uint4v xv[CH], bv[CH], wv[CH];
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int i = min(c * NT + t, nch - 1);
+    xv[c] = xr[i];
+    if (ADD) bv[c] = br[i];
+    if (HAS_W) wv[c] = reinterpret_cast<const uint4v*>(w)[i];
+  }
+  __builtin_amdgcn_sched_barrier(0);
   float f[CH][8];
   float ss = 0.f;
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
-    const int i = c * 256 + t;
-    uint4v xv = {0u, 0u, 0u, 0u}, bv = {0u, 0u, 0u, 0u};
-    if (i < nch) {
-      xv = xr[i];
-      if (ADD) bv = br[i];
-    }
-    const half8v xh = __builtin_bit_cast(half8v, xv), bh = __builtin_bit_cast(half8v, bv);
+    const bool live = c * NT + t < nch;
+    const half8v xh = __builtin_bit_cast(half8v, xv[c]);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      f[c][e] = ADD ? (float)xh[e] + (float)bh[e] * bs : (float)xh[e];
+      float v = (float)xh[e];
+      if (ADD) v += (float)__builtin_bit_cast(half8v, bv[c])[e] * bs;
+      f[c][e] = live ? v : 0.f;
       ss = fmaf(f[c][e], f[c][e], ss);
     }
   }
   ss = wave_sum(ss);
   if ((t & 63) == 0) part[t >> 6] = ss;
   __syncthreads();
-  const float r = rsqrtf((part[0] + part[1] + part[2] + part[3]) / (float)n + eps);
-  if (rstd_out != nullptr && t == 0) rstd_out[row] = r;
-  if (y == nullptr) return;
-  uint4v* yr = reinterpret_cast<uint4v*>(y + (int64_t)row * ldy);
+  float sum = part[0];
 #pragma unroll
-  for (int c = 0; c < CH; ++c) {
-    const int i = c * 256 + t;
-    if (i >= nch) continue;
-    half8v o;
-    if (w != nullptr) {
-      const half8v wh = __builtin_bit_cast(half8v, reinterpret_cast<const uint4v*>(w)[i]);
+  for (int i = 1; i < NT / 64; ++i) sum += part[i];
+  const float r = rsqrtf(sum / (float)n + eps);
+  if (y != nullptr) {
+    uint4v* yr = reinterpret_cast<uint4v*>(y + (int64_t)row * ldy);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = (half_t)(f[c][e] * r * (float)wh[e]);
-    } else {
+    for (int c = 0; c < CH; ++c) {
+      const int i = c * NT + t;
+      half8v o;
+      if (HAS_W) {
+        const half8v wh = __builtin_bit_cast(half8v, wv[c]);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = (half_t)(f[c][e] * r);
+        for (int e = 0; e < 8; ++e) o[e] = (half_t)(f[c][e] * r * (float)wh[e]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = (half_t)(f[c][e] * r);
+      }
+      if (i < nch) yr[i] = __builtin_bit_cast(uint4v, o);
     }
-    yr[i] = __builtin_bit_cast(uint4v, o);
   }
+  if (rstd_out != nullptr && t == 0) rstd_out[row] = r;
 }
 
 template <bool ADD>
@@ -192,13 +203,26 @@ static void launch_block_rows(const half_t* x, int64_t ldx, const half_t* b, int
                               const half_t* w, half_t* y, int64_t ldy, float* rstd_out, int rows, int n, float eps,
                               hipStream_t stream) {
   const int ch = (n / 8 + 255) / 256;
-#define TRI_RMSB(C)                                                                                                \
-  hipLaunchKernelGGL((rmsnorm_block_kernel<C, ADD>), dim3(rows), dim3(256), 0, stream, x, ldx, b, ldb, bscale, w, y, ldy, \
-                     rstd_out, n, eps)
-  if (ch <= 1) TRI_RMSB(1);
-  else if (ch <= 2) TRI_RMSB(2);
-  else if (ch <= 3) TRI_RMSB(3);
-  else TRI_RMSB(4);
+#define TRI_RMSB(C, NT, W)                                                                                          \
+  hipLaunchKernelGGL((rmsnorm_block_kernel<C, NT, ADD, W>), dim3(rows), dim3(NT), 0, stream, x, ldx, b, ldb, bscale, w, y, \
+                     ldy, rstd_out, n, eps)
+// three waves where their chunks cover the row as well as four waves' would (n = 4544: 568 of 576 lanes' chunks hold
+// something instead of 568 of 768)
+#define TRI_RMSB_CH(C)                                                       \
+  do {                                                                       \
+    if (C > 1 && n / 8 <= C * 192) {                                         \
+      if (w != nullptr && y != nullptr) TRI_RMSB(C, 192, true);              \
+      else TRI_RMSB(C, 192, false);                                          \
+    } else {                                                                 \
+      if (w != nullptr && y != nullptr) TRI_RMSB(C, 256, true);              \
+      else TRI_RMSB(C, 256, false);                                          \
+    }                                                                        \
+  } while (0)
+  if (ch <= 1) TRI_RMSB_CH(1);
+  else if (ch <= 2) TRI_RMSB_CH(2);
+  else if (ch <= 3) TRI_RMSB_CH(3);
+  else TRI_RMSB_CH(4);
+#undef TRI_RMSB_CH
 #undef TRI_RMSB
 }
 
