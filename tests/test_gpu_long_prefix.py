@@ -36,6 +36,8 @@ def test_parts_of_the_key_axis(dev, S, Hq, Hkv, D, P):
     (16, 8, 2, 128, 2048), (13, 10, 2, 64, 2111),   # 64 rows per KV head, and 65: half tiles per wave end here
     (4, 4, 1, 128, 2050), (5, 4, 1, 128, 2050),     # runs of two tiles, and of four
     (33, 4, 2, 64, 2100), (70, 4, 4, 128, 2241),    # pairs of tiles: an odd last tile, and none
+    (9, 8, 1, 64, 28650), (9, 8, 1, 64, 28740),     # 72 rows, fp8: either side of seven tiles a run, from where pairs
+    (17, 4, 1, 128, 28671),                         # ... with a last tile of 48 keys beside a full one
 ])
 @pytest.mark.parametrize("fp8", [False, True])
 def test_rows_and_tiles_of_a_run(dev, S, Hq, Hkv, D, P, fp8):

@@ -1085,6 +1085,7 @@ constexpr int kSplitTargetWorkgroups = 512;
 constexpr int kSplitMaxRuns = 32, kSplitMaxRunsFew = 64, kSplitFewBase = 2;
 constexpr int kSplitMinTiles = 4, kSplitMinTilesDecode = 2, kSplitDecodeTokens = 4;
 constexpr int kSplitHalvesRows = 64;  // two query groups of 32
+constexpr int kSplitPairWorkgroups = 256, kSplitPairTiles = 7;  // (one workgroup per CU; tiles per run)
 template <int D, int KF, bool FP8, int HALVES, int KW>
 static int launch_attn_split_h(const AttnArgs& a, int nwg, hipStream_t stream) {
   constexpr int LDS = KW * AttnLds<D>::BYTES;
@@ -1101,8 +1102,15 @@ static int launch_attn_split_t(const AttnArgs& a, int nwg, hipStream_t stream) {
   // 6000 keys 83.8 -> 77.7 us for the whole block, 48 against 6000 39.6 -> 35.7, 100 x 71 heads against 9000 51 -> 46)
   if constexpr (!FP8)
     if (a.S > kFewMaxQueries) return launch_attn_split_h<D, KF, FP8, 1, 2>(a, nwg, stream);
-  return (a.Hq / a.Hkv) * a.S <= kSplitHalvesRows ? launch_attn_split_h<D, KF, FP8, 2, 1>(a, nwg, stream)
-                                                  : launch_attn_split_h<D, KF, FP8, 1, 1>(a, nwg, stream);
+  if ((a.Hq / a.Hkv) * a.S <= kSplitHalvesRows) return launch_attn_split_h<D, KF, FP8, 2, 1>(a, nwg, stream);
+  // fp8 with whole tiles per wave keeps one tile on its way: where a CU has one workgroup at most and a long run to walk,
+  // eight waves on pairs of tiles keep two (Llama-3-8B heads, 28 tokens against 32000 keys 48.0 -> 45.1 us for the whole
+  // block; 71 heads on one, one token against 30000 keys, 7 tiles a run, 27.1 -> 26.3; three against 20000, 4.9 tiles,
+  // 26.1 -> 26.5; 16-bit tiles, which do not pass through registers, 53.5 -> 54.9 for the first of these)
+  if constexpr (FP8)
+    if (nwg <= kSplitPairWorkgroups && (a.P + a.S) / kKeyTile >= kSplitPairTiles * a.split_runs)
+      return launch_attn_split_h<D, KF, FP8, 1, 2>(a, nwg, stream);
+  return launch_attn_split_h<D, KF, FP8, 1, 1>(a, nwg, stream);
 }
 
 // Number of runs for a call; false: the call is not of this kind, which takes at least kSplitMinKeys
