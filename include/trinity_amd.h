@@ -187,10 +187,14 @@ int tri_validate_ffn_block(const tri_tensor* o2, const tri_tensor* wo, const tri
                            const tri_tensor* attn_o2, const tri_tensor* row_scratch, const tri_tensor* ff1,
                            const tri_tensor* ff2, const tri_tensor* o_ff_norm, const tri_tensor* workspace);
 
-/* Bytes of scratch tri_qkv_attention / tri_keyformer / tri_roco need for the
- * given parameters (n_model = columns of X).  Negative = tri_status.  The
- * attention entry points want at least one new token: p->seq < 1 is
- * TRI_ERR_SHAPE here and there. */
+/* Bytes of scratch with which tri_qkv_attention / tri_keyformer / tri_roco run
+ * their fastest plans for the given parameters (n_model = columns of X).
+ * Negative = tri_status.  The attention entry points want at least one new
+ * token: p->seq < 1 is TRI_ERR_SHAPE here and there.  They also accept a smaller
+ * buffer and shrink the workspaces in it, which only let faster plans run (same
+ * results to rounding), as long as everything else has room (TRI_ERR_SCRATCH
+ * otherwise).  A buffer of this size serves every call with fewer tokens behind
+ * the same prefix, although their own fastest plans may ask for more. */
 int64_t tri_qkv_scratch_bytes(const tri_attn_params* p, int64_t n_model);
 
 /* Fused QKV projection + KV-cache append + softmax attention: Vanilla,

@@ -96,6 +96,27 @@ def test_scratch_size_query_rejects_what_the_launchers_reject():
     assert q(**dict(ok, seq=0)) == -3
 
 
+def _host(*shape, dtype=torch.float16):
+    return torch.empty(*shape, dtype=dtype)  # (never touched: the checks look at shapes, strides and pointers only)
+
+
+@pytest.mark.parametrize("longest", [64, 128, 512, 1024, 2048])
+@pytest.mark.parametrize("P", [0, 1000, 4096])
+@pytest.mark.parametrize("Hq,Hkv,D,N", [(71, 1, 64, 4544), (32, 8, 128, 4096)])
+def test_scratch_of_the_longest_call_serves_shorter_ones(Hq, Hkv, D, N, P, longest):
+    """The size for the fastest plan peaks in the middle of the range of token counts; a buffer sized for the longest
+    call of a program is accepted for each shorter one all the same, behind the prefix it was sized for or none."""
+    raw = torch.empty(ext.qkv_scratch_bytes(ext.attn_params(Hq, Hkv, D, longest, kv_prefix=P), N) + 256, dtype=torch.uint8)
+    lead = (-raw.data_ptr()) % 256
+    scratch = raw[lead:lead + raw.numel() - 256]
+    x, wq, wk, wv, out = _host(longest, N), _host(N, Hq * D), _host(N, Hkv * D), _host(N, Hkv * D), _host(longest, Hq * D)
+    kc, vc = _host(Hkv, P + longest, D), _host(Hkv, P + longest, D)
+    for prefix in {0, P}:
+        for s in list(range(1, min(longest, 100))) + list(range(100, longest, 53)):
+            p = ext.attn_params(Hq, Hkv, D, s, kv_prefix=prefix)
+            assert ext.qkv_attention(x[:s], None, wq, wk, wv, kc, vc, scratch, None, out[:s], p, validate_only=True) == 0, s
+
+
 def test_static_scratch_entry_point_checks_before_touching_the_gpu():
     """tri_qkv_attention_static refuses a call that does not fit its array, and any bad argument, on the host."""
     S, N, Hq, Hkv, D = 8192, 4096, 32, 8, 128

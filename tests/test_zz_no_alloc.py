@@ -164,3 +164,37 @@ def test_static_scratch_holds_calls_without_full_workspaces(dev, S, Hq, Hkv, D, 
     ext.qkv_attention_static(x, None, wq, wk, wv, kc, vc, None, got, p)
     torch.cuda.synchronize()
     assert (got.float() - want.float()).abs().max().item() <= 2.0 ** -7 * max(1.0, want.float().abs().max().item())
+
+
+@pytest.mark.parametrize("S,Hq,Hkv,D,P,fp8", [
+    (400, 71, 1, 64, 0, False),      # part of the room that the projection's parts want (a buffer for 1024 tokens)
+    (200, 32, 8, 128, 0, False), (300, 32, 8, 128, 4096, False),  # ... none for the parts of a chunk's attention
+    (20, 32, 8, 128, 2100, True),    # the fewest runs of the key-split attention, fp8 rows
+    (33, 32, 8, 128, 4096, True),
+])
+def test_caller_scratch_of_the_least_size(dev, S, Hq, Hkv, D, P, fp8):
+    """The smallest buffer a call is accepted with: the results of the whole layout, and no byte past its end touched.
+    Tolerance as above: sums in another order, one step of a new row's fp8 code."""
+    N = 4544 if D == 64 else 4096
+    g = torch.Generator().manual_seed(6)
+    rn = lambda *shape, std=1.0: (torch.randn(*shape, generator=g) * std).half().to(dev)
+    x, wq, wk, wv = rn(S, N), rn(N, Hq * D, std=0.02), rn(N, Hkv * D, std=0.02), rn(N, Hkv * D, std=0.02)
+    kc, vc = rn(Hkv, P + S, D), rn(Hkv, P + S, D)
+    if fp8:
+        kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
+    p = ext.attn_params(Hq, Hkv, D, S, kv_prefix=P, causal=True, kv_fp8=fp8, k_scale=1.0, v_scale=1.0)
+    whole = ext.qkv_scratch_bytes(p, N)
+    scratch = torch.full((whole,), 0x7F, dtype=torch.uint8, device=dev)
+    want, got = (torch.zeros(S, Hq * D, dtype=torch.float16, device=dev) for _ in range(2))
+    accepted = lambda n: ext.qkv_attention(x, None, wq, wk, wv, kc, vc, scratch[:n], None, got, p, validate_only=True) == 0
+    lo, hi = 0, whole // 256
+    while lo < hi:
+        mid = (lo + hi) // 2
+        lo, hi = (lo, mid) if accepted(mid * 256) else (mid + 1, hi)
+    assert hi * 256 < whole
+    ext.qkv_attention(x, None, wq, wk, wv, kc.clone(), vc.clone(), scratch[:hi * 256], None, got, p)
+    torch.cuda.synchronize()
+    assert (scratch[hi * 256:] == 0x7F).all()
+    ext.qkv_attention(x, None, wq, wk, wv, kc, vc, scratch, None, want, p)
+    torch.cuda.synchronize()
+    assert (got.float() - want.float()).abs().max().item() <= 2.0 ** -7 * max(1.0, want.float().abs().max().item())

@@ -69,12 +69,33 @@ struct Scratch {
 
 inline int64_t align256(int64_t x) { return (x + 255) & ~(int64_t)255; }
 
-// Layout in at most `budget` bytes.  The two workspaces (partial sums of the projection, partial results of the
-// key-split attention) only let faster plans run: where the whole layout does not fit, the second shrinks to the size
-// that every plan accepts and the first to what is left.  The total may exceed the budget all the same.
-Scratch scratch_layout(const tri_attn_params* p, int64_t n_model, int64_t budget = INT64_MAX) {
+// Partial results of the key-split attention of a call of S tokens, for every run the key axis would be cut into, for the
+// fewest, or what the call cannot do without: up to 32 tokens the attention kernels (the only ones that read fp8 rows)
+// always leave parts.
+enum AttnParts { kAllRuns, kFewestRuns, kNoRuns };
+int64_t attn_parts_bytes(const tri_attn_params* p, int S, AttnParts runs) {
+  const int Hq = p->n_q_heads, Hkv = p->n_kv_heads, D = p->head_dim, L = p->kv_prefix + S;
+  if (runs == kNoRuns && S > tri::kFewMaxQueries) return 0;
+  const int64_t split = split_attn_workspace_bytes(S, Hq, Hkv, D, L, runs != kAllRuns);
+  if (runs == kNoRuns && split > 0) return split;
+  const int64_t few = few_attn_workspace_bytes(S, Hq, D, L);
+  return few > split ? few : split;
+}
+
+// 33 to 64 tokens: one part of the projection is asked for whether or not its plan has parts (without it this would be
+// the one range that needs less than its shorter calls, whose attention cannot do without parts).
+int64_t proj_part_bytes(const tri_attn_params* p, int64_t n_model, int64_t S) {
+  if (S <= tri::kFewMaxQueries || S > 64 || n_model < 64 || n_model % 32 != 0) return 0;
+  return S * (p->n_q_heads + 2 * (int64_t)p->n_kv_heads) * p->head_dim * 4;
+}
+
+// Layout of a call of S tokens in at most `budget` bytes, those of the buffer it is given.  Its two workspaces (partial
+// sums of the projection, partial results of attention) only let faster plans run: where the whole layout does not fit,
+// attention is left the fewest runs, or none, and the projection what remains.  The total may exceed the budget all the
+// same.
+Scratch scratch_layout(const tri_attn_params* p, int64_t n_model, int64_t S, int64_t budget) {
   Scratch s{};
-  const int64_t S = p->seq, Hq = p->n_q_heads, Hkv = p->n_kv_heads, D = p->head_dim;
+  const int64_t Hq = p->n_q_heads, Hkv = p->n_kv_heads, D = p->head_dim;
   int64_t off = 0;
   s.q_off = off; off = align256(off + S * Hq * D * 2);
   s.k_off = off; off = align256(off + Hkv * S * D * 2);
@@ -82,22 +103,21 @@ Scratch scratch_layout(const tri_attn_params* p, int64_t n_model, int64_t budget
   s.xn_off = off; off = align256(off + (p->prenorm ? S * n_model * 2 : 0));
   s.lse_off = off; off = align256(off + Hq * S * 4);
   s.lsep_off = off; off = align256(off + Hq * S * 4);
-  // few or middling tokens: room for the partial sums of the projection and for the partial results of the
-  // key-split attention (separate: the attention kernel merges the former while it writes the latter)
-  s.ws_bytes = qkv_workspace_bytes((int)S, (int)n_model, (int)((Hq + 2 * Hkv) * D), p->qknorm ? (int)D : 1);
-  const int64_t few = few_attn_workspace_bytes((int)S, (int)Hq, (int)D, (int)(p->kv_prefix + S));
-  auto attn_bytes = [&](bool least) {
-    const int64_t split = split_attn_workspace_bytes((int)S, (int)Hq, (int)Hkv, (int)D, (int)(p->kv_prefix + S), least);
-    return few > split ? few : split;
-  };
-  s.aws_bytes = attn_bytes(false);
   // fp8 caches: 16-bit copies of all P + S rows for the kernels that read 16-bit K / V tiles
   const int64_t copy = p->kv_fp8 ? Hkv * ((int64_t)p->kv_prefix + S) * D * 2 : 0;
-  const int64_t rest = off + 2 * align256(copy);
-  if (rest + align256(s.ws_bytes) + align256(s.aws_bytes) > budget) {
-    s.aws_bytes = attn_bytes(true);
-    const int64_t left = (budget - rest - align256(s.aws_bytes)) & ~(int64_t)255;
-    s.ws_bytes = left <= 0 ? 0 : (s.ws_bytes < left ? s.ws_bytes : left);
+  const int64_t left = budget - off - 2 * align256(copy);  // for the workspaces
+  // (separate: the attention kernel merges the projection's parts while it writes its own)
+  s.ws_bytes = proj_part_bytes(p, n_model, S);
+  if (left > 0) {
+    const int64_t parts = qkv_workspace_bytes((int)S, (int)n_model, (int)((Hq + 2 * Hkv) * D), p->qknorm ? (int)D : 1);
+    s.ws_bytes = parts > s.ws_bytes ? parts : s.ws_bytes;
+  }
+  s.aws_bytes = attn_parts_bytes(p, (int)S, kAllRuns);
+  if (align256(s.ws_bytes) + align256(s.aws_bytes) > left) {
+    s.aws_bytes = attn_parts_bytes(p, (int)S, kFewestRuns);
+    if (align256(s.aws_bytes) > left) s.aws_bytes = attn_parts_bytes(p, (int)S, kNoRuns);
+    const int64_t rest = (left - align256(s.aws_bytes)) & ~(int64_t)255;
+    s.ws_bytes = rest <= 0 ? 0 : (s.ws_bytes < rest ? s.ws_bytes : rest);
   }
   s.ws_off = off; off = align256(off + s.ws_bytes);
   s.aws_off = off; off = align256(off + s.aws_bytes);
@@ -105,6 +125,16 @@ Scratch scratch_layout(const tri_attn_params* p, int64_t n_model, int64_t budget
   s.vd_off = off; off = align256(off + copy);
   s.total = off;
   return s;
+}
+
+// Bytes without which a call of S tokens is refused: everything but the workspaces, and what is always asked for of them.
+int64_t scratch_least(const tri_attn_params* p, int64_t n_model, int64_t S) {
+  return scratch_layout(p, n_model, S, 0).total + align256(proj_part_bytes(p, n_model, S));
+}
+
+// bytes of a 1-D scratch buffer
+int64_t scratch_bytes(const tri_tensor* t) {
+  return t->shape[0] * (t->dtype == TRI_U8 || t->dtype == TRI_FP8_E4M3 ? 1 : (t->dtype == TRI_F32 ? 4 : 2));
 }
 
 // element type of a call: fp16 or bf16, taken from its first activation tensor (every other 16-bit tensor of the
@@ -258,12 +288,22 @@ int validate_qkv_common(const tri_tensor* x, const tri_tensor* norm_w, const tri
   }
   if (scratch == nullptr || scratch->ptr == nullptr) return TRI_ERR_NULL;
   if (scratch->ndim != 1 || (scratch->shape[0] > 1 && scratch->stride[0] != 1)) return TRI_ERR_STRIDE;
-  {
-    const int64_t esz = (scratch->dtype == TRI_U8) ? 1 : (scratch->dtype == TRI_F32 ? 4 : 2);
-    if (scratch->shape[0] * esz < scratch_layout(p, N).total) return TRI_ERR_SCRATCH;
-    if (((uintptr_t)scratch->ptr & 255u) != 0) return TRI_ERR_ALIGN;
-  }
+  if (scratch_bytes(scratch) < scratch_least(p, N, S)) return TRI_ERR_SCRATCH;
+  if (((uintptr_t)scratch->ptr & 255u) != 0) return TRI_ERR_ALIGN;
   TRI_TRY(check_mat(out, S, Hq * D, dt));
+  return TRI_OK;
+}
+
+// the limits of validate_qkv_common, so that a size is only returned for parameters the launchers accept
+int check_scratch_params(const tri_attn_params* p, int64_t n_model) {
+  if (p == nullptr) return TRI_ERR_NULL;
+  if (p->head_dim != 64 && p->head_dim != 128) return TRI_ERR_UNSUPPORTED;
+  if (p->seq <= 0 || p->kv_prefix < 0 || p->n_q_heads <= 0 || p->n_kv_heads <= 0 ||
+      p->n_q_heads % p->n_kv_heads != 0 || n_model < 0 || n_model >= ((int64_t)1 << 31))
+    return TRI_ERR_SHAPE;
+  const int64_t S = p->seq, D = p->head_dim, L = (int64_t)p->kv_prefix + S;
+  if (S * p->n_q_heads * D * 2 >= ((int64_t)1 << 31)) return TRI_ERR_UNSUPPORTED;
+  if (L * D * 2 >= ((int64_t)1 << 31)) return TRI_ERR_UNSUPPORTED;  // a head's cache rows fit a buffer descriptor
   return TRI_OK;
 }
 
@@ -435,16 +475,16 @@ int tri_ffn_block(const tri_tensor* o2, const tri_tensor* wo, const tri_tensor* 
 
 // ---------------------------------------------------------------- attention
 int64_t tri_qkv_scratch_bytes(const tri_attn_params* p, int64_t n_model) {
-  if (p == nullptr) return TRI_ERR_NULL;
-  // the limits of validate_qkv_common, so that a size is only returned for parameters the launchers accept
-  if (p->head_dim != 64 && p->head_dim != 128) return TRI_ERR_UNSUPPORTED;
-  if (p->seq <= 0 || p->kv_prefix < 0 || p->n_q_heads <= 0 || p->n_kv_heads <= 0 ||
-      p->n_q_heads % p->n_kv_heads != 0 || n_model < 0 || n_model >= ((int64_t)1 << 31))
-    return TRI_ERR_SHAPE;
-  const int64_t S = p->seq, D = p->head_dim, L = (int64_t)p->kv_prefix + S;
-  if (S * p->n_q_heads * D * 2 >= ((int64_t)1 << 31)) return TRI_ERR_UNSUPPORTED;
-  if (L * D * 2 >= ((int64_t)1 << 31)) return TRI_ERR_UNSUPPORTED;  // a head's cache rows fit a buffer descriptor
-  return scratch_layout(p, n_model).total;
+  TRI_TRY(check_scratch_params(p, n_model));
+  // The whole layout need not grow with the number of tokens (Falcon-7B heads: 33.8 MB at 512, 9.9 MB at 1000), nor does
+  // what a call cannot do without (the parts of up to 32 tokens): a buffer made for the longest call of a program has to
+  // serve its shorter ones.
+  int64_t bytes = scratch_layout(p, n_model, p->seq, INT64_MAX).total;
+  for (int s = 1; s < p->seq && s <= 64; ++s) {
+    const int64_t least = scratch_least(p, n_model, s);
+    bytes = bytes > least ? bytes : least;
+  }
+  return bytes;
 }
 
 int tri_validate_qkv_attention(const tri_tensor* x, const tri_tensor* norm_w, const tri_tensor* wq,
@@ -470,15 +510,13 @@ int tri_qkv_attention_static(const tri_tensor* x, const tri_tensor* norm_w, cons
   if (x == nullptr || p == nullptr) return TRI_ERR_NULL;
   if (x->ndim != 2) return TRI_ERR_SHAPE;
   // the size first: a call that does not fit the array is refused before anything else is looked at
-  const int64_t need = tri_qkv_scratch_bytes(p, x->shape[1]);
-  if (need < 0) return (int)need;
-  if (need > kStaticScratchBytes && scratch_layout(p, x->shape[1], kStaticScratchBytes).total > kStaticScratchBytes)
-    return TRI_ERR_SCRATCH;
+  TRI_TRY(check_scratch_params(p, x->shape[1]));
+  if (scratch_layout(p, x->shape[1], p->seq, kStaticScratchBytes).total > kStaticScratchBytes) return TRI_ERR_SCRATCH;
   // every other argument is checked against a stand-in for the array (right size and alignment, never
   // dereferenced), so that a bad call fails without touching the GPU
   tri_tensor scratch{};
   scratch.ptr = reinterpret_cast<void*>(static_cast<uintptr_t>(256));
-  scratch.shape[0] = need > kStaticScratchBytes ? need : kStaticScratchBytes;
+  scratch.shape[0] = INT64_MAX / 8;
   scratch.stride[0] = 1;
   scratch.ndim = 1;
   scratch.dtype = TRI_U8;

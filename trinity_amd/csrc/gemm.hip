@@ -427,15 +427,18 @@ static TilePlan big_plan(int M, int N, int epi, bool kcontig) {
 // (1 row x [4096, 14336 x 2] with 64 x 64 tiles 82 us, with 128 columns 43 us).
 constexpr int kGatedMinBn = 128;
 
-// Up to 64 rows the size of one part is returned even where the best plan has no parts: callers take a size of zero
-// to mean "not a few-row shape".
-static int64_t plan_workspace_bytes(int M, int K, int ncols, int unit, int min_bn) {
+// workspace of the best plan, if it has at least `least` parts (0 otherwise)
+static int64_t plan_workspace_bytes(int M, int K, int ncols, int unit, int min_bn, int least) {
   const RingPlan plan = ring_plan(M, K, ncols, unit, min_bn, INT64_MAX);
-  return plan.tile < 0 || (plan.ksplit == 1 && M > 64) ? 0 : (int64_t)plan.ksplit * M * ncols * 4;
+  return plan.tile < 0 || plan.ksplit < least ? 0 : (int64_t)plan.ksplit * M * ncols * 4;
 }
 
+// Up to 64 rows the size of one part is returned even where the best plan has no parts: callers take a size of zero
+// to mean "not a few-row shape".
 int64_t gemm_workspace_bytes(int M, int K, int ncols) {
-  const int64_t any = plan_workspace_bytes(M, K, ncols, 1, 0), gated = plan_workspace_bytes(M, K, ncols, 1, kGatedMinBn);
+  const int least = M > 64 ? 2 : 1;
+  const int64_t any = plan_workspace_bytes(M, K, ncols, 1, 0, least);
+  const int64_t gated = plan_workspace_bytes(M, K, ncols, 1, kGatedMinBn, least);
   return any > gated ? any : gated;
 }
 
@@ -532,7 +535,7 @@ static int launch_qkv_d(const QkvProjArgs& a, hipStream_t stream) {
   }
 }
 
-int64_t qkv_workspace_bytes(int S, int K, int ncols, int unit) { return plan_workspace_bytes(S, K, ncols, unit, 0); }
+int64_t qkv_workspace_bytes(int S, int K, int ncols, int unit) { return plan_workspace_bytes(S, K, ncols, unit, 0, 2); }
 
 int launch_qkv_proj(const QkvProjArgs& a, hipStream_t stream, int* deferred_ksplit, bool* appended) {
   if (deferred_ksplit != nullptr) *deferred_ksplit = 0;
