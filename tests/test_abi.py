@@ -152,6 +152,18 @@ def test_rmsnorm_validation():
     assert ext.lib().tri_validate_rmsnorm(None, None, None, ctypes.c_float(0)) == -1
 
 
+def test_launching_calls_take_tensor_descriptors():
+    """Tensors and their descriptors (ext.as_tri) are the same to every call; what is neither is refused."""
+    x, y, w = _h(0, 64), _h(0, 64), _h(64)  # no rows: nothing is launched
+    d = ext.as_tri
+    call = lambda *tensors: ext.native().rmsnorm(*tensors, 1e-5, 0)
+    assert call(x, w, y) == call(d(x), d(w), d(y)) == call(x, d(w), y) == 0
+    assert call(x, w, _h(0, 32)) == call(d(x), d(w), d(_h(0, 32))) == -3
+    for other in (bytes(ctypes.sizeof(ext.TriTensor)), ext.attn_params(1, 1, 64, 1), 0):
+        with pytest.raises(TypeError):
+            call(x, other, y)
+
+
 def test_ffn_validation():
     x, wg, wu, wd, hid, out = _h(16, 64), _h(64, 128), _h(64, 128), _h(128, 64), _h(16, 128), _h(16, 64)
     assert ext.ffn_swiglu(x, wg, wu, wd, hid, out, validate_only=True) == 0

@@ -4,9 +4,12 @@
 // 25 us per call, more than most kernels of a decode step run (RMSNorm of 16 rows: 10.2 us a call of which the GPU
 // worked 3.0).  Reading sizes and strides from the tensor object takes some 20 ns.
 //
-// Every function takes the tensors in the order of the C entry point (None where it allows NULL), then its scalars, then
-// the stream as an integer, and returns the status; trinity_amd/ext.py turns a status into an exception.
+// Every function takes the tensors (or descriptors of them) in the order of the C entry point (None where it allows
+// NULL), then its scalars, then the stream as an integer, and returns the status; trinity_amd/ext.py turns a status into
+// an exception.
 #include <torch/csrc/autograd/python_variable.h>
+
+#include <cstring>
 
 #include "../../include/trinity_amd.h"
 
@@ -19,15 +22,24 @@ struct Tensors {
   tri_tensor* p[kMaxTensors];
 };
 
-// a[i] = tensor or None
+// a[i] = tensor, None, or a tensor's descriptor as ext.as_tri makes it
 bool to_tri(PyObject* o, tri_tensor& v, tri_tensor*& p) {
   if (o == Py_None) {
     p = nullptr;
     return true;
   }
   if (!THPVariable_Check(o)) {
-    PyErr_Format(PyExc_TypeError, "expected a tensor or None, got %.100s", Py_TYPE(o)->tp_name);
-    return false;
+    Py_buffer b;
+    if (strcmp(Py_TYPE(o)->tp_name, "TriTensor") != 0 || PyObject_GetBuffer(o, &b, PyBUF_SIMPLE) != 0) {
+      PyErr_Format(PyExc_TypeError, "expected a tensor or None, got %.100s", Py_TYPE(o)->tp_name);
+      return false;
+    }
+    const bool whole = b.len == (Py_ssize_t)sizeof v;
+    if (whole) memcpy(&v, b.buf, sizeof v);
+    else PyErr_SetString(PyExc_TypeError, "not the TriTensor of this library");
+    PyBuffer_Release(&b);
+    p = &v;
+    return whole;
   }
   const at::Tensor& t = THPVariable_Unpack(o);
   switch (t.scalar_type()) {
