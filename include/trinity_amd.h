@@ -133,8 +133,9 @@ int tri_validate_ffn_swiglu(const tri_tensor* x, const tri_tensor* w_gate, const
                             const tri_tensor* w_down, const tri_tensor* hidden, const tri_tensor* out,
                             const tri_tensor* workspace);
 
-/* Workspace of products with few or middling rows (1 to about 1100; the
- * reference's own regime is M = 16 new tokens, convert_eval_rms.py:61-107).
+/* Workspace of products with few or middling rows (1 to about 1100, up to 8192
+ * where the outputs are few and the sums long; the reference's own regime is
+ * M = 16 new tokens, convert_eval_rms.py:61-107).
  * Such a product is bound by streaming w from HBM once; where whole tiles
  * would leave part of the chip idle the library cuts the K axis into parts,
  * which needs room for fp32 partial sums.  Every FFN entry point takes that

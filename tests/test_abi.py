@@ -45,6 +45,13 @@ def test_workspace_sizes():
     assert ext.ffn_gelu(x, wg, wd, hid, out, workspace=ws.view(2, 512), validate_only=True) == -3
 
 
+@pytest.mark.parametrize("M,K,N", [(1101, 4096, 1024), (1536, 14336, 1024), (3000, 14336, 1024), (1200, 14336, 4096)])
+def test_narrow_products_of_many_rows_run_in_parts(M, K, N):
+    """Few large tiles, each over a deep K, leave most of the chip idle: such products are cut into parts."""
+    assert ext.gemm_workspace_bytes(M, K, N) >= 2 * M * N * 4
+    assert ext.gemm_workspace_bytes(M, K, N) % (M * N * 4) == 0
+
+
 def _h(*shape):
     return torch.zeros(*shape, dtype=torch.float16)
 

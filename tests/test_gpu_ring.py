@@ -32,6 +32,8 @@ def check(got, want, what):
     (129, 4096, 6144), (160, 4544, 18176), (161, 1056, 5000),        # row blocks with a remainder; K = 16.5 k tiles
     (300, 14336, 4096), (333, 18176, 4544), (700, 4096, 6144),
     (1100, 4096, 4096), (1101, 512, 1024),                           # the largest rows of the family, and one more
+    (1101, 2048, 1024), (1500, 14336, 520), (2049, 4544, 1000),      # beyond them: narrow outputs over a deep K
+    (8192, 2048, 72), (8193, 2048, 72),
 ])
 @pytest.mark.parametrize("kcontig", [False, True])
 @pytest.mark.parametrize("with_ws", [False, True])

@@ -394,10 +394,13 @@ static TilePlan best_plan(int M, int N, int& which) {
 // of 256 x 256 tiles (Llama-3-8B and Falcon-7B products, 256 to 1536 rows: within 12 %).
 static float plan_us(const TilePlan& p, int K) { return 6.0f + 0.0272f * (float)K * (float)p.cost; }
 
-// The ring kernels' plan for a product, if it beats a tile plan of big_us.
+// The ring kernels' plan for a product, if it beats a tile plan of big_us.  Beyond the rows that the costs were fitted
+// over, by a quarter: 14336 -> 1024, 2048 rows 162 -> 70 us (0.39 by the costs), 14336 -> 4096, 1200 rows 187 -> 142
+// (0.74), but 4096 rows of 4096 -> 1024 43.0 -> 45.8 (0.76), 3072 of 14336 -> 4096 310 -> 370 (0.86).
+constexpr float kRingMarginNarrow = 0.75f;
 static bool ring_wins(float big_us, int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes, RingPlan& plan) {
   plan = ring_plan(M, K, ncols, unit, min_bn, ws_bytes);
-  return plan.tile >= 0 && plan.us < big_us;
+  return plan.tile >= 0 && plan.us < (M <= kRingMaxRows ? big_us : kRingMarginNarrow * big_us);
 }
 
 // plain and GELU epilogues on the direct-to-LDS path: pick the cheapest plan
@@ -436,6 +439,13 @@ static int64_t plan_workspace_bytes(int M, int K, int ncols, int unit, int min_b
 // Up to 64 rows the size of one part is returned even where the best plan has no parts: callers take a size of zero
 // to mean "not a few-row shape".
 int64_t gemm_workspace_bytes(int M, int K, int ncols) {
+  if (M > kRingMaxRows) {  // (plain and GELU products only; the tile plan over K-contiguous weights is the dearer one)
+    RingPlan plan;
+    if (M > kRingMaxRowsNarrow || ncols > kRingMaxColsNarrow ||
+        !ring_wins(plan_us(big_plan(M, ncols, EPI_NONE, true), K), M, K, ncols, 1, 0, INT64_MAX, plan))
+      return 0;
+    return plan_workspace_bytes(M, K, ncols, 1, 0, 2);
+  }
   const int least = M > 64 ? 2 : 1;
   const int64_t any = plan_workspace_bytes(M, K, ncols, 1, 0, least);
   const int64_t gated = plan_workspace_bytes(M, K, ncols, 1, kGatedMinBn, least);
@@ -470,8 +480,10 @@ static int launch_gemm_big(const GemmArgs& a, hipStream_t stream) {
 int launch_gemm(const GemmArgs& a, hipStream_t stream) {
   if (a.M <= 0 || a.N <= 0) return 0;
   RingPlan plan;
-  if (ring_wins(plan_us(big_plan(a.M, a.N, a.epi, a.w_kcontig != 0), a.K), a.M, a.K, a.epi == EPI_SWIGLU ? 2 * a.N : a.N, 1,
-                a.epi == EPI_SWIGLU && !a.w_kcontig ? kGatedMinBn : 0, a.ws != nullptr ? a.ws_bytes : 0, plan))
+  const bool gated = a.epi == EPI_SWIGLU;
+  if (!(gated && a.M > kRingMaxRows) &&
+      ring_wins(plan_us(big_plan(a.M, a.N, a.epi, a.w_kcontig != 0), a.K), a.M, a.K, gated ? 2 * a.N : a.N, 1,
+                gated && !a.w_kcontig ? kGatedMinBn : 0, a.ws != nullptr ? a.ws_bytes : 0, plan))
     return launch_ring_gemm(a, plan, stream);
   const int rc = launch_gemm_big(a, stream);
   if (rc != 0 || a.rowstat_out == nullptr) return rc;
@@ -535,7 +547,9 @@ static int launch_qkv_d(const QkvProjArgs& a, hipStream_t stream) {
   }
 }
 
-int64_t qkv_workspace_bytes(int S, int K, int ncols, int unit) { return plan_workspace_bytes(S, K, ncols, unit, 0, 2); }
+int64_t qkv_workspace_bytes(int S, int K, int ncols, int unit) {
+  return S > kRingMaxRows ? 0 : plan_workspace_bytes(S, K, ncols, unit, 0, 2);
+}
 
 int launch_qkv_proj(const QkvProjArgs& a, hipStream_t stream, int* deferred_ksplit, bool* appended) {
   if (deferred_ksplit != nullptr) *deferred_ksplit = 0;
@@ -548,7 +562,8 @@ int launch_qkv_proj(const QkvProjArgs& a, hipStream_t stream, int* deferred_kspl
   const TilePlan big = a.w_kcontig ? qkv_plan_kcontig(a.S, ncols) : qkv_plan(a.S, ncols, a.qknorm ? a.D : 0, which);
   // (its weights are small enough to come from the Infinity Cache when the caller uses them again: the large tiles
   // are then a tenth faster than over weights from HBM, the ring kernels hardly - 658 to 1000 rows, both within 2 %)
-  if (ring_wins(0.9f * plan_us(big, a.K), a.S, a.K, ncols, a.qknorm ? a.D : 1, 0, a.ws != nullptr ? a.ws_bytes : 0, plan))
+  if (a.S <= kRingMaxRows &&
+      ring_wins(0.9f * plan_us(big, a.K), a.S, a.K, ncols, a.qknorm ? a.D : 1, 0, a.ws != nullptr ? a.ws_bytes : 0, plan))
     return launch_ring_qkv(a, plan, stream, deferred_ksplit, appended);
   return a.D == 128 ? launch_qkv_d<128>(a, stream) : launch_qkv_d<64>(a, stream);
 }

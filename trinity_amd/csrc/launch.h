@@ -91,7 +91,10 @@ struct RingPlan {
   int tile, ksplit;
   float us;
 };
-constexpr int kRingMaxRows = 1100;  // beyond this the large tiles fill the chip (and the cost model was not fitted)
+constexpr int kRingMaxRows = 1100;  // the range that the cost model was fitted over, and some more
+// ... and that of products with so few large tiles, each with so much to sum, that these leave most of the chip idle
+// (ring_wins in gemm.hip)
+constexpr int kRingMaxRowsNarrow = 8192, kRingMaxColsNarrow = 1 << 16, kRingMinKNarrow = 2048;
 // ncols: weight columns (gate and up, or q, k and v, together).  Tiles must be a multiple of `unit` wide (whole heads; 1
 // otherwise) and at least min_bn.  ws_bytes: fp32 workspace for partial results, ksplit * M * ncols * 4 bytes (1: none).
 RingPlan ring_plan(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes);

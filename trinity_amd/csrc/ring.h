@@ -1,4 +1,5 @@
-// Main loop and tile family of the GEMMs with few and middling rows (1 to about 1000 tokens), shared by ring.hip
+// Main loop and tile family of the GEMMs with few and middling rows (1 to about 1000 tokens, more of narrow products over
+// a deep K), shared by ring.hip
 // (FFN products) and ring_qkv.hip (Q/K/V projection).
 //
 // What bounds them: streaming the weights once.  To keep 5 TB/s coming from HBM a CU needs some 60 KB of weights in

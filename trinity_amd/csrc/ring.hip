@@ -323,7 +323,8 @@ static RingPlan ring_plan_search(int M, int K, int ncols, int unit, int min_bn, 
 // The search is a pure function of its arguments and takes 5 to 10 us, longer than a launch; each thread keeps the
 // answers it was last given.
 RingPlan ring_plan(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes) {
-  if (M < 1 || M > kRingMaxRows || K % 32 != 0 || K < 64 || ncols < 8) return RingPlan{-1, 1, 1e30f};
+  if (M < 1 || K % 32 != 0 || K < 64 || ncols < 8) return RingPlan{-1, 1, 1e30f};
+  if (M > kRingMaxRows && (M > kRingMaxRowsNarrow || ncols > kRingMaxColsNarrow || K < kRingMinKNarrow)) return RingPlan{-1, 1, 1e30f};
   struct Entry { int M, K, ncols, unit, min_bn; int64_t ws_bytes; RingPlan plan; };
   static thread_local Entry memo[256] = {};
   uint64_t h = (uint64_t)M;
