@@ -383,6 +383,24 @@ def test_qkv_validation_randomised(s, hq, group, d, p, causal, short_scratch, dt
         assert rc == 0
 
 
+def test_the_library_builds_without_what_only_the_binding_needs(monkeypatch, tmp_path, capsys):
+    """No C++ compiler of its own: the C library is built all the same, and what is missing is said."""
+    import shutil
+    import subprocess
+
+    from trinity_amd import build
+
+    ran = []
+    monkeypatch.setattr(build.subprocess, "run",
+                        lambda cmd, **kw: ran.append(cmd) or subprocess.CompletedProcess(cmd, 0, "", ""))
+    monkeypatch.setattr(build, "NATIVE", str(tmp_path / "_native.so"))
+    hipcc = build.hipcc()
+    monkeypatch.setattr(shutil, "which", lambda name, *a, **kw: hipcc if name == "hipcc" else None)
+    assert build.build() == build.LIB
+    assert len(ran) == len(build.UNITS) + 1 and all(cmd[0] == hipcc for cmd in ran)
+    assert "binding" in capsys.readouterr().err
+
+
 def test_header_is_plain_c_and_links(tmp_path):
     """include/trinity_amd.h compiles as C99 with warnings as errors, and a C program linked against the library
     reaches the entry points (no GPU work: version, status strings, a validator, a size query)."""

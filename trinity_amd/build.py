@@ -1,4 +1,4 @@
-"""Build libtrinity_amd.so (gfx950) in-tree with hipcc.
+"""Build libtrinity_amd.so (gfx950) in-tree with hipcc, and its Python binding where torch and a C++ compiler are there.
 
 Usage: python -m trinity_amd.build            (also called by __graft_entry__.build)
 """
@@ -46,10 +46,23 @@ def hipcc():
 
 
 def cxx():
-    exe = shutil.which("g++")
-    if exe is None:
-        raise RuntimeError("g++ not found; the Python binding cannot be built")
-    return exe
+    """The C++ compiler of the binding: g++, or else the clang++ that hipcc drives (None: neither)."""
+    rocm = os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(hipcc()))), "llvm", "bin", "clang++")
+    return shutil.which("g++") or shutil.which(rocm)
+
+
+def binding_obstacle():
+    """What keeps the Python binding from being built here (None: nothing).  The C library does without it."""
+    import importlib.util
+    import sysconfig
+
+    if cxx() is None:
+        return "no C++ compiler (g++ or ROCm's clang++)"
+    if importlib.util.find_spec("torch") is None:
+        return "torch is not installed"
+    if not os.path.exists(os.path.join(sysconfig.get_paths()["include"], "Python.h")):
+        return "the Python headers are not installed"
+    return None
 
 
 def torch_libs():
@@ -69,11 +82,11 @@ def compile_binding(obj):
     cmd = [cxx(), "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI]
     r = subprocess.run(cmd + inc + ["-c", os.path.join(CSRC, "bind.cpp"), "-o", obj], capture_output=True, text=True)
     if r.returncode != 0:
-        raise RuntimeError("g++ failed on bind.cpp:\n%s\n%s" % (r.stdout, r.stderr))
+        raise RuntimeError("%s failed on bind.cpp:\n%s\n%s" % (cmd[0], r.stdout, r.stderr))
 
 
 def build(verbose=True, jobs=7):
-    """Compile every translation unit and link the shared library."""
+    """Compile every translation unit and link the shared library, then its Python binding."""
     from concurrent.futures import ThreadPoolExecutor
 
     objdir = os.path.join(HERE, "build")
@@ -93,8 +106,9 @@ def build(verbose=True, jobs=7):
         return obj
 
     bind_obj = os.path.join(objdir, "bind.o")
+    obstacle = binding_obstacle()
     with ThreadPoolExecutor(max_workers=jobs) as ex:
-        binding = ex.submit(compile_binding, bind_obj)
+        binding = ex.submit(compile_binding, bind_obj) if obstacle is None else None
         objs = list(ex.map(compile_one, UNITS))
     cmd = [cc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs
     r = subprocess.run(cmd, capture_output=True, text=True)
@@ -104,6 +118,11 @@ def build(verbose=True, jobs=7):
     import ctypes
 
     ctypes.CDLL(LIB)
+    if binding is None:
+        if os.path.exists(NATIVE):
+            os.remove(NATIVE)  # (of another build of the library)
+        sys.stderr.write("built %s without its Python binding, which trinity_amd.ext needs: %s\n" % (LIB, obstacle))
+        return LIB
     binding.result()
     cmd = [cxx(), "-shared", "-o", NATIVE, bind_obj, "-L" + HERE, "-ltrinity_amd", "-Wl,-rpath,$ORIGIN"] + torch_libs()
     r = subprocess.run(cmd, capture_output=True, text=True)

@@ -15,6 +15,7 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libtrinity_amd.so")
+NATIVE_PATH = os.path.join(_HERE, "_native.so")
 
 TRI_F16, TRI_BF16, TRI_F32, TRI_U8, TRI_FP8_E4M3 = 0, 1, 2, 3, 4
 _DTYPES = {torch.float16: TRI_F16, torch.bfloat16: TRI_BF16, torch.float32: TRI_F32, torch.uint8: TRI_U8,
