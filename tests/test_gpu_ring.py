@@ -62,6 +62,23 @@ def test_gated_with_row_scale(rn, M, K, F, kcontig):
         check(out, a * torch.sigmoid(a) * b, "gated")
 
 
+@pytest.mark.parametrize("M,N", [(1, 64), (16, 512), (33, 1024), (64, 4096)])
+def test_few_rows_in_place(rn, M, N):
+    """With a workspace a product of up to 64 rows may overwrite its input, also where its plan has one part."""
+    x, wg, wu = rn(M, N), rn(N, N, std=N ** -0.5), rn(N, N, std=N ** -0.5)
+    ws = torch.empty(ext.gemm_workspace_bytes(M, N, 2 * N), dtype=torch.uint8, device="cuda:0")
+    a, b = x.float() @ wg.float(), x.float() @ wu.float()
+    for call, want in ((lambda t: ext.matmul(t, wg, None, t, workspace=ws), a),
+                       (lambda t: ext.gateup_swiglu(t, wg, wu, None, t, workspace=ws), a * torch.sigmoid(a) * b)):
+        t = x.clone()
+        call(t)
+        check(t, want, "in place")
+    # two views of one buffer: neighbouring columns, not in place
+    buf = torch.cat([x, torch.zeros_like(x)], 1)
+    ext.matmul(buf[:, :N], wg, None, buf[:, N:], workspace=ws)
+    check(buf, torch.cat([x.float(), a], 1), "side by side")
+
+
 @pytest.mark.parametrize("S,N,Hq,Hkv,D", [
     (1, 64, 4, 4, 64), (33, 96, 5, 1, 128), (100, 4096, 32, 8, 128), (260, 4096, 32, 8, 128), (200, 4544, 71, 1, 64),
     (700, 128, 32, 8, 128), (1000, 128, 71, 1, 64), (1100, 160, 32, 4, 128),  # a tile across two weight matrices

@@ -436,8 +436,8 @@ static int64_t plan_workspace_bytes(int M, int K, int ncols, int unit, int min_b
   return plan.tile < 0 || plan.ksplit < least ? 0 : (int64_t)plan.ksplit * M * ncols * 4;
 }
 
-// Up to 64 rows the size of one part is returned even where the best plan has no parts: callers take a size of zero
-// to mean "not a few-row shape".
+// Up to 64 rows the size of one part is returned even where the best plan has no parts: with it such a product may
+// overwrite its own input (launch_ring_gemm).
 int64_t gemm_workspace_bytes(int M, int K, int ncols) {
   if (M > kRingMaxRows) {  // (plain and GELU products only; the tile plan over K-contiguous weights is the dearer one)
     RingPlan plan;
