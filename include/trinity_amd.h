@@ -145,9 +145,9 @@ int tri_validate_ffn_swiglu(const tri_tensor* x, const tri_tensor* w_gate, const
  * product [M, K] x [K, ncols] (ncols = 2 F for the gate/up pair);
  * tri_ffn_workspace_bytes for a whole FFN (x [M, N], hidden width F, including
  * the N x N output projection of tri_ffn_block).  Both return 0 when no
- * product of the shape is cut into parts, except that up to 64 rows at least
- * the size of one part is returned: given that much, a product may overwrite
- * its own input.  The attention entry points carry the same room inside their
+ * product of the shape is cut into parts, except that up to 64 rows (128 with
+ * at most 64 MB of weights; K >= 64) at least the size of one part is returned:
+ * given that much, a product may overwrite its own input.  The attention entry points carry the same room inside their
  * scratch buffer (tri_qkv_scratch_bytes), next to
  * the partial results of their key-split attention kernels (few new tokens,
  * or a chunk of tokens against thousands of cached keys). */

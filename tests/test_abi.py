@@ -107,6 +107,13 @@ def _host(*shape, dtype=torch.float16):
     return torch.empty(*shape, dtype=dtype)  # (never touched: the checks look at shapes, strides and pointers only)
 
 
+@pytest.mark.parametrize("M,K,N", [(1, 64, 8), (64, 14336, 4096), (65, 64, 64), (74, 416, 8), (100, 1024, 1024),
+                                   (128, 4096, 8192)])
+def test_few_rows_get_the_room_to_work_in_place(M, K, N):
+    """Up to 64 rows, and up to 128 with at most 64 MB of weights, there is room for one part at least."""
+    assert ext.gemm_workspace_bytes(M, K, N) >= M * N * 4
+
+
 @pytest.mark.parametrize("longest", [64, 128, 512, 1024, 2048])
 @pytest.mark.parametrize("P", [0, 1000, 4096])
 @pytest.mark.parametrize("Hq,Hkv,D,N", [(71, 1, 64, 4544), (32, 8, 128, 4096)])

@@ -62,9 +62,9 @@ def test_gated_with_row_scale(rn, M, K, F, kcontig):
         check(out, a * torch.sigmoid(a) * b, "gated")
 
 
-@pytest.mark.parametrize("M,N", [(1, 64), (16, 512), (33, 1024), (64, 4096)])
+@pytest.mark.parametrize("M,N", [(1, 64), (16, 512), (33, 1024), (64, 4096), (65, 1024), (128, 736)])
 def test_few_rows_in_place(rn, M, N):
-    """With a workspace a product of up to 64 rows may overwrite its input, also where its plan has one part."""
+    """With a workspace a product of few rows may overwrite its input, also where its plan has one part."""
     x, wg, wu = rn(M, N), rn(N, N, std=N ** -0.5), rn(N, N, std=N ** -0.5)
     ws = torch.empty(ext.gemm_workspace_bytes(M, N, 2 * N), dtype=torch.uint8, device="cuda:0")
     a, b = x.float() @ wg.float(), x.float() @ wu.float()

@@ -436,8 +436,10 @@ static int64_t plan_workspace_bytes(int M, int K, int ncols, int unit, int min_b
   return plan.tile < 0 || plan.ksplit < least ? 0 : (int64_t)plan.ksplit * M * ncols * 4;
 }
 
-// Up to 64 rows the size of one part is returned even where the best plan has no parts: with it such a product may
-// overwrite its own input (launch_ring_gemm).
+// Up to 64 rows, and up to 128 where the weights are at most 64 MB, the size of one part is returned even where the best
+// plan has no parts: with it such a product may overwrite its own input (launch_ring_gemm).
+constexpr int kInPlaceRows = 64, kInPlaceRowsSmall = 128;
+constexpr int64_t kInPlaceSmallBytes = (int64_t)64 << 20;
 int64_t gemm_workspace_bytes(int M, int K, int ncols) {
   if (M > kRingMaxRows) {  // (plain and GELU products only; the tile plan over K-contiguous weights is the dearer one)
     RingPlan plan;
@@ -446,7 +448,8 @@ int64_t gemm_workspace_bytes(int M, int K, int ncols) {
       return 0;
     return plan_workspace_bytes(M, K, ncols, 1, 0, 2);
   }
-  const int least = M > 64 ? 2 : 1;
+  const bool one_part = M <= kInPlaceRows || (M <= kInPlaceRowsSmall && 2 * (int64_t)K * ncols <= kInPlaceSmallBytes);
+  const int least = one_part ? 1 : 2;
   const int64_t any = plan_workspace_bytes(M, K, ncols, 1, 0, least);
   const int64_t gated = plan_workspace_bytes(M, K, ncols, 1, kGatedMinBn, least);
   return any > gated ? any : gated;
@@ -482,8 +485,9 @@ int launch_gemm(const GemmArgs& a, hipStream_t stream) {
   RingPlan plan;
   const bool gated = a.epi == EPI_SWIGLU;
   if (!(gated && a.M > kRingMaxRows) &&
-      ring_wins(plan_us(big_plan(a.M, a.N, a.epi, a.w_kcontig != 0), a.K), a.M, a.K, gated ? 2 * a.N : a.N, 1,
-                gated && !a.w_kcontig ? kGatedMinBn : 0, a.ws != nullptr ? a.ws_bytes : 0, plan))
+      (ring_wins(plan_us(big_plan(a.M, a.N, a.epi, a.w_kcontig != 0), a.K), a.M, a.K, gated ? 2 * a.N : a.N, 1,
+                 gated && !a.w_kcontig ? kGatedMinBn : 0, a.ws != nullptr ? a.ws_bytes : 0, plan) ||
+       (plan.tile >= 0 && ring_gemm_in_place(a))))  // (the tile plans store while other tiles still read)
     return launch_ring_gemm(a, plan, stream);
   const int rc = launch_gemm_big(a, stream);
   if (rc != 0 || a.rowstat_out == nullptr) return rc;

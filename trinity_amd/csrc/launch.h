@@ -99,6 +99,7 @@ constexpr int kRingMaxRowsNarrow = 8192, kRingMaxColsNarrow = 1 << 16, kRingMinK
 // otherwise) and at least min_bn.  ws_bytes: fp32 workspace for partial results, ksplit * M * ncols * 4 bytes (1: none).
 RingPlan ring_plan(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes);
 int launch_ring_gemm(const GemmArgs& a, const RingPlan& plan, hipStream_t stream);
+bool ring_gemm_in_place(const GemmArgs& a);  // out overlaps x, and the workspace holds the one part it takes to allow that
 // workspace that lets launch_gemm take its best plan for [M, K] x [K, ncols] (0: no plan in parts)
 int64_t gemm_workspace_bytes(int M, int K, int ncols);
 // the same for the Q/K/V projection; unit as in ring_plan

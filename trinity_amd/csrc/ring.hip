@@ -336,7 +336,7 @@ RingPlan ring_plan(int M, int K, int ncols, int unit, int min_bn, int64_t ws_byt
 }
 
 // out shares memory with x (views of one buffer whose columns do not meet share none)
-static bool in_place(const GemmArgs& a) {
+static bool shares_memory(const GemmArgs& a) {
   const half_t *xend = a.x + (a.M - 1) * a.ldx + a.K, *oend = a.out + (a.M - 1) * a.ldo + a.N;
   if (oend <= a.x || xend <= a.out) return false;
   if (a.ldx != a.ldo) return true;
@@ -344,12 +344,16 @@ static bool in_place(const GemmArgs& a) {
   return d < a.K || d + a.N > a.ldx;
 }
 
+// (Callers have that room up to 64 rows or more, see gemm_workspace_bytes.)
+bool ring_gemm_in_place(const GemmArgs& a) {
+  return a.ws != nullptr && a.ws_bytes >= (int64_t)a.M * (a.epi == EPI_SWIGLU ? 2 * a.N : a.N) * 4 && shares_memory(a);
+}
+
 int launch_ring_gemm(const GemmArgs& a, const RingPlan& plan, hipStream_t stream) {
   const bool gated = a.epi == EPI_SWIGLU;
   // A product that overwrites its own input goes through the workspace also in one part: the tiles of the epilogue
-  // kernel would store while others still read.  (Callers have that room up to 64 rows, see gemm_workspace_bytes.)
-  const bool via_ws = a.ws != nullptr && a.ws_bytes >= (int64_t)a.M * (gated ? 2 * a.N : a.N) * 4 && in_place(a);
-  if (plan.ksplit == 1 && !via_ws) {
+  // kernel would store while others still read.
+  if (plan.ksplit == 1 && !ring_gemm_in_place(a)) {
     int rc = -1;
     switch (a.epi) {
       case EPI_NONE: rc = launch_epi<EPI_NONE>(a, plan.tile, stream); break;
