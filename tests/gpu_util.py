@@ -9,6 +9,13 @@ def scratch_for(params, n_model, dev):
     return torch.empty(ext.qkv_scratch_bytes(params, n_model), dtype=torch.uint8, device=dev)
 
 
+def projection_parts(n_model, S, Hq, Hkv, D, P, **kw):
+    """Parts of K that the plan of a call's Q/K/V projection has, from the room they take in the scratch buffer: that of
+    n_model = 64, one k tile, has one.  (A little less than the number where a shorter call decides the other size.)"""
+    size = lambda n: ext.qkv_scratch_bytes(ext.attn_params(Hq, Hkv, D, S, kv_prefix=P, **kw), n)
+    return (size(n_model) - size(64)) / (S * (Hq + 2 * Hkv) * D * 4)
+
+
 def run_qkv(t, dev, *, Hq, Hkv, D, P=0, scale=None, causal=True, prenorm=False, norm_weight=True, qknorm=False,
             eps=0.0, variant="vanilla", noise=None, seed=0, tau=1.0, want_lse=False, mean_var=False,
             keep_scratch=False):

@@ -8,8 +8,9 @@ import pytest
 import torch
 
 import oracle
+from gpu_util import projection_parts
 from trinity_amd import ext
-from util import assert_close, attn_inputs, ffn_inputs, gen
+from util import assert_close, attn_inputs, ffn_inputs, gen, proj_std
 
 pytestmark = pytest.mark.gpu
 BF = torch.bfloat16
@@ -38,7 +39,7 @@ def test_rmsnorm_bf16(dev):
         assert_close(y, oracle.rmsnorm(xx, w, 1e-5, out_dtype=BF), 1e-2, 1e-2, "rmsnorm bf16 %d rows" % rows)
 
 
-@pytest.mark.parametrize("T,N,F", [(300, 512, 1088), (16, 512, 1088), (2048, 512, 4544)])
+@pytest.mark.parametrize("T,N,F", [(300, 512, 1088), (16, 512, 1088), (16, 2048, 2176), (2048, 512, 4544)])  # (the third: in parts)
 def test_ffn_bf16(dev, T, N, F):
     t = _bf(ffn_inputs(T, N, F, w_std=0.05))
     d = {k: v.to(dev) for k, v in t.items()}
@@ -62,9 +63,11 @@ CASES = [
     # S,  N,   Hq, Hkv, D,  P,  causal
     (192, 256, 4, 2, 128, 0, True),
     (200, 256, 4, 4, 64, 0, True),
-    (16, 256, 4, 4, 64, 300, False),     # few-token regime: split-K projection, key-split attention
+    (16, 256, 4, 4, 64, 300, False),     # few-token regime: key-split attention
+    (16, 4544, 4, 4, 64, 300, False),    # ... which sums the parts of the projection itself
     (40, 256, 2, 2, 128, 70, True),
-    (16, 128, 4, 2, 128, 300, True),     # few tokens, head dimension 128: the projection's own merge kernel
+    (16, 128, 4, 2, 128, 300, True),     # few tokens, head dimension 128
+    (16, 4096, 4, 2, 128, 300, True),    # ... with a projection in parts and its merge kernel
     (16, 128, 4, 2, 128, 4200, True),    # long prefix: the looping key-split kernel, heads stacked
     (20, 128, 6, 1, 64, 2500, False),
 ]
@@ -102,7 +105,9 @@ def _run(t, dev, variant, Hq, Hkv, D, P, scale, causal, **kw):
 @pytest.mark.parametrize("variant,prenorm,qknorm", [("vanilla", False, False), ("vanilla", True, False), ("vanilla", False, True),
                                                      ("roco", False, False), ("keyformer", False, False)])
 def test_attention_bf16(dev, S, N, Hq, Hkv, D, P, causal, variant, prenorm, qknorm):
-    t = _bf(attn_inputs(S, N, Hq, Hkv, D, P=P, w_std=0.06))
+    if N > 320:
+        assert projection_parts(N, S, Hq, Hkv, D, P, qknorm=qknorm) > 1
+    t = _bf(attn_inputs(S, N, Hq, Hkv, D, P=P, w_std=proj_std(N)))
     scale = 1.0 / math.sqrt(D)
     want = oracle.qkv_attention(t["x"], t["wq"], t["wk"], t["wv"], n_q_heads=Hq, n_kv_heads=Hkv, head_dim=D, scale=scale,
                                 causal=causal, kv_prefix=P, k_cache=t.get("k_cache"), v_cache=t.get("v_cache"),

@@ -11,10 +11,10 @@ import pytest
 import torch
 
 import oracle
-from gpu_util import scratch_for
+from gpu_util import projection_parts, scratch_for
 from test_gpu_attention import assert_scores
 from trinity_amd import ext
-from util import assert_close, attn_inputs, gen
+from util import assert_close, attn_inputs, proj_std
 
 pytestmark = pytest.mark.gpu
 F8 = torch.float8_e4m3fn
@@ -22,7 +22,7 @@ K_SCALE, V_SCALE = 0.04, 0.015
 
 
 def _fp8_inputs(S, N, Hq, Hkv, D, P, dtype=torch.float16):
-    t = attn_inputs(S, N, Hq, Hkv, D, P=P, w_std=0.06, with_cache=True)
+    t = attn_inputs(S, N, Hq, Hkv, D, P=P, w_std=proj_std(N), with_cache=True)
     t = {k: (v.to(dtype) if v.dtype == torch.float16 else v) for k, v in t.items()}
     kc = (t["k_cache"].float() / K_SCALE).clamp(-448, 448).to(F8)
     vc = (t["v_cache"].float() / V_SCALE).clamp(-448, 448).to(F8)
@@ -77,11 +77,22 @@ CASES = [
     (16, 128, 4, 2, 128, 4200, True),    # long prefix: the looping key-split kernel converts the fp8 tiles itself
     (20, 128, 6, 1, 64, 3001, False),    # ... 120 stacked rows, ragged last tile
 ]
+# models so wide that the projection runs in parts: their merge converts and appends the new rows
+PARTS = [
+    (16, 4096, 4, 2, 128, 300, True),
+    (3, 4544, 6, 1, 64, 70, False),
+    (1, 4096, 4, 4, 128, 0, True),
+    (16, 4096, 4, 2, 128, 4200, True),   # ... in front of the looping key-split kernel
+    (40, 4096, 2, 2, 128, 70, True),     # ... and of the 16-bit copy
+    (200, 4544, 5, 1, 64, 33, True),
+]
 
 
-@pytest.mark.parametrize("S,N,Hq,Hkv,D,P,causal", CASES)
+@pytest.mark.parametrize("S,N,Hq,Hkv,D,P,causal", CASES + PARTS)
 @pytest.mark.parametrize("qknorm", [False, True])
 def test_fp8_cache_vanilla(dev, S, N, Hq, Hkv, D, P, causal, qknorm):
+    if N > 320:
+        assert projection_parts(N, S, Hq, Hkv, D, P, qknorm=qknorm, kv_fp8=True, k_scale=K_SCALE, v_scale=V_SCALE) > 1
     t = _fp8_inputs(S, N, Hq, Hkv, D, P)
     kw = dict(n_q_heads=Hq, n_kv_heads=Hkv, head_dim=D, scale=1 / math.sqrt(D), causal=causal, kv_prefix=P,
               k_cache=t["k_cache"], v_cache=t["v_cache"], kv_fp8=True, k_scale=K_SCALE, v_scale=V_SCALE)
@@ -94,7 +105,7 @@ def test_fp8_cache_vanilla(dev, S, N, Hq, Hkv, D, P, causal, qknorm):
     assert_close(got["O2"], want["O2"], 1e-2, 1e-2, "O2")
 
 
-@pytest.mark.parametrize("S,N,Hq,Hkv,D,P,causal", [CASES[0], CASES[2], CASES[4], CASES[6]])
+@pytest.mark.parametrize("S,N,Hq,Hkv,D,P,causal", [CASES[0], CASES[2], CASES[4], CASES[6], PARTS[0], PARTS[5]])
 def test_fp8_cache_scores(dev, S, N, Hq, Hkv, D, P, causal):
     t = _fp8_inputs(S, N, Hq, Hkv, D, P)
     kw = dict(n_q_heads=Hq, n_kv_heads=Hkv, head_dim=D, scale=1 / math.sqrt(D), causal=causal, kv_prefix=P,
@@ -117,8 +128,9 @@ def test_fp8_cache_scores(dev, S, N, Hq, Hkv, D, P, causal):
     assert_scores(got["score"], want["score"], "score")
 
 
-def test_fp8_cache_bf16_elements(dev):
-    S, N, Hq, Hkv, D, P = 16, 256, 4, 2, 128, 300
+@pytest.mark.parametrize("N", [256, 4096])
+def test_fp8_cache_bf16_elements(dev, N):
+    S, Hq, Hkv, D, P = 16, 4, 2, 128, 300
     t = _fp8_inputs(S, N, Hq, Hkv, D, P, dtype=torch.bfloat16)
     want = oracle.qkv_attention(t["x"], t["wq"], t["wk"], t["wv"], n_q_heads=Hq, n_kv_heads=Hkv, head_dim=D,
                                 scale=1 / math.sqrt(D), causal=False, kv_prefix=P, k_cache=t["k_cache"],

@@ -9,9 +9,9 @@ import pytest
 import torch
 
 import oracle
-from gpu_util import run_qkv
+from gpu_util import projection_parts, run_qkv
 from test_gpu_attention import assert_scores
-from util import assert_close, attn_inputs
+from util import assert_close, attn_inputs, proj_std
 
 pytestmark = pytest.mark.gpu
 RTOL = ATOL = 1e-2
@@ -26,6 +26,20 @@ def _draw(seed):
     S = r.randint(1, 32) if few else r.randint(33, 300)
     P = r.choice([0, 0, r.randint(1, 700)]) if few else r.choice([0, 0, r.randint(1, 200)])
     N = 8 * r.randint(8, 40)
+    causal = r.random() < 0.6
+    return S, N, Hq, Hkv, D, P, causal
+
+
+def _draw_parts(seed):
+    """Few new tokens of a model so wide that the projection runs in parts of K: the merge kernel of their q/k/v rows
+    (128-wide heads) or the attention kernel (64-wide ones) sums them."""
+    r = random.Random(seed)
+    D = r.choice([64, 128])
+    Hkv = r.choice([1, 2, 3])
+    Hq = Hkv * r.choice([1, 2, 4])
+    S = r.randint(1, 32)
+    P = r.choice([0, r.randint(1, 700)])
+    N = 32 * r.randint(64, 142)
     causal = r.random() < 0.6
     return S, N, Hq, Hkv, D, P, causal
 
@@ -59,6 +73,13 @@ def _draw_prefill(seed, lo, hi):
 @pytest.mark.parametrize("seed", range(24))
 def test_random_shape_all_variants(dev, seed):
     _check_all_variants(dev, seed, _draw(seed))
+
+
+@pytest.mark.parametrize("seed", range(100, 110))
+def test_random_parts_all_variants(dev, seed):
+    cfg = _draw_parts(seed)
+    assert projection_parts(cfg[1], cfg[0], *cfg[2:6]) > 1
+    _check_all_variants(dev, seed, cfg)
 
 
 @pytest.mark.parametrize("seed,lo,hi", [(2000 + i, 129, 900) for i in range(8)] + [(4000 + i, 900, 2600) for i in range(4)] +
@@ -134,7 +155,7 @@ def _check_all_variants(dev, seed, cfg):
     S, N, Hq, Hkv, D, P, causal = cfg
     r = random.Random(1000 + seed)
     prenorm, qknorm = r.random() < 0.4, r.random() < 0.4
-    t = attn_inputs(S, N, Hq, Hkv, D, P=P, w_std=0.06)
+    t = attn_inputs(S, N, Hq, Hkv, D, P=P, w_std=proj_std(N))
     scale = 1.0 / math.sqrt(D)
     kw = dict(n_q_heads=Hq, n_kv_heads=Hkv, head_dim=D, scale=scale, causal=causal, kv_prefix=P,
               k_cache=t.get("k_cache"), v_cache=t.get("v_cache"))
@@ -179,7 +200,7 @@ def _draw_ffn(seed):
     T = {"few": r.randint(1, 64), "mid": r.randint(65, 300), "many": r.randint(301, 1100)}[kind]
     N = 8 * r.randint(4, 96)
     F = 8 * r.randint(4, 200)
-    if r.random() < 0.5:  # multiples of 32 in the reduction dimension open the split-K paths
+    if r.random() < 0.5:  # multiples of 32 in the reduction dimension: the direct-to-LDS kernels
         N, F = 32 * max(N // 32, 1), 32 * max(F // 32, 1)
     return T, N, F
 

@@ -219,41 +219,53 @@ def _ws(dev, nbytes):
     return torch.zeros(max(nbytes, 16), dtype=torch.uint8, device=dev)
 
 
-@pytest.mark.parametrize("T,N,F,N2", [
-    (16, 512, 1088, 512),       # the reference's token count; F not a multiple of the 128-column slab
-    (1, 64, 64, 64),
-    (33, 4544, 1024, 4544),     # Falcon width, second row tile partly filled
-    (64, 256, 2048, 256),       # the largest few-row case
+def _within_a_rounding(got, want, what):
+    """fp16 results of fp32 sums against the same product in fp32: one rounding (2^-11 of the value, four times that
+    allowed) and the order of the sums."""
+    assert ((got.float() - want).abs() <= 2.0 ** -9 * want.abs() + 1e-4).all(), what
+
+
+@pytest.mark.parametrize("T,N,F,N2,parts", [
+    (16, 512, 1088, 512, False),       # the reference's token count; F not a multiple of the tiles' columns
+    (1, 64, 64, 64, False),
+    (33, 4544, 1024, 4544, False),     # Falcon width, second row tile partly filled; its second product in one part
+    (64, 256, 2048, 256, False),
+    (16, 2048, 2176, 512, True),       # every product deep enough to run in parts
+    (1, 2048, 3072, 72, True),
+    (33, 4544, 2048, 4544, True),
+    (64, 2080, 2048, 264, True),       # (half a k tile at the end)
 ])
-def test_ffn_few_rows_split_k_parity(dev, T, N, F, N2):
-    """With a workspace the few-row (split-K) kernels run; they must agree with the oracle and with the
-    large-tile kernels (no workspace)."""
+def test_ffn_few_rows_split_k_parity(dev, T, N, F, N2, parts):
+    """With a workspace products over a deep K run in parts, without one in one part; both must agree with the oracle
+    and with fp32 products of the same operands."""
     t = ffn_inputs(T, N, F, N2, w_std=0.05)
     d = {k: v.to(dev) for k, v in t.items()}
     nbytes = ext.ffn_workspace_bytes(T, N, F)
     assert nbytes > 0
-    ws = _ws(dev, nbytes)
+    if parts:
+        for k, cols in ((N, 2 * F), (N, F), (F, N2)):
+            assert ext.gemm_workspace_bytes(T, k, cols) >= 2 * T * cols * 4
+    a32 = d["x"].float() @ d["w1"].float()
     for act in ("swiglu", "gelu"):
-        hid, out = (torch.zeros(T, F, dtype=torch.float16, device=dev), torch.zeros(T, N2, dtype=torch.float16, device=dev))
-        hid0, out0 = torch.zeros_like(hid), torch.zeros_like(out)
         if act == "swiglu":
             want, want_h = oracle.ffn_swiglu(t["x"], t["w1"], t["w_up"], t["w2"])
-            ext.ffn_swiglu(d["x"], d["w1"], d["w_up"], d["w2"], hid, out, workspace=ws)
-            ext.ffn_swiglu(d["x"], d["w1"], d["w_up"], d["w2"], hid0, out0)
+            h32 = a32 * torch.sigmoid(a32) * (d["x"].float() @ d["w_up"].float())
         else:
             want, want_h = oracle.ffn_gelu(t["x"], t["w1"], t["w2"])
-            ext.ffn_gelu(d["x"], d["w1"], d["w2"], hid, out, workspace=ws)
-            ext.ffn_gelu(d["x"], d["w1"], d["w2"], hid0, out0)
-        torch.cuda.synchronize()
-        assert_close(hid, want_h, RTOL, ATOL, act + " hidden")
-        assert_close(out, want, RTOL, ATOL, act + " out")
-        assert_close(hid, hid0.cpu(), 2e-3, 2e-3, act + " hidden vs large tiles")
-    # a workspace that is too small silently selects the large-tile kernels
-    small = _ws(dev, 64)
-    out1 = torch.zeros(T, N2, dtype=torch.float16, device=dev)
-    ext.ffn_gelu(d["x"], d["w1"], d["w2"], hid, out1, workspace=small)
-    torch.cuda.synchronize()
-    assert_close(out1, want, RTOL, ATOL, "gelu out, small workspace")
+            h32 = torch.nn.functional.gelu(a32)
+        # (a workspace that is too small is as good as none)
+        for ws in (_ws(dev, max(nbytes, ext.gemm_workspace_bytes(T, F, N2))), None, _ws(dev, 64)):
+            hid = torch.zeros(T, F, dtype=torch.float16, device=dev)
+            out = torch.zeros(T, N2, dtype=torch.float16, device=dev)
+            if act == "swiglu":
+                ext.ffn_swiglu(d["x"], d["w1"], d["w_up"], d["w2"], hid, out, workspace=ws)
+            else:
+                ext.ffn_gelu(d["x"], d["w1"], d["w2"], hid, out, workspace=ws)
+            torch.cuda.synchronize()
+            assert_close(hid, want_h, RTOL, ATOL, act + " hidden")
+            assert_close(out, want, RTOL, ATOL, act + " out")
+            _within_a_rounding(hid, h32, act + " hidden")
+            _within_a_rounding(out, hid.float() @ d["w2"].float(), act + " out")
 
 
 def test_matmul_residual_and_rowscale_few_rows(dev):
@@ -310,7 +322,7 @@ def test_activation_functions_pointwise(dev):
     out = torch.zeros(T, N, dtype=torch.float16, device=dev)
     xd = x.to(dev)
     a = x.double()[:, : N - 1]
-    for ws in (None, _ws(dev, ext.ffn_workspace_bytes(T, N, N))):                     # T > 64: both use the large tiles
+    for ws in (None, _ws(dev, ext.ffn_workspace_bytes(T, N, N))):                     # 512 rows; one k tile is not cut into parts
         ext.ffn_gelu(xd, eye.to(dev), eye.to(dev), hid, out, workspace=ws)
         torch.cuda.synchronize()
         want = (0.5 * a * (1 + torch.erf(a / math.sqrt(2.0)))).half()
@@ -323,7 +335,7 @@ def test_activation_functions_pointwise(dev):
         got = hid.cpu()[:, : N - 1]
         ulp = torch.maximum(want.abs().float() * 2 ** -10, torch.tensor(2.0 ** -24))
         assert ((got.float() - want.float()).abs() <= ulp).all(), "silu"
-    # the few-row kernels share the functions
+    # tiles of 32 rows share the functions
     ws = _ws(dev, ext.ffn_workspace_bytes(16, N, N))
     ext.ffn_gelu(xd[:16], eye.to(dev), eye.to(dev), hid[:16], out[:16], workspace=ws)
     torch.cuda.synchronize()
@@ -348,9 +360,11 @@ def test_large_split_k_ragged_shape_with_residual(dev):
 @pytest.mark.parametrize("M,K,N", [
     (2048, 1024, 4544),   # 256 x 160 tiles (17.75 column tiles of 256 fill the chip badly)
     (2048, 512, 6144),    # 256 x 192 tiles
-    (1024, 512, 6144),    # 256 x 96 tiles
+    (1200, 512, 4096),    # 256 x 96 tiles
+    (1101, 512, 4104),    # ... the fewest rows that come here, a ragged last row block and column tile
     (2048, 512, 18176),   # full rounds of 256 x 256 tiles plus a narrower remainder
-    (1000, 512, 4672),    # ragged rows and a ragged last column tile
+    (1024, 512, 6144),    # 128 x 192 tiles (ring.hip)
+    (1000, 512, 4672),    # ... ragged rows and a ragged last column tile
 ])
 def test_matmul_tile_plan_family(dev, M, K, N):
     """Shapes that make the launcher pick each second tile shape of its plan family."""

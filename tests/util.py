@@ -15,6 +15,11 @@ def randn(g, *shape, std=1.0, mean=0.0):
     return (torch.randn(*shape, generator=g) * std + mean).to(torch.float16)
 
 
+def proj_std(N):
+    """Weight scale of the attention tests: projected values of order one also where the model is wide."""
+    return 0.06 if N <= 320 else 0.96 * N ** -0.5
+
+
 def attn_inputs(S, N, Hq, Hkv, D, P=0, seed=42, x_std=1.0, w_std=0.02, cache_std=1.0, with_cache=None):
     g = gen(seed)
     t = {
