@@ -1078,9 +1078,12 @@ static int launch_attn_kf(const AttnArgs& a, int kf, hipStream_t stream) {
 // Workgroups aimed at (eight waves per CU) and the most runs the key axis is cut into: every run adds a partial result
 // per (head, token) that the merge kernel reads, eight runs per round trip.  16 tokens, 32768 keys: Llama-3-8B's 8 KV
 // heads 55.1 us for the whole block with 64 runs, 51.3 with 32; 32 KV heads want the 512 workgroups (9000 keys 54.0 us,
-// 55.3 with 256).  One or two workgroups per run leave the chip so idle that 64 runs pay (71 heads on one KV head, one
-// token, 30000 fp8 keys 33.4 -> 29.2 us).  A run has at least four tiles, or two where its partial result is small
-// (one token: 2500 keys, 71 heads 21.5 -> 20.2 us, 4096 keys, 32 heads 23.5 -> 23.0; 16 tokens, 4000 keys 26.3 -> 27.0).
+// 55.3 with 256).  One or two workgroups per run leave the chip so idle that 64 runs pay from some 10000 keys on (71 heads
+// on one KV head, 6000 / 16000 / 32000 keys: one token 20.2 -> 20.7, 24.2 -> 22.5, 30.7 -> 25.9 us, two tokens 21.6 -> 22.1,
+// 25.8 -> 24.4, 31.7 -> 27.7); with three (4 tokens) 10000 keys are slower, 24.1 -> 25.3, 16000 level, 32000 faster,
+// 32.1 -> 28.6.  A run has at least four tiles, or two where its partial result is small: that pays below 6000 keys (8 KV
+// heads, 2100 / 4000 keys: one token 23.5 -> 22.2, 23.9 -> 23.3, four 23.8 -> 22.9, 24.3 -> 24.1, eight 24.4 -> 23.7 but
+// 25.3 -> 25.7; 71 heads on one: one token 20.7 -> 19.2, 20.6 -> 19.3; 16 tokens, 4000 keys 26.3 -> 27.0).
 constexpr int kSplitTargetWorkgroups = 512;
 constexpr int kSplitMaxRuns = 32, kSplitMaxRunsFew = 64, kSplitFewBase = 2;
 constexpr int kSplitMinTiles = 4, kSplitMinTilesDecode = 2, kSplitDecodeTokens = 4;
@@ -1104,9 +1107,10 @@ static int launch_attn_split_t(const AttnArgs& a, int nwg, hipStream_t stream) {
     if (a.S > kFewMaxQueries) return launch_attn_split_h<D, KF, FP8, 1, 2>(a, nwg, stream);
   if ((a.Hq / a.Hkv) * a.S <= kSplitHalvesRows) return launch_attn_split_h<D, KF, FP8, 2, 1>(a, nwg, stream);
   // fp8 with whole tiles per wave keeps one tile on its way: where a CU has one workgroup at most and a long run to walk,
-  // eight waves on pairs of tiles keep two (Llama-3-8B heads, 28 tokens against 32000 keys 48.0 -> 45.1 us for the whole
-  // block; 71 heads on one, one token against 30000 keys, 7 tiles a run, 27.1 -> 26.3; three against 20000, 4.9 tiles,
-  // 26.1 -> 26.5; 16-bit tiles, which do not pass through registers, 53.5 -> 54.9 for the first of these)
+  // eight waves on pairs of tiles keep two: from seven tiles a run (whole calls at some 4.5, 6 and 8 tiles a run: 71 heads
+  // on one, one token 23.8 -> 24.2, 25.6 level, 26.4 -> 25.7 us, 4 tokens 24.1 -> 24.8, 25.1 -> 24.9, 26.9 -> 26.4;
+  // Llama-3-8B heads, 24 tokens 35.0 -> 35.8, 34.8 level, 36.9 -> 36.2, 32 tokens 37.1 -> 38.7, 37.6 -> 38.1, 40.0 -> 39.6;
+  // 28 against 32000 keys, 16 tiles, 48.0 -> 45.1; 16-bit tiles, which do not pass through registers, 53.5 -> 54.9 there)
   if constexpr (FP8)
     if (nwg <= kSplitPairWorkgroups && (a.P + a.S) / kKeyTile >= kSplitPairTiles * a.split_runs)
       return launch_attn_split_h<D, KF, FP8, 1, 2>(a, nwg, stream);
