@@ -114,6 +114,13 @@ def test_few_rows_get_the_room_to_work_in_place(M, K, N):
     assert ext.gemm_workspace_bytes(M, K, N) >= M * N * 4
 
 
+@pytest.mark.skipif(torch.cuda.is_available(), reason="a GPU is visible")
+def test_one_row_of_stride_zero_in_place_reaches_the_launch():
+    x, w = torch.empty(512, dtype=torch.float16).as_strided((1, 512), (0, 1)), _host(512, 512)
+    ws = _host(ext.gemm_workspace_bytes(1, 512, 512), dtype=torch.uint8)
+    assert ext.native().matmul(x, w, None, x, ws, 0) == -8  # (there is no device to launch on)
+
+
 @pytest.mark.parametrize("longest", [64, 128, 512, 1024, 2048])
 @pytest.mark.parametrize("P", [0, 1000, 4096])
 @pytest.mark.parametrize("Hq,Hkv,D,N", [(71, 1, 64, 4544), (32, 8, 128, 4096)])

@@ -79,6 +79,17 @@ def test_few_rows_in_place(rn, M, N):
     check(buf, torch.cat([x.float(), a], 1), "side by side")
 
 
+@pytest.mark.parametrize("stride", [0, 8, 512])
+def test_one_row_of_any_stride_in_place(rn, stride):
+    """A single row's stride means nothing: zero, or less than the row, as a view may have it."""
+    x, w = rn(1, 512), rn(512, 512, std=512 ** -0.5)
+    want = x.float() @ w.float()
+    ws = torch.empty(ext.gemm_workspace_bytes(1, 512, 512), dtype=torch.uint8, device="cuda:0")
+    t = x.as_strided((1, 512), (stride, 1))
+    ext.matmul(t, w, None, t, workspace=ws)
+    check(t, want, "in place")
+
+
 @pytest.mark.parametrize("S,N,Hq,Hkv,D", [
     (1, 64, 4, 4, 64), (33, 96, 5, 1, 128), (100, 4096, 32, 8, 128), (260, 4096, 32, 8, 128), (200, 4544, 71, 1, 64),
     (700, 128, 32, 8, 128), (1000, 128, 71, 1, 64), (1100, 160, 32, 4, 128),  # a tile across two weight matrices

@@ -339,7 +339,7 @@ RingPlan ring_plan(int M, int K, int ncols, int unit, int min_bn, int64_t ws_byt
 static bool shares_memory(const GemmArgs& a) {
   const half_t *xend = a.x + (a.M - 1) * a.ldx + a.K, *oend = a.out + (a.M - 1) * a.ldo + a.N;
   if (oend <= a.x || xend <= a.out) return false;
-  if (a.ldx != a.ldo) return true;
+  if (a.M == 1 || a.ldx != a.ldo) return true;  // (the stride of a single row may be anything, zero too)
   const int64_t d = ((a.out - a.x) % a.ldx + a.ldx) % a.ldx;
   return d < a.K || d + a.N > a.ldx;
 }
