@@ -36,13 +36,13 @@ CASES = [
     (1, 128, 2, 1, 64, 0, True),
 ]
 
-# few new tokens against a long cached prefix: the key-split kernels and the split-K projection
+# few new tokens against a long cached prefix: the key-split kernels (projections in parts: test_gpu_random_shapes.py)
 FEW_CASES = [
     (16, 256, 4, 2, 128, 1024, False),   # the reference's regime, several key splits
     (32, 256, 2, 2, 64, 500, True),      # most queries the few-query path takes; causal over a prefix
     (5, 128, 2, 1, 64, 253, True),       # ragged: P + S not a multiple of four (noise rows unaligned)
     (16, 128, 3, 3, 128, 300, False),
-    (20, 128, 4, 2, 64, 0, True),        # no caches: the merged k / v rows go to the scratch buffer; GQA
+    (20, 128, 4, 2, 64, 0, True),        # no caches: the new k / v rows go to the scratch buffer; GQA
     (32, 128, 6, 2, 128, 255, False),    # the first new key is the last key of a split
     (16, 128, 2, 2, 64, 2000, True),     # the longest prefix the one-tile-per-wave kernel still takes
 ]

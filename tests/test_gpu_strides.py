@@ -7,9 +7,9 @@ import pytest
 import torch
 
 import oracle
-from gpu_util import scratch_for
+from gpu_util import projection_parts, scratch_for
 from trinity_amd import ext
-from util import assert_close, attn_inputs, ffn_inputs
+from util import assert_close, attn_inputs, ffn_inputs, proj_std
 
 pytestmark = pytest.mark.gpu
 RTOL = ATOL = 1e-2
@@ -58,11 +58,15 @@ def test_ffn_strided(dev, T, N, F, with_ws):
 
 @pytest.mark.parametrize("S,N,Hq,Hkv,D,P,causal", [
     (150, 256, 4, 2, 128, 40, True),     # many tokens
-    (16, 256, 4, 4, 64, 300, False),     # few tokens: split-K projection, key-split attention
+    (16, 256, 4, 4, 64, 300, False),     # few tokens: key-split attention
+    (16, 4544, 4, 4, 64, 300, False),    # ... which sums the parts of the projection and stores the new rows
+    (16, 4096, 4, 2, 128, 300, True),    # ... with a projection in parts and its merge kernel
 ])
 @pytest.mark.parametrize("variant", ["vanilla", "roco", "keyformer"])
 def test_attention_strided(dev, S, N, Hq, Hkv, D, P, causal, variant):
-    t = attn_inputs(S, N, Hq, Hkv, D, P=P, w_std=0.06)
+    if N > 256:
+        assert projection_parts(N, S, Hq, Hkv, D, P) > 1
+    t = attn_inputs(S, N, Hq, Hkv, D, P=P, w_std=proj_std(N))
     x, xb = _wide(t["x"], dev)
     wq, _ = _wide(t["wq"], dev)
     wk, _ = _wide(t["wk"], dev)

@@ -33,7 +33,7 @@ def _both(dev, S, N, Hq, Hkv, D, P, causal, prenorm=False, qknorm=False, seed=1)
     return res
 
 
-# (many tokens: large tiles + prefill attention) then (few tokens: split-K projection + key-split attention), each
+# (many tokens: large tiles + prefill attention) then (few tokens: key-split attention), each
 # followed by a smaller call of the same kind that reuses the array
 CALLS = [
     dict(S=384, N=512, Hq=8, Hkv=2, D=128, P=64, causal=True),
