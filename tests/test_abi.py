@@ -138,6 +138,21 @@ def test_scratch_of_the_longest_call_serves_shorter_ones(Hq, Hkv, D, N, P, longe
             assert ext.qkv_attention(x[:s], None, wq, wk, wv, kc, vc, scratch, None, out[:s], p, validate_only=True) == 0, s
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,N", [(32, 32, 128, 4096), (71, 1, 64, 4544), (32, 8, 128, 4096)])
+@pytest.mark.parametrize("longest,P", [(33, 4096), (33, 2100), (64, 4096), (16, 4096)])
+def test_scratch_serves_shorter_prefixes(Hq, Hkv, D, N, longest, P):
+    """Fewer keys may be cut into more runs (32 KV heads: 16 for 64 tiles of keys, 13 for 65)."""
+    raw = torch.empty(ext.qkv_scratch_bytes(ext.attn_params(Hq, Hkv, D, longest, kv_prefix=P), N) + 256, dtype=torch.uint8)
+    lead = (-raw.data_ptr()) % 256
+    scratch = raw[lead:lead + raw.numel() - 256]
+    x, wq, wk, wv, out = _host(longest, N), _host(N, Hq * D), _host(N, Hkv * D), _host(N, Hkv * D), _host(longest, Hq * D)
+    kc, vc = _host(Hkv, P + longest, D), _host(Hkv, P + longest, D)
+    for prefix in range(0, P + 1, 50):
+        for s in {1, 5, 31, 32, longest} & set(range(longest + 1)):
+            p = ext.attn_params(Hq, Hkv, D, s, kv_prefix=prefix)
+            assert ext.qkv_attention(x[:s], None, wq, wk, wv, kc, vc, scratch, None, out[:s], p, validate_only=True) == 0, (s, prefix)
+
+
 def test_static_scratch_entry_point_checks_before_touching_the_gpu():
     """tri_qkv_attention_static refuses a call that does not fit its array, and any bad argument, on the host."""
     S, N, Hq, Hkv, D = 8192, 4096, 32, 8, 128

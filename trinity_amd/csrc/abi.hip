@@ -71,14 +71,16 @@ inline int64_t align256(int64_t x) { return (x + 255) & ~(int64_t)255; }
 
 // Partial results of the key-split attention of a call of S tokens, for every run the key axis would be cut into, for the
 // fewest, or what the call cannot do without: up to 32 tokens the attention kernels (the only ones that read fp8 rows)
-// always leave parts.
-enum AttnParts { kAllRuns, kFewestRuns, kNoRuns };
+// always leave parts (kNoRunsAnyPrefix: a bound of that over all prefixes up to the call's).
+enum AttnParts { kAllRuns, kFewestRuns, kNoRuns, kNoRunsAnyPrefix };
 int64_t attn_parts_bytes(const tri_attn_params* p, int S, AttnParts runs) {
   const int Hq = p->n_q_heads, Hkv = p->n_kv_heads, D = p->head_dim, L = p->kv_prefix + S;
-  if (runs == kNoRuns && S > tri::kFewMaxQueries) return 0;
-  const int64_t split = split_attn_workspace_bytes(S, Hq, Hkv, D, L, runs != kAllRuns);
+  if (runs >= kNoRuns && S > tri::kFewMaxQueries) return 0;
+  const bool fewest = runs == kFewestRuns || runs == kNoRuns;
+  const int64_t split = split_attn_workspace_bytes(S, Hq, Hkv, D, L, fewest);
   if (runs == kNoRuns && split > 0) return split;
-  const int64_t few = few_attn_workspace_bytes(S, Hq, D, L);
+  const bool no_few = runs == kNoRunsAnyPrefix && L >= tri::kSplitMinKeys;  // (the split kernel takes these keys)
+  const int64_t few = few_attn_workspace_bytes(S, Hq, D, no_few ? tri::kSplitMinKeys - 1 : L);
   return few > split ? few : split;
 }
 
@@ -479,9 +481,11 @@ int64_t tri_qkv_scratch_bytes(const tri_attn_params* p, int64_t n_model) {
   // The whole layout need not grow with the number of tokens (Falcon-7B heads: 33.8 MB at 512, 9.9 MB at 1000), nor does
   // what a call cannot do without (the parts of up to 32 tokens): a buffer made for the longest call of a program has to
   // serve its shorter ones.
+  // The same holds for shorter prefixes: the fewest runs are 13 for 65 tiles of keys and 16 for 64.
   int64_t bytes = scratch_layout(p, n_model, p->seq, INT64_MAX).total;
   for (int s = 1; s < p->seq && s <= 64; ++s) {
-    const int64_t least = scratch_least(p, n_model, s);
+    const int64_t here = attn_parts_bytes(p, s, kNoRuns), any = attn_parts_bytes(p, s, kNoRunsAnyPrefix);
+    const int64_t least = scratch_least(p, n_model, s) + (any > here ? align256(any) - align256(here) : 0);
     bytes = bytes > least ? bytes : least;
   }
   return bytes;
