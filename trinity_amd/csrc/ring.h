@@ -1,13 +1,13 @@
 // Main loop and tile family of the GEMMs with few and middling rows (1 to about 1000 tokens, more of narrow products over
-// a deep K), shared by ring.hip
-// (FFN products) and ring_qkv.hip (Q/K/V projection).
+// a deep K), shared by ring.hip (FFN products) and ring_qkv.hip (Q/K/V projection).
 //
-// What bounds them: streaming the weights once.  To keep 5 TB/s coming from HBM a CU needs some 60 KB of weights in
-// flight at any time, whatever else it does, so the LDS is one ring of NST stages, each holding a 64-deep k tile of
-// both operands, and a stage is requested again as soon as the barrier has freed it: NST - 1 tiles are always on
-// their way.  (The large-tile loop of gemm_core.h keeps its activations in two buffers and loads complete in order,
-// so its weights are never more than about one tile ahead: 64 rows x [4096, 28672] 59 us there and in the split-K
-// kernel, 44 us here = 5.3 TB/s; 128 rows 64 -> 51 us.)
+// What bounds them: streaming the weights once.  The LDS is one ring of NST stages, each holding a 64-deep k tile of both
+// operands, and a stage is requested again as soon as the barrier has freed it, so that NST - 1 tiles are on their way
+// whatever else a CU does.  (The large-tile loop of gemm_core.h keeps its activations in two buffers and loads complete in
+// order, so its weights are never more than about one tile ahead: 64 rows x [4096, 28672] 59 us there and in the split-K
+// kernel, 44 us here = 5.3 TB/s; 128 rows 64 -> 51 us.)  How many it takes was measured for 32 x 128 tiles with a CU to
+// themselves, 16 rows x [4096, 28672]: 32 KB of weights on their way per CU (three stages) 43.0 us, 48 KB (four, as built)
+// 44.5, 64 KB 44.7, 96 KB 45.2 - more than 32 KB buy nothing there.
 //
 // 64-deep k tiles: an activation row, and a K-contiguous weight column, is then read in whole 128-byte lines.
 // Both operands go global -> LDS without passing through registers (1 KB per wave instruction), XOR-swizzled by the
