@@ -114,6 +114,12 @@ def test_few_rows_get_the_room_to_work_in_place(M, K, N):
     assert ext.gemm_workspace_bytes(M, K, N) >= M * N * 4
 
 
+@pytest.mark.parametrize("M,K,F", [(16, 1024, 4096), (16, 2048, 5632), (48, 2048, 5632), (64, 3072, 8192)])
+def test_gated_products_of_few_row_blocks_run_in_parts(M, K, F):
+    """Whole columns leave most CUs without work, and one that has some streams no faster for it."""
+    assert ext.gemm_workspace_bytes(M, K, 2 * F) >= 2 * M * 2 * F * 4
+
+
 @pytest.mark.skipif(torch.cuda.is_available(), reason="a GPU is visible")
 def test_one_row_of_stride_zero_in_place_reaches_the_launch():
     x, w = torch.empty(512, dtype=torch.float16).as_strided((1, 512), (0, 1)), _host(512, 512)

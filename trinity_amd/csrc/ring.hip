@@ -287,6 +287,13 @@ static const RingCost kRingCost[kRingTiles] = {
     {128, 256, TRI_RING_PER_CU(128, 256, 3), 0.743f, 0.755f}, {160, 256, TRI_RING_PER_CU(160, 256, 3), 0.914f, 1.006f},
     {32, 128, TRI_RING_PER_CU(32, 128, 4), 0.264f, 0.222f}};
 constexpr int kRingTileOneBlock = 8;  // the non-temporal tile, for a single row block
+// Gate and up columns over row-major weights in one part: however few workgroups there are, one streams no faster than
+// about this many bytes per us (16 rows x [2048, 5632 x 2], 88 workgroups: 22.0 us, 16.0 in two parts; x [1024, 4096 x 2],
+// 64: 12.0 and 10.1 in four; the costs above, fitted where 200 and more workgroups share the memory's rate, say 14.9 and
+// 7.8).  Over 84 products of 1 to 100 rows and K of 512 to 8192 the plan picked is 1.3 % slower than the best of the
+// family with this bound and 4.5 % without.  Above 64 rows the costs hold as they are.
+constexpr float kRingGatedChainRate = 36e3f;
+constexpr int kRingGatedChainRows = 64;
 
 static RingPlan ring_plan_search(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes) {
   RingPlan best = {-1, 1, 1e30f};
@@ -307,7 +314,11 @@ static RingPlan ring_plan_search(int M, int K, int ncols, int unit, int min_bn, 
       last_per = per;
       const int wg = tiles * ks, share = (wg + 255) / 256;
       const float even = share == 1 ? 1.0f : sqrtf((float)wg / (256.0f * share));
-      const float mem = wbytes / (8e6f * even) + (ks > 1 ? ks * obytes : 0.5f * obytes) / 3e6f;
+      float mem = wbytes / (8e6f * even) + (ks > 1 ? ks * obytes : 0.5f * obytes) / 3e6f;
+      if (ks == 1 && share == 1 && min_bn > 0 && M <= kRingGatedChainRows) {
+        const float chain = per * c.bn * 128.0f / kRingGatedChainRate;
+        mem = mem > chain ? mem : chain;
+      }
       const float it = share == 1 ? c.alone : (c.alone > c.shared * share ? c.alone : c.shared * share);
       const float comp = per * it;
       const float loads = (float)wg * per * (c.bm + c.bn) * 128.0f / 37e6f;
