@@ -114,10 +114,19 @@ def test_few_rows_get_the_room_to_work_in_place(M, K, N):
     assert ext.gemm_workspace_bytes(M, K, N) >= M * N * 4
 
 
-@pytest.mark.parametrize("M,K,F", [(16, 1024, 4096), (16, 2048, 5632), (48, 2048, 5632), (64, 3072, 8192)])
+@pytest.mark.parametrize("M,K,F", [(16, 1024, 4096), (16, 2048, 5632), (48, 2048, 5632), (32, 3072, 8192)])
 def test_gated_products_of_few_row_blocks_run_in_parts(M, K, F):
     """Whole columns leave most CUs without work, and one that has some streams no faster for it."""
     assert ext.gemm_workspace_bytes(M, K, 2 * F) >= 2 * M * 2 * F * 4
+
+
+@pytest.mark.parametrize("S,N,Hq,Hkv,parts", [(1, 1024, 16, 4, True), (4, 1024, 16, 4, True), (4, 768, 12, 12, True),
+                                             (16, 2048, 32, 32, True), (32, 1024, 16, 4, False)])
+def test_projections_whose_parts_attention_sums(S, N, Hq, Hkv, parts):
+    """64-wide heads, short prefix: parts cost no launch, but every head's workgroups sum its rows again (fewer tokens,
+    more parts)."""
+    size = lambda n: ext.qkv_scratch_bytes(ext.attn_params(Hq, Hkv, 64, S, kv_prefix=100), n)
+    assert (size(N) >= size(64) + 2 * S * (Hq + 2 * Hkv) * 64 * 4) == parts
 
 
 @pytest.mark.skipif(torch.cuda.is_available(), reason="a GPU is visible")

@@ -75,6 +75,14 @@ def test_random_shape_all_variants(dev, seed):
     _check_all_variants(dev, seed, _draw(seed))
 
 
+@pytest.mark.parametrize("cfg", [(1, 1024, 16, 4, 64, 100, True), (4, 1024, 16, 4, 64, 300, False), (4, 768, 12, 12, 64, 1100, True),
+                                 (16, 2048, 32, 32, 64, 40, True)])
+def test_narrow_models_parts_summed_by_attention(dev, cfg):
+    """Narrow models: a few tokens' projection runs in parts because the attention kernel sums them at little cost."""
+    assert projection_parts(cfg[1], cfg[0], *cfg[2:6]) > 1
+    _check_all_variants(dev, 3, cfg)
+
+
 @pytest.mark.parametrize("seed", range(100, 110))
 def test_random_parts_all_variants(dev, seed):
     cfg = _draw_parts(seed)

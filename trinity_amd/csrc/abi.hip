@@ -84,6 +84,11 @@ int64_t attn_parts_bytes(const tri_attn_params* p, int S, AttnParts runs) {
   return few > split ? few : split;
 }
 
+// The few-token attention kernel sums the projection's parts itself (16-bit caches, 64-wide heads, short prefixes).
+inline bool attn_may_merge_proj(const tri_attn_params* p, int S) {
+  return !p->kv_fp8 && S <= tri::kFewMaxQueries && p->head_dim == 64 && p->kv_prefix + S < tri::kSplitMinKeys;
+}
+
 // 33 to 64 tokens: one part of the projection is asked for whether or not its plan has parts (without it this would be
 // the one range that needs less than its shorter calls, whose attention cannot do without parts).
 int64_t proj_part_bytes(const tri_attn_params* p, int64_t n_model, int64_t S) {
@@ -111,7 +116,8 @@ Scratch scratch_layout(const tri_attn_params* p, int64_t n_model, int64_t S, int
   // (separate: the attention kernel merges the projection's parts while it writes its own)
   s.ws_bytes = proj_part_bytes(p, n_model, S);
   if (left > 0) {
-    const int64_t parts = qkv_workspace_bytes((int)S, (int)n_model, (int)((Hq + 2 * Hkv) * D), p->qknorm ? (int)D : 1);
+    const int64_t parts = qkv_workspace_bytes((int)S, (int)n_model, (int)((Hq + 2 * Hkv) * D), p->qknorm ? (int)D : 1,
+                                              attn_may_merge_proj(p, (int)S));
     s.ws_bytes = parts > s.ws_bytes ? parts : s.ws_bytes;
   }
   s.aws_bytes = attn_parts_bytes(p, (int)S, kAllRuns);

@@ -398,8 +398,9 @@ static float plan_us(const TilePlan& p, int K) { return 6.0f + 0.0272f * (float)
 // over, by a quarter: 14336 -> 1024, 2048 rows 162 -> 70 us (0.39 by the costs), 14336 -> 4096, 1200 rows 187 -> 142
 // (0.74), but 4096 rows of 4096 -> 1024 43.0 -> 45.8 (0.76), 3072 of 14336 -> 4096 310 -> 370 (0.86).
 constexpr float kRingMarginNarrow = 0.75f;
-static bool ring_wins(float big_us, int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes, RingPlan& plan) {
-  plan = ring_plan(M, K, ncols, unit, min_bn, ws_bytes);
+static bool ring_wins(float big_us, int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes, RingPlan& plan,
+                      float merge_us = kRingMergeUs) {
+  plan = ring_plan(M, K, ncols, unit, min_bn, ws_bytes, merge_us);
   return plan.tile >= 0 && plan.us < (M <= kRingMaxRows ? big_us : kRingMarginNarrow * big_us);
 }
 
@@ -431,8 +432,8 @@ static TilePlan big_plan(int M, int N, int epi, bool kcontig) {
 constexpr int kGatedMinBn = 128;
 
 // workspace of the best plan, if it has at least `least` parts (0 otherwise)
-static int64_t plan_workspace_bytes(int M, int K, int ncols, int unit, int min_bn, int least) {
-  const RingPlan plan = ring_plan(M, K, ncols, unit, min_bn, INT64_MAX);
+static int64_t plan_workspace_bytes(int M, int K, int ncols, int unit, int min_bn, int least, float merge_us = kRingMergeUs) {
+  const RingPlan plan = ring_plan(M, K, ncols, unit, min_bn, INT64_MAX, merge_us);
   return plan.tile < 0 || plan.ksplit < least ? 0 : (int64_t)plan.ksplit * M * ncols * 4;
 }
 
@@ -551,8 +552,13 @@ static int launch_qkv_d(const QkvProjArgs& a, hipStream_t stream) {
   }
 }
 
-int64_t qkv_workspace_bytes(int S, int K, int ncols, int unit) {
-  return S > kRingMaxRows ? 0 : plan_workspace_bytes(S, K, ncols, unit, 0, 2);
+// What it costs the attention kernel to merge the projection's parts itself: no launch, but each workgroup sums the rows
+// of its own head again.  One part is 1.1 to 2.3 us slower than four for one to four tokens (16 heads on 4, 1024 columns),
+// 0.3 faster to 0.7 slower for 16, 2.9 to 3.8 faster for 32.
+static float deferred_merge_us(int S) { return 1.2f + 0.12f * (float)S; }
+
+int64_t qkv_workspace_bytes(int S, int K, int ncols, int unit, bool deferred) {
+  return S > kRingMaxRows ? 0 : plan_workspace_bytes(S, K, ncols, unit, 0, 2, deferred ? deferred_merge_us(S) : kRingMergeUs);
 }
 
 int launch_qkv_proj(const QkvProjArgs& a, hipStream_t stream, int* deferred_ksplit, bool* appended) {
@@ -567,7 +573,8 @@ int launch_qkv_proj(const QkvProjArgs& a, hipStream_t stream, int* deferred_kspl
   // (its weights are small enough to come from the Infinity Cache when the caller uses them again: the large tiles
   // are then a tenth faster than over weights from HBM, the ring kernels hardly - 658 to 1000 rows, both within 2 %)
   if (a.S <= kRingMaxRows &&
-      ring_wins(0.9f * plan_us(big, a.K), a.S, a.K, ncols, a.qknorm ? a.D : 1, 0, a.ws != nullptr ? a.ws_bytes : 0, plan))
+      ring_wins(0.9f * plan_us(big, a.K), a.S, a.K, ncols, a.qknorm ? a.D : 1, 0, a.ws != nullptr ? a.ws_bytes : 0, plan,
+                deferred_ksplit != nullptr ? deferred_merge_us(a.S) : kRingMergeUs))
     return launch_ring_qkv(a, plan, stream, deferred_ksplit, appended);
   return a.D == 128 ? launch_qkv_d<128>(a, stream) : launch_qkv_d<64>(a, stream);
 }

@@ -97,13 +97,15 @@ constexpr int kRingMaxRows = 1100;  // the range that the cost model was fitted 
 constexpr int kRingMaxRowsNarrow = 8192, kRingMaxColsNarrow = 1 << 16, kRingMinKNarrow = 2048;
 // ncols: weight columns (gate and up, or q, k and v, together).  Tiles must be a multiple of `unit` wide (whole heads; 1
 // otherwise) and at least min_bn.  ws_bytes: fp32 workspace for partial results, ksplit * M * ncols * 4 bytes (1: none).
-RingPlan ring_plan(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes);
+// merge_us: what the merge of parts takes beside its bytes.
+constexpr float kRingMergeUs = 3.5f;
+RingPlan ring_plan(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes, float merge_us = kRingMergeUs);
 int launch_ring_gemm(const GemmArgs& a, const RingPlan& plan, hipStream_t stream);
 bool ring_gemm_in_place(const GemmArgs& a);  // out overlaps x, and the workspace holds the one part it takes to allow that
 // workspace that lets launch_gemm take its best plan for [M, K] x [K, ncols] (0: no plan in parts)
 int64_t gemm_workspace_bytes(int M, int K, int ncols);
-// the same for the Q/K/V projection; unit as in ring_plan
-int64_t qkv_workspace_bytes(int S, int K, int ncols, int unit);
+// the same for the Q/K/V projection; unit as in ring_plan; deferred: the attention kernel merges the parts
+int64_t qkv_workspace_bytes(int S, int K, int ncols, int unit, bool deferred);
 
 // [Q | K | V] = X . [Wq | Wk | Wv], optional per-head RMSNorm of Q and K,
 // scattered to q [S, Hq*D] and the head-major k/v buffers.

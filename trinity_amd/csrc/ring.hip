@@ -274,7 +274,7 @@ static int launch_epi(const GemmArgs& a, int tile, hipStream_t stream) {
 //             one more to stream - and what is written;
 //   compute   k tiles in a row on the busiest CU, by tile and by whether workgroups share a CU;
 //   loads     every byte that passes from L2 to LDS, at 37 TB/s over the chip;
-// and per wave of workgroups 2 us of first loads and epilogue.  Parts cost a merge: 3.5 us and their bytes at 6 TB/s.
+// and per wave of workgroups 2 us of first loads and epilogue.  Parts cost a merge: 3.5 us (kRingMergeUs) and their bytes at 6 TB/s.
 struct RingCost {
   int bm, bn, per_cu;   // per_cu: workgroups that fit a CU's LDS
   float alone, shared;  // us per k tile of a workgroup with a CU to itself / of each of several
@@ -287,15 +287,18 @@ static const RingCost kRingCost[kRingTiles] = {
     {128, 256, TRI_RING_PER_CU(128, 256, 3), 0.743f, 0.755f}, {160, 256, TRI_RING_PER_CU(160, 256, 3), 0.914f, 1.006f},
     {32, 128, TRI_RING_PER_CU(32, 128, 4), 0.264f, 0.222f}};
 constexpr int kRingTileOneBlock = 8;  // the non-temporal tile, for a single row block
-// Gate and up columns over row-major weights in one part: however few workgroups there are, one streams no faster than
-// about this many bytes per us (16 rows x [2048, 5632 x 2], 88 workgroups: 22.0 us, 16.0 in two parts; x [1024, 4096 x 2],
-// 64: 12.0 and 10.1 in four; the costs above, fitted where 200 and more workgroups share the memory's rate, say 14.9 and
-// 7.8).  Over 84 products of 1 to 100 rows and K of 512 to 8192 the plan picked is 1.3 % slower than the best of the
-// family with this bound and 4.5 % without.  Above 64 rows the costs hold as they are.
-constexpr float kRingGatedChainRate = 36e3f;
-constexpr int kRingGatedChainRows = 64;
+// A plan in one part on few workgroups: one streams no faster than about this many bytes of weights per us (16 rows x
+// [2048, 5632 x 2] as gate/up, 88 workgroups: 22.0 us, 16.0 in two parts; x [1024, 4096 x 2], 64: 12.0 and 10.1 in four; the
+// costs above, fitted where 200 and more workgroups share the memory's rate, say 14.9 and 7.8).  Up to 64 rows and 192
+// workgroups; beyond either the costs hold as they are (one row x K-contiguous [4096, 14336 x 2], 224 workgroups, would be
+// cut with the bound: the whole FFN 66.3 -> 72.4 us; 48 rows x [2048, 5632 x 2], 176, have to be cut: 22.2 -> 18.7).  What
+// the plan picked is slower than the best of the family on average, with this bound and without: gated products of 16 to
+// 100 rows, K of 512 to 8192, 2.1 % and 4.7; Q/K/V projections of 768- to 4544-wide models, up to 32 rows, 0.5 and 1.1;
+// plain products of such sizes 0.4 either way.
+constexpr float kRingStreamRate = 34e3f;
+constexpr int kRingStreamRows = 64, kRingStreamWorkgroups = 192;
 
-static RingPlan ring_plan_search(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes) {
+static RingPlan ring_plan_search(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes, float merge_us) {
   RingPlan best = {-1, 1, 1e30f};
   const int KT = K / 64;
   const float wbytes = 2.0f * (float)K * (float)ncols, obytes = 4.0f * (float)M * (float)ncols;
@@ -314,17 +317,14 @@ static RingPlan ring_plan_search(int M, int K, int ncols, int unit, int min_bn, 
       last_per = per;
       const int wg = tiles * ks, share = (wg + 255) / 256;
       const float even = share == 1 ? 1.0f : sqrtf((float)wg / (256.0f * share));
-      float mem = wbytes / (8e6f * even) + (ks > 1 ? ks * obytes : 0.5f * obytes) / 3e6f;
-      if (ks == 1 && share == 1 && min_bn > 0 && M <= kRingGatedChainRows) {
-        const float chain = per * c.bn * 128.0f / kRingGatedChainRate;
-        mem = mem > chain ? mem : chain;
-      }
+      const float mem = wbytes / (8e6f * even) + (ks > 1 ? ks * obytes : 0.5f * obytes) / 3e6f;
       const float it = share == 1 ? c.alone : (c.alone > c.shared * share ? c.alone : c.shared * share);
-      const float comp = per * it;
+      float comp = per * it;
+      if (ks == 1 && wg <= kRingStreamWorkgroups && M <= kRingStreamRows) comp = fmaxf(comp, per * c.bn * 128.0f / kRingStreamRate);
       const float loads = (float)wg * per * (c.bm + c.bn) * 128.0f / 37e6f;
       const float sum = cbrtf(mem * sqrtf(mem) + comp * sqrtf(comp) + loads * sqrtf(loads));
       const float us = 1.1f + 1.9f * ((share + c.per_cu - 1) / c.per_cu) + sum * sum +
-                       (ks > 1 ? 3.5f + ks * obytes / 6e6f : 0.f);
+                       (ks > 1 ? merge_us + ks * obytes / 6e6f : 0.f);
       if (us < best.us) { best.tile = tile; best.ksplit = ks; best.us = us; }
     }
   }
@@ -333,16 +333,17 @@ static RingPlan ring_plan_search(int M, int K, int ncols, int unit, int min_bn, 
 
 // The search is a pure function of its arguments and takes 5 to 10 us, longer than a launch; each thread keeps the
 // answers it was last given.
-RingPlan ring_plan(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes) {
+RingPlan ring_plan(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes, float merge_us) {
   if (M < 1 || K % 32 != 0 || K < 64 || ncols < 8) return RingPlan{-1, 1, 1e30f};
   if (M > kRingMaxRows && (M > kRingMaxRowsNarrow || ncols > kRingMaxColsNarrow || K < kRingMinKNarrow)) return RingPlan{-1, 1, 1e30f};
-  struct Entry { int M, K, ncols, unit, min_bn; int64_t ws_bytes; RingPlan plan; };
+  struct Entry { int M, K, ncols, unit, min_bn; int64_t ws_bytes; float merge_us; RingPlan plan; };
   static thread_local Entry memo[256] = {};
   uint64_t h = (uint64_t)M;
-  for (const uint64_t v : {(uint64_t)K, (uint64_t)ncols, (uint64_t)unit, (uint64_t)min_bn, (uint64_t)ws_bytes}) h = (h ^ v) * 0x9E3779B97F4A7C15ull;
+  for (const uint64_t v : {(uint64_t)K, (uint64_t)ncols, (uint64_t)unit, (uint64_t)min_bn, (uint64_t)ws_bytes, (uint64_t)(merge_us * 64.0f)}) h = (h ^ v) * 0x9E3779B97F4A7C15ull;
   Entry& e = memo[h >> 56];
-  if (e.M != M || e.K != K || e.ncols != ncols || e.unit != unit || e.min_bn != min_bn || e.ws_bytes != ws_bytes)
-    e = Entry{M, K, ncols, unit, min_bn, ws_bytes, ring_plan_search(M, K, ncols, unit, min_bn, ws_bytes)};
+  if (e.M != M || e.K != K || e.ncols != ncols || e.unit != unit || e.min_bn != min_bn || e.ws_bytes != ws_bytes ||
+      e.merge_us != merge_us)
+    e = Entry{M, K, ncols, unit, min_bn, ws_bytes, merge_us, ring_plan_search(M, K, ncols, unit, min_bn, ws_bytes, merge_us)};
   return e.plan;
 }
 
