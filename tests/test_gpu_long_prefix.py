@@ -11,7 +11,8 @@ import pytest
 import torch
 
 import oracle
-from gpu_util import run_qkv
+from gpu_util import projection_parts, run_qkv
+from test_gpu_attention import assert_scores
 from test_gpu_fp8_kv import K_SCALE, V_SCALE, _fp8_inputs, _run
 from util import assert_close, attn_inputs
 
@@ -88,3 +89,37 @@ def test_a_lost_tile_shows(S, Hq, Hkv, D, P, fp8):
     for k0 in range(0, P + S, 64):
         lost = (p[:, :, k0:k0 + 64] @ v[:, k0:k0 + 64]).abs()
         assert (lost > rel * o2.abs() + abs_).any(), "the tile at key %d" % k0
+
+
+# ---- projections in parts that attention sums itself: up to eight rows per KV head and four tokens here, eight tokens of
+# 128-wide heads against shorter prefixes
+FUSED = [
+    (1, 8, 1, 128, 2048), (2, 8, 2, 128, 2111),   # the new key opens a tile; two new keys in two tiles
+    (4, 2, 1, 64, 2110), (3, 4, 2, 64, 2300), (4, 4, 4, 128, 2047),
+    (8, 4, 2, 128, 300), (1, 4, 4, 128, 60), (7, 2, 1, 128, 252),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,Hq,Hkv,D,P", FUSED)
+@pytest.mark.parametrize("variant,qknorm", [("vanilla", False), ("vanilla", True), ("roco", False), ("keyformer", True)])
+def test_new_rows_from_partial_sums(dev, S, Hq, Hkv, D, P, variant, qknorm):
+    """Only the new rows have values, so that O2 is theirs alone, and what the caches hold in their places is not a number.
+    Tolerance: roundings of q, k, v, p and O2 to 2^-11 of a value each; a logit of up to about eight moves by q's and k's."""
+    n = 1024
+    assert projection_parts(n, S, Hq, Hkv, D, P, qknorm=qknorm) > 1.5
+    t = attn_inputs(S, n, Hq, Hkv, D, P=P, w_std=0.96 * n ** -0.5)
+    t["v_cache"][:, :P] = 0
+    t["k_cache"][:, P:], t["v_cache"][:, P:] = math.nan, math.nan
+    kw = dict(scale=1.0 / math.sqrt(D), causal=True, qknorm=qknorm, eps=1e-5)
+    clean = {k: t[k].nan_to_num(0.0) for k in ("k_cache", "v_cache")}
+    okw = dict(n_q_heads=Hq, n_kv_heads=Hkv, head_dim=D, scale=kw["scale"], causal=True, kv_prefix=P, qknorm=qknorm, rms_eps=1e-5)
+    more = {"roco": dict(roco=True), "keyformer": dict(keyformer=True, noise_seed=5, tau=1.0)}.get(variant, {})
+    want = oracle.qkv_attention(t["x"], t["wq"], t["wk"], t["wv"], **okw, **clean, **more)
+    got = run_qkv(t, dev, Hq=Hq, Hkv=Hkv, D=D, P=P, variant=variant, seed=5, **kw)
+    assert_close(got["O2"], want["O2"], 1e-2, 1e-2 * want["O2"].float().std().item(), "O2")
+    assert_close(got["k_cache"][:, P:], want["k_new"], 2e-3, 2e-3, "k rows")
+    assert_close(got["v_cache"][:, P:], want["v_new"], 2e-3, 2e-3, "v rows")
+    for name in ("s1", "s2", "score"):
+        if name in got:
+            assert_scores(got[name], want[name], name)

@@ -20,6 +20,7 @@
 #include "common.h"
 #include "launch.h"
 #include "philox.h"
+#include "proj_merge.h"
 
 
 namespace tri {
@@ -96,13 +97,19 @@ __device__ __forceinline__ void attn_wg_map(int id, int Hq, int nqb, int& qb, in
 // With FP8 (SPLIT only) K and V come from fp8 (e4m3) caches: a tile travels global -> registers while the tile (HALVES:
 // the two tiles) before it is worked on, and is converted to the 16-bit element type on its way into the same swizzled
 // LDS places (exact; the scales ride on a.scale and a.out_scale).
-template <int D, int QT, int KF, int KW, bool SPLIT = false, bool FP8 = false, int HALVES = 1>
+//
+// FUSED (SPLIT, 16-bit caches, at most kSplitFusedRows rows): q and the new rows of k / v come from the partial sums of a
+// split-K projection (AttnArgs::pj).  Every workgroup sums its q rows, those whose tiles hold new keys the new k / v
+// rows too, which then replace the stale rows of the tile in LDS; one workgroup each stores them where the unfused
+// projection would have.  One launch less, against one round trip to the partial sums in every workgroup.
+template <int D, int QT, int KF, int KW, bool SPLIT = false, bool FP8 = false, int HALVES = 1, bool FUSED = false>
 __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, const half_t* __restrict__ qglob) {
   // (qglob = a.q; the qualifier is what keeps the compiler from waiting for the loads in flight before the
   // first LDS transpose read of a tile - see attn_fwd_pipe_body)
   static_assert(!SPLIT || QT == 1, "the split variant: 32 rows per wave");
   static_assert(!FP8 || SPLIT, "fp8 caches are read by the split variant only");
   static_assert(HALVES == 1 || SPLIT, "half tiles per wave: the split variant only");
+  static_assert(!FUSED || (SPLIT && !FP8 && KW == 1), "the fused merge: the split variant on 16-bit caches");
   constexpr bool KEYFORMER = KF != 0;
   constexpr bool kf_fast = KF == 2;
   // a wave may meet tiles without a visible key before it has met one (its state is then still -inf / 0)
@@ -161,9 +168,11 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, co
     q = q < rows ? q : rows - 1;
     qtok[nt] = SPLIT ? q % a.S : q;
     qhead[nt] = SPLIT ? h + q / a.S : h;
-    const half_t* qp = qglob + (int64_t)qtok[nt] * a.ldq + qhead[nt] * D + g * 8;
+    if (!FUSED) {
+      const half_t* qp = qglob + (int64_t)qtok[nt] * a.ldq + qhead[nt] * D + g * 8;
 #pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) qf[nt][ks] = *reinterpret_cast<const half8v*>(qp + ks * 16);
+      for (int ks = 0; ks < KSTEPS; ++ks) qf[nt][ks] = *reinterpret_cast<const half8v*>(qp + ks * 16);
+    }
   }
 
   // ---- key range of this workgroup
@@ -457,10 +466,48 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, co
     }
   } else {
     issue(0);
+    // FUSED: rows of q, of new k and of new v behind the stages
+    half_t *const stage_q = lds + 2 * L::STAGE_HALFS, *const stage_k = stage_q + kSplitFusedRows * D, *const stage_v = stage_k + kSplitFusedRows * D;
+    bool has_new = false;
+    if (FUSED) {
+      for (int kt = a.P / kKeyTile; kt <= (Ltot - 1) / kKeyTile; ++kt) has_new |= kt % a.split_runs == split;
+      const int nq = a.Hq * D, nkv = a.Hkv * D;
+      const bool q_writer = split == 0 && a.q_w != nullptr;
+      merge_projection<D, 1, NWAVE * 64>(a, rows + (has_new ? 2 * a.S : 0), [&](int i) {
+        if (i < rows) {
+          const int m = i % a.S, head = h + i / a.S;
+          return MergeRow{m, head * D, true, stage_q + i * D, q_writer ? a.q_w + (int64_t)m * a.ldq + head * D : nullptr};
+        }
+        const int m = (i - rows) % a.S;
+        if (i - rows < a.S) return MergeRow{m, nq + hk * D, true, stage_k + m * D, a.k_w + (int64_t)hk * a.k_sh + (int64_t)(a.P + m) * a.k_sr};
+        return MergeRow{m, nq + nkv + hk * D, false, stage_v + m * D, a.v_w + (int64_t)hk * a.v_sh + (int64_t)(a.P + m) * a.v_sr};
+      });
+      __syncthreads();
+#pragma unroll
+      for (int nt = 0; nt < QT; ++nt) {
+        const int i = min(qidx[nt], rows - 1);  // (lanes without a row repeat the last one)
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ++ks) qf[nt][ks] = *reinterpret_cast<const half8v*>(stage_q + i * D + g * 8 + ks * 16);
+      }
+    }
     for (int step = 0; step < nsteps; ++step) {
       __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's share of the stage has landed
       __builtin_amdgcn_s_barrier();        // ... and everybody's; the stage before is retired
       if (step + 1 < nsteps) issue(step + 1);
+      if (FUSED) {
+        const int kt = step_tile(step), r0 = a.P - kt * kKeyTile;  // row of the tile that token 0 has
+        if (has_new && r0 < kKeyTile && r0 + a.S > 0) {
+          half_t *const ks = lds + (step & 1) * L::STAGE_HALFS, *const vs = ks + L::K_HALFS;
+          for (int p = t; p < a.S * L::CPR; p += NWAVE * 64) {
+            const int m = p / L::CPR, c = p % L::CPR, row = r0 + m;
+            if (row < 0 || row >= kKeyTile) continue;
+            *reinterpret_cast<half8v*>(ks + row * D + ((c ^ L::fk(row)) << 3)) = *reinterpret_cast<const half8v*>(stage_k + m * D + c * 8);
+            *reinterpret_cast<half8v*>(vs + row * D + ((c ^ L::fv(row)) << 3)) = *reinterpret_cast<const half8v*>(stage_v + m * D + c * 8);
+          }
+          __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the next tile's loads stay in flight
+          __builtin_amdgcn_s_barrier();
+        }
+      }
       work(step);
     }
   }
@@ -1048,10 +1095,10 @@ __global__ __launch_bounds__(256 * KW * QW) __attribute__((amdgpu_waves_per_eu(2
   else attn_fwd_body<D, QT, KF, KW>(a, lds, a.q);
 }
 
-template <int D, int KF, bool FP8, int HALVES, int KW>
+template <int D, int KF, bool FP8, int HALVES, int KW, bool FUSED>
 __global__ __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_split_kernel(AttnArgs a) {
   extern __shared__ __attribute__((aligned(16))) half_t lds[];
-  attn_fwd_body<D, 1, KF, KW, true, FP8, HALVES>(a, lds, a.q);
+  attn_fwd_body<D, 1, KF, KW, true, FP8, HALVES, FUSED>(a, lds, a.q);
 }
 
 template <int D, int QT, int KF, int KW, int QW = 1>
@@ -1089,11 +1136,11 @@ constexpr int kSplitMaxRuns = 32, kSplitMaxRunsFew = 64, kSplitFewBase = 2;
 constexpr int kSplitMinTiles = 4, kSplitMinTilesDecode = 2, kSplitDecodeTokens = 4;
 constexpr int kSplitHalvesRows = 64;  // two query groups of 32
 constexpr int kSplitPairWorkgroups = 256, kSplitPairTiles = 7;  // (one workgroup per CU; tiles per run)
-template <int D, int KF, bool FP8, int HALVES, int KW>
+template <int D, int KF, bool FP8, int HALVES, int KW, bool FUSED = false>
 static int launch_attn_split_h(const AttnArgs& a, int nwg, hipStream_t stream) {
-  constexpr int LDS = KW * AttnLds<D>::BYTES;
+  constexpr int LDS = KW * AttnLds<D>::BYTES + (FUSED ? 3 * kSplitFusedRows * D * 2 : 0);
   static_assert(KW * 2 * (D / 2 + 4) * 64 * 4 <= LDS, "the merge area fits the K/V stages");
-  constexpr auto kern = attn_split_kernel<D, KF, FP8, HALVES, KW>;
+  constexpr auto kern = attn_split_kernel<D, KF, FP8, HALVES, KW, FUSED>;
   if (set_max_lds<kern, LDS>() != 0) return -1;
   hipLaunchKernelGGL(kern, dim3(nwg), dim3(256 * KW), LDS, stream, a);
   return hipGetLastError() == hipSuccess ? 0 : -1;
@@ -1101,6 +1148,8 @@ static int launch_attn_split_h(const AttnArgs& a, int nwg, hipStream_t stream) {
 
 template <int D, int KF, bool FP8>
 static int launch_attn_split_t(const AttnArgs& a, int nwg, hipStream_t stream) {
+  if constexpr (!FP8)
+    if (a.pj != nullptr) return launch_attn_split_h<D, KF, FP8, 2, 1, true>(a, nwg, stream);
   // chunks: eight waves on two tiles at a time, half the runs and with them half the partial results (300 tokens against
   // 6000 keys 83.8 -> 77.7 us for the whole block, 48 against 6000 39.6 -> 35.7, 100 x 71 heads against 9000 51 -> 46)
   if constexpr (!FP8)
@@ -1154,7 +1203,7 @@ int64_t split_attn_workspace_bytes(int S, int Hq, int Hkv, int D, int Ltot, bool
 static int launch_attn_split(const AttnArgs& a, hipStream_t stream) {
   const int Ltot = a.P + a.S;
   const int kf = a.lse_pert == nullptr ? 0 : ((a.noise == nullptr && a.tau == 1.0f) ? 2 : 1);
-  if (a.pj != nullptr || a.ws == nullptr || (a.D != 64 && a.D != 128) || (a.k8 != nullptr && (a.v8 == nullptr || kf != 0)))
+  if ((a.pj != nullptr && (a.S > kSplitFusedTokens || a.S * (a.Hq / a.Hkv) > kSplitFusedRows || a.k8 != nullptr || a.k_w == nullptr || a.v_w == nullptr)) || a.ws == nullptr || (a.D != 64 && a.D != 128) || (a.k8 != nullptr && (a.v8 == nullptr || kf != 0)))
     return 1;
   int nsplit, fewest;
   if (!split_plan(a.S, a.Hq, a.Hkv, Ltot, &nsplit, &fewest)) return 1;
@@ -1190,7 +1239,8 @@ int launch_attention(const AttnArgs& a, hipStream_t stream, int* merge_parts) {
     const int r = launch_attention_few(a, stream, merge_parts);
     if (r <= 0) return r;
   }
-  if (a.k == nullptr || a.v == nullptr) return -1;  // (fp8 caches are read by the two variants above only)
+  // (fp8 caches and projections in parts are read by the two variants above only)
+  if (a.k == nullptr || a.v == nullptr || a.pj != nullptr) return -1;
   const int kf = a.lse_pert == nullptr ? 0 : ((a.noise == nullptr && a.tau == 1.0f) ? 2 : 1);
   // At most one workgroup per CU and a long key axis: eight waves per workgroup walk the keys two tiles at a
   // time (Llama-3-8B, four-wave -> eight-wave kernel: S = 1024 26 -> 20.8 us, S = 768 20.0 -> 17.5 us, S = 512

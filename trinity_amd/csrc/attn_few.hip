@@ -16,6 +16,7 @@
 #include "common.h"
 #include "launch.h"
 #include "philox.h"
+#include "proj_merge.h"
 
 namespace tri {
 
@@ -26,85 +27,6 @@ constexpr int kFewWaves = kFewKeysPerWg / kFewTile;
 
 template <int D>
 __device__ __forceinline__ int few_fv(int row) { return D == 128 ? ((row & 3) << 2) : (((row >> 1) & 1) << 2); }
-
-// Merge of a split-K projection for this workgroup: rows [0, S) x D columns of `nseg` column blocks (q head; new k
-// rows; new v rows) starting at columns col0[], each the sum of the splits in a fixed order, rounded to the element
-// type, RMS-normalised per row when `norm` (q and k only) - the arithmetic of the projection's own merge kernel -
-// stored to LDS dst_lds[seg] [row][D] and, where dst_g[seg] is given, to global rows of stride g_stride[seg].
-// Every thread takes up to R groups of four columns and has the loads of all of them in flight together: the
-// partial sums sit in other XCDs' caches, one round trip instead of one per block.  Called by all NT threads of the workgroup.
-template <int D, int R, int NT>
-__device__ __forceinline__ void few_merge_projection(const AttnArgs& a, int nseg, const int (&col0)[3], bool norm,
-                                                     half_t* const (&dst_lds)[3], half_t* const (&dst_g)[3],
-                                                     const int64_t (&g_stride)[3]) {
-  constexpr int LPH = D / 4;  // lanes per row
-  const int per = a.S * LPH, total = nseg * per;
-  const int64_t split_stride = (int64_t)a.S * a.pj_ntot;
-  for (int base = 0; base < total; base += NT * R) {
-    bool live[R];
-    int seg[R], m[R], li[R];
-    const float* src[R];
-    float4v acc[R];
-#pragma unroll
-    for (int u = 0; u < R; ++u) {
-      const int idx = base + u * NT + (int)threadIdx.x;
-      live[u] = idx < total;
-      seg[u] = live[u] ? idx / per : 0;
-      const int rem = live[u] ? idx - seg[u] * per : 0;
-      m[u] = rem / LPH;
-      li[u] = rem % LPH;
-      const int c0 = seg[u] == 0 ? col0[0] : (seg[u] == 1 ? col0[1] : col0[2]);
-      src[u] = a.pj + (int64_t)m[u] * a.pj_ntot + c0 + li[u] * 4;
-      acc[u] = float4v{0.f, 0.f, 0.f, 0.f};
-    }
-    // eight splits at a time (past the last split the last one is re-read and ignored)
-    for (int i0 = 0; i0 < a.pj_ksplit; i0 += 8) {
-      float4v p[R][8];
-#pragma unroll
-      for (int u = 0; u < R; ++u)
-        if (live[u]) {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const int i = i0 + j < a.pj_ksplit ? i0 + j : a.pj_ksplit - 1;
-            p[u][j] = *reinterpret_cast<const float4v*>(src[u] + i * split_stride);
-          }
-        }
-#pragma unroll
-      for (int u = 0; u < R; ++u)
-        if (live[u]) {
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            if (i0 + j < a.pj_ksplit) {
-#pragma unroll
-              for (int e = 0; e < 4; ++e) acc[u][e] += p[u][j][e];
-            }
-        }
-    }
-#pragma unroll
-    for (int u = 0; u < R; ++u) {
-      half4v h = {(half_t)acc[u][0], (half_t)acc[u][1], (half_t)acc[u][2], (half_t)acc[u][3]};
-      if (norm) {  // uniform; every lane takes part in the reduction
-        float ss = 0.f;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) ss = fmaf((float)h[e], (float)h[e], ss);
-#pragma unroll
-        for (int o = LPH / 2; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
-        if (seg[u] < 2) {
-          const float nrm = rsqrtf(ss / (float)D + a.eps);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) h[e] = (half_t)((float)h[e] * nrm);
-        }
-      }
-      if (live[u]) {
-        half_t* dl = seg[u] == 0 ? dst_lds[0] : (seg[u] == 1 ? dst_lds[1] : dst_lds[2]);
-        half_t* dg = seg[u] == 0 ? dst_g[0] : (seg[u] == 1 ? dst_g[1] : dst_g[2]);
-        const int64_t gs = seg[u] == 0 ? g_stride[0] : (seg[u] == 1 ? g_stride[1] : g_stride[2]);
-        *reinterpret_cast<half4v*>(dl + m[u] * D + li[u] * 4) = h;
-        if (dg != nullptr) *reinterpret_cast<half4v*>(dg + (int64_t)m[u] * gs + li[u] * 4) = h;
-      }
-    }
-  }
-}
 
 // FP8: K and V come from fp8 (e4m3) caches (a.k8 / a.v8) and are converted on the way in - K rows in registers, V
 // rows while they are staged in LDS; their scales are folded into a.scale and a.out_scale by the caller.
@@ -203,13 +125,12 @@ __device__ __forceinline__ void attn_few_body(const AttnArgs& a, half_t* lds) {
     // the k / v rows too when some of this workgroup's keys are new
     const bool kv = split * KPW < Ltot && (split + 1) * KPW > a.P;
     const bool writer = split == a.P / KPW && h % group == 0;
-    const int col0[3] = {h * D, nq + hk * D, nq + nkv + hk * D};
-    half_t* const dst_lds[3] = {stage_q, stage_k, stage_v};
-    half_t* const dst_g[3] = {(split == 0 && a.q_w != nullptr) ? a.q_w + h * D : nullptr,
-                              writer ? a.k_w + (int64_t)hk * a.k_sh + (int64_t)a.P * a.k_sr : nullptr,
-                              writer ? a.v_w + (int64_t)hk * a.v_sh + (int64_t)a.P * a.v_sr : nullptr};
-    const int64_t g_stride[3] = {a.ldq, a.k_sr, a.v_sr};
-    few_merge_projection<D, 3, NW * 64>(a, kv ? 3 : 1, col0, a.qknorm != 0, dst_lds, dst_g, g_stride);
+    merge_projection<D, 3, NW * 64>(a, (kv ? 3 : 1) * a.S, [&](int i) {
+      const int seg = i / a.S, m = i % a.S;  // q rows, new k rows, new v rows
+      if (seg == 0) return MergeRow{m, h * D, true, stage_q + m * D, split == 0 && a.q_w != nullptr ? a.q_w + (int64_t)m * a.ldq + h * D : nullptr};
+      if (seg == 1) return MergeRow{m, nq + hk * D, true, stage_k + m * D, writer ? a.k_w + (int64_t)hk * a.k_sh + (int64_t)(a.P + m) * a.k_sr : nullptr};
+      return MergeRow{m, nq + nkv + hk * D, false, stage_v + m * D, writer ? a.v_w + (int64_t)hk * a.v_sh + (int64_t)(a.P + m) * a.v_sr : nullptr};
+    });
     __syncthreads();
   }
 

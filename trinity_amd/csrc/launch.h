@@ -159,7 +159,7 @@ struct AttnArgs {
   // fp8 (e4m3) caches read directly - few-query path only; k / v are then unused.  Strides in elements = bytes.
   const uint8_t *k8, *v8;
   int64_t k8_sh, k8_sr, v8_sh, v8_sr;
-  // Few-query path fused with the merge of a split-K projection (pj != nullptr; launch_attention_few only): q and
+  // Few-query paths fused with the merge of a split-K projection (pj != nullptr): q and
   // the S new rows of k / v are not read from memory but summed from the projection's partial results
   // pj [pj_ksplit][S][pj_ntot] (columns [q heads | k heads | v heads]), rounded, RMS-normalised per head when
   // qknorm (q and k), and stored to q_w and to rows [P, P+S) of k_w / v_w (the buffers k / v point to) on the way.
@@ -187,6 +187,9 @@ int64_t split_attn_workspace_bytes(int S, int Hq, int Hkv, int D, int Ltot, bool
 // 16 tokens: at 1040 keys the two are level, at 2064 keys the looping kernel is 2-5 us ahead, at 32784 keys
 // 2.3x (8 KV heads, head dimension 128) to 3x (1 KV head, 64) on the whole block.
 constexpr int kSplitMinKeys = 2048;
+// Most tokens, and rows (heads of a group x tokens), whose projection's partial sums that kernel adds up itself; most
+// tokens of 128-wide heads for the one-tile-per-wave kernel (attn_may_merge_proj has the measurements).
+constexpr int kSplitFusedRows = 8, kSplitFusedTokens = 4, kFewFusedTokens = 8;
 
 // fp8 (OCP e4m3) KV caches, value = scale * fp8: append of the new rows, and 16-bit copies (without the scale)
 // for the kernels that read 16-bit K / V tiles.
