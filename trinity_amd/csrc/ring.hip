@@ -12,6 +12,8 @@
 
 #include <math.h>
 
+#include <type_traits>
+
 namespace tri {
 
 template <class T, bool WT>
@@ -67,7 +69,7 @@ __global__ __launch_bounds__(T::NT) void ring_epi_kernel(GemmArgs a) {
   constexpr int OUT_BN = GATED ? T::BN / 2 : T::BN;
   const int nrb = (a.M + T::BM - 1) / T::BM, ntn = (a.N + OUT_BN - 1) / OUT_BN;
   int rb, tn, split;
-  ring_coords(blockIdx.x, nrb, ntn, 1, nrb > 1 || T::BM >= 96, rb, tn, split);
+  ring_coords(blockIdx.x, nrb, ntn, 1, nrb > 1 || T::BM >= 96 || std::is_same<T, RingTileKContig>::value, rb, tn, split);
   const int m0 = rb * T::BM, n0 = tn * OUT_BN;
   auto wmap = [&](int c, int64_t& ldw) -> const half_t* {
     const int nloc = WT ? c : c * 8;
@@ -254,8 +256,11 @@ static int launch_epi_t(const GemmArgs& a, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+constexpr int kRingTileOneBlock = 8;  // the non-temporal tile, for a single row block
 template <int EPI>
 static int launch_epi(const GemmArgs& a, int tile, hipStream_t stream) {
+  if (a.w_kcontig && tile == kRingTileOneBlock && ((a.ldw | (EPI == EPI_SWIGLU ? a.ldw2 : 0)) & 4095) == 0)
+    return launch_epi_t<RingTileKContig, EPI, true>(a, stream);
   switch (tile) {
 #define TRI_RING_CASE(id, bm, bn, wm, wn, nst, nt)                                                       \
   case id:                                                                                           \
@@ -286,7 +291,6 @@ static const RingCost kRingCost[kRingTiles] = {
     {128, 128, TRI_RING_PER_CU(128, 128, 5), 0.480f, 0.490f}, {128, 192, TRI_RING_PER_CU(128, 192, 4), 0.660f, 0.691f},
     {128, 256, TRI_RING_PER_CU(128, 256, 3), 0.743f, 0.755f}, {160, 256, TRI_RING_PER_CU(160, 256, 3), 0.914f, 1.006f},
     {32, 128, TRI_RING_PER_CU(32, 128, 4), 0.264f, 0.222f}};
-constexpr int kRingTileOneBlock = 8;  // the non-temporal tile, for a single row block
 // A plan in one part on few workgroups: one streams no faster than about this many bytes of weights per us (16 rows x
 // [2048, 5632 x 2] as gate/up, 88 workgroups: 22.0 us, 16.0 in two parts; x [1024, 4096 x 2], 64: 12.0 and 10.1 in four; the
 // costs above, fitted where 200 and more workgroups share the memory's rate, say 14.9 and 7.8).  Up to 64 rows and 192
