@@ -134,3 +134,36 @@ def test_ffn_block_row_statistic(rn, M, N, F):
     check(attn, o2.float() @ wo.float() + x.float(), "attn_O2")
     want = torch.rsqrt((attn.double() ** 2).mean(1)).float()
     assert ((rows - want).abs() <= 1e-5 * want).all()  # fp32 sums of N squares
+
+
+@pytest.mark.parametrize("M,K,N", [
+    (1, 512, 4096), (16, 544, 4096), (7, 608, 1000),        # one 128-deep piece a wave; K ends 32 and 96 into a piece
+    (3, 640, 24), (5, 1152, 8), (16, 2016, 520),            # waves with a piece more than others; less than 16 columns
+    (16, 4096, 4104), (17, 4096, 4096), (2, 4544, 18176),   # a ragged last strip; one row too many; several a CU
+])
+def test_strips_over_k_contiguous_weights(rn, M, K, N):
+    """Row strides beyond the columns, residual and GELU; what lies between the rows stays as it is."""
+    x, r = rn(M, K + 24)[:, 8:K + 8], rn(M, N + 8)[:, :N]
+    w = rn(N, K + 8, std=K ** -0.5)[:, :K].t()
+    ws = torch.empty(ext.gemm_workspace_bytes(M, K, N), dtype=torch.uint8, device="cuda:0")
+    buf = torch.full((M, N + 16), 7.0, dtype=torch.float16, device="cuda:0")
+    out = buf[:, 8:N + 8]
+    for workspace in (ws, None):
+        out.fill_(float("nan"))
+        ext.matmul(x, w, r, out, workspace=workspace)
+        check(out, x.float() @ w.float() + r.float(), "x.w + r")
+        assert (buf[:, :8] == 7).all() and (buf[:, N + 8:] == 7).all()
+    w2 = rn(N, 64, std=N ** -0.5) if N % 32 else rn(64, N, std=N ** -0.5).t()  # (K-contiguous: K % 32 == 0)
+    y = torch.empty(M, 64, dtype=torch.float16, device="cuda:0")
+    ext.ffn_gelu(x, w, w2, out, y, workspace=None)
+    want = torch.nn.functional.gelu(x.float() @ w.float())
+    check(out, want, "gelu(x.w)")
+    check(y, out.float() @ w2.float(), "hidden.w2")
+
+
+def test_strips_and_a_product_over_its_own_input(rn):
+    x, w = rn(4, 1024), rn(1024, 1024, std=1 / 32).t()
+    want = x.float() @ w.float()
+    ws = torch.empty(ext.gemm_workspace_bytes(4, 1024, 1024), dtype=torch.uint8, device="cuda:0")
+    ext.matmul(x, w, None, x, workspace=ws)
+    check(x, want, "x = x.w")

@@ -101,6 +101,9 @@ constexpr int kRingMaxRowsNarrow = 8192, kRingMaxColsNarrow = 1 << 16, kRingMinK
 constexpr float kRingMergeUs = 3.5f;
 RingPlan ring_plan(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes, float merge_us = kRingMergeUs);
 int launch_ring_gemm(const GemmArgs& a, const RingPlan& plan, hipStream_t stream);
+// few rows over K-contiguous weights in one part (strip.hip): what it should take (us; 1e30: not for it), and the launch
+float strip_us(const GemmArgs& a);
+int launch_strip(const GemmArgs& a, hipStream_t stream);
 bool ring_gemm_in_place(const GemmArgs& a);  // out overlaps x, and the workspace holds the one part it takes to allow that
 // workspace that lets launch_gemm take its best plan for [M, K] x [K, ncols] (0: no plan in parts)
 int64_t gemm_workspace_bytes(int M, int K, int ncols);

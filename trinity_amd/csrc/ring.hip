@@ -366,6 +366,7 @@ bool ring_gemm_in_place(const GemmArgs& a) {
 }
 
 int launch_ring_gemm(const GemmArgs& a, const RingPlan& plan, hipStream_t stream) {
+  if (strip_us(a) < 0.97f * plan.us && !shares_memory(a)) return launch_strip(a, stream);
   const bool gated = a.epi == EPI_SWIGLU;
   // A product that overwrites its own input goes through the workspace also in one part: the tiles of the epilogue
   // kernel would store while others still read.
