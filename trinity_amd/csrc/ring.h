@@ -6,8 +6,8 @@
 // whatever else a CU does.  (The large-tile loop of gemm_core.h keeps its activations in two buffers and loads complete in
 // order, so its weights are never more than about one tile ahead: 64 rows x [4096, 28672] 59 us there and in the split-K
 // kernel, 44 us here = 5.3 TB/s; 128 rows 64 -> 51 us.)  How many it takes was measured for 32 x 128 tiles with a CU to
-// themselves, 16 rows x [4096, 28672]: 32 KB of weights on their way per CU (three stages) 43.0 us, 48 KB (four, as built)
-// 44.5, 64 KB 44.7, 96 KB 45.2 - more than 32 KB buy nothing there.
+// themselves, 16 rows x [4096, 28672]: 32 KB of weights on their way per CU (three stages, as built) 43.0 us, 48 KB (four)
+// 44.5, 64 KB 44.7, 96 KB 45.2 - more than 32 KB cost time there.
 //
 // 64-deep k tiles: an activation row, and a K-contiguous weight column, is then read in whole 128-byte lines.
 // Both operands go global -> LDS without passing through registers (1 KB per wave instruction), XOR-swizzled by the
@@ -49,6 +49,8 @@ struct RingTile {
 // other's LDS reads: 128 x 256 at 512 rows 138 -> 136 us, 64 x 128 at 64 rows of [4096, 14336 x 2] 44.7 -> 44.2 us).
 // Non-temporal weights where one block of at most 32 rows sees them: 16 rows x [18176, 4544] in 7 parts 29.6 -> 27.1 us
 // (6.1 TB/s), x [14336, 4096] in 8 parts 22.6 -> 21.2 us; at 64 rows the gain is gone (42.7 -> 43.6, 25.1 -> 23.6 us).
+// That tile has three stages, not four: whole calls of 16 tokens, Llama-3-8B FFN block 83.2 -> 80.4 us, Q/K/V block against
+// 1024 keys 39.2 -> 38.9, one token against 4095 keys 21.6 -> 21.4; others of 1 to 32 rows level to 3 % faster, none slower.
 #define TRI_RING_TILES(X)        \
   X(0, 32, 128, 1, 4, 4, false)  \
   X(1, 64, 64, 2, 2, 5, false)   \
@@ -58,7 +60,7 @@ struct RingTile {
   X(5, 128, 192, 2, 2, 4, false) \
   X(6, 128, 256, 2, 4, 3, false) \
   X(7, 160, 256, 1, 4, 3, false) \
-  X(8, 32, 128, 1, 4, 4, true)
+  X(8, 32, 128, 1, 4, 3, true)
 constexpr int kRingTiles = 9;
 // A product in one part of tile 8 over K-contiguous weights whose columns lie a multiple of 8 KB apart runs on this one
 // instead: two waves, 64 columns, and an XCD's workgroups on neighbouring columns.  At such distances the memory is slow

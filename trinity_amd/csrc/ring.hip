@@ -290,7 +290,7 @@ static const RingCost kRingCost[kRingTiles] = {
     {64, 128, TRI_RING_PER_CU(64, 128, 3), 0.354f, 0.272f},  {96, 128, TRI_RING_PER_CU(96, 128, 5), 0.429f, 0.431f},
     {128, 128, TRI_RING_PER_CU(128, 128, 5), 0.480f, 0.490f}, {128, 192, TRI_RING_PER_CU(128, 192, 4), 0.660f, 0.691f},
     {128, 256, TRI_RING_PER_CU(128, 256, 3), 0.743f, 0.755f}, {160, 256, TRI_RING_PER_CU(160, 256, 3), 0.914f, 1.006f},
-    {32, 128, TRI_RING_PER_CU(32, 128, 4), 0.264f, 0.222f}};
+    {32, 128, TRI_RING_PER_CU(32, 128, 3), 0.264f, 0.222f}};
 // A plan in one part on few workgroups: one streams no faster than about this many bytes of weights per us (16 rows x
 // [2048, 5632 x 2] as gate/up, 88 workgroups: 22.0 us, 16.0 in two parts; x [1024, 4096 x 2], 64: 12.0 and 10.1 in four; the
 // costs above, fitted where 200 and more workgroups share the memory's rate, say 14.9 and 7.8).  Up to 64 rows and 192
