@@ -139,3 +139,41 @@ def test_fp8_cache_bf16_elements(dev, N):
     got = _run(t, dev, "vanilla", Hq=Hq, Hkv=Hkv, D=D, P=P, causal=False, dtype=torch.bfloat16)
     assert_close(got["O2"], want["O2"], 3e-2, 3e-2, "O2 (bf16 elements)")
     _codes_match(got["k_cache"][:, P:P + S], want["k_new"], "appended k")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("group,S,P", [(1, 1, 300), (1, 1, 2100), (2, 16, 4100), (1, 32, 2500), (40, 2, 2300)])
+def test_every_code_is_converted_exactly(dev, dtype, D, group, S, P):
+    """Zero activations make all weights equal, and every key holds the same codes, all finite ones among its columns: an
+    output is its column's value (or the average of P of them and the new rows' zeros), rounded once."""
+    Hkv, N = 256 // D, 256  # a column for every code
+    Hq = group * Hkv
+    codes = torch.arange(Hkv * D, dtype=torch.int32) % 256
+    codes[(codes & 0x7F) == 0x7F] = 0  # NaN
+    vrow = codes.to(torch.uint8).view(F8).reshape(Hkv, 1, D)
+    vc = vrow.view(torch.uint8).repeat(1, P + S, 1).view(F8).contiguous().to(dev)
+    kc = torch.zeros(Hkv, P + S, D, dtype=torch.uint8).view(F8).to(dev)
+    x = torch.zeros(S, N, dtype=dtype, device=dev)
+    w = lambda h: torch.zeros(N, h * D, dtype=dtype, device=dev)
+    p = ext.attn_params(Hq, Hkv, D, S, kv_prefix=P, causal=True, rms_eps=1e-5, kv_fp8=True, k_scale=1.0, v_scale=1.0)
+    out = torch.zeros(S, Hq * D, dtype=dtype, device=dev)
+    ext.qkv_attention(x, None, w(Hq), w(Hkv), w(Hkv), kc, vc, scratch_for(p, N, dev), None, out, p)
+    visible = (P + 1 + torch.arange(S, dtype=torch.float64)).reshape(S, 1, 1)
+    want = (vrow.float().double().reshape(1, Hkv, 1, D) * (P / visible).reshape(S, 1, 1, 1)).expand(S, Hkv, Hq // Hkv, D).reshape(S, Hq * D)
+    # one rounding to the element type, and fp32 sums of at most P + S equal terms: 1e-5 is above both sums' error
+    eps = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+    assert_close(out.cpu().double(), want, rtol=eps + 1e-5, atol=0.0)
+
+
+@pytest.mark.parametrize("S,D", [(16, 128), (1, 128), (3, 64)])
+@pytest.mark.parametrize("P", [2048, 2200, 2331, 2600, 3100])
+def test_odd_and_even_numbers_of_tile_steps(dev, S, D, P):
+    """Runs of two to seven tiles, some a tile shorter than others: tiles of even and odd steps travel in registers of their own."""
+    Hq, Hkv = 64, 16  # (512 workgroups over 16 KV heads: up to 32 runs of two tiles for one token, of four for more)
+    t = _fp8_inputs(S, 256, Hq, Hkv, D, P)
+    want = oracle.qkv_attention(t["x"], t["wq"], t["wk"], t["wv"], n_q_heads=Hq, n_kv_heads=Hkv, head_dim=D, scale=1 / math.sqrt(D),
+                                causal=True, kv_prefix=P, k_cache=t["k_cache"], v_cache=t["v_cache"], kv_fp8=True,
+                                k_scale=K_SCALE, v_scale=V_SCALE)
+    got = _run(t, dev, "vanilla", Hq=Hq, Hkv=Hkv, D=D, P=P, causal=True)
+    assert_close(got["O2"], want["O2"], 1e-2, 1e-2, "O2")

@@ -94,7 +94,7 @@ __device__ __forceinline__ void attn_wg_map(int id, int Hq, int nqb, int& qb, in
 // kernel there is not HBM but the chain of LDS reads, MFMAs and exponentials of a tile step (64 rows, 32768 fp8 keys,
 // 8 KV heads: 27.8 -> 22.2 us = 3.0 TB/s; two tiles per step for eight waves are level with this).
 //
-// With FP8 (SPLIT only) K and V come from fp8 (e4m3) caches: a tile travels global -> registers while the tile (HALVES:
+// With FP8 (SPLIT only) K and V come from fp8 (e4m3) caches: a tile travels global -> registers while the tile (TWO_SETS:
 // the two tiles) before it is worked on, and is converted to the 16-bit element type on its way into the same swizzled
 // LDS places (exact; the scales ride on a.scale and a.out_scale).
 //
@@ -224,7 +224,11 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, co
   struct Raw8 {
     uint4v k[PIECES], v[PIECES];
   };
-  Raw8 raw_even, raw_odd;  // (HALVES) tiles of even and of odd steps: two tiles are on their way at any time
+  // TWO_SETS: tiles of even and of odd steps, two of them on their way at any time.  Whole tiles of 128-wide heads have no
+  // registers for that (24 tokens against 32752 keys 28.1 -> 39.1 us, the compiler spills); 64-wide heads, 71 on one, 16
+  // tokens against 8000 keys 12.9 -> 12.1, against 32752 27.4 -> 26.5.
+  constexpr bool TWO_SETS = HALVES == 2 || D == 64;
+  Raw8 raw_even, raw_odd;
   auto fetch8 = [&](int step, Raw8& raw) {
     const int kt = step_tile(step);
 #pragma unroll
@@ -232,8 +236,11 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, co
       const int piece = i * NWAVE * 64 + t;
       // (past the last key: the last one again - its scores are masked, and an unconditional load lets the waits count)
       const int key = min(kt * kKeyTile + piece / PPR, Ltot - 1), j = piece % PPR;
-      raw.k[i] = *reinterpret_cast<const uint4v*>(a.k8 + (int64_t)hk * a.k8_sh + (int64_t)key * a.k8_sr + j * 16);
-      raw.v[i] = *reinterpret_cast<const uint4v*>(a.v8 + (int64_t)hk * a.v8_sh + (int64_t)key * a.v8_sr + j * 16);
+      const uint4v* kp = reinterpret_cast<const uint4v*>(a.k8 + (int64_t)hk * a.k8_sh + (int64_t)key * a.k8_sr + j * 16);
+      const uint4v* vp = reinterpret_cast<const uint4v*>(a.v8 + (int64_t)hk * a.v8_sh + (int64_t)key * a.v8_sr + j * 16);
+      // (HALVES: a single block of rows reads the cache, each line once; 32 tokens on 32 KV heads, 32752 keys, 56.8 -> 47.1 us)
+      raw.k[i] = HALVES == 2 ? __builtin_nontemporal_load(kp) : *kp;
+      raw.v[i] = HALVES == 2 ? __builtin_nontemporal_load(vp) : *vp;
     }
   };
   auto commit8 = [&](int step, const Raw8& raw) {
@@ -439,7 +446,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, co
     const bool need_mask = (key0 + kKeyTile > Ltot) || (a.causal && key0 + kKeyTile - 1 > a.P + (SPLIT ? 0 : qw0));
     if (active) tile(step, kt, need_mask);
   };
-  if (FP8 && HALVES == 1) {
+  if (FP8 && !TWO_SETS) {
     fetch8(0, raw_even);
     for (int step = 0; step < nsteps; ++step) {
       commit8(step, raw_even);
@@ -456,14 +463,15 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, co
     };
     fetch8(0, raw_even);
     fetch8(1, raw_odd);
-    // (left from the middle: were the second half skipped instead, the wait at the loop's head would have to assume
-    // that the tile it needs is the one requested last)
-    for (int step = 0;; step += 2) {
+    // Two steps a turn, an odd last one behind the loop: a loop that may be left in its middle makes the compiler wait at its
+    // head as if the tile it needs were the one requested last, and one tile is on its way instead of two (one token against
+    // 32752 keys, 8 KV heads, 19.1 -> 18.4 us, 16 tokens 23.7 -> 22.9, both with two values converted per instruction).
+    int step = 0;
+    for (; step + 1 < nsteps; step += 2) {
       step8(step, raw_even);
-      if (step + 1 >= nsteps) break;
       step8(step + 1, raw_odd);
-      if (step + 2 >= nsteps) break;
     }
+    if (step < nsteps) step8(step, raw_even);
   } else {
     issue(0);
     // FUSED: rows of q, of new k and of new v behind the stages
