@@ -50,7 +50,8 @@ struct RingTile {
 // Non-temporal weights where one block of at most 32 rows sees them: 16 rows x [18176, 4544] in 7 parts 29.6 -> 27.1 us
 // (6.1 TB/s), x [14336, 4096] in 8 parts 22.6 -> 21.2 us; at 64 rows the gain is gone (42.7 -> 43.6, 25.1 -> 23.6 us).
 // That tile has three stages, not four: whole calls of 16 tokens, Llama-3-8B FFN block 83.2 -> 80.4 us, Q/K/V block against
-// 1024 keys 39.2 -> 38.9, one token against 4095 keys 21.6 -> 21.4; others of 1 to 32 rows level to 3 % faster, none slower.
+// 1024 keys 39.2 -> 38.9, one token against 4095 keys 21.6 -> 21.4; others of 1 to 32 rows level to 3 % faster - but for
+// row-major weights whose rows are no multiple of 256 bytes (RingTileStraddle).
 #define TRI_RING_TILES(X)        \
   X(0, 32, 128, 1, 4, 4, false)  \
   X(1, 64, 64, 2, 2, 5, false)   \
@@ -62,6 +63,11 @@ struct RingTile {
   X(7, 160, 256, 1, 4, 3, false) \
   X(8, 32, 128, 1, 4, 3, true)
 constexpr int kRingTiles = 9;
+// Tile 8 with a fourth stage, for row-major weights whose rows are no multiple of 256 bytes apart: a tile's 256 bytes of a
+// row then lie across two such blocks of memory, and 48 KB on their way are worth more than 32 (16 rows x [4544, 4544 x 2]
+// 17.0 -> 16.4 us, x [4544, 4544 x 3] 22.5 -> 21.7, x [18176, 4544] level).
+using RingTileStraddle = RingTile<32, 128, 1, 4, 4, true>;
+inline bool ring_rows_straddle(int64_t ldw) { return (ldw & 127) != 0; }  // (several distances or-ed together)
 // A product in one part of tile 8 over K-contiguous weights whose columns lie a multiple of 8 KB apart runs on this one
 // instead: two waves, 64 columns, and an XCD's workgroups on neighbouring columns.  At such distances the memory is slow
 // (a kernel that only reads [4096, 28672]: 45.4 us with 224 workgroups of 128 columns, 39.9 with 448 of 64, 37.9 with
