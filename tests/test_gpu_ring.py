@@ -167,3 +167,14 @@ def test_strips_and_a_product_over_its_own_input(rn):
     ws = torch.empty(ext.gemm_workspace_bytes(4, 1024, 1024), dtype=torch.uint8, device="cuda:0")
     ext.matmul(x, w, None, x, workspace=ws)
     check(x, want, "x = x.w")
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 4096, 4096), (5, 1152, 8), (16, 544, 4096)])
+def test_strips_in_bf16(rn, M, K, N):
+    """As above with an element of 8 bits: two of its ulps, 2^-6 of the value, in place of fp16's 2^-9."""
+    x, r, w = rn(M, K).bfloat16(), rn(M, N).bfloat16(), rn(N, K, std=K ** -0.5).bfloat16().t()
+    out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda:0")
+    ext.matmul(x, w, r, out, workspace=None)
+    want = x.float() @ w.float() + r.float()
+    torch.cuda.synchronize()
+    assert ((out.float() - want).abs() <= 2.0 ** -6 * want.abs() + ABS).all()
