@@ -178,3 +178,49 @@ def test_strips_in_bf16(rn, M, K, N):
     want = x.float() @ w.float() + r.float()
     torch.cuda.synchronize()
     assert ((out.float() - want).abs() <= 2.0 ** -6 * want.abs() + ABS).all()
+
+
+def check_bf16(got, want, what):
+    """check() for an element of 8 bits: 2^-6 of the value in place of 2^-9."""
+    torch.cuda.synchronize()
+    assert ((got.float() - want).abs() <= 2.0 ** -6 * want.abs() + ABS).all(), what
+
+
+# up to 32 rows on 32 x 128 tiles; which of them run three stages and which four follows from the workgroups of the last round
+# (two a CU) and the distance between rows: 133 workgroups, 257, 399 and 195 in three parts, 144 in four
+@pytest.mark.parametrize("M,K,N", [(24, 544, 17000), (17, 1056, 32776), (20, 2080, 17000), (24, 4544, 8200), (32, 2080, 4552)])
+@pytest.mark.parametrize("kcontig", [False, True])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_stages_of_plain_products(rn, M, K, N, kcontig, bf16):
+    el, ok = (torch.bfloat16, check_bf16) if bf16 else (torch.float16, check)
+    x, r = rn(M, K).to(el), rn(M, N).to(el)
+    w = (rn(N, K, std=K ** -0.5).t() if kcontig else rn(K, N, std=K ** -0.5)).to(el)
+    ws = torch.empty(ext.gemm_workspace_bytes(M, K, N), dtype=torch.uint8, device="cuda:0")
+    for workspace in (ws, None):
+        out = torch.full((M, N), float("nan"), dtype=el, device="cuda:0")
+        ext.matmul(x, w, r, out, workspace=workspace)
+        ok(out, x.float() @ w.float() + r.float(), "x.w + r")
+
+
+# 225 workgroups, 257, and 213 and 387 in three parts
+@pytest.mark.parametrize("M,K,F", [(17, 1056, 14344), (32, 544, 16400), (8, 1056, 4544), (3, 2080, 8200)])
+@pytest.mark.parametrize("kcontig", [False, True])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_stages_of_gated_products(rn, M, K, F, kcontig, bf16):
+    el, ok = (torch.bfloat16, check_bf16) if bf16 else (torch.float16, check)
+    x = rn(M, K).to(el)
+    wg, wu = ((rn(F, K, std=K ** -0.5).t() if kcontig else rn(K, F, std=K ** -0.5)).to(el) for _ in range(2))
+    ws = torch.empty(ext.gemm_workspace_bytes(M, K, 2 * F), dtype=torch.uint8, device="cuda:0")
+    a, b = x.float() @ wg.float(), x.float() @ wu.float()
+    for workspace in (ws, None):
+        out = torch.full((M, F), float("nan"), dtype=el, device="cuda:0")
+        ext.gateup_swiglu(x, wg, wu, None, out, workspace=workspace)
+        ok(out, a * torch.sigmoid(a) * b, "gated")
+
+
+# 134, 208 and 258 workgroups in one part, and 64-wide heads
+@pytest.mark.parametrize("S,N,Hq,Hkv,D", [(20, 544, 130, 2, 128), (32, 544, 192, 8, 128), (17, 544, 252, 3, 128), (20, 544, 260, 4, 64)])
+@pytest.mark.parametrize("qknorm", [False, True])
+@pytest.mark.parametrize("kcontig", [False, True])
+def test_stages_of_the_projection(rn, S, N, Hq, Hkv, D, qknorm, kcontig):
+    test_qkv_projection(rn, S, N, Hq, Hkv, D, qknorm, kcontig)

@@ -6,8 +6,8 @@
 // whatever else a CU does.  (The large-tile loop of gemm_core.h keeps its activations in two buffers and loads complete in
 // order, so its weights are never more than about one tile ahead: 64 rows x [4096, 28672] 59 us there and in the split-K
 // kernel, 44 us here = 5.3 TB/s; 128 rows 64 -> 51 us.)  How many it takes was measured for 32 x 128 tiles with a CU to
-// themselves, 16 rows x [4096, 28672]: 32 KB of weights on their way per CU (three stages, as built) 43.0 us, 48 KB (four)
-// 44.5, 64 KB 44.7, 96 KB 45.2 - more than 32 KB cost time there.
+// themselves, 16 rows x [4096, 14336 x 2], 224 workgroups: 32 KB of weights on their way per CU (three stages) 43.0 us, 48 KB
+// (four) 44.5, 64 KB 44.7, 96 KB 45.2 - but with fewer workgroups, or other distances in memory, 48 KB (ring_fourth_stage).
 //
 // 64-deep k tiles: an activation row, and a K-contiguous weight column, is then read in whole 128-byte lines.
 // Both operands go global -> LDS without passing through registers (1 KB per wave instruction), XOR-swizzled by the
@@ -49,9 +49,7 @@ struct RingTile {
 // other's LDS reads: 128 x 256 at 512 rows 138 -> 136 us, 64 x 128 at 64 rows of [4096, 14336 x 2] 44.7 -> 44.2 us).
 // Non-temporal weights where one block of at most 32 rows sees them: 16 rows x [18176, 4544] in 7 parts 29.6 -> 27.1 us
 // (6.1 TB/s), x [14336, 4096] in 8 parts 22.6 -> 21.2 us; at 64 rows the gain is gone (42.7 -> 43.6, 25.1 -> 23.6 us).
-// That tile has three stages, not four: whole calls of 16 tokens, Llama-3-8B FFN block 83.2 -> 80.4 us, Q/K/V block against
-// 1024 keys 39.2 -> 38.9, one token against 4095 keys 21.6 -> 21.4; others of 1 to 32 rows level to 3 % faster - but for
-// row-major weights whose rows are no multiple of 256 bytes (RingTileStraddle).
+// That tile has three stages, or four (ring_fourth_stage).
 #define TRI_RING_TILES(X)        \
   X(0, 32, 128, 1, 4, 4, false)  \
   X(1, 64, 64, 2, 2, 5, false)   \
@@ -63,11 +61,31 @@ struct RingTile {
   X(7, 160, 256, 1, 4, 3, false) \
   X(8, 32, 128, 1, 4, 3, true)
 constexpr int kRingTiles = 9;
-// Tile 8 with a fourth stage, for row-major weights whose rows are no multiple of 256 bytes apart: a tile's 256 bytes of a
-// row then lie across two such blocks of memory, and 48 KB on their way are worth more than 32 (16 rows x [4544, 4544 x 2]
-// 17.0 -> 16.4 us, x [4544, 4544 x 3] 22.5 -> 21.7, x [18176, 4544] level).
-using RingTileStraddle = RingTile<32, 128, 1, 4, 4, true>;
-inline bool ring_rows_straddle(int64_t ldw) { return (ldw & 127) != 0; }  // (several distances or-ed together)
+constexpr int kRingTileOneBlock = 8;  // the non-temporal tile, for a single row block
+// Tile 8 with a fourth stage: 48 KB of weights on their way per workgroup in place of 32.  A CU with two workgroups has
+// enough with three stages, and more costs time; one with a single workgroup, or none, leaves memory bandwidth unused, the
+// more so the faster the memory is at the distance between rows.  What counts is the last round of workgroups (two a CU).
+// us with three / four stages, one row unless said otherwise:
+//   K-contiguous: [4096, 11008 x 2] in 4 parts, 688 workgroups, 44.3 / 40.1, [2048, 5632 x 2], 176, 14.9 / 14.2, [5120, 13824 x 2],
+//     216, 46.4 / 44.4, [8192, 28672 x 2], 448, 156 / 167, [8192, 8192 x 2], 512, 68.1 / 73.0
+//   rows no multiple of 256 bytes: 16 rows x [4544, 4544], 216, 13.2 / 12.9, [4096, 13632], 107, 30.6 / 25.2, rows 4544 apart x
+//     [4096, 4096], 512, 11.6 / 11.8; no multiple of 1 KB: [4544, 9088 x 2], 142, 36.1 / 32.0, [4096, 18176], 142, 32.2 / 28.4,
+//     [4096, 32000], 250, 40.8 / 42.2
+//   else: [4096, 8192], 64, 29.1 / 26.3, [4096, 12288], 192, 22.1 / 22.1, 16 rows x [4096, 6144], 240, 14.1 / 14.6, x [4096, 28672],
+//     224, 38.4 / 39.6; halves (a tile takes 128 bytes of a row from each of two matrices) [4096, 8192 x 2], 128, 35.6 / 36.2
+// Over 960 K-contiguous and 1170 row-major plans (K 1024 to 18176, 1 to 32 rows) the rule's choice is on average 0.3 and 0.1 %
+// slower than the better of the two, at worst 10 % (K-contiguous, K = 14336 in 7 parts, 504 workgroups) and 2.5 %; three
+// everywhere 2.3 and 0.4 %, four everywhere 0.7 and 1.5 %.  A column view whose first element is 128 bytes into a line of 256
+// changes nothing ([4096, 4096] three / four 11.6 / 11.9 with it, 11.8 / 12.0 without).
+using RingTileFour = RingTile<32, 128, 1, 4, 4, true>;
+// (ld: distances between rows or columns, several or-ed together)
+inline bool ring_fourth_stage(int workgroups, int64_t ld, bool kcontig, bool halves) {
+  const int last = (workgroups - 1) % 512 + 1;
+  if (kcontig) return last <= 256;
+  if ((ld & 127) != 0) return last < 256;
+  if ((ld & 511) != 0) return last < 224;
+  return !halves && workgroups < 176;
+}
 // A product in one part of tile 8 over K-contiguous weights whose columns lie a multiple of 8 KB apart runs on this one
 // instead: two waves, 64 columns, and an XCD's workgroups on neighbouring columns.  At such distances the memory is slow
 // (a kernel that only reads [4096, 28672]: 45.4 us with 224 workgroups of 128 columns, 39.9 with 448 of 64, 37.9 with

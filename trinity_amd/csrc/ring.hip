@@ -234,10 +234,9 @@ static int launch_partial_t(const RingArgs& a, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-constexpr int kRingTileOneBlock = 8;  // the non-temporal tile, for a single row block
-
 int launch_ring_partial(const RingArgs& a, int tile, bool kcontig, hipStream_t stream) {
-  if (!kcontig && tile == kRingTileOneBlock && ring_rows_straddle(a.ldw[0] | a.ldw[1] | a.ldw[2])) return launch_partial_t<RingTileStraddle, false>(a, stream);
+  if (tile == kRingTileOneBlock && ring_fourth_stage((a.ncols + 127) / 128 * a.ksplit, a.ldw[0] | a.ldw[1] | a.ldw[2], kcontig, false))
+    return kcontig ? launch_partial_t<RingTileFour, true>(a, stream) : launch_partial_t<RingTileFour, false>(a, stream);
   switch (tile) {
 #define TRI_RING_CASE(id, bm, bn, wm, wn, nst, nt)                                                  \
   case id:                                                                                      \
@@ -261,10 +260,11 @@ static int launch_epi_t(const GemmArgs& a, hipStream_t stream) {
 
 template <int EPI>
 static int launch_epi(const GemmArgs& a, int tile, hipStream_t stream) {
-  if (a.w_kcontig && tile == kRingTileOneBlock && ((a.ldw | (EPI == EPI_SWIGLU ? a.ldw2 : 0)) & 4095) == 0)
-    return launch_epi_t<RingTileKContig, EPI, true>(a, stream);
-  if (!a.w_kcontig && tile == kRingTileOneBlock && ring_rows_straddle(a.ldw | (EPI == EPI_SWIGLU ? a.ldw2 : 0)))
-    return launch_epi_t<RingTileStraddle, EPI, false>(a, stream);
+  constexpr bool GATED = EPI == EPI_SWIGLU;
+  const int64_t ld = a.ldw | (GATED ? a.ldw2 : 0);
+  if (a.w_kcontig && tile == kRingTileOneBlock && (ld & 4095) == 0) return launch_epi_t<RingTileKContig, EPI, true>(a, stream);
+  if (tile == kRingTileOneBlock && ring_fourth_stage(((GATED ? 2 : 1) * a.N + 127) / 128, ld, a.w_kcontig != 0, GATED))
+    return a.w_kcontig ? launch_epi_t<RingTileFour, EPI, true>(a, stream) : launch_epi_t<RingTileFour, EPI, false>(a, stream);
   switch (tile) {
 #define TRI_RING_CASE(id, bm, bn, wm, wn, nst, nt)                                                       \
   case id:                                                                                           \
