@@ -224,3 +224,41 @@ def test_stages_of_gated_products(rn, M, K, F, kcontig, bf16):
 @pytest.mark.parametrize("kcontig", [False, True])
 def test_stages_of_the_projection(rn, S, N, Hq, Hkv, D, qknorm, kcontig):
     test_qkv_projection(rn, S, N, Hq, Hkv, D, qknorm, kcontig)
+
+
+# K-contiguous columns 8 KB apart, 64 a workgroup: ragged last tiles, grids that are no multiple of the eight XCDs, plans in one
+# part and (24 rows x [4096, 16392]) a plan in parts that this tile replaces; 1025 workgroups
+@pytest.mark.parametrize("M,K,N", [(24, 544, 17000), (17, 1056, 32776), (24, 4096, 16392), (1, 1056, 28680), (32, 1088, 17032)])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_narrow_tiles(rn, M, K, N, bf16):
+    el, ok = (torch.bfloat16, check_bf16) if bf16 else (torch.float16, check)
+    x, r = rn(M, K).to(el), rn(M, N).to(el)
+    w = rn(N, 4096, std=K ** -0.5).to(el)[:, :K].t()
+    ws = torch.empty(ext.gemm_workspace_bytes(M, K, N), dtype=torch.uint8, device="cuda:0")
+    for workspace in (ws, None):
+        buf = torch.full((M, N + 16), 7.0, dtype=el, device="cuda:0")
+        out = buf[:, 8:N + 8]
+        ext.matmul(x, w, r, out, workspace=workspace)
+        ok(out, x.float() @ w.float() + r.float(), "x.w + r")
+        assert (buf[:, :8] == 7).all() and (buf[:, N + 8:] == 7).all()
+    if N % 32 == 0 or bf16:
+        return
+    y = torch.empty(M, 64, dtype=el, device="cuda:0")
+    ext.ffn_gelu(x, w, rn(N, 64, std=N ** -0.5), out, y, workspace=ws)
+    ok(out, torch.nn.functional.gelu(x.float() @ w.float()), "gelu(x.w)")
+
+
+# 449 workgroups, 276 in place of a plan in parts, and 512, whose gate and up columns lie a multiple of 8 KB apart or 4 KB off that
+@pytest.mark.parametrize("M,K,F,shift", [(1, 1056, 14344, 0), (32, 1056, 14344, 0), (17, 4096, 8808, 0), (32, 544, 16384, 0), (32, 544, 16384, 2048)])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_narrow_gated_tiles(rn, M, K, F, shift, bf16):
+    el, ok = (torch.bfloat16, check_bf16) if bf16 else (torch.float16, check)
+    x, rs = rn(M, K).to(el), torch.rand(M, device="cuda:0") + 0.5
+    both = rn(2 * F * 4096 + shift, std=K ** -0.5).to(el)
+    wg, wu = both[:F * 4096].view(F, 4096)[:, :K].t(), both[F * 4096 + shift:].view(F, 4096)[:, :K].t()
+    ws = torch.empty(ext.gemm_workspace_bytes(M, K, 2 * F), dtype=torch.uint8, device="cuda:0")
+    a, b = (x.float() @ wg.float()) * rs[:, None], (x.float() @ wu.float()) * rs[:, None]
+    for workspace in (ws, None):
+        out = torch.full((M, F), float("nan"), dtype=el, device="cuda:0")
+        ext.gateup_swiglu(x, wg, wu, rs, out, workspace=workspace)
+        ok(out, a * torch.sigmoid(a) * b, "gated")

@@ -86,13 +86,9 @@ inline bool ring_fourth_stage(int workgroups, int64_t ld, bool kcontig, bool hal
   if ((ld & 511) != 0) return last < 224;
   return !halves && workgroups < 176;
 }
-// A product in one part of tile 8 over K-contiguous weights whose columns lie a multiple of 8 KB apart runs on this one
-// instead: two waves, 64 columns, and an XCD's workgroups on neighbouring columns.  At such distances the memory is slow
-// (a kernel that only reads [4096, 28672]: 45.4 us with 224 workgroups of 128 columns, 39.9 with 448 of 64, 37.9 with
-// neighbours on one XCD).  Whole launches: 1 row x [4096, 14336 x 2] 42.5 -> 40.2 us, 32 rows 45.4 -> 43.3, 4 rows x
-// [8192, 28672 x 2] 172 -> 151, x [4096, 32768] 58.1 -> 47.6, [8192, 8192 x 2] and [16384, 4096 x 2] level, but
-// [4096, 16384 x 2] 52.0 -> 53.8; other distances are faster on tile 8 (K = 5120, 13824 x 2 46.6 -> 48.9, 3072 32.1 -> 33.0,
-// 2048 46.2 -> 48.1, 10240 96.0 -> 98.0, 4544 level), but for 6144 (65.1 -> 59.5).
+// K-contiguous weights whose columns lie a multiple of 8 KB apart, up to 32 rows (ring_takes_narrow): two waves, 64 columns, and
+// an XCD's workgroups on neighbouring columns.  At such distances the memory is slow (a kernel that only reads [4096, 28672]: 45.4 us
+// with 224 workgroups of 128 columns, 39.9 with 448 of 64, 37.9 with neighbours on one XCD).
 using RingTileKContig = RingTile<32, 64, 1, 2, 5, true>;
 
 // Workgroup id -> (row block, column tile, split): row blocks fastest, so that the workgroups that stream the same

@@ -258,11 +258,13 @@ static int launch_epi_t(const GemmArgs& a, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+constexpr int kRingTileNarrow = kRingTiles;  // (not planned by ring_plan: RingTileKContig)
+
 template <int EPI>
 static int launch_epi(const GemmArgs& a, int tile, hipStream_t stream) {
   constexpr bool GATED = EPI == EPI_SWIGLU;
   const int64_t ld = a.ldw | (GATED ? a.ldw2 : 0);
-  if (a.w_kcontig && tile == kRingTileOneBlock && (ld & 4095) == 0) return launch_epi_t<RingTileKContig, EPI, true>(a, stream);
+  if (tile == kRingTileNarrow) return launch_epi_t<RingTileKContig, EPI, true>(a, stream);
   if (tile == kRingTileOneBlock && ring_fourth_stage(((GATED ? 2 : 1) * a.N + 127) / 128, ld, a.w_kcontig != 0, GATED))
     return a.w_kcontig ? launch_epi_t<RingTileFour, EPI, true>(a, stream) : launch_epi_t<RingTileFour, EPI, false>(a, stream);
   switch (tile) {
@@ -369,21 +371,57 @@ bool ring_gemm_in_place(const GemmArgs& a) {
   return a.ws != nullptr && a.ws_bytes >= (int64_t)a.M * (a.epi == EPI_SWIGLU ? 2 * a.N : a.N) * 4 && shares_memory(a);
 }
 
+// Estimated us of a product in one part on RingTileKContig at columns a power of two apart: the 4-norm of its loads on the
+// busiest CU and of the weights at 6.3 TB/s (K = 4096 and 8192, 1 to 32 rows, 2048 to 57344 columns: 4.7 % rms).
+static float ring_narrow_us(const GemmArgs& a) {
+  const int cols = a.epi == EPI_SWIGLU ? 2 * a.N : a.N, share = ((cols + 63) / 64 + 255) / 256;
+  const float mem = 2.0f * (float)a.K * (float)cols / 6.3e6f, cu = (float)a.K / 64.0f * (share == 1 ? 0.249f : 0.231f * share);
+  const float m2 = mem * mem, c2 = cu * cu;
+  return 3.35f + sqrtf(sqrtf(m2 * m2 + c2 * c2));
+}
+
+// Whether a product takes RingTileKContig, in one part, in place of its plan.  At columns a power of two apart (8, 16, 32 KB) in
+// place of a plan in one part on 128 columns, and of one that its estimate beats by 5 % (the plans' costs know nothing of the
+// slow distances).  us of the 128-column plan / of this tile, one row unless said otherwise: [4096, 14336 x 2] 45.7 / 42.1, 32 rows
+// 46.7 / 44.0, [4096, 32768] 59.5 / 48.2, [8192, 28672 x 2] 156 / 148, 4 rows x [16384, 14336 x 2] 162 / 146; in parts
+// [4096, 6912 x 2] 30.5 / 23.2, [4096, 12288 x 2] 43.0 / 36.7, 24 rows x [4096, 16384] 38.3 / 27.2; of 197 plans one is 4 % slower
+// ([4096, 18176 x 2], 60.6 / 63.0).  Not where the workgroups fill the chip twice and gate and up columns 8 KB apart also lie a
+// multiple of 8 KB from each other, and so meet on the same memory: [4096, 16384 x 2] 56.1 / 58.9, but 55.4 / 48.3 with up 68 KB
+// behind the end of gate; 16 KB apart [8192, 16384 x 2] is 116 / 92.6 all the same.  At other multiples of 8 KB beyond two
+// workgroups a CU only: 4 rows x [12288, 17408 x 2] 174 / 163, but [12288, 14336 x 2] 109 / 111, [12288, 16384 x 2] 122 / 137,
+// [20480, 14336 x 2] 167 / 175.  12 KB apart it is ahead too, by 3 to 14 % (4 rows x [6144, 14336 x 2] 68.2 / 61.3); 4, 20 and 28 KB
+// are mixed ([2048, 14336 x 2] 28.1 / 26.9, [2048, 16384 x 2] 31.5 / 38.5).
+static bool ring_takes_narrow(const GemmArgs& a, const RingPlan& plan) {
+  const bool gated = a.epi == EPI_SWIGLU;
+  const int64_t ld = a.ldw | (gated ? a.ldw2 : 0);
+  if (!a.w_kcontig || a.M > RingTileKContig::BM || (ld & 4095) != 0) return false;
+  const bool whole = plan.tile == kRingTileOneBlock && plan.ksplit == 1;
+  const int wg = ((gated ? 2 : 1) * a.N + RingTileKContig::BN - 1) / RingTileKContig::BN;
+  if (whole && wg > 512) return true;
+  if ((ld & (ld - 1)) != 0) return false;
+  if (gated && ld == 4096 && wg > 480 && wg <= 512 && ((a.w2 - a.w) & 4095) == 0) return false;
+  return whole || ring_narrow_us(a) < 0.95f * plan.us;
+}
+
+// over the whole of K, by the epilogue kernel
+static int launch_whole(const GemmArgs& a, int tile, hipStream_t stream) {
+  int rc = -1;
+  switch (a.epi) {
+    case EPI_NONE: rc = launch_epi<EPI_NONE>(a, tile, stream); break;
+    case EPI_GELU: rc = launch_epi<EPI_GELU>(a, tile, stream); break;
+    case EPI_SWIGLU: rc = launch_epi<EPI_SWIGLU>(a, tile, stream); break;
+  }
+  if (rc != 0 || a.rowstat_out == nullptr) return rc;
+  return launch_rmsnorm(a.out, a.ldo, nullptr, nullptr, 0, a.rowstat_out, a.M, a.N, 0.f, stream);
+}
+
 int launch_ring_gemm(const GemmArgs& a, const RingPlan& plan, hipStream_t stream) {
   if (strip_us(a) < 0.97f * plan.us && !shares_memory(a)) return launch_strip(a, stream);
+  if (ring_takes_narrow(a, plan) && !shares_memory(a)) return launch_whole(a, kRingTileNarrow, stream);
   const bool gated = a.epi == EPI_SWIGLU;
   // A product that overwrites its own input goes through the workspace also in one part: the tiles of the epilogue
   // kernel would store while others still read.
-  if (plan.ksplit == 1 && !ring_gemm_in_place(a)) {
-    int rc = -1;
-    switch (a.epi) {
-      case EPI_NONE: rc = launch_epi<EPI_NONE>(a, plan.tile, stream); break;
-      case EPI_GELU: rc = launch_epi<EPI_GELU>(a, plan.tile, stream); break;
-      case EPI_SWIGLU: rc = launch_epi<EPI_SWIGLU>(a, plan.tile, stream); break;
-    }
-    if (rc != 0 || a.rowstat_out == nullptr) return rc;
-    return launch_rmsnorm(a.out, a.ldo, nullptr, nullptr, 0, a.rowstat_out, a.M, a.N, 0.f, stream);
-  }
+  if (plan.ksplit == 1 && !ring_gemm_in_place(a)) return launch_whole(a, plan.tile, stream);
   RingArgs r = {};
   r.x = a.x; r.ldx = a.ldx; r.M = a.M; r.K = a.K; r.ncols = gated ? 2 * a.N : a.N; r.ksplit = plan.ksplit; r.partial = a.ws;
   r.w[0] = a.w; r.ldw[0] = a.ldw; r.seg_begin[0] = 0;
