@@ -123,3 +123,11 @@ def test_new_rows_from_partial_sums(dev, S, Hq, Hkv, D, P, variant, qknorm):
     for name in ("s1", "s2", "score"):
         if name in got:
             assert_scores(got[name], want[name], name)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,Hq,Hkv,D,P", [(8, 64, 2, 128, 1790), (4, 66, 2, 128, 1800), (5, 66, 2, 128, 1800), (8, 66, 2, 128, 1800)])
+@pytest.mark.parametrize("variant", ["vanilla", "keyformer"])
+def test_new_rows_with_many_workgroups(dev, S, Hq, Hkv, D, P, variant):
+    """512 workgroups, two a CU, and 528, from where more than four tokens are merged by the projection."""
+    test_new_rows_from_partial_sums(dev, S, Hq, Hkv, D, P, variant, True)

@@ -87,14 +87,17 @@ int64_t attn_parts_bytes(const tri_attn_params* p, int S, AttnParts runs) {
 // The few-token attention kernels sum the projection's parts themselves (16-bit caches), one launch less against a round
 // trip to the parts in every workgroup, as long as a workgroup has few of them to read.  Fewer than 2048 keys: 64-wide heads
 // always; 128-wide up to eight tokens (Llama-3-8B heads, 500 keys, whole calls: one token 23.7 -> 21.1 us, 4 24.3 -> 22.0,
-// 8 24.2 -> 23.1; 16 against 1000 25.2 -> 29.1, 32 heads on 32 34.7 -> 35.7, 31 tokens 36.2 -> 43.2).  Beyond: up to four
+// 8 24.2 -> 23.1; 16 against 1000 25.2 -> 29.1, 32 heads on 32 34.7 -> 35.7, 31 tokens 36.2 -> 43.2), or four with more than two
+// workgroups a CU (96 heads on 8, 2000 keys: 4 tokens 60.9 -> 60.0, 8 61.7 -> 62.6).  Beyond: up to four
 // tokens and eight rows of a KV head (one token against 4095 keys 23.1 -> 21.7, two 22.7 -> 21.9; 32 heads on 32, 6000 keys:
 // 44.1 -> 42.0 and, 4 tokens, 44.6 -> 44.1, but 8 45.6 -> 46.7; 16 rows, Llama's at 4 tokens, level; 71 rows of a Falcon
 // token 21.6 -> 24.4).
 inline bool attn_may_merge_proj(const tri_attn_params* p, int S) {
   if (p->kv_fp8) return false;
   if (p->kv_prefix + S >= tri::kSplitMinKeys) return S <= tri::kSplitFusedTokens && S * (p->n_q_heads / p->n_kv_heads) <= tri::kSplitFusedRows;
-  return S <= (p->head_dim == 64 ? tri::kFewMaxQueries : tri::kFewFusedTokens);
+  if (p->head_dim == 64) return S <= tri::kFewMaxQueries;
+  const int64_t wg = (int64_t)((p->kv_prefix + S + tri::kFewKeysPerWg - 1) / tri::kFewKeysPerWg) * p->n_q_heads;
+  return S <= (wg > tri::kFewFusedWorkgroups ? tri::kFewFusedTokensMany : tri::kFewFusedTokens);
 }
 
 // 33 to 64 tokens: one part of the projection is asked for whether or not its plan has parts (without it this would be

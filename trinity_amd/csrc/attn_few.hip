@@ -21,9 +21,13 @@
 namespace tri {
 
 constexpr int kFewTile = 64;        // keys per wave
-constexpr int kFewKeysPerWg = 256;  // keys per workgroup
 constexpr float kNegBig = -1.0e30f; // "no key seen yet" (finite, so that differences stay defined)
 constexpr int kFewWaves = kFewKeysPerWg / kFewTile;
+// FUSED: most tokens, and the room kept for merged rows.  128-wide heads: 72 KB in all, so that a CU holds two workgroups; with room
+// for 32 tokens it held one (64 heads on 8, one token against 2000 keys: whole calls 35.0 -> 31.7 us, unfused 34.0; 8 tokens 36.9
+// -> 32.9, unfused 34.1; level up to 256 workgroups).
+template <int D>
+constexpr int kFewFusedRows = D == 128 ? kFewFusedTokens : kFewMaxQueries;
 
 template <int D>
 __device__ __forceinline__ int few_fv(int row) { return D == 128 ? ((row & 3) << 2) : (((row >> 1) & 1) << 2); }
@@ -57,10 +61,10 @@ __device__ __forceinline__ void attn_few_body(const AttnArgs& a, half_t* lds) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[dt][r] = 0.f;
 
-  // FUSED: merged rows [32][D] of q, new k, new v behind the V tiles and the statistics
+  // FUSED: merged rows of q, new k, new v behind the V tiles and the statistics
   half_t* stage_q = lds + NW * kFewTile * D + NW * 32 * 4 * 2;
-  half_t* stage_k = stage_q + 32 * D;
-  half_t* stage_v = stage_k + 32 * D;
+  half_t* stage_k = stage_q + kFewFusedRows<D> * D;
+  half_t* stage_v = stage_k + kFewFusedRows<D> * D;
   const int qq = l32 < a.S ? l32 : a.S - 1;
   half8v qf[KSTEPS], kf[2][KSTEPS];
 
@@ -679,7 +683,7 @@ int64_t few_attn_workspace_bytes(int S, int Hq, int D, int Ltot) {
 
 template <int D, bool KF, bool FP8, bool FUSED = false, int NW = kFewWaves>
 static int launch_few_t(const AttnArgs& a, hipStream_t stream, int* merge_parts) {
-  constexpr int LDS = NW * kFewTile * D * 2 + NW * 32 * 4 * 4 + (FUSED ? 3 * 32 * D * 2 : 0);
+  constexpr int LDS = NW * kFewTile * D * 2 + NW * 32 * 4 * 4 + (FUSED ? 3 * kFewFusedRows<D> * D * 2 : 0);
   const int nsplit = (a.P + a.S + NW * kFewTile - 1) / (NW * kFewTile);
   constexpr auto kern = attn_few_kernel<D, KF, FP8, FUSED, NW>;
   if (set_max_lds<kern, LDS>() != 0) return -1;
@@ -707,7 +711,7 @@ int launch_attention_few(const AttnArgs& a, hipStream_t stream, int* merge_parts
     return a.D == 128 ? launch_few_t<128, false, true>(a, stream, merge_parts) : launch_few_t<64, false, true>(a, stream, merge_parts);
   }
   if (a.pj != nullptr) {  // q and the new k / v rows are still partial sums of the projection
-    if (a.pj_ksplit < 1 || a.k_w == nullptr || a.v_w == nullptr) return -1;
+    if (a.pj_ksplit < 1 || a.k_w == nullptr || a.v_w == nullptr || a.S > (a.D == 128 ? kFewFusedRows<128> : kFewFusedRows<64>)) return -1;
     if (a.D == 128)
       return kf ? launch_few_t<128, true, false, true>(a, stream, merge_parts) : launch_few_t<128, false, false, true>(a, stream, merge_parts);
     return kf ? launch_few_t<64, true, false, true>(a, stream, merge_parts) : launch_few_t<64, false, false, true>(a, stream, merge_parts);

@@ -179,6 +179,7 @@ int launch_attention(const AttnArgs& a, hipStream_t stream, int* merge_parts = n
 // With at most kFewMaxQueries queries attention is bound by reading the K/V cache once; it then runs split
 // over the key axis (partial results in the workspace) followed by a merge kernel.
 constexpr int kFewMaxQueries = 32;
+constexpr int kFewKeysPerWg = 256;  // keys per workgroup
 int64_t few_attn_workspace_bytes(int S, int Hq, int D, int Ltot);
 int launch_attention_few(const AttnArgs& a, hipStream_t stream, int* merge_parts = nullptr);
 int launch_attention_few_combine(const AttnArgs& a, int nsplit, hipStream_t stream);  // the merge kernel alone
@@ -191,8 +192,9 @@ int64_t split_attn_workspace_bytes(int S, int Hq, int Hkv, int D, int Ltot, bool
 // 2.3x (8 KV heads, head dimension 128) to 3x (1 KV head, 64) on the whole block.
 constexpr int kSplitMinKeys = 2048;
 // Most tokens, and rows (heads of a group x tokens), whose projection's partial sums that kernel adds up itself; most
-// tokens of 128-wide heads for the one-tile-per-wave kernel (attn_may_merge_proj has the measurements).
-constexpr int kSplitFusedRows = 8, kSplitFusedTokens = 4, kFewFusedTokens = 8;
+// tokens of 128-wide heads for the one-tile-per-wave kernel, and where it has more than kFewFusedWorkgroups (two a CU)
+// workgroups (attn_may_merge_proj has the measurements).
+constexpr int kSplitFusedRows = 8, kSplitFusedTokens = 4, kFewFusedTokens = 8, kFewFusedTokensMany = 4, kFewFusedWorkgroups = 512;
 
 // fp8 (OCP e4m3) KV caches, value = scale * fp8: append of the new rows, and 16-bit copies (without the scale)
 // for the kernels that read 16-bit K / V tiles.
