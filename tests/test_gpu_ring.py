@@ -202,8 +202,8 @@ def test_stages_of_plain_products(rn, M, K, N, kcontig, bf16):
         ok(out, x.float() @ w.float() + r.float(), "x.w + r")
 
 
-# 225 workgroups, 257, and 213 and 387 in three parts
-@pytest.mark.parametrize("M,K,F", [(17, 1056, 14344), (32, 544, 16400), (8, 1056, 4544), (3, 2080, 8200)])
+# 225 workgroups, 257, and 213, 387 and 457 in three parts (of 4 KB of a K-contiguous column)
+@pytest.mark.parametrize("M,K,F", [(17, 1056, 14344), (32, 544, 16400), (8, 1056, 4544), (3, 2080, 8200), (3, 6144, 9736)])
 @pytest.mark.parametrize("kcontig", [False, True])
 @pytest.mark.parametrize("bf16", [False, True])
 def test_stages_of_gated_products(rn, M, K, F, kcontig, bf16):

@@ -66,8 +66,13 @@ constexpr int kRingTileOneBlock = 8;  // the non-temporal tile, for a single row
 // enough with three stages, and more costs time; one with a single workgroup, or none, leaves memory bandwidth unused, the
 // more so the faster the memory is at the distance between rows.  What counts is the last round of workgroups (two a CU).
 // us with three / four stages, one row unless said otherwise:
-//   K-contiguous: [4096, 11008 x 2] in 4 parts, 688 workgroups, 44.3 / 40.1, [2048, 5632 x 2], 176, 14.9 / 14.2, [5120, 13824 x 2],
-//     216, 46.4 / 44.4, [8192, 28672 x 2], 448, 156 / 167, [8192, 8192 x 2], 512, 68.1 / 73.0
+//   K-contiguous: [3072, 11008 x 2] in 4 parts, 688 workgroups, 32.1 / 28.9, [2048, 5632 x 2], 176, 14.9 / 14.2, [5120, 13824 x 2],
+//     216, 46.4 / 44.4, [14336, 8192 x 2] in 4 parts, 512, 77.2 / 80.7; columns a multiple of 4 KB apart and parts of as many, from 384
+//     on: [6144, 9728 x 2] in three, 456, 51.6 / 49.1, [14336, 4544 x 2] in seven, 497, 58.1 / 54.1, [2048, 28672 x 2], 448, 47.4 / 44.1,
+//     but [6144, 17408 x 2], 272, 97.8 / 102.3; a power of two of 8 KB and more: 16 rows x [8192, 5120 x 2] in three parts, 240, 36.3 /
+//     38.1, [8192, 28672 x 2], 448, 156 / 167, [8192, 8192 x 2], 512, 68.1 / 73.0, but parts of 4096, 4 rows x
+//     [16384, 15904] in four, 500, 109 / 102, [4096, 32400 x 2], 507, 108 / 96.  (22 KB, K = 11008, would have four there too: 4 rows x
+//     [11008, 28672 x 2], 448, 223 / 214.)
 //   rows no multiple of 256 bytes: 16 rows x [4544, 4544], 216, 13.2 / 12.9, [4096, 13632], 107, 30.6 / 25.2, rows 4544 apart x
 //     [4096, 4096], 512, 11.6 / 11.8; no multiple of 1 KB: [4544, 9088 x 2], 142, 36.1 / 32.0, [4096, 18176], 142, 32.2 / 28.4,
 //     [4096, 32000], 250, 40.8 / 42.2
@@ -78,10 +83,13 @@ constexpr int kRingTileOneBlock = 8;  // the non-temporal tile, for a single row
 // everywhere 2.3 and 0.4 %, four everywhere 0.7 and 1.5 %.  A column view whose first element is 128 bytes into a line of 256
 // changes nothing ([4096, 4096] three / four 11.6 / 11.9 with it, 11.8 / 12.0 without).
 using RingTileFour = RingTile<32, 128, 1, 4, 4, true>;
-// (ld: distances between rows or columns, several or-ed together)
-inline bool ring_fourth_stage(int workgroups, int64_t ld, bool kcontig, bool halves) {
+// (ld: distances between rows or columns, several or-ed together; k_part: K of a workgroup)
+inline bool ring_fourth_stage(int workgroups, int64_t ld, int k_part, bool kcontig, bool halves) {
   const int last = (workgroups - 1) % 512 + 1;
-  if (kcontig) return last <= 256;
+  if (kcontig) {
+    if (ld >= 4096 && (ld & (ld - 1)) == 0) return last < 224 || (last >= 384 && k_part == 4096);
+    return last <= 256 || (last >= 384 && ld % 2048 == 0 && k_part % 2048 == 0);
+  }
   if ((ld & 127) != 0) return last < 256;
   if ((ld & 511) != 0) return last < 224;
   return !halves && workgroups < 176;

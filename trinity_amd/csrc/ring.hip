@@ -235,7 +235,7 @@ static int launch_partial_t(const RingArgs& a, hipStream_t stream) {
 }
 
 int launch_ring_partial(const RingArgs& a, int tile, bool kcontig, hipStream_t stream) {
-  if (tile == kRingTileOneBlock && ring_fourth_stage((a.ncols + 127) / 128 * a.ksplit, a.ldw[0] | a.ldw[1] | a.ldw[2], kcontig, false))
+  if (tile == kRingTileOneBlock && ring_fourth_stage((a.ncols + 127) / 128 * a.ksplit, a.ldw[0] | a.ldw[1] | a.ldw[2], ring_kt_per_part(a.K, a.ksplit) * 64, kcontig, false))
     return kcontig ? launch_partial_t<RingTileFour, true>(a, stream) : launch_partial_t<RingTileFour, false>(a, stream);
   switch (tile) {
 #define TRI_RING_CASE(id, bm, bn, wm, wn, nst, nt)                                                  \
@@ -265,7 +265,7 @@ static int launch_epi(const GemmArgs& a, int tile, hipStream_t stream) {
   constexpr bool GATED = EPI == EPI_SWIGLU;
   const int64_t ld = a.ldw | (GATED ? a.ldw2 : 0);
   if (tile == kRingTileNarrow) return launch_epi_t<RingTileKContig, EPI, true>(a, stream);
-  if (tile == kRingTileOneBlock && ring_fourth_stage(((GATED ? 2 : 1) * a.N + 127) / 128, ld, a.w_kcontig != 0, GATED))
+  if (tile == kRingTileOneBlock && ring_fourth_stage(((GATED ? 2 : 1) * a.N + 127) / 128, ld, a.K, a.w_kcontig != 0, GATED))
     return a.w_kcontig ? launch_epi_t<RingTileFour, EPI, true>(a, stream) : launch_epi_t<RingTileFour, EPI, false>(a, stream);
   switch (tile) {
 #define TRI_RING_CASE(id, bm, bn, wm, wn, nst, nt)                                                       \
@@ -380,27 +380,28 @@ static float ring_narrow_us(const GemmArgs& a) {
   return 3.35f + sqrtf(sqrtf(m2 * m2 + c2 * c2));
 }
 
-// Whether a product takes RingTileKContig, in one part, in place of its plan.  At columns a power of two apart (8, 16, 32 KB) in
-// place of a plan in one part on 128 columns, and of one that its estimate beats by 5 % (the plans' costs know nothing of the
-// slow distances).  us of the 128-column plan / of this tile, one row unless said otherwise: [4096, 14336 x 2] 45.7 / 42.1, 32 rows
-// 46.7 / 44.0, [4096, 32768] 59.5 / 48.2, [8192, 28672 x 2] 156 / 148, 4 rows x [16384, 14336 x 2] 162 / 146; in parts
-// [4096, 6912 x 2] 30.5 / 23.2, [4096, 12288 x 2] 43.0 / 36.7, 24 rows x [4096, 16384] 38.3 / 27.2; of 197 plans one is 4 % slower
-// ([4096, 18176 x 2], 60.6 / 63.0).  Not where the workgroups fill the chip twice and gate and up columns 8 KB apart also lie a
-// multiple of 8 KB from each other, and so meet on the same memory: [4096, 16384 x 2] 56.1 / 58.9, but 55.4 / 48.3 with up 68 KB
-// behind the end of gate; 16 KB apart [8192, 16384 x 2] is 116 / 92.6 all the same.  At other multiples of 8 KB beyond two
-// workgroups a CU only: 4 rows x [12288, 17408 x 2] 174 / 163, but [12288, 14336 x 2] 109 / 111, [12288, 16384 x 2] 122 / 137,
-// [20480, 14336 x 2] 167 / 175.  12 KB apart it is ahead too, by 3 to 14 % (4 rows x [6144, 14336 x 2] 68.2 / 61.3); 4, 20 and 28 KB
-// are mixed ([2048, 14336 x 2] 28.1 / 26.9, [2048, 16384 x 2] 31.5 / 38.5).
+// Whether a product takes RingTileKContig, in one part, in place of its plan (us of the 128-column plan / of this tile, one row
+// unless said otherwise).  Columns a power of two apart (8, 16, 32 KB): in place of a plan in one part on 128 columns
+// ([4096, 14336 x 2] 45.7 / 42.1, 32 rows 46.7 / 44.0, [4096, 32768] 59.5 / 48.2, [8192, 28672 x 2] 156 / 148, 4 rows x
+// [16384, 14336 x 2] 162 / 146) and of any plan that its estimate beats by 5 %, as the plans' costs know nothing of the slow distances
+// (in parts [4096, 6912 x 2] 30.5 / 23.2, [4096, 12288 x 2] 43.0 / 36.7, 24 rows x [4096, 16384] 38.3 / 27.2; with few workgroups beyond
+// two a CU the estimate is too low, [4096, 18176 x 2] in 3 parts 60.6 / 63.0).  But not where the workgroups just fill the chip (512,
+// two a CU, or 1024) and gate and up columns 8 KB apart also lie a multiple of 8 KB from each other, and so meet on the same memory:
+// [4096, 16384 x 2] 56.1 / 58.9, [4096, 32768 x 2] 99.6 / 113, while with up 68 KB behind the end of gate [4096, 16384 x 2] is 55.4 /
+// 48.3, and 16 KB apart [8192, 16384 x 2] 116 / 92.6 all the same.  At other multiples of 8 KB in place of
+// a plan in one part, gated ones beyond two workgroups a CU: [12288, 28672] 116 / 111, [12288, 17408 x 2] 174 / 163, but
+// [12288, 14336 x 2] 109 / 111, [12288, 16384 x 2] 122 / 137, [20480, 14336 x 2] 167 / 175.  12 KB apart it is ahead too, by 3 to 14 %
+// (4 rows x [6144, 14336 x 2] 68.2 / 61.3); 4, 20 and 28 KB are mixed ([2048, 14336 x 2] 28.1 / 26.9, [2048, 16384 x 2] 31.5 / 38.5).
 static bool ring_takes_narrow(const GemmArgs& a, const RingPlan& plan) {
   const bool gated = a.epi == EPI_SWIGLU;
   const int64_t ld = a.ldw | (gated ? a.ldw2 : 0);
   if (!a.w_kcontig || a.M > RingTileKContig::BM || (ld & 4095) != 0) return false;
   const bool whole = plan.tile == kRingTileOneBlock && plan.ksplit == 1;
   const int wg = ((gated ? 2 : 1) * a.N + RingTileKContig::BN - 1) / RingTileKContig::BN;
-  if (whole && wg > 512) return true;
-  if ((ld & (ld - 1)) != 0) return false;
-  if (gated && ld == 4096 && wg > 480 && wg <= 512 && ((a.w2 - a.w) & 4095) == 0) return false;
-  return whole || ring_narrow_us(a) < 0.95f * plan.us;
+  if ((ld & (ld - 1)) != 0) return whole && (!gated || wg > 512);
+  const bool just_full = (wg - 1) % 512 >= 496 || (wg > 512 && wg <= 528);
+  if (gated && ld == 4096 && just_full && ((a.w2 - a.w) & 4095) == 0) return false;
+  return whole || ((wg <= 512 || wg > 576) && ring_narrow_us(a) < 0.95f * plan.us);
 }
 
 // over the whole of K, by the epilogue kernel
