@@ -417,7 +417,7 @@ static int launch_whole(const GemmArgs& a, int tile, hipStream_t stream) {
 }
 
 int launch_ring_gemm(const GemmArgs& a, const RingPlan& plan, hipStream_t stream) {
-  if (strip_us(a) < 0.97f * plan.us && !shares_memory(a)) return launch_strip(a, stream);
+  if (strip_us(a) < (plan.tile == 1 && plan.ksplit == 1 ? 0.88f : 0.92f) * plan.us && !shares_memory(a)) return launch_strip(a, stream);
   if (ring_takes_narrow(a, plan) && !shares_memory(a)) return launch_whole(a, kRingTileNarrow, stream);
   const bool gated = a.epi == EPI_SWIGLU;
   // A product that overwrites its own input goes through the workspace also in one part: the tiles of the epilogue

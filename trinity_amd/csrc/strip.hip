@@ -8,6 +8,8 @@
 #include "gemm_core.h"
 #include "launch.h"
 
+#include <math.h>
+
 namespace tri {
 
 // D[16 x 16] += A[16 x 32] * B[32 x 16].  Lane l supplies row (l % 16) of A and column (l % 16) of B, eight consecutive k
@@ -121,18 +123,21 @@ __global__ __launch_bounds__(kStripWaves * 64) void strip_kernel(GemmArgs a) {
   *reinterpret_cast<half4v*>(a.out + (int64_t)c * a.ldo + n) = h;
 }
 
-// Estimated us of a product (1e30: not for this kernel), to compare with a ring plan's: the weights at 6.1 TB/s, or what
-// the busiest CU has to load, activations included, at 38 GB/s (up to two workgroups a CU everything is placed at once, more
-// even out), and half a us to start each workgroup of a CU.  Estimated, measured and the ring kernels' time with their
-// merge: one row x [4096, 4096] 9.0, 7.6, 13.7 us, [4096, 14336] 24, 20.7, 30.5, [14336, 4096] 23, 21, 26, [5120, 5120] 13,
-// 13.2, 15.7; 8 rows x [2048, 2048] 5.6, 5.3, 7.9, 4 x [4544, 18176] 29, 27.3, 32; not taken: 16 rows x [14336, 4096] 28, 27,
-// 26, one row x [18176, 4544] (284 workgroups) 36, 36, 32, 8 x [13824, 5120] 39, 34, 27, 4 x [1024, 16384] 11, 9.0, 8.0.
+// Estimated us of a product (1e30: not for this kernel), to compare with a ring plan's: of the weights at 12 TB/s and of what the
+// busiest CU has to load, activations included, at 58 GB/s the 3/2-norm (up to three workgroups a CU everything is placed at once,
+// more even out), and 0.6 us to start each workgroup of a CU.  Over 1690 products (1 to 16 rows, K 512 to 18176, 512 to 32768
+// columns) 1 % low on average with a deviation of 7 %; the ring plans' costs are 8 % high there for 64 x 64 tiles in one part and 4 to
+// 6 % for most others.  Taken below 0.88 and 0.92 of those (launch_ring_gemm): 888 of the 1690, 51 of them slower than the plan by more
+// than 2 %, at worst 13.  us, and those of the ring kernels with their merge: one row x [4096, 4096] 7.6, 13.7, [4096, 14336] 21.0,
+// 29.6, [14336, 4096] 21.9, 24.0, 12 rows 24.7, 23.9, 4 x [4544, 18176] 27.6, 32.5; not taken: 14 x [14336, 4096] 25.6, 23.9, 12 x
+// [2048, 9728] 13.4, 11.8, 10 x [512, 4672] 5.5, 4.8, 6 x [14336, 9728] 53.6, 46.3.
 float strip_us(const GemmArgs& a) {
   if (!a.w_kcontig || a.epi == EPI_SWIGLU || a.rowstat_out != nullptr || a.M > 16 || a.K < 512 || a.K % 32 != 0 || a.N % 8 != 0) return 1e30f;
   const int wg = (a.N + kStripCols - 1) / kStripCols;
-  const float share = wg <= 512 ? (float)((wg + 255) / 256) : (float)wg / 256.0f + 0.5f;
-  const float hbm = 2.0f * (float)a.K * (float)a.N / 6.1e6f, cu = share * (float)(kStripCols + a.M) * 2.0f * (float)a.K / 38e3f;
-  return 3.0f + (float)wg / 512.0f + (hbm > cu ? hbm : cu);
+  const float per = (float)wg / 256.0f, share = wg <= 768 ? (float)((wg + 255) / 256) : per + 0.5f;
+  const float hbm = 2.0f * (float)a.K * (float)a.N / 12e6f, cu = share * ((float)kStripCols + 1.25f * (float)a.M) * 2.0f * (float)a.K / 58e3f;
+  const float sum = cbrtf(hbm * sqrtf(hbm) + cu * sqrtf(cu));
+  return 2.8f + 0.6f * per + sum * sum;
 }
 
 template <int EPI>
