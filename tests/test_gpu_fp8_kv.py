@@ -177,3 +177,28 @@ def test_odd_and_even_numbers_of_tile_steps(dev, S, D, P):
                                 k_scale=K_SCALE, v_scale=V_SCALE)
     got = _run(t, dev, "vanilla", Hq=Hq, Hkv=Hkv, D=D, P=P, causal=True)
     assert_close(got["O2"], want["O2"], 1e-2, 1e-2, "O2")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("group,S,P", [(1, 1, 300), (1, 1, 2100), (40, 2, 2300), (1, 40, 200)])
+def test_a_nan_code_stays_nan(dev, dtype, D, group, S, P):
+    """Both NaN codes in one row of V: their columns are NaN for every token, all others are the average of ones."""
+    Hkv, N = 2, 256
+    Hq = group * Hkv
+    vc = torch.ones(Hkv, P + S, D).to(F8)
+    vc.view(torch.uint8)[0, P // 2, 3], vc.view(torch.uint8)[0, P // 2, D - 1] = 0x7F, 0xFF
+    kc = torch.zeros(Hkv, P + S, D).to(F8).to(dev)
+    w = lambda h: torch.zeros(N, h * D, dtype=dtype, device=dev)
+    p = ext.attn_params(Hq, Hkv, D, S, kv_prefix=P, causal=True, rms_eps=1e-5, kv_fp8=True, k_scale=1.0, v_scale=1.0)
+    out = torch.zeros(S, Hq * D, dtype=dtype, device=dev)
+    ext.qkv_attention(torch.zeros(S, N, dtype=dtype, device=dev), None, w(Hq), w(Hkv), w(Hkv), kc, vc.to(dev), scratch_for(p, N, dev), None, out, p)
+    got = out.cpu().float().view(S, Hkv, group, D)
+    bad = torch.zeros(Hkv, D, dtype=torch.bool)
+    bad[0, 3] = bad[0, D - 1] = True
+    assert torch.equal(got.isnan(), bad.view(1, Hkv, 1, D).expand_as(got))
+    want = (P / (P + 1.0 + torch.arange(S))).view(S, 1, 1, 1).expand_as(got)
+    ok = ~got.isnan()
+    # (one rounding to the element type, and fp32 sums of at most P + S equal terms)
+    eps = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+    assert ((got - want)[ok].abs() <= (eps + 1e-5) * want[ok]).all()

@@ -11,9 +11,10 @@ import pytest
 import torch
 
 import oracle
-from gpu_util import projection_parts, run_qkv
+from gpu_util import projection_parts, run_qkv, scratch_for
 from test_gpu_attention import assert_scores
 from test_gpu_fp8_kv import K_SCALE, V_SCALE, _fp8_inputs, _run
+from trinity_amd import ext
 from util import assert_close, attn_inputs
 
 N = 64
@@ -131,3 +132,53 @@ def test_new_rows_from_partial_sums(dev, S, Hq, Hkv, D, P, variant, qknorm):
 def test_new_rows_with_many_workgroups(dev, S, Hq, Hkv, D, P, variant):
     """512 workgroups, two a CU, and 528, from where more than four tokens are merged by the projection."""
     test_new_rows_from_partial_sums(dev, S, Hq, Hkv, D, P, variant, True)
+
+
+FORMS = ["bf16", "bf16 keyformer", "noise", "tau", "unmasked", "strided", "fewest runs"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,Hq,Hkv,D,P", FUSED)
+@pytest.mark.parametrize("form", FORMS)
+def test_forms_of_calls_that_merge_the_projection(dev, S, Hq, Hkv, D, P, form):
+    """As above (the prefix has no values, the new rows' places hold NaN): bf16 elements, a noise tensor or temperature of
+    the caller's (the kernels' general noise), no mask, caches with padded rows and heads, and scratch memory that has room for
+    the fewest runs of the key axis only.  bf16 rounds to 2^-8 in place of 2^-11: eight times the tolerances."""
+    n, bf = 1024, form.startswith("bf16")
+    el, wide = (torch.bfloat16, 8.0) if bf else (torch.float16, 1.0)
+    assert projection_parts(n, S, Hq, Hkv, D, P) > 1.5
+    t = {k: v.to(el) for k, v in attn_inputs(S, n, Hq, Hkv, D, P=P, w_std=0.96 * n ** -0.5).items()}
+    t["v_cache"][:, :P] = 0
+    t["k_cache"][:, P:], t["v_cache"][:, P:] = math.nan, math.nan
+    clean = {k: t[k].nan_to_num(0.0) for k in ("k_cache", "v_cache")}
+    causal, tau = form != "unmasked", 1.5 if form == "tau" else 1.0
+    keyformer = form in ("bf16 keyformer", "noise", "tau")
+    noise = -torch.log(-torch.log(torch.rand(Hq, S, P + S).clamp(1e-6, 1 - 1e-6))).to(el) if form == "noise" else None
+    scale = 1.0 / math.sqrt(D)
+    more = dict(keyformer=True, noise=noise, noise_seed=None if noise is not None else 5, tau=tau) if keyformer else {}
+    want = oracle.qkv_attention(t["x"], t["wq"], t["wk"], t["wv"], n_q_heads=Hq, n_kv_heads=Hkv, head_dim=D, scale=scale, causal=causal,
+                                kv_prefix=P, elem=el, **clean, **more)
+    d = {k: v.to(dev) for k, v in t.items()}
+    pad = (3, 16) if form == "strided" else (0, 0)
+    bufs = [torch.full((Hkv, P + S + pad[0], D + pad[1]), 7.0, dtype=el, device=dev) for _ in range(2)]
+    kc, vc = (b[:, :P + S, :D].copy_(d[c]) for b, c in zip(bufs, ("k_cache", "v_cache")))
+    p = ext.attn_params(Hq, Hkv, D, S, kv_prefix=P, scale=scale, causal=causal, tau=tau, noise_seed=5)
+    scratch = scratch_for(p, n, dev)
+    if form == "fewest runs":
+        scratch = scratch[:-256]
+    out = torch.full((S, Hq * D), math.nan, dtype=el, device=dev)
+    score = torch.full((Hq, P + S), math.nan, dtype=torch.float32, device=dev)
+    if keyformer:
+        ext.keyformer(d["x"], None, d["wq"], d["wk"], d["wv"], kc, vc, scratch, noise.to(dev) if noise is not None else None, out, score, p)
+    else:
+        ext.qkv_attention(d["x"], None, d["wq"], d["wk"], d["wv"], kc, vc, scratch, None, out, p)
+    torch.cuda.synchronize()
+    assert_close(out, want["O2"], 1e-2 * wide, 1e-2 * wide * want["O2"].float().std().item(), "O2")
+    assert_close(kc[:, P:], want["k_new"], 2e-3 * wide, 2e-3 * wide, "k rows")
+    assert_close(vc[:, P:], want["v_new"], 2e-3 * wide, 2e-3 * wide, "v rows")
+    if keyformer:
+        a, e = score.cpu().double(), want["score"].double()
+        assert ((a - e).abs() <= wide * (1e-3 * e.abs() + 1e-4 * e.abs().amax(-1, keepdim=True)) + 1e-7).all(), "score"
+    for b in bufs:
+        assert (b[:, P + S:] == 7).all() and (b[:, :, D:] == 7).all()
+    assert torch.equal(kc[:, :P].cpu(), t["k_cache"][:, :P])
