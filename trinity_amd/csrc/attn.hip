@@ -100,8 +100,9 @@ __device__ __forceinline__ void attn_wg_map(int id, int Hq, int nqb, int& qb, in
 //
 // FUSED (SPLIT, 16-bit caches, at most kSplitFusedRows rows): q and the new rows of k / v come from the partial sums of a
 // split-K projection (AttnArgs::pj).  Every workgroup sums its q rows, those whose tiles hold new keys the new k / v
-// rows too, which then replace the stale rows of the tile in LDS; one workgroup each stores them where the unfused
-// projection would have.  One launch less, against one round trip to the partial sums in every workgroup.
+// rows too, which then replace the stale rows of the tile in LDS.  q is stored by the first run's workgroups, k / v by those of
+// every run that has a tile with new keys - two where these lie across a tile's end, which store the same values.  One launch
+// less, against one round trip to the partial sums in every workgroup.
 template <int D, int QT, int KF, int KW, bool SPLIT = false, bool FP8 = false, int HALVES = 1, bool FUSED = false>
 __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, half_t* lds, const half_t* __restrict__ qglob) {
   // (qglob = a.q; the qualifier is what keeps the compiler from waiting for the loads in flight before the
@@ -1163,11 +1164,12 @@ static int launch_attn_split_t(const AttnArgs& a, int nwg, hipStream_t stream) {
   if constexpr (!FP8)
     if (a.S > kFewMaxQueries) return launch_attn_split_h<D, KF, FP8, 1, 2>(a, nwg, stream);
   if ((a.Hq / a.Hkv) * a.S <= kSplitHalvesRows) return launch_attn_split_h<D, KF, FP8, 2, 1>(a, nwg, stream);
-  // fp8 with whole tiles per wave keeps one tile on its way: where a CU has one workgroup at most and a long run to walk,
-  // eight waves on pairs of tiles keep two: from seven tiles a run (whole calls at some 4.5, 6 and 8 tiles a run: 71 heads
-  // on one, one token 23.8 -> 24.2, 25.6 level, 26.4 -> 25.7 us, 4 tokens 24.1 -> 24.8, 25.1 -> 24.9, 26.9 -> 26.4;
-  // Llama-3-8B heads, 24 tokens 35.0 -> 35.8, 34.8 level, 36.9 -> 36.2, 32 tokens 37.1 -> 38.7, 37.6 -> 38.1, 40.0 -> 39.6;
-  // 28 against 32000 keys, 16 tiles, 48.0 -> 45.1; 16-bit tiles, which do not pass through registers, 53.5 -> 54.9 there)
+  // fp8 where a CU has one workgroup at most and a long run to walk: eight waves on pairs of tiles.  128-wide heads keep two tiles
+  // on their way with them, one without; 64-wide heads two either way.  Both are ahead from seven tiles a run (whole calls at some
+  // 4.5, 6 and 8 tiles a run: Llama-3-8B heads, 24 tokens 35.0 -> 35.8 us, 34.8 level, 36.9 -> 36.2, 32 tokens 37.1 -> 38.7, 37.6 -> 38.1,
+  // 40.0 -> 39.6, 28 against 32000 keys, 16 tiles, 48.0 -> 45.1; 71 heads of 64 on one, 4 tokens 25.4 -> 26.0, 26.2 -> 26.0, 27.8 -> 27.2,
+  // 16 tiles 34.0 -> 31.7, one token, 4, 6 and 8 tiles, 24.3 -> 24.4, 25.9 -> 25.6, 27.2 -> 26.4; 64 of 64 on 8, 16 tokens 29.1 -> 29.7,
+  // 30.1 -> 30.6, 33.0 -> 32.4; 16-bit tiles, which do not pass through registers, 28 against 32000 keys 53.5 -> 54.9)
   if constexpr (FP8)
     if (nwg <= kSplitPairWorkgroups && (a.P + a.S) / kKeyTile >= kSplitPairTiles * a.split_runs)
       return launch_attn_split_h<D, KF, FP8, 1, 2>(a, nwg, stream);
