@@ -70,7 +70,7 @@ constexpr int kRingTileOneBlock = 8;  // the non-temporal tile, for a single row
 //     216, 46.4 / 44.4, [14336, 8192 x 2] in 4 parts, 512, 77.2 / 80.7; columns a multiple of 4 KB apart and parts of as many, from 384
 //     on: [6144, 9728 x 2] in three, 456, 51.6 / 49.1, [14336, 4544 x 2] in seven, 497, 58.1 / 54.1, [2048, 28672 x 2], 448, 47.4 / 44.1,
 //     but [6144, 17408 x 2], 272, 97.8 / 102.3; a power of two of 8 KB and more: 16 rows x [8192, 5120 x 2] in three parts, 240, 36.3 /
-//     38.1, [8192, 28672 x 2], 448, 156 / 167, [8192, 8192 x 2], 512, 68.1 / 73.0, but parts of 4096, 4 rows x
+//     38.1, [4096, 12288 x 2] in four, 768, 44.6 / 43.0, [8192, 28672 x 2], 448, 156 / 167, [8192, 8192 x 2], 512, 68.1 / 73.0, but parts of 4096, 4 rows x
 //     [16384, 15904] in four, 500, 109 / 102, [4096, 32400 x 2], 507, 108 / 96.  (22 KB, K = 11008, would have four there too: 4 rows x
 //     [11008, 28672 x 2], 448, 223 / 214.)
 //   rows no multiple of 256 bytes: 16 rows x [4544, 4544], 216, 13.2 / 12.9, [4096, 13632], 107, 30.6 / 25.2, rows 4544 apart x
@@ -83,11 +83,13 @@ constexpr int kRingTileOneBlock = 8;  // the non-temporal tile, for a single row
 // everywhere 2.3 and 0.4 %, four everywhere 0.7 and 1.5 %.  A column view whose first element is 128 bytes into a line of 256
 // changes nothing ([4096, 4096] three / four 11.6 / 11.9 with it, 11.8 / 12.0 without).
 using RingTileFour = RingTile<32, 128, 1, 4, 4, true>;
+// K-contiguous columns a power of two of 8 KB and more apart: the memory is slow there.
+inline bool ring_slow_columns(int64_t ld) { return ld >= 4096 && (ld & (ld - 1)) == 0; }
 // (ld: distances between rows or columns, several or-ed together; k_part: K of a workgroup)
 inline bool ring_fourth_stage(int workgroups, int64_t ld, int k_part, bool kcontig, bool halves) {
   const int last = (workgroups - 1) % 512 + 1;
   if (kcontig) {
-    if (ld >= 4096 && (ld & (ld - 1)) == 0) return last < 224 || (last >= 384 && k_part == 4096);
+    if (ring_slow_columns(ld)) return last < (workgroups <= 256 ? 224 : 257) || (last >= 384 && k_part == 4096);
     return last <= 256 || (last >= 384 && ld % 2048 == 0 && k_part % 2048 == 0);
   }
   if ((ld & 127) != 0) return last < 256;

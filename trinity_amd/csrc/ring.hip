@@ -384,12 +384,13 @@ static float ring_narrow_us(const GemmArgs& a) {
 // unless said otherwise).  Columns a power of two apart (8, 16, 32 KB): in place of a plan in one part on 128 columns
 // ([4096, 14336 x 2] 45.7 / 42.1, 32 rows 46.7 / 44.0, [4096, 32768] 59.5 / 48.2, [8192, 28672 x 2] 156 / 148, 4 rows x
 // [16384, 14336 x 2] 162 / 146) and of any plan that its estimate beats by 5 %, as the plans' costs know nothing of the slow distances
-// (in parts [4096, 6912 x 2] 30.5 / 23.2, [4096, 12288 x 2] 43.0 / 36.7, 24 rows x [4096, 16384] 38.3 / 27.2; with few workgroups beyond
-// two a CU the estimate is too low, [4096, 18176 x 2] in 3 parts 60.6 / 63.0).  But not where the workgroups just fill the chip (512,
-// two a CU, or 1024) and gate and up columns 8 KB apart also lie a multiple of 8 KB from each other, and so meet on the same memory:
-// [4096, 16384 x 2] 56.1 / 58.9, [4096, 32768 x 2] 99.6 / 113, while with up 68 KB behind the end of gate [4096, 16384 x 2] is 55.4 /
-// 48.3, and 16 KB apart [8192, 16384 x 2] 116 / 92.6 all the same.  At other multiples of 8 KB in place of
-// a plan in one part, gated ones beyond two workgroups a CU: [12288, 28672] 116 / 111, [12288, 17408 x 2] 174 / 163, but
+// (in parts [4096, 6912 x 2] 30.5 / 23.2, 32 rows x [4096, 12288 x 2] 50.1 / 40.6, 24 x [4096, 16384] 38.3 / 27.2; of 185 products 67
+// take it, none slower; others would be faster, one row x [4096, 12288 x 2] 43.0 / 36.7, but by a margin of 0 some slower, 32 rows x
+// [4096, 9728 x 2] 36.9 / 39.7; with few workgroups beyond two a CU the estimate is too low, [4096, 18176 x 2] 60.6 / 63.0).  But not
+// where the workgroups just fill the chip (512, two a CU, or 1024) and gate and up columns 8 KB apart also lie a multiple of 8 KB
+// from each other, and so meet on the same memory: [4096, 16384 x 2] 56.1 / 58.9, [4096, 32768 x 2] 99.6 / 113, while with up 68 KB
+// behind the end of gate [4096, 16384 x 2] is 55.4 / 48.3, and 16 KB apart [8192, 16384 x 2] 116 / 92.6 all the same.  At other
+// multiples of 8 KB in place of a plan in one part, gated ones beyond two workgroups a CU: [12288, 28672] 116 / 111, [12288, 17408 x 2] 174 / 163, but
 // [12288, 14336 x 2] 109 / 111, [12288, 16384 x 2] 122 / 137, [20480, 14336 x 2] 167 / 175.  12 KB apart it is ahead too, by 3 to 14 %
 // (4 rows x [6144, 14336 x 2] 68.2 / 61.3); 4, 20 and 28 KB are mixed ([2048, 14336 x 2] 28.1 / 26.9, [2048, 16384 x 2] 31.5 / 38.5).
 static bool ring_takes_narrow(const GemmArgs& a, const RingPlan& plan) {
@@ -398,7 +399,7 @@ static bool ring_takes_narrow(const GemmArgs& a, const RingPlan& plan) {
   if (!a.w_kcontig || a.M > RingTileKContig::BM || (ld & 4095) != 0) return false;
   const bool whole = plan.tile == kRingTileOneBlock && plan.ksplit == 1;
   const int wg = ((gated ? 2 : 1) * a.N + RingTileKContig::BN - 1) / RingTileKContig::BN;
-  if ((ld & (ld - 1)) != 0) return whole && (!gated || wg > 512);
+  if (!ring_slow_columns(ld)) return whole && (!gated || wg > 512);
   const bool just_full = (wg - 1) % 512 >= 496 || (wg > 512 && wg <= 528);
   if (gated && ld == 4096 && just_full && ((a.w2 - a.w) & 4095) == 0) return false;
   return whole || ((wg <= 512 || wg > 576) && ring_narrow_us(a) < 0.95f * plan.us);
@@ -417,8 +418,11 @@ static int launch_whole(const GemmArgs& a, int tile, hipStream_t stream) {
 }
 
 int launch_ring_gemm(const GemmArgs& a, const RingPlan& plan, hipStream_t stream) {
-  if (strip_us(a) < (plan.tile == 1 && plan.ksplit == 1 ? 0.88f : 0.92f) * plan.us && !shares_memory(a)) return launch_strip(a, stream);
-  if (ring_takes_narrow(a, plan) && !shares_memory(a)) return launch_whole(a, kRingTileNarrow, stream);
+  // the plans' costs are 8 % high for 64 x 64 tiles in one part, 4 to 6 % for most others, and 2 % low at slow distances (strip.hip)
+  const float strip = strip_us(a), margin = plan.tile == 1 && plan.ksplit == 1 ? 0.88f : (ring_slow_columns(a.ldw) ? 1.0f : 0.92f);
+  const bool narrow = ring_takes_narrow(a, plan);
+  if (strip < margin * plan.us && !(narrow && ring_narrow_us(a) < strip) && !shares_memory(a)) return launch_strip(a, stream);
+  if (narrow && !shares_memory(a)) return launch_whole(a, kRingTileNarrow, stream);
   const bool gated = a.epi == EPI_SWIGLU;
   // A product that overwrites its own input goes through the workspace also in one part: the tiles of the epilogue
   // kernel would store while others still read.

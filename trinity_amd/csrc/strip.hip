@@ -126,11 +126,12 @@ __global__ __launch_bounds__(kStripWaves * 64) void strip_kernel(GemmArgs a) {
 // Estimated us of a product (1e30: not for this kernel), to compare with a ring plan's: of the weights at 12 TB/s and of what the
 // busiest CU has to load, activations included, at 58 GB/s the 3/2-norm (up to three workgroups a CU everything is placed at once,
 // more even out), and 0.6 us to start each workgroup of a CU.  Over 1690 products (1 to 16 rows, K 512 to 18176, 512 to 32768
-// columns) 1 % low on average with a deviation of 7 %; the ring plans' costs are 8 % high there for 64 x 64 tiles in one part and 4 to
-// 6 % for most others.  Taken below 0.88 and 0.92 of those (launch_ring_gemm): 888 of the 1690, 51 of them slower than the plan by more
-// than 2 %, at worst 13.  us, and those of the ring kernels with their merge: one row x [4096, 4096] 7.6, 13.7, [4096, 14336] 21.0,
-// 29.6, [14336, 4096] 21.9, 24.0, 12 rows 24.7, 23.9, 4 x [4544, 18176] 27.6, 32.5; not taken: 14 x [14336, 4096] 25.6, 23.9, 12 x
-// [2048, 9728] 13.4, 11.8, 10 x [512, 4672] 5.5, 4.8, 6 x [14336, 9728] 53.6, 46.3.
+// columns) 1 % low on average with a deviation of 7 %; the ring plans' costs are 8 % high there for 64 x 64 tiles in one part, 4 to 6 %
+// for most others, and 2 % low, with a deviation of 10, at columns a power of two of 8 KB apart.  Taken below 0.88, 0.92 and 1.0 of
+// those (launch_ring_gemm): 940 of the 1690, 56 of them slower than the plan by more than 2 %, at worst 13.  us, and those of the ring
+// kernels with their merge: one row x [4096, 4096] 7.6, 13.7, [4096, 14336] 21.0, 29.6, [14336, 4096] 21.9, 24.0, 12 rows 24.7, 23.9, 4 x
+// [4544, 18176] 27.6, 32.5, 9 x [16384, 8192] 46.7, 78.8; not taken: 14 x [14336, 4096] 25.6, 23.9, 12 x [2048, 9728] 13.4, 11.8, 10 x
+// [512, 4672] 5.5, 4.8, 6 x [14336, 9728] 53.6, 46.3.
 float strip_us(const GemmArgs& a) {
   if (!a.w_kcontig || a.epi == EPI_SWIGLU || a.rowstat_out != nullptr || a.M > 16 || a.K < 512 || a.K % 32 != 0 || a.N % 8 != 0) return 1e30f;
   const int wg = (a.N + kStripCols - 1) / kStripCols;
