@@ -280,7 +280,10 @@ static int launch_epi(const GemmArgs& a, int tile, hipStream_t stream) {
 
 // Cost of a plan in us, fitted to 4100 timings on the card (the Q/K/V, output, FFN up and FFN down products of
 // Llama-3-8B and Falcon-7B sizes, 16 to 1024 rows, both weight layouts, up to 16 parts): 4 % rms, and the plan it picks
-// is 1.3 % slower on average than the best plan of the family.  Three times add up in part (as a 3/2-norm):
+// is 1.3 % slower on average than the best plan of the family.  (Those timings had the 32 x 128 tile with four stages throughout.  As it
+// runs now, ring_fourth_stage, the costs of plans of 1 to 32 rows on it are 7 % high, deviation 7, over 1170 row-major ones, 6 and 7 over
+// 980 K-contiguous ones, and 4 % low, deviation 9, over 190 with columns 8 or 16 KB apart.)  Three times add up in part (as a
+// 3/2-norm):
 //   memory    the weights once at 8 TB/s - less when the workgroups do not divide evenly over the CUs and some CUs have
 //             one more to stream - and what is written;
 //   compute   k tiles in a row on the busiest CU, by tile and by whether workgroups share a CU;
