@@ -187,8 +187,8 @@ def check_bf16(got, want, what):
 
 
 # up to 32 rows on 32 x 128 tiles; which of them run three stages and which four follows from the workgroups of the last round
-# (two a CU) and the distance between rows: 133 workgroups, 257, 399 and 195 in three parts, 144 in four
-@pytest.mark.parametrize("M,K,N", [(24, 544, 17000), (17, 1056, 32776), (20, 2080, 17000), (24, 4544, 8200), (32, 2080, 4552)])
+# (two a CU) and the distance between rows: 133 workgroups, 257, 399 and 195 in three parts, 144 in four, 504 in fourteen
+@pytest.mark.parametrize("M,K,N", [(24, 544, 17000), (17, 1056, 32776), (20, 2080, 17000), (24, 4544, 8200), (32, 2080, 4552), (4, 5152, 4552)])
 @pytest.mark.parametrize("kcontig", [False, True])
 @pytest.mark.parametrize("bf16", [False, True])
 def test_stages_of_plain_products(rn, M, K, N, kcontig, bf16):

@@ -70,12 +70,13 @@ constexpr int kRingTileOneBlock = 8;  // the non-temporal tile, for a single row
 //     216, 46.4 / 44.4, [14336, 8192 x 2] in 4 parts, 512, 77.2 / 80.7; columns a multiple of 4 KB apart and parts of as many, from 384
 //     on: [6144, 9728 x 2] in three, 456, 51.6 / 49.1, [14336, 4544 x 2] in seven, 497, 58.1 / 54.1, [2048, 28672 x 2], 448, 47.4 / 44.1,
 //     but [6144, 17408 x 2], 272, 97.8 / 102.3; a power of two of 8 KB and more: 16 rows x [8192, 5120 x 2] in three parts, 240, 36.3 /
-//     38.1, [4096, 12288 x 2] in four, 768, 44.6 / 43.0, [8192, 28672 x 2], 448, 156 / 167, [8192, 8192 x 2], 512, 68.1 / 73.0, but parts of 4096, 4 rows x
-//     [16384, 15904] in four, 500, 109 / 102, [4096, 32400 x 2], 507, 108 / 96.  (22 KB, K = 11008, would have four there too: 4 rows x
-//     [11008, 28672 x 2], 448, 223 / 214.)
-//   rows no multiple of 256 bytes: 16 rows x [4544, 4544], 216, 13.2 / 12.9, [4096, 13632], 107, 30.6 / 25.2, rows 4544 apart x
-//     [4096, 4096], 512, 11.6 / 11.8; no multiple of 1 KB: [4544, 9088 x 2], 142, 36.1 / 32.0, [4096, 18176], 142, 32.2 / 28.4,
-//     [4096, 32000], 250, 40.8 / 42.2
+//     38.1, [4096, 12288 x 2] in four, 768, 44.6 / 43.0, [8192, 28672 x 2], 448, 156 / 167, [8192, 8192 x 2], 512, 68.1 / 73.0, but parts of
+//     4096, 4 rows x [16384, 15904] in four, 500, 109 / 102, [4096, 32400 x 2], 507, 108 / 96.  (22 KB, K = 11008, would have four
+//     there too: 4 rows x [11008, 28672 x 2], 448, 223 / 214.)
+//   rows no multiple of 256 bytes: 16 rows x [4544, 4544], 216, 13.2 / 12.9, [4096, 13632], 107, 30.6 / 25.2, [4096, 12288] out of
+//     18112, 288, 24.4 / 25.4, 16 rows x [18176, 4672], 481, 1.1 % slower; up to eight rows and nearly two on every CU level or better:
+//     [18176, 4544], 504, the whole Falcon-7B FFN 63.1 / 62.8; no multiple of 1 KB: [4544, 9088 x 2], 142, 36.1 / 32.0, [4096, 18176],
+//     142, 32.2 / 28.4, [4096, 32000], 250, 40.8 / 42.2
 //   else: [4096, 8192], 64, 29.1 / 26.3, [4096, 12288], 192, 22.1 / 22.1, 16 rows x [4096, 6144], 240, 14.1 / 14.6, x [4096, 28672],
 //     224, 38.4 / 39.6; halves (a tile takes 128 bytes of a row from each of two matrices) [4096, 8192 x 2], 128, 35.6 / 36.2
 // Over 960 K-contiguous and 1170 row-major plans (K 1024 to 18176, 1 to 32 rows) the rule's choice is on average 0.3 and 0.1 %
@@ -86,13 +87,13 @@ using RingTileFour = RingTile<32, 128, 1, 4, 4, true>;
 // K-contiguous columns a power of two of 8 KB and more apart: the memory is slow there.
 inline bool ring_slow_columns(int64_t ld) { return ld >= 4096 && (ld & (ld - 1)) == 0; }
 // (ld: distances between rows or columns, several or-ed together; k_part: K of a workgroup)
-inline bool ring_fourth_stage(int workgroups, int64_t ld, int k_part, bool kcontig, bool halves) {
+inline bool ring_fourth_stage(int rows, int workgroups, int64_t ld, int k_part, bool kcontig, bool halves) {
   const int last = (workgroups - 1) % 512 + 1;
   if (kcontig) {
     if (ring_slow_columns(ld)) return last < (workgroups <= 256 ? 224 : 257) || (last >= 384 && k_part == 4096);
     return last <= 256 || (last >= 384 && ld % 2048 == 0 && k_part % 2048 == 0);
   }
-  if ((ld & 127) != 0) return last < 256;
+  if ((ld & 127) != 0) return last < 256 || (rows <= 8 && last > 480);
   if ((ld & 511) != 0) return last < 224;
   return !halves && workgroups < 176;
 }

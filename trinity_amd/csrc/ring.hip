@@ -235,7 +235,7 @@ static int launch_partial_t(const RingArgs& a, hipStream_t stream) {
 }
 
 int launch_ring_partial(const RingArgs& a, int tile, bool kcontig, hipStream_t stream) {
-  if (tile == kRingTileOneBlock && ring_fourth_stage((a.ncols + 127) / 128 * a.ksplit, a.ldw[0] | a.ldw[1] | a.ldw[2], ring_kt_per_part(a.K, a.ksplit) * 64, kcontig, false))
+  if (tile == kRingTileOneBlock && ring_fourth_stage(a.M, (a.ncols + 127) / 128 * a.ksplit, a.ldw[0] | a.ldw[1] | a.ldw[2], ring_kt_per_part(a.K, a.ksplit) * 64, kcontig, false))
     return kcontig ? launch_partial_t<RingTileFour, true>(a, stream) : launch_partial_t<RingTileFour, false>(a, stream);
   switch (tile) {
 #define TRI_RING_CASE(id, bm, bn, wm, wn, nst, nt)                                                  \
@@ -265,7 +265,7 @@ static int launch_epi(const GemmArgs& a, int tile, hipStream_t stream) {
   constexpr bool GATED = EPI == EPI_SWIGLU;
   const int64_t ld = a.ldw | (GATED ? a.ldw2 : 0);
   if (tile == kRingTileNarrow) return launch_epi_t<RingTileKContig, EPI, true>(a, stream);
-  if (tile == kRingTileOneBlock && ring_fourth_stage(((GATED ? 2 : 1) * a.N + 127) / 128, ld, a.K, a.w_kcontig != 0, GATED))
+  if (tile == kRingTileOneBlock && ring_fourth_stage(a.M, ((GATED ? 2 : 1) * a.N + 127) / 128, ld, a.K, a.w_kcontig != 0, GATED))
     return a.w_kcontig ? launch_epi_t<RingTileFour, EPI, true>(a, stream) : launch_epi_t<RingTileFour, EPI, false>(a, stream);
   switch (tile) {
 #define TRI_RING_CASE(id, bm, bn, wm, wn, nst, nt)                                                       \
