@@ -46,9 +46,31 @@ def test_plain_and_residual(rn, M, K, N, kcontig, with_ws):
     check(out, x.float() @ w.float() + r.float(), "x.w + r")
 
 
+# Tiles whose loads have waves of their own - 128 x 192, 192 x 128, 192 x 192, 256 x 128 - in one part and in parts: a last row
+# block of one row and full ones, ragged columns, K = 16.5 and 64.5 k tiles (the last one begins half way back), one k tile
+# and two (fewer than the three stages that are requested ahead)
+@pytest.mark.parametrize("M,K,N", [
+    (193, 4128, 6144), (1000, 1056, 6144), (1000, 64, 6144), (150, 4128, 6136), (385, 1056, 9000), (384, 96, 9000),
+    (385, 4544, 4544), (700, 1056, 9000), (768, 64, 9000), (333, 18176, 4544), (576, 1056, 11264), (560, 128, 12000),
+])
+@pytest.mark.parametrize("kcontig", [False, True])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_loading_waves(rn, M, K, N, kcontig, bf16):
+    dt, tol = (torch.bfloat16, 2.0 ** -6) if bf16 else (torch.float16, REL)  # (bf16: two ulps of 2^-8)
+    x = rn(M, K).to(dt)
+    w = (rn(N, K, std=K ** -0.5).to(dt).t() if kcontig else rn(K, N, std=K ** -0.5).to(dt))
+    want = x.float() @ w.float()
+    for ws in (None, torch.empty(ext.gemm_workspace_bytes(M, K, N), dtype=torch.uint8, device="cuda:0")):
+        out = torch.full((M, N), float("nan"), dtype=dt, device="cuda:0")
+        ext.matmul(x, w, None, out, workspace=ws)
+        torch.cuda.synchronize()
+        assert not ((out.float() - want).abs() > tol * want.abs() + 1e-4).any()
+
+
 @pytest.mark.parametrize("M,K,F", [
     (1, 4096, 14336), (16, 96, 72), (48, 4096, 14336), (90, 4096, 14336), (130, 4096, 14336), (300, 4096, 14336),
     (100, 4544, 4544), (256, 4544, 4544), (500, 1024, 4000),
+    (150, 1056, 14336), (190, 4128, 3000), (1000, 96, 3064), (576, 1056, 5632),  # tiles whose loads have waves of their own
 ])
 @pytest.mark.parametrize("kcontig", [False, True])
 def test_gated_with_row_scale(rn, M, K, F, kcontig):
@@ -93,6 +115,7 @@ def test_one_row_of_any_stride_in_place(rn, stride):
 @pytest.mark.parametrize("S,N,Hq,Hkv,D", [
     (1, 64, 4, 4, 64), (33, 96, 5, 1, 128), (100, 4096, 32, 8, 128), (260, 4096, 32, 8, 128), (200, 4544, 71, 1, 64),
     (700, 128, 32, 8, 128), (1000, 128, 71, 1, 64), (1100, 160, 32, 4, 128),  # a tile across two weight matrices
+    (150, 4128, 32, 8, 128), (1000, 1056, 71, 1, 64), (1000, 1056, 32, 8, 128),  # loads in waves of their own
 ])
 @pytest.mark.parametrize("qknorm", [False, True])
 @pytest.mark.parametrize("kcontig", [False, True])

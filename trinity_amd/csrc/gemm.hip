@@ -395,9 +395,9 @@ static TilePlan best_plan(int M, int N, int& which) {
 static float plan_us(const TilePlan& p, int K) { return 6.0f + 0.0272f * (float)K * (float)p.cost; }
 
 // The ring kernels' plan for a product, if it beats a tile plan of big_us.  Beyond the rows that the costs were fitted
-// over, by a quarter: 14336 -> 1024, 2048 rows 162 -> 70 us (0.39 by the costs), 14336 -> 4096, 1200 rows 187 -> 142
-// (0.74), but 4096 rows of 4096 -> 1024 43.0 -> 45.8 (0.76), 3072 of 14336 -> 4096 310 -> 370 (0.86).
-constexpr float kRingMarginNarrow = 0.75f;
+// over, by three tenths: 14336 -> 1024, 2048 rows 162 -> 70 us (0.36 by the costs), 14336 -> 4096, 1200 rows 187 -> 142
+// (0.67), but 4096 rows of 4096 -> 1024 43.0 -> 45.8 (0.73), 3072 of 14336 -> 4096 310 -> 370 (0.79).
+constexpr float kRingMarginNarrow = 0.70f;
 static bool ring_wins(float big_us, int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes, RingPlan& plan,
                       float merge_us = kRingMergeUs) {
   plan = ring_plan(M, K, ncols, unit, min_bn, ws_bytes, merge_us);

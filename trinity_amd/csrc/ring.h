@@ -16,7 +16,8 @@
 //   row-major weights [64][BN]: chunk c of row k at slot c ^ ((k & 3) << 2), or c ^ (((k >> 1) & 1) << 2) where a
 //   row is not a multiple of 256 bytes - the four rows of a transpose read then fall on different banks.
 // One barrier per k tile, in front of its last k16 step, when the next tile must have landed; the loads of a tile are
-// spread one by one between the MFMAs of the four steps after the barrier that freed their stage.
+// spread one by one between the MFMAs of the four steps after the barrier that freed their stage, or (RingTile::NP) are left
+// to waves that do nothing else.
 #if (defined(TRI_BF16) && !defined(TRI_RING_H_BF16)) || (!defined(TRI_BF16) && !defined(TRI_RING_H_F16))
 #ifdef TRI_BF16
 #define TRI_RING_H_BF16
@@ -29,40 +30,52 @@
 namespace tri {
 
 // NTW: the weights are requested non-temporally (each line is wanted once: a single row block).
-template <int BM_, int BN_, int WM_, int WN_, int NST_, bool NTW_ = false>
+// NP: that many further waves do nothing but request tiles; the WM x WN waves then only read fragments and multiply.
+template <int BM_, int BN_, int WM_, int WN_, int NST_, bool NTW_ = false, int NP_ = 0>
 struct RingTile {
-  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, NST = NST_, BK = 64;
+  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, NST = NST_, BK = 64, NP = NP_;
   static constexpr bool NTW = NTW_;
-  static constexpr int NW = WM * WN, NT = NW * 64;
+  static constexpr int NW = WM * WN, NT = (NW + NP) * 64, LW = NP > 0 ? NP : NW;  // LW: waves that request tiles
   static constexpr int TM = BM / WM, TN = BN / WN, MI = TM / 32, NI = TN / 32;
   static constexpr int X_HALFS = BM * BK, STAGE = (BM + BN) * BK;
   static constexpr int LDS_BYTES = NST * STAGE * 2;
-  static constexpr int XI = BM / 8 / NW, WI = BN / 8 / NW, L = XI + WI;  // 1 KB load instructions per wave and k tile
+  static constexpr int XI = BM / 8 / LW, WI = BN / 8 / LW, L = XI + WI;  // 1 KB load instructions per loading wave and k tile
   static constexpr int CPR = BN / 8;                                     // 16-byte chunks per row-major weight row
-  static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0 && TM % 32 == 0 && TN % 32 == 0, "tile split");
+  static_assert(BM % (8 * LW) == 0 && BN % (8 * LW) == 0 && TM % 32 == 0 && TN % 32 == 0, "tile split");
   static_assert(NST >= 3 && LDS_BYTES <= 160 * 1024, "LDS budget");
-  static_assert((NST - 2) * L + L / 4 < 64, "loads in flight fit vmcnt");
+  static_assert(NP > 0 ? (NST - 1) * L < 64 : (NST - 2) * L + L / 4 < 64, "loads in flight fit vmcnt");
 };
 
 // The family (planned by ring_plan below).  Waves are arranged so that every tile has at least one wave per SIMD
 // and an accumulator of at most 160 registers; eight waves where the tile is large enough to share (they hide each
 // other's LDS reads: 128 x 256 at 512 rows 138 -> 136 us, 64 x 128 at 64 rows of [4096, 14336 x 2] 44.7 -> 44.2 us).
+// Tiles of 24 K to 36 K outputs but for 128 x 256: four waves multiply and four do nothing but load.  A wave that does both
+// stalls with its MFMAs behind a load that the CU has no room for (a CU keeps 32 KB of misses in flight, however deep the
+// ring: a kernel that only streams gets 13 bytes a clock and CU from HBM, 31 from the last-level cache, 63 from its L2); a loop
+// without MFMAs and fragment reads takes as long as the whole one then.  192 x 128, 192 x 192 and 256 x 128 are in the family
+// because of it: 150 rows x [4096, 14336 x 2] 68 -> 62 us, 192 x [14336, 4096] in eight parts 41.6 -> 38.4, 333 x [18176, 4544]
+// in parts 74.7 -> 72.9, 1000 x [4544, 4672] 52.4 -> 48.3 (the best of the family without / with them); 128 x 192 in place
+// of four waves that do both 48.0 -> 46.5 (800 x [4096, 6144]); 128 x 256 with four loading waves is level with eight waves
+// that do both (333 x [4544, 18176] 64.0 and 64.2), 128 x 128 behind it, 96 x 256 behind 192 x 128.  Two loading waves are
+// too few (loads alone, all from the L2, 38 against 31 us).
 // Non-temporal weights where one block of at most 32 rows sees them: 16 rows x [18176, 4544] in 7 parts 29.6 -> 27.1 us
 // (6.1 TB/s), x [14336, 4096] in 8 parts 22.6 -> 21.2 us; at 64 rows the gain is gone (42.7 -> 43.6, 25.1 -> 23.6 us).
 // That tile has three stages, or four (ring_fourth_stage).
-#define TRI_RING_TILES(X)        \
-  X(0, 32, 128, 1, 4, 4, false)  \
-  X(1, 64, 64, 2, 2, 5, false)   \
-  X(2, 64, 128, 2, 4, 3, false)  \
-  X(3, 96, 128, 1, 4, 5, false)  \
-  X(4, 128, 128, 2, 4, 5, false) \
-  X(5, 128, 192, 2, 2, 4, false) \
-  X(6, 128, 256, 2, 4, 3, false) \
-  X(7, 160, 256, 1, 4, 3, false) \
-  X(8, 32, 128, 1, 4, 3, true)
-constexpr int kRingTiles = 9;
-constexpr int kRingTileOneBlock = 8;  // the non-temporal tile, for a single row block
-// Tile 8 with a fourth stage: 48 KB of weights on their way per workgroup in place of 32.  A CU with two workgroups has
+#define TRI_RING_TILES(X)            \
+  X(0, 32, 128, 1, 4, 3, true, 0)    \
+  X(1, 64, 64, 2, 2, 5, false, 0)    \
+  X(2, 64, 128, 2, 4, 3, false, 0)   \
+  X(3, 96, 128, 1, 4, 5, false, 0)   \
+  X(4, 128, 128, 2, 4, 5, false, 0)  \
+  X(5, 128, 192, 2, 2, 3, false, 4)  \
+  X(6, 128, 256, 2, 4, 3, false, 0)  \
+  X(7, 160, 256, 1, 4, 3, false, 0)  \
+  X(8, 192, 128, 2, 2, 3, false, 4)  \
+  X(9, 192, 192, 2, 2, 3, false, 4)  \
+  X(10, 256, 128, 2, 2, 3, false, 4)
+constexpr int kRingTiles = 11;
+constexpr int kRingTileOneBlock = 0;  // the non-temporal tile, for a single row block of up to 32 rows
+// That tile with a fourth stage: 48 KB of weights on their way per workgroup in place of 32.  A CU with two workgroups has
 // enough with three stages, and more costs time; one with a single workgroup, or none, leaves memory bandwidth unused, the
 // more so the faster the memory is at the distance between rows.  What counts is the last round of workgroups (two a CU).
 // us with three / four stages, one row unless said otherwise:
@@ -127,12 +140,13 @@ __device__ __forceinline__ void ring_coords(int pid, int nrb, int ntn, int kspli
 template <class T, bool NTL, bool SWAP, class WMap>
 __device__ __forceinline__ void gemm_mainloop_ring(const half_t* __restrict__ x, int64_t ldx, int m0, int M, int K,
                                                    WMap wmap, half_t* lds, float16v (&acc)[T::NI][T::MI]) {
-  constexpr int NW = T::NW, BK = T::BK, BN = T::BN, NST = T::NST, XI = T::XI, WI = T::WI, L = T::L, CPR = T::CPR;
+  constexpr int NW = T::NW, LW = T::LW, BK = T::BK, BN = T::BN, NST = T::NST, XI = T::XI, WI = T::WI, L = T::L, CPR = T::CPR;
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int wm = wave % T::WM, wn = wave / T::WM;
   const int l32 = lane & 31, g = lane >> 5;
   const int KT = (K + BK - 1) / BK;
+  const int lw = T::NP > 0 ? max(wave - NW, 0) : wave;  // which of the loading waves
 
   const half_t* xsrc[XI];
   const half_t* wsrc[WI];
@@ -142,7 +156,7 @@ __device__ __forceinline__ void gemm_mainloop_ring(const half_t* __restrict__ x,
   int64_t ldw[NLD];
 #pragma unroll
   for (int i = 0; i < XI; ++i) {
-    const int rloc = (i * NW + wave) * 8 + (lane >> 3);
+    const int rloc = (i * LW + lw) * 8 + (lane >> 3);
     int row = m0 + rloc;
     row = row < M ? row : M - 1;
     xsrc[i] = x + (int64_t)row * ldx + ((lane & 7) ^ ((rloc >> 1) & 7)) * 8;
@@ -150,10 +164,10 @@ __device__ __forceinline__ void gemm_mainloop_ring(const half_t* __restrict__ x,
 #pragma unroll
   for (int i = 0; i < WI; ++i) {
     if constexpr (NTL) {
-      const int nloc = (i * NW + wave) * 8 + (lane >> 3);
+      const int nloc = (i * LW + lw) * 8 + (lane >> 3);
       wsrc[i] = wmap(nloc, ldw[0]) + ((lane & 7) ^ ((nloc >> 1) & 7)) * 8;
     } else {
-      const int p = (i * NW + wave) * 64 + lane;
+      const int p = (i * LW + lw) * 64 + lane;
       const int krow = p / CPR, slot = p % CPR;
       const int chunk = CPR % 16 == 0 ? slot ^ ((krow & 3) << 2) : slot ^ (((krow >> 1) & 1) << 2);
       wsrc[i] = wmap(chunk, ldw[i % NLD]) + (int64_t)krow * ldw[i % NLD];
@@ -183,9 +197,39 @@ __device__ __forceinline__ void gemm_mainloop_ring(const half_t* __restrict__ x,
   };
   auto load_one = [&](const KPos& o, int st, int i) {
     half_t* b = lds + st * T::STAGE;
-    if (i < XI) load_to_lds16(xsrc[i] + o.k, b + (i * NW + wave) * 512);
-    else load_to_lds16<T::NTW>(wsrc[i - XI] + o.w[(i - XI) % NLD], b + T::X_HALFS + ((i - XI) * NW + wave) * 512);
+    if (i < XI) load_to_lds16(xsrc[i] + o.k, b + (i * LW + lw) * 512);
+    else load_to_lds16<T::NTW>(wsrc[i - XI] + o.w[(i - XI) % NLD], b + T::X_HALFS + ((i - XI) * LW + lw) * 512);
   };
+  KPos pos;
+  pos.k = 0;
+#pragma unroll
+  for (int j = 0; j < NLD; ++j) pos.w[j] = 0;
+
+  // ---- waves that only load: a tile goes out as soon as the barrier has freed its stage, and the barrier of tile kt waits for
+  // their loads of tile kt + 1.  (Barriers: one before tile 0, then one per tile but the last - the others' below.)
+  if (T::NP > 0 && wave >= NW) {
+    auto load_tile = [&](int st) {
+#pragma unroll
+      for (int i = 0; i < L; ++i) load_one(pos, st, i);
+    };
+#pragma unroll
+    for (int s = 0; s < NST; ++s) {
+      load_tile(s);
+      advance(pos, s + 1);
+    }
+    TRI_WAIT_VMCNT((NST - 1) * L);
+    __builtin_amdgcn_s_barrier();
+    int st = 0;
+    for (int kt = 0; kt < KT - 1; ++kt) {
+      TRI_WAIT_VMCNT((NST - 2) * L);
+      __builtin_amdgcn_s_barrier();
+      load_tile(st);  // tile kt + NST
+      advance(pos, kt + NST + 1);
+      st = st == NST - 1 ? 0 : st + 1;
+    }
+    TRI_WAIT_VMCNT(0);
+    return;
+  }
 
   // ---- fragment read offsets (halfs)
   const int sx = (l32 >> 1) & 7;
@@ -247,20 +291,18 @@ __device__ __forceinline__ void gemm_mainloop_ring(const half_t* __restrict__ x,
       for (int r = 0; r < 16; ++r) acc[ni][mi][r] = 0.f;
 
   // a quarter of tile kt + NST's loads is issued in the last step of tile kt, the rest in the first three of kt + 1
-  constexpr int L0 = L / 4, L1 = L / 2, L2 = 3 * L / 4;
-  KPos pos;
-  pos.k = 0;
+  constexpr int LE = T::NP > 0 ? 0 : L, L0 = LE / 4, L1 = LE / 2, L2 = 3 * LE / 4;
+  if constexpr (T::NP == 0) {
 #pragma unroll
-  for (int j = 0; j < NLD; ++j) pos.w[j] = 0;
+    for (int s = 0; s < NST - 1; ++s) {
 #pragma unroll
-  for (int s = 0; s < NST - 1; ++s) {
+      for (int i = 0; i < L; ++i) load_one(pos, s, i);
+      advance(pos, s + 1);
+    }
 #pragma unroll
-    for (int i = 0; i < L; ++i) load_one(pos, s, i);
-    advance(pos, s + 1);
+    for (int i = 0; i < L0; ++i) load_one(pos, NST - 1, i);
+    TRI_WAIT_VMCNT((NST - 2) * L + L0);
   }
-#pragma unroll
-  for (int i = 0; i < L0; ++i) load_one(pos, NST - 1, i);
-  TRI_WAIT_VMCNT((NST - 2) * L + L0);
   __builtin_amdgcn_s_barrier();
 #pragma unroll
   for (int i = 0; i < NF; ++i) read_one(0, 0, 0, i);
@@ -271,12 +313,17 @@ __device__ __forceinline__ void gemm_mainloop_ring(const half_t* __restrict__ x,
     __builtin_amdgcn_sched_barrier(0);
     step(0, pos, sp, L0, L1, st, 1);
     step(1, pos, sp, L1, L2, st, 2);
-    step(0, pos, sp, L2, L, st, 3);
-    // this wave's reads of tile kt are over and its share of tile kt + 1 has landed; kt + 2 .. kt + NST - 1 in flight
-    constexpr int V = (NST - 2) * L;
-    __builtin_amdgcn_s_waitcnt((V & 15) | ((V >> 4) << 14) | 0x0070);  // vmcnt(V) lgkmcnt(0)
-    __builtin_amdgcn_s_barrier();
-    advance(pos, kt + NST);
+    step(0, pos, sp, L2, LE, st, 3);
+    if constexpr (T::NP > 0) {
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's reads of tile kt are over
+      __builtin_amdgcn_s_barrier();
+    } else {
+      // this wave's reads of tile kt are over and its share of tile kt + 1 has landed; kt + 2 .. kt + NST - 1 in flight
+      constexpr int V = (NST - 2) * L;
+      __builtin_amdgcn_s_waitcnt((V & 15) | ((V >> 4) << 14) | 0x0070);  // vmcnt(V) lgkmcnt(0)
+      __builtin_amdgcn_s_barrier();
+      advance(pos, kt + NST);
+    }
     __builtin_amdgcn_sched_barrier(0);
     step(1, pos, st, 0, L0, sn, 0);
     st = sn;
@@ -290,7 +337,7 @@ __device__ __forceinline__ void gemm_mainloop_ring(const half_t* __restrict__ x,
   }
   step(0, pos, 0, 0, 0, st, 3);
   step(1, pos, 0, 0, 0, st, -1);
-  TRI_WAIT_VMCNT(0);
+  if constexpr (T::NP == 0) TRI_WAIT_VMCNT(0);
 }
 
 // k tiles per part of a plan (the last part takes what is left, and the odd 32 of a K that is not a multiple of 64)

@@ -41,6 +41,7 @@ __global__ __launch_bounds__(T::NT) void ring_partial_kernel(RingArgs a) {
 
   // lanes run along the columns: 128 bytes of a row per half wave and store
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (T::NP > 0 && wave >= T::NW) return;  // (a wave that only loads)
   const int wm = wave % T::WM, wn = wave / T::WM;
   const int l32 = lane & 31, g = lane >> 5;
   float* base = a.partial + (int64_t)split * a.M * a.ncols;
@@ -97,7 +98,8 @@ __global__ __launch_bounds__(T::NT) void ring_epi_kernel(GemmArgs a) {
   constexpr int US = OUT_BN + 4;  // floats per row of the up half
   static_assert(T::BM * RS * 2 <= T::LDS_BYTES && (!GATED || (T::BM * US * 4 <= T::LDS_BYTES && T::WN % 2 == 0)), "the staged tile fits the ring");
   float* up = reinterpret_cast<float*>(lds);
-  const bool up_wave = GATED && wn >= T::WN / 2;
+  const bool loader = T::NP > 0 && wave >= T::NW;  // (holds no part of the tile, but stores rows of it below)
+  const bool up_wave = GATED && !loader && wn >= T::WN / 2, out_wave = !up_wave && !loader;
   __syncthreads();  // every wave is done with the ring (and every load into it has landed)
   if (up_wave) {
 #pragma unroll
@@ -111,7 +113,7 @@ __global__ __launch_bounds__(T::NT) void ring_epi_kernel(GemmArgs a) {
         }
   }
   if (GATED) __syncthreads();
-  if (!up_wave) {
+  if (out_wave) {
 #pragma unroll
     for (int mi = 0; mi < T::MI; ++mi) {
       const int mloc = wm * T::TM + mi * 32 + l32, m = m0 + mloc;
@@ -140,7 +142,7 @@ __global__ __launch_bounds__(T::NT) void ring_epi_kernel(GemmArgs a) {
     }
   }
   if (GATED) __syncthreads();  // the up half has been read
-  if (!up_wave) {
+  if (out_wave) {
 #pragma unroll
     for (int mi = 0; mi < T::MI; ++mi)
 #pragma unroll
@@ -238,10 +240,10 @@ int launch_ring_partial(const RingArgs& a, int tile, bool kcontig, hipStream_t s
   if (tile == kRingTileOneBlock && ring_fourth_stage(a.M, (a.ncols + 127) / 128 * a.ksplit, a.ldw[0] | a.ldw[1] | a.ldw[2], ring_kt_per_part(a.K, a.ksplit) * 64, kcontig, false))
     return kcontig ? launch_partial_t<RingTileFour, true>(a, stream) : launch_partial_t<RingTileFour, false>(a, stream);
   switch (tile) {
-#define TRI_RING_CASE(id, bm, bn, wm, wn, nst, nt)                                                  \
+#define TRI_RING_CASE(id, bm, bn, wm, wn, nst, nt, np)                                                  \
   case id:                                                                                      \
-    return kcontig ? launch_partial_t<RingTile<bm, bn, wm, wn, nst, nt>, true>(a, stream) \
-                   : launch_partial_t<RingTile<bm, bn, wm, wn, nst, nt>, false>(a, stream);
+    return kcontig ? launch_partial_t<RingTile<bm, bn, wm, wn, nst, nt, np>, true>(a, stream) \
+                   : launch_partial_t<RingTile<bm, bn, wm, wn, nst, nt, np>, false>(a, stream);
     TRI_RING_TILES(TRI_RING_CASE)
 #undef TRI_RING_CASE
   }
@@ -268,58 +270,70 @@ static int launch_epi(const GemmArgs& a, int tile, hipStream_t stream) {
   if (tile == kRingTileOneBlock && ring_fourth_stage(a.M, ((GATED ? 2 : 1) * a.N + 127) / 128, ld, a.K, a.w_kcontig != 0, GATED))
     return a.w_kcontig ? launch_epi_t<RingTileFour, EPI, true>(a, stream) : launch_epi_t<RingTileFour, EPI, false>(a, stream);
   switch (tile) {
-#define TRI_RING_CASE(id, bm, bn, wm, wn, nst, nt)                                                       \
+#define TRI_RING_CASE(id, bm, bn, wm, wn, nst, nt, np)                                                       \
   case id:                                                                                           \
-    return a.w_kcontig ? launch_epi_t<RingTile<bm, bn, wm, wn, nst, nt>, EPI, true>(a, stream) \
-                       : launch_epi_t<RingTile<bm, bn, wm, wn, nst, nt>, EPI, false>(a, stream);
+    return a.w_kcontig ? launch_epi_t<RingTile<bm, bn, wm, wn, nst, nt, np>, EPI, true>(a, stream) \
+                       : launch_epi_t<RingTile<bm, bn, wm, wn, nst, nt, np>, EPI, false>(a, stream);
     TRI_RING_TILES(TRI_RING_CASE)
 #undef TRI_RING_CASE
   }
   return -1;
 }
 
-// Cost of a plan in us, fitted to 4100 timings on the card (the Q/K/V, output, FFN up and FFN down products of
-// Llama-3-8B and Falcon-7B sizes, 16 to 1024 rows, both weight layouts, up to 16 parts): 4 % rms, and the plan it picks
-// is 1.3 % slower on average than the best plan of the family.  (Those timings had the 32 x 128 tile with four stages throughout.  As it
-// runs now, ring_fourth_stage, the costs of plans of 1 to 32 rows on it are 7 % high, deviation 7, over 1170 row-major ones, 6 and 7 over
-// 980 K-contiguous ones, and 4 % low, deviation 9, over 190 with columns 8 or 16 KB apart.)  Three times add up in part (as a
-// 3/2-norm):
-//   memory    the weights once at 8 TB/s - less when the workgroups do not divide evenly over the CUs and some CUs have
+// Cost of a plan in us.  Three times add up in part (as a 3/2-norm up to 32 rows, as a 4/3-norm above):
+//   memory    the weights once - less fast when the workgroups do not divide evenly over the CUs and some CUs have
 //             one more to stream - and what is written;
 //   compute   k tiles in a row on the busiest CU, by tile and by whether workgroups share a CU;
-//   loads     every byte that passes from L2 to LDS, at 37 TB/s over the chip;
-// and per wave of workgroups 2 us of first loads and epilogue.  Parts cost a merge: 3.5 us (kRingMergeUs) and their bytes at 6 TB/s.
+//   loads     every byte that passes from L2 to LDS;
+// and per wave of workgroups 2 us of first loads and epilogue.  Parts cost a merge and their bytes.
+// Up to 32 rows: weights at 8 TB/s, loads at 37, fitted to 4100 timings on the card, 16 to 1024 rows, when the 32 x 128 tile had four
+// stages throughout; 4 % rms then, the plan it picks 1.3 % slower on average than the best plan of the family.  As that tile
+// runs now, ring_fourth_stage, the costs of plans on it are 7 % high, deviation 7, over 1170 row-major ones, 6 and 7 over
+// 980 K-contiguous ones, and 4 % low, deviation 9, over 190 with columns 8 or 16 KB apart.
+// Above: weights at 12 TB/s, loads at 62, fitted to 8800 timings of 600 products (33 to 1100 rows, K 1024 to 18176, 512 to 28672 columns,
+// plain and gated, both layouts, up to 16 parts; most out of HBM, 48 of Q/K/V projections out of the last-level cache): 7 % rms,
+// its choice, tile plans included, is 1.5 % slower than the best on average, at worst 19 % (800 rows x [4544, 4672], 52.8 / 44.4); over
+// the first 386 of them 1.3 %, where the constants of up to 32 rows throughout, without the tiles whose loads have waves of
+// their own, came to 2.9 %.
 struct RingCost {
   int bm, bn, per_cu;   // per_cu: workgroups that fit a CU's LDS
   float alone, shared;  // us per k tile of a workgroup with a CU to itself / of each of several
+  float few_alone, few_shared;  // the same in the fit for up to 32 rows (0: not for them)
 };
 #define TRI_RING_PER_CU(bm, bn, nst) ((160 * 1024) / (((bm) + (bn)) * 128 * (nst)))
 static const RingCost kRingCost[kRingTiles] = {
-    {32, 128, TRI_RING_PER_CU(32, 128, 4), 0.264f, 0.222f},  {64, 64, TRI_RING_PER_CU(64, 64, 5), 0.215f, 0.181f},
-    {64, 128, TRI_RING_PER_CU(64, 128, 3), 0.354f, 0.272f},  {96, 128, TRI_RING_PER_CU(96, 128, 5), 0.429f, 0.431f},
-    {128, 128, TRI_RING_PER_CU(128, 128, 5), 0.480f, 0.490f}, {128, 192, TRI_RING_PER_CU(128, 192, 4), 0.660f, 0.691f},
-    {128, 256, TRI_RING_PER_CU(128, 256, 3), 0.743f, 0.755f}, {160, 256, TRI_RING_PER_CU(160, 256, 3), 0.914f, 1.006f},
-    {32, 128, TRI_RING_PER_CU(32, 128, 3), 0.264f, 0.222f}};
+    {32, 128, TRI_RING_PER_CU(32, 128, 3), 0.264f, 0.222f, 0.264f, 0.222f},
+    {64, 64, TRI_RING_PER_CU(64, 64, 5), 0.224f, 0.198f, 0.215f, 0.181f},
+    {64, 128, TRI_RING_PER_CU(64, 128, 3), 0.360f, 0.302f, 0.354f, 0.272f},
+    {96, 128, TRI_RING_PER_CU(96, 128, 5), 0.406f, 0.396f, 0.429f, 0.431f},
+    {128, 128, TRI_RING_PER_CU(128, 128, 5), 0.473f, 0.473f, 0.f, 0.f},
+    {128, 192, TRI_RING_PER_CU(128, 192, 3), 0.609f, 0.700f, 0.f, 0.f},
+    {128, 256, TRI_RING_PER_CU(128, 256, 3), 0.750f, 0.760f, 0.f, 0.f},
+    {160, 256, TRI_RING_PER_CU(160, 256, 3), 0.829f, 0.904f, 0.f, 0.f},
+    {192, 128, TRI_RING_PER_CU(192, 128, 3), 0.567f, 0.680f, 0.f, 0.f},
+    {192, 192, TRI_RING_PER_CU(192, 192, 3), 0.770f, 0.850f, 0.f, 0.f},
+    {256, 128, TRI_RING_PER_CU(256, 128, 3), 0.670f, 0.747f, 0.f, 0.f}};
 // A plan in one part on few workgroups: one streams no faster than about this many bytes of weights per us (16 rows x
 // [2048, 5632 x 2] as gate/up, 88 workgroups: 22.0 us, 16.0 in two parts; x [1024, 4096 x 2], 64: 12.0 and 10.1 in four; the
-// costs above, fitted where 200 and more workgroups share the memory's rate, say 14.9 and 7.8).  Up to 64 rows and 192
-// workgroups; beyond either the costs hold as they are (one row x K-contiguous [4096, 14336 x 2], 224 workgroups, would be
+// costs above, fitted where 200 and more workgroups share the memory's rate, say 14.9 and 7.8).  Up to 96 rows and 192
+// workgroups (75 rows x K-contiguous [4544, 18176], 142, 45.0 in three parts, 47.0 in one); beyond either the costs hold as they are (one row x K-contiguous [4096, 14336 x 2], 224 workgroups, would be
 // cut with the bound: the whole FFN 66.3 -> 72.4 us; 48 rows x [2048, 5632 x 2], 176, have to be cut: 22.2 -> 18.7).  What
 // the plan picked is slower than the best of the family on average, with this bound and without: gated products of 16 to
 // 100 rows, K of 512 to 8192, 2.1 % and 4.7; Q/K/V projections of 768- to 4544-wide models, up to 32 rows, 0.5 and 1.1;
 // plain products of such sizes 0.4 either way.
 constexpr float kRingStreamRate = 34e3f;
-constexpr int kRingStreamRows = 64, kRingStreamWorkgroups = 192;
+constexpr int kRingStreamRows = 96, kRingStreamWorkgroups = 192;
 
 static RingPlan ring_plan_search(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes, float merge_us) {
   RingPlan best = {-1, 1, 1e30f};
   const int KT = K / 64;
   const float wbytes = 2.0f * (float)K * (float)ncols, obytes = 4.0f * (float)M * (float)ncols;
+  const bool few = M <= kRingCost[kRingTileOneBlock].bm;
   for (int tile = 0; tile < kRingTiles; ++tile) {
     const RingCost& c = kRingCost[tile];
     if (c.bn % unit != 0 || c.bn < min_bn) continue;
-    if (tile == kRingTileOneBlock && M > c.bm) continue;
-    if (tile == 0 && M <= c.bm) continue;  // (the non-temporal twin serves these)
+    if (few ? c.few_alone == 0.f : tile == kRingTileOneBlock) continue;
+    const float alone = few ? c.few_alone : c.alone, shared = few ? c.few_shared : c.shared;
     const int tiles = ((M + c.bm - 1) / c.bm) * ((ncols + c.bn - 1) / c.bn);
     int last_per = 0;
     for (int s = 1; s <= 16; ++s) {
@@ -330,14 +344,21 @@ static RingPlan ring_plan_search(int M, int K, int ncols, int unit, int min_bn, 
       last_per = per;
       const int wg = tiles * ks, share = (wg + 255) / 256;
       const float even = share == 1 ? 1.0f : sqrtf((float)wg / (256.0f * share));
-      const float mem = wbytes / (8e6f * even) + (ks > 1 ? ks * obytes : 0.5f * obytes) / 3e6f;
-      const float it = share == 1 ? c.alone : (c.alone > c.shared * share ? c.alone : c.shared * share);
+      const float it = share == 1 ? alone : (alone > shared * share ? alone : shared * share);
       float comp = per * it;
       if (ks == 1 && wg <= kRingStreamWorkgroups && M <= kRingStreamRows) comp = fmaxf(comp, per * c.bn * 128.0f / kRingStreamRate);
-      const float loads = (float)wg * per * (c.bm + c.bn) * 128.0f / 37e6f;
-      const float sum = cbrtf(mem * sqrtf(mem) + comp * sqrtf(comp) + loads * sqrtf(loads));
-      const float us = 1.1f + 1.9f * ((share + c.per_cu - 1) / c.per_cu) + sum * sum +
-                       (ks > 1 ? merge_us + ks * obytes / 6e6f : 0.f);
+      const float waves = (float)((share + c.per_cu - 1) / c.per_cu), loaded = (float)wg * per * (c.bm + c.bn) * 128.0f;
+      const float written = ks > 1 ? ks * obytes : 0.5f * obytes;
+      float us;
+      if (few) {
+        const float mem = wbytes / (8e6f * even) + written / 3e6f, loads = loaded / 37e6f;
+        const float sum = cbrtf(mem * sqrtf(mem) + comp * sqrtf(comp) + loads * sqrtf(loads));
+        us = 1.1f + 1.9f * waves + sum * sum + (ks > 1 ? merge_us + ks * obytes / 6e6f : 0.f);
+      } else {
+        const float mem = wbytes / (12e6f * even) + written / 2.4e6f, loads = loaded / 62e6f;
+        const float sum = sqrtf(mem * cbrtf(mem) + comp * cbrtf(comp) + loads * cbrtf(loads));
+        us = 1.6f + 1.75f * waves + sum * sqrtf(sum) + (ks > 1 ? merge_us + 1.25f + ks * obytes / 10e6f : 0.f);
+      }
       if (us < best.us) { best.tile = tile; best.ksplit = ks; best.us = us; }
     }
   }

@@ -32,17 +32,19 @@ __global__ __launch_bounds__(T::NT) void ring_qkv_kernel(QkvProjArgs a) {
   constexpr int RS = T::BN + 8;  // halfs per staged row
   static_assert(T::BM * RS * 2 <= T::LDS_BYTES, "the staged output tile fits the ring");
   __syncthreads();
+  if (T::NP == 0 || wave < T::NW) {  // (a wave that only loads holds no part of the tile)
 #pragma unroll
-  for (int mi = 0; mi < T::MI; ++mi)
+    for (int mi = 0; mi < T::MI; ++mi)
 #pragma unroll
-    for (int ni = 0; ni < T::NI; ++ni)
+      for (int ni = 0; ni < T::NI; ++ni)
 #pragma unroll
-      for (int rq = 0; rq < 4; ++rq) {
-        half4v h;
+        for (int rq = 0; rq < 4; ++rq) {
+          half4v h;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) h[e] = (half_t)acc[ni][mi][rq * 4 + e];
-        *reinterpret_cast<half4v*>(lds + (wm * T::TM + mi * 32 + l32) * RS + wn * T::TN + ni * 32 + rq * 8 + g * 4) = h;
-      }
+          for (int e = 0; e < 4; ++e) h[e] = (half_t)acc[ni][mi][rq * 4 + e];
+          *reinterpret_cast<half4v*>(lds + (wm * T::TM + mi * 32 + l32) * RS + wn * T::TN + ni * 32 + rq * 8 + g * 4) = h;
+        }
+  }
   __syncthreads();
   constexpr int CH = T::BN / 8;  // 16-byte chunks per staged row
   static_assert(T::BM * CH % T::NT == 0, "every thread takes part in every pass (head sums run across lanes)");
@@ -132,10 +134,10 @@ static int launch_qkv_tile(const QkvProjArgs& a, int tile, hipStream_t stream) {
   if (tile == kRingTileOneBlock && ring_fourth_stage(a.S, ((a.Hq + 2 * a.Hkv) * D + 127) / 128, a.ldwq | a.ldwk | a.ldwv, a.K, a.w_kcontig != 0, false))
     return a.w_kcontig ? launch_qkv_t<RingTileFour, D, true>(a, stream) : launch_qkv_t<RingTileFour, D, false>(a, stream);
   switch (tile) {
-#define TRI_RING_CASE(id, bm, bn, wm, wn, nst, nt)                                                    \
+#define TRI_RING_CASE(id, bm, bn, wm, wn, nst, nt, np)                                                    \
   case id:                                                                                        \
-    return a.w_kcontig ? launch_qkv_t<RingTile<bm, bn, wm, wn, nst, nt>, D, true>(a, stream) \
-                       : launch_qkv_t<RingTile<bm, bn, wm, wn, nst, nt>, D, false>(a, stream);
+    return a.w_kcontig ? launch_qkv_t<RingTile<bm, bn, wm, wn, nst, nt, np>, D, true>(a, stream) \
+                       : launch_qkv_t<RingTile<bm, bn, wm, wn, nst, nt, np>, D, false>(a, stream);
     TRI_RING_TILES(TRI_RING_CASE)
 #undef TRI_RING_CASE
   }
