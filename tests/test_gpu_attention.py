@@ -56,6 +56,34 @@ LONG_NARROW_CASES = [
 ]
 
 
+# somewhat more than a round of eight-wave workgroups under a causal mask: whole query blocks in place of folded ones
+# (258 and 264 workgroups, a ragged last block, a short prefix; the last case is past the prefix that takes it)
+TURN_CASES = [
+    (641, 128, 43, 1, 128, 0, True),     # 6 blocks x 43 heads = 258 workgroups, the last block with one row
+    (700, 128, 44, 4, 128, 300, True),
+    (700, 128, 44, 4, 128, 360, True),
+]
+
+
+@pytest.mark.parametrize("S,N,Hq,Hkv,D,P,causal", TURN_CASES)
+@pytest.mark.parametrize("variant", ["vanilla", "keyformer"])
+def test_more_than_a_round_of_two_key_ways(dev, S, N, Hq, Hkv, D, P, causal, variant):
+    t = attn_inputs(S, N, Hq, Hkv, D, P=P, w_std=0.06)
+    scale = 1.0 / math.sqrt(D)
+    kw = dict(n_q_heads=Hq, n_kv_heads=Hkv, head_dim=D, scale=scale, causal=causal, kv_prefix=P,
+              k_cache=t.get("k_cache"), v_cache=t.get("v_cache"))
+    run = dict(Hq=Hq, Hkv=Hkv, D=D, P=P, scale=scale, causal=causal)
+    if variant == "vanilla":
+        want = oracle.qkv_attention(t["x"], t["wq"], t["wk"], t["wv"], want_lse=True, **kw)
+        got = run_qkv(t, dev, want_lse=True, **run)
+        assert_close(got["lse"], want["lse"], 1e-3, 2e-3, "lse")
+    else:
+        want = oracle.qkv_attention(t["x"], t["wq"], t["wk"], t["wv"], keyformer=True, noise_seed=11, tau=1.0, **kw)
+        got = run_qkv(t, dev, variant="keyformer", seed=11, tau=1.0, **run)
+        assert_scores(got["score"], want["score"], "perturbed scores")
+    assert_close(got["O2"], want["O2"], RTOL, ATOL, "O2")
+
+
 # few new tokens against thousands of cached keys: the looping key-split kernel with the query heads of a KV head
 # stacked along the query axis
 LONG_PREFIX_CASES = [

@@ -55,6 +55,7 @@ constexpr int kAttnStageRow = D + 8;  // halfs per row of an output tile staged 
 // taken against the same reference value, so the result is unchanged.
 constexpr float kLazyMax = 8.0f;
 constexpr int kTwoWayMaxWorkgroups = 256, kTwoWayMinKeys = 640;  // when the eight-wave variant runs
+constexpr int kTwoWayRoundsPlain = 352, kTwoWayRoundsSeeded = 448;  // ... and how far beyond a round (launch_attention)
 constexpr int kEightGroupMinWorkgroups = 129, kEightGroupMaxWorkgroups = 256;  // (of 256 queries each)
 constexpr int kWideMinWorkgroups = 768;  // 64 queries per wave (head dimension 64) from this many workgroups on
 
@@ -675,7 +676,8 @@ __device__ __forceinline__ void attn_fwd_pipe_body(const AttnArgs& a, half_t* ld
   const int hk = h / group;
   const int Ltot = a.P + a.S;
   int qw0 = qb * BQ + wave * 32 * QT, qend = qb * BQ + BQ;
-  if (KW == 2 && a.causal) {  // the folded half blocks of attn_fwd_body
+  // the folded half blocks of attn_fwd_body, within a round; beyond it whole blocks, which leave no wave idle
+  if (KW == 2 && a.causal && (int)gridDim.x <= kTwoWayMaxWorkgroups) {
     const int nhb = (a.S + 63) / 64, hb_long = nhb - 1 - qb, hb_short = qb;
     qw0 = wave < 2 ? hb_long * 64 + wave * 32 : (hb_short < hb_long ? hb_short * 64 + (wave - 2) * 32 : a.S);
     qend = hb_long * 64 + 64;
@@ -1254,10 +1256,17 @@ int launch_attention(const AttnArgs& a, hipStream_t stream, int* merge_parts) {
   const int kf = a.lse_pert == nullptr ? 0 : ((a.noise == nullptr && a.tau == 1.0f) ? 2 : 1);
   // At most one workgroup per CU and a long key axis: eight waves per workgroup walk the keys two tiles at a
   // time (Llama-3-8B, four-wave -> eight-wave kernel: S = 1024 26 -> 20.8 us, S = 768 20.0 -> 17.5 us, S = 512
-  // 14.4 -> 14.3 us, S = 256 9.6 -> 11.0 us; with more than one workgroup per CU the four-wave kernel is ahead:
-  // S = 1280 33 vs 43 us)
+  // 14.4 -> 14.3 us, S = 256 9.6 -> 11.0 us).
   const int64_t wgs = (int64_t)((a.S + 127) / 128) * a.Hq;
-  const bool two = wgs <= kTwoWayMaxWorkgroups && a.P + a.S >= kTwoWayMinKeys;
+  // Causal, 128-wide heads, somewhat more than a round: eight waves take whole query blocks, longest first, all of them
+  // busy to a block's end, where the eight query groups below leave a late wave alone on its SIMD.  Whole calls of 32
+  // heads on 8, eight groups -> this: plain, S = 1030 86.8 -> 83.4 us, 1152 89.8 -> 86.4, 1408 (352 workgroups) 112.9 ->
+  // 109.4, 1472 113.5 -> 113.3, 2048 142.9 -> 145.1, 2304 182 -> 189; seeded KeyFormer, 1408 161.6 -> 154.8, 1664 (416)
+  // 180.5 -> 174.3, 2048 211.2 -> 210.2.  A cached prefix evens the blocks out: 1100 tokens behind 1100 keys level,
+  // 1280 behind 3000 169.5 -> 176.4.  64-wide heads lose (71 heads, S = 768 57.8 -> 60.6).
+  const int rounds = kf == 2 ? kTwoWayRoundsSeeded : kTwoWayRoundsPlain;
+  const bool turns = a.D == 128 && a.causal && kf != 1 && 2 * a.P <= a.S && wgs <= rounds;
+  const bool two = (wgs <= kTwoWayMaxWorkgroups || turns) && a.P + a.S >= kTwoWayMinKeys;
   // One round of four-wave workgroups under a causal mask: eight query groups per workgroup instead (128-wide
   // heads; with 64-wide heads it is level at best: 71 heads S = 768 17.2 -> 17.7 us, 32 heads S = 2048 36.3 -> 35.5)
   const int64_t wgs8 = (int64_t)((a.S + 255) / 256) * a.Hq;
