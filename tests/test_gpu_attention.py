@@ -249,6 +249,39 @@ def test_keyformer_parity(dev, S, N, Hq, Hkv, D, P, causal, mode):
     assert torch.allclose(got["score"].sum(-1), torch.full((Hq,), float(S)), rtol=1e-3)
 
 
+# the score kernel's workgroups: one block of 64 keys each (64-key blocks x heads up to 256), two of them (up to twice
+# that, an odd number among them), two blocks of 128 keys beyond; odd numbers of query tiles, ragged ends, a prefix
+SCORE_CASES = [
+    (500, 128, 32, 8, 128, 0, True),     # 8 blocks x 32 heads: 256
+    (513, 128, 32, 8, 128, 0, True),     # 9 blocks, the middle one alone
+    (65, 128, 32, 8, 64, 900, True),     # 16 blocks in pairs, two query tiles, the second with one row
+    (200, 128, 32, 8, 128, 833, False),  # 17 blocks: 288 pairs of 64 keys are too many
+    (129, 128, 40, 8, 64, 700, True),
+]
+
+
+@pytest.mark.parametrize("S,N,Hq,Hkv,D,P,causal", SCORE_CASES)
+@pytest.mark.parametrize("variant", ["roco", "seeded", "tensor"])
+def test_score_workgroups(dev, S, N, Hq, Hkv, D, P, causal, variant):
+    t = attn_inputs(S, N, Hq, Hkv, D, P=P, w_std=0.06)
+    scale = 1.0 / math.sqrt(D)
+    kw = dict(n_q_heads=Hq, n_kv_heads=Hkv, head_dim=D, scale=scale, causal=causal, kv_prefix=P,
+              k_cache=t.get("k_cache"), v_cache=t.get("v_cache"))
+    run = dict(Hq=Hq, Hkv=Hkv, D=D, P=P, scale=scale, causal=causal)
+    if variant == "roco":
+        want = oracle.qkv_attention(t["x"], t["wq"], t["wk"], t["wv"], roco=True, **kw)
+        got = run_qkv(t, dev, variant="roco", **run)
+        assert_scores(got["s1"], want["s1"], "s1")
+        assert_scores(got["s2"], want["s2"], "s2")
+        return
+    noise = torch.randn(Hq, S, P + S, generator=gen(7)).half() if variant == "tensor" else None
+    kw.update(dict(noise=noise, tau=1.5) if variant == "tensor" else dict(noise_seed=5, tau=1.0))
+    run.update(dict(noise=noise, tau=1.5) if variant == "tensor" else dict(seed=5, tau=1.0))
+    want = oracle.qkv_attention(t["x"], t["wq"], t["wk"], t["wv"], keyformer=True, **kw)
+    got = run_qkv(t, dev, variant="keyformer", **run)
+    assert_scores(got["score"], want["score"], "score")
+
+
 # ----------------------------------------------------------------- numerically hard inputs and closed forms
 @pytest.mark.parametrize("S,P,D", [(300, 0, 128), (16, 500, 64), (200, 77, 64)])
 def test_large_logits_stay_finite_and_exact(dev, S, P, D):

@@ -12,6 +12,10 @@
 // Under the causal mask key block b only meets queries >= its first key, so
 // the work per block falls linearly with b; every workgroup therefore takes
 // block b and block (n - 1 - b), which makes all workgroups equally long.
+//
+// Where such workgroups leave CUs empty (up to 1024 keys x 32 heads) the kernel's time is one workgroup's chain of
+// tiles: there a workgroup owns 64 keys, its waves are two groups of keys times two query groups that take the tiles of
+// the query axis in turn, a step moves a pair of tiles, and the two groups' sums meet in LDS (QG = 2).
 #include "common.h"
 #include "launch.h"
 #include "philox.h"
@@ -20,9 +24,12 @@
 namespace tri {
 
 constexpr int kQTile = 64;
-constexpr int kKeysPerWg = 128;
+constexpr int kKeysPerWg = 128;  // (half of them with two query groups)
 
-constexpr int kScoreStages = 4;  // Q tiles in LDS
+constexpr int kScoreStages = 4;         // steps (a Q tile per query group) in LDS
+constexpr int kScoreMergeFloats = 64;   // sums a wave of the second query group hands over
+constexpr int kScoreRound = 256;        // workgroups that have a CU each
+constexpr int kScoreBlockTiles = 4;
 
 // s_waitcnt vmcnt(n) leaving the other counters unconstrained (gfx9 encoding)
 #define TRI_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | 0x0F70)
@@ -55,25 +62,28 @@ __device__ __forceinline__ float half_wave_sum_dpp(float x) {
 // itself the compiler puts all MFMAs of a tile first, each waiting for its LDS read, and the arithmetic after.
 // The chain of (tile t + 1, first half) runs during step t, so a Q tile must be in LDS one step before its own:
 // four LDS stages, tiles loaded three steps ahead (tiles past the last one read as zero and are never used).
-template <int D, int MODE_>
+template <int D, int MODE_, int QG>
 __device__ __forceinline__ void score_body(const ScoreArgs& a, half_t* lds) {
   constexpr int MODE = MODE_ == 0 ? 0 : 1;
   constexpr bool kf_fast = MODE_ == 2;  // seeded noise at temperature 1: exp(s + g) = exp(s) / (-ln u)
-  constexpr int STAGE = kQTile * D;  // halfs; unpadded, XOR-swizzled (chunk c of row r at slot c ^ f(r))
+  constexpr int TILE = kQTile * D;   // halfs; unpadded, XOR-swizzled (chunk c of row r at slot c ^ f(r))
+  constexpr int STAGE = QG * TILE;   // a step's tiles, one per query group
+  constexpr int KEYS = kKeysPerWg / QG, KWAVES = 4 / QG;
   constexpr int KSTEPS = D / 16;
-  constexpr int CPR = D / 8, INSTR = kQTile * D * 2 / 1024 / 4;
+  constexpr int CPR = D / 8, INSTR = QG * kQTile * D * 2 / 1024 / 4;
   constexpr int PD = 3, RING = 4;  // LDS reads run PD slots ahead of their MFMAs
   constexpr int GPS = 8 / KSTEPS;  // groups of two scores per MFMA slot
   static_assert(KSTEPS % RING == 0 && PD < KSTEPS, "the fragment ring keeps its phase from chain to chain");
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int kgroup = wave % KWAVES, qgroup = wave / KWAVES;
   const int l32 = lane & 31, g = lane >> 5;
   const int Ltot = a.P + a.S;
-  const int nkb = (Ltot + kKeysPerWg - 1) / kKeysPerWg;
+  const int nkb = (Ltot + KEYS - 1) / KEYS;
   // Linear workgroup id -> (head, pair of key blocks).  Workgroups go to the eight XCDs round-robin by id; with a
   // multiple of eight heads XCD x takes heads [x Hq / 8, (x + 1) Hq / 8), so that its L2 streams the Q rows of
   // those heads only (all workgroups of a head read the same Q).
-  const int nbx = (nkb + 1) / 2;
+  const int nbx = a.lone ? nkb : (nkb + 1) / 2;
   int h, bx;
   if (a.Hq % 8 == 0) {
     const int x = (int)blockIdx.x % 8, sidx = (int)blockIdx.x / 8;
@@ -108,21 +118,21 @@ __device__ __forceinline__ void score_body(const ScoreArgs& a, half_t* lds) {
   int qb[KSTEPS];
 #pragma unroll
   for (int ks = 0; ks < KSTEPS; ++ks) {
-    qb[ks] = (l32 * D + (((ks * 2 + g) ^ swz(l32)) << 3)) * 2;
+    qb[ks] = (qgroup * TILE + l32 * D + (((ks * 2 + g) ^ swz(l32)) << 3)) * 2;
     asm volatile("" : "+v"(qb[ks]));
   }
   const char* const ldsb = reinterpret_cast<const char*>(lds);
-  // fragment (tile qt, query half u, k step ks)
-  auto frag = [&](int qt, int u, int ks) {
-    return *reinterpret_cast<const half8v*>(ldsb + qb[ks] + ((qt & (kScoreStages - 1)) * STAGE + u * 32 * D) * 2);
+  // fragment (this wave's tile of step st, query half u, k step ks)
+  auto frag = [&](int st, int u, int ks) {
+    return *reinterpret_cast<const half8v*>(ldsb + qb[ks] + ((st & (kScoreStages - 1)) * STAGE + u * 32 * D) * 2);
   };
 
   for (int half = 0; half < 2; ++half) {
     // the two key blocks of this workgroup: b and n-1-b (the middle one only once)
     const int kb = half == 0 ? bx : nkb - 1 - bx;
-    if (half == 1 && kb <= bx) break;
-    const int kb0 = kb * kKeysPerWg;
-    const int kw0 = kb0 + wave * 32;
+    if (half == 1 && (a.lone || kb <= bx)) break;
+    const int kb0 = kb * KEYS;
+    const int kw0 = kb0 + kgroup * 32;
 
     // K fragments: MFMA source 0, rows = this wave's 32 keys
     half8v kf[KSTEPS];
@@ -140,19 +150,21 @@ __device__ __forceinline__ void score_body(const ScoreArgs& a, half_t* lds) {
       qstart = qstart > 0 ? (qstart / kQTile) * kQTile : 0;
     }
     const int nqt = qstart < a.S ? (a.S - qstart + kQTile - 1) / kQTile : 0;
-    auto issue = [&](int qt) {   // (qt may lie past the last tile: those rows are past S and read as zero)
+    const int nsteps = (nqt + QG - 1) / QG;
+    auto issue = [&](int st) {   // (st may lie past the last step: those rows are past S and read as zero)
 #pragma unroll
       for (int i = 0; i < INSTR; ++i)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            qrsrc, (TRI_LDS void*)(lds + (qt & (kScoreStages - 1)) * STAGE + (i * 4 + wave) * 512), 16,
-            // (unsigned: tiles up to three past the last one are issued, and for a Q buffer close to 2 GiB their
+            qrsrc, (TRI_LDS void*)(lds + (st & (kScoreStages - 1)) * STAGE + (i * 4 + wave) * 512), 16,
+            // (unsigned: steps up to three past the last one are issued, and for a Q buffer close to 2 GiB their
             // offsets pass 2^31; they stay beyond the descriptor's size and read as zero)
-            (int)((uint32_t)ld_off[i] + (uint32_t)(qstart / kQTile + qt) * (uint32_t)qtile_bytes), 0, 0, 0);
+            (int)((uint32_t)ld_off[i] + (uint32_t)(qstart / kQTile + st * QG) * (uint32_t)qtile_bytes), 0, 0, 0);
     };
-    auto load_lse = [&](int qt, float (&v)[2]) {
+    auto tile_of = [&](int st) { return st * QG + qgroup; };  // the wave's tile of a step
+    auto load_lse = [&](int st, float (&v)[2]) {
 #pragma unroll
       for (int nt = 0; nt < 2; ++nt) {
-        int q = qstart + qt * kQTile + nt * 32 + l32;
+        int q = qstart + tile_of(st) * kQTile + nt * 32 + l32;
         q = q < a.S ? q : a.S - 1;
         v[nt] = a.lse[(int64_t)h * a.S + q];
       }
@@ -162,10 +174,10 @@ __device__ __forceinline__ void score_body(const ScoreArgs& a, half_t* lds) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) { acc1[r] = 0.f; acc2[r] = 0.f; }
 
-    // vector arithmetic of scores 2 i and 2 i + 1 of a half tile (tile qt, query half u); st: its S^T block
+    // vector arithmetic of scores 2 i and 2 i + 1 of a half tile (step n, query half u); st: its S^T block
     uint32_t rnd[4] = {0u, 0u, 0u, 0u};
-    auto group = [&](const float16v& st, int qt, int u, float lse_q, int i, const bool MASK) {
-      const int q = qstart + qt * kQTile + u * 32 + l32;
+    auto group = [&](const float16v& st, int n, int u, float lse_q, int i, const bool MASK) {
+      const int q = qstart + tile_of(n) * kQTile + u * 32 + l32;
       const int qq = q < a.S ? q : a.S - 1;
       const int qlim = a.causal ? a.P + qq : Ltot;
       const float lse2 = lse_q * kLog2e;
@@ -206,9 +218,9 @@ __device__ __forceinline__ void score_body(const ScoreArgs& a, half_t* lds) {
       issue(0);
       issue(1);
       issue(2);
-      TRI_WAIT_VMCNT(2 * INSTR);     // lse(0) and this wave's share of tile 0
+      TRI_WAIT_VMCNT(2 * INSTR);     // lse(0) and this wave's share of step 0
       __builtin_amdgcn_s_barrier();
-      // ---- S^T of (tile 0, first half) on its own; the first fragments of its second half
+      // ---- S^T of (step 0, first half) on its own; the first fragments of its second half
 #pragma unroll
       for (int r = 0; r < 16; ++r) sa[r] = 0.f;
 #pragma unroll
@@ -216,18 +228,18 @@ __device__ __forceinline__ void score_body(const ScoreArgs& a, half_t* lds) {
 #pragma unroll
       for (int j = 0; j < PD; ++j) fr[j] = frag(0, 1, j);
 
-      // One step: [chain (qt, second half) beside the arithmetic of (qt, first half)], then
-      // [chain (qt + 1, first half) beside the arithmetic of (qt, second half)].
-      auto step = [&](int qt, const bool MASK) __attribute__((always_inline)) {
+      // One step: [chain (st, second half) beside the arithmetic of (st, first half)], then
+      // [chain (st + 1, first half) beside the arithmetic of (st, second half)].
+      auto step = [&](int st, const bool MASK) __attribute__((always_inline)) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) sb[r] = 0.f;
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < KSTEPS; ++i) {
-          fr[(i + PD) % RING] = (i + PD < KSTEPS) ? frag(qt, 1, i + PD) : frag(qt + 1, 0, i + PD - KSTEPS);
+          fr[(i + PD) % RING] = (i + PD < KSTEPS) ? frag(st, 1, i + PD) : frag(st + 1, 0, i + PD - KSTEPS);
           sb = mfma32(kf[i], fr[i % RING], sb);
 #pragma unroll
-          for (int x = 0; x < GPS; ++x) group(sa, qt, 0, lse_cur[0], i * GPS + x, MASK);
+          for (int x = 0; x < GPS; ++x) group(sa, st, 0, lse_cur[0], i * GPS + x, MASK);
           __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
@@ -235,58 +247,78 @@ __device__ __forceinline__ void score_body(const ScoreArgs& a, half_t* lds) {
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < KSTEPS; ++i) {
-          fr[(i + PD) % RING] = (i + PD < KSTEPS) ? frag(qt + 1, 0, i + PD) : frag(qt + 1, 1, i + PD - KSTEPS);
+          fr[(i + PD) % RING] = (i + PD < KSTEPS) ? frag(st + 1, 0, i + PD) : frag(st + 1, 1, i + PD - KSTEPS);
           sa = mfma32(kf[i], fr[i % RING], sa);
 #pragma unroll
-          for (int x = 0; x < GPS; ++x) group(sb, qt, 1, lse_cur[1], i * GPS + x, MASK);
+          for (int x = 0; x < GPS; ++x) group(sb, st, 1, lse_cur[1], i * GPS + x, MASK);
           __builtin_amdgcn_sched_barrier(0);
         }
       };
 
-      // Tiles [q0, q1), every one with or every one without masking.  The walk over the tiles is cut into such
+      // Steps [q0, q1), every one with or every one without masking.  The walk over the steps is cut into such
       // runs - the tiles on the causal diagonal come first, a ragged last tile last, and in between nothing is
       // masked - because one loop that chose between the two copies of the step tile by tile made the compiler keep
       // the sums and the S^T blocks in different registers in the two copies and move them at every turn: 62
       // register moves per tile beside 128 instructions of arithmetic (RoCo, S = 4096: 448 -> 440 us).
       auto run = [&](int q0, int q1, const bool MASK) __attribute__((always_inline)) {
-        for (int qt = q0; qt < q1; ++qt) {
+        for (int st = q0; st < q1; ++st) {
           // Two workgroups share a CU, and a SIMD serves the older of its two waves first whenever both are ready:
           // left alone, the older workgroup runs at the pace of a lone one, the younger on what is left, and then
           // finishes on its own, one wave per SIMD (S = 4096: one done after 76 us, the other after 110 us).  So the
           // two waves of a SIMD take turns at the higher priority, tile by tile, and stay side by side.
-          if ((qt ^ slot) & 1) __builtin_amdgcn_s_setprio(1);
+          if ((st ^ slot) & 1) __builtin_amdgcn_s_setprio(1);
           else __builtin_amdgcn_s_setprio(0);
-          // this wave's share of tile qt + 1 has landed (the loads of a wave complete in order; those of tile
-          // qt + 2 may still be in flight)
+          // this wave's share of step st + 1 has landed (the loads of a wave complete in order; those of step
+          // st + 2 may still be in flight)
           TRI_WAIT_VMCNT(INSTR);
-          __builtin_amdgcn_s_barrier();  // ... and everybody's; tile qt - 1 is retired
-          load_lse(qt + 1, lse_nxt);
-          issue(qt + 3);
-          step(qt, MASK);
+          __builtin_amdgcn_s_barrier();  // ... and everybody's; step st - 1 is retired
+          load_lse(st + 1, lse_nxt);
+          issue(st + 3);
+          step(st, MASK);
           lse_cur[0] = lse_nxt[0];
           lse_cur[1] = lse_nxt[1];
         }
       };
-      // masking is needed where the causal diagonal crosses this wave's keys - tile qt with
+      // masking is needed where the causal diagonal crosses this wave's keys - a tile qt with
       // kw0 + 31 > P + qstart + 64 qt - and at the ragged ends (keys past the last one: every tile; queries past
-      // S: the last tile).  Every wave walks all nqt tiles, one barrier each, whatever its runs are.
+      // S: the last tile, and one past it).  Every wave walks all steps, one barrier each, whatever its runs are.
+      auto steps_before = [&](int qt) { return min(nsteps, max(0, (qt - qgroup + QG - 1) / QG)); };  // the wave's, on tiles before qt
       int n_diag = 0;
-      if (kw0 + 32 > Ltot) n_diag = nqt;
-      else if (a.causal) n_diag = min(nqt, max(0, (kw0 + 31 - a.P - qstart + kQTile - 1) / kQTile));
-      const int n_plain_end = max(n_diag, (qstart + nqt * kQTile > a.S) ? nqt - 1 : nqt);
+      if (kw0 + 32 > Ltot) n_diag = nsteps;
+      else if (a.causal) n_diag = steps_before(max(0, (kw0 + 31 - a.P - qstart + kQTile - 1) / kQTile));
+      const int n_plain_end = max(n_diag, steps_before((qstart + nqt * kQTile > a.S) ? nqt - 1 : nqt));
       run(0, n_diag, true);
       run(n_diag, n_plain_end, false);
-      run(n_plain_end, nqt, true);
+      run(n_plain_end, nsteps, true);
       __builtin_amdgcn_s_setprio(0);
-      TRI_WAIT_VMCNT(0);  // (the loads past the last tile)
+      TRI_WAIT_VMCNT(0);  // (the loads past the last step)
     }
 
     // ---- reduce over the 32 query lanes; lane (l32 == 16) of each half writes
     const float invS = 1.0f / (float)a.S;
+    float* const other = reinterpret_cast<float*>(lds + kScoreStages * STAGE) + kgroup * kScoreMergeFloats;  // sums of query group 1
+    if (QG == 2) {
+      if (qgroup == 1) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float s1 = half_wave_sum_dpp(acc1[r]), s2 = MODE == 0 ? half_wave_sum_dpp(acc2[r]) : 0.f;
+          if (l32 == 16) {
+            other[g * 32 + r] = s1;
+            if (MODE == 0) other[g * 32 + 16 + r] = s2;
+          }
+        }
+      }
+      __syncthreads();  // (the next block's sums are written behind its barriers)
+      if (qgroup == 1) continue;
+    }
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const float s1 = half_wave_sum_dpp(acc1[r]) * ((MODE == 1 && kf_fast) ? kInvNegLnScale : 1.0f);
-      const float s2 = (MODE == 0) ? half_wave_sum_dpp(acc2[r]) : 0.f;
+      float s1 = half_wave_sum_dpp(acc1[r]), s2 = MODE == 0 ? half_wave_sum_dpp(acc2[r]) : 0.f;
+      if (QG == 2) {
+        s1 += other[g * 32 + r];
+        if (MODE == 0) s2 += other[g * 32 + 16 + r];
+      }
+      if (MODE == 1 && kf_fast) s1 *= kInvNegLnScale;
       const int key = kw0 + (r >> 2) * 8 + g * 4 + (r & 3);
       if (l32 == 16 && key < Ltot) {
         if (MODE == 0) {
@@ -307,10 +339,45 @@ __device__ __forceinline__ void score_body(const ScoreArgs& a, half_t* lds) {
 }
 
 // (body in a device function: see the note at attn_fwd_kernel)
-template <int D, int MODE>
+template <int D, int MODE, int QG>
 __global__ __launch_bounds__(256) void score_kernel(ScoreArgs a) {
-  __shared__ __attribute__((aligned(16))) half_t lds[kScoreStages * kQTile * D];
-  score_body<D, MODE>(a, lds);
+  extern __shared__ __attribute__((aligned(16))) half_t lds[];
+  score_body<D, MODE, QG>(a, lds);
+}
+
+template <int D, int MODE, int QG>
+static int launch_score_t(ScoreArgs a, bool lone, hipStream_t stream) {
+  constexpr int LDS = kScoreStages * QG * kQTile * D * 2 + (QG == 2 ? 2 * kScoreMergeFloats * 4 : 0);
+  constexpr auto kern = score_kernel<D, MODE, QG>;
+  if (set_max_lds<kern, LDS>() != 0) return -1;
+  const int nkb = (a.P + a.S + kKeysPerWg / QG - 1) / (kKeysPerWg / QG);
+  a.lone = lone;
+  hipLaunchKernelGGL(kern, dim3((lone ? nkb : (nkb + 1) / 2) * a.Hq), dim3(256), LDS, stream, a);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+// One block a workgroup or two, of 128 keys or of 64 with two query groups: the shortest chain of those whose workgroups
+// have a CU each, a block's first loads and last sums taken for kScoreBlockTiles tiles.  Two blocks of 128 keys as the only
+// form -> this, whole calls of 32 heads on 8: RoCo, 130 tokens (one of 64, 96 workgroups) 39.1 -> 36.7 us, 512 (one of 64,
+// 256) 63.5 -> 57.7, 640 (one of 128, 160; two of 64: 70.2) 69.9 -> 64.8, 1000 (two of 64, 256) 89.6 -> 86.8, 64 against
+// 300 keys (one of 128, 96; one of 64: 33.6) 35.6 -> 32.0; KeyFormer 200 49.8 -> 43.5, 1024 100.4 -> 93.6, 300 against 600
+// 71.6 -> 63.5; 71 heads of 64, 100 against 200 keys 33.9 -> 30.4.
+template <int D, int MODE>
+static int launch_score_d(const ScoreArgs& a, hipStream_t stream) {
+  int qg = 1, least = 1 << 30;
+  bool lone = false;
+  for (int g = 1; g <= 2; ++g) {
+    const int keys = kKeysPerWg / g, nkb = (a.P + a.S + keys - 1) / keys;
+    auto steps = [&](int kb) {  // of key block kb
+      const int q0 = a.causal ? kb * keys - a.P : 0;
+      const int tiles = (a.S - (q0 > 0 ? q0 / kQTile * kQTile : 0) + kQTile - 1) / kQTile;
+      return kScoreBlockTiles + (tiles + g - 1) / g;
+    };
+    const int one = steps(0), two = nkb > 1 ? one + steps(nkb - 1) : one;
+    if ((int64_t)nkb * a.Hq <= kScoreRound && one < least) { least = one; qg = g; lone = true; }
+    if ((int64_t)(nkb + 1) / 2 * a.Hq <= kScoreRound && two < least) { least = two; qg = g; lone = false; }
+  }
+  return qg == 2 ? launch_score_t<D, MODE, 2>(a, lone, stream) : launch_score_t<D, MODE, 1>(a, lone, stream);
 }
 
 int launch_scores(const ScoreArgs& a, hipStream_t stream) {
@@ -319,22 +386,13 @@ int launch_scores(const ScoreArgs& a, hipStream_t stream) {
     const int r = launch_scores_few(a, stream);
     if (r <= 0) return r;
   }
-  const int Ltot = a.P + a.S;
-  const int nkb = (Ltot + kKeysPerWg - 1) / kKeysPerWg;
-  const dim3 grid(((nkb + 1) / 2) * a.Hq), block(256);
-  const bool fast = a.mode == 1 && a.noise == nullptr && a.tau == 1.0f;
-  if (a.D == 128) {
-    if (a.mode == 0) hipLaunchKernelGGL((score_kernel<128, 0>), grid, block, 0, stream, a);
-    else if (fast) hipLaunchKernelGGL((score_kernel<128, 2>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((score_kernel<128, 1>), grid, block, 0, stream, a);
-  } else if (a.D == 64) {
-    if (a.mode == 0) hipLaunchKernelGGL((score_kernel<64, 0>), grid, block, 0, stream, a);
-    else if (fast) hipLaunchKernelGGL((score_kernel<64, 2>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((score_kernel<64, 1>), grid, block, 0, stream, a);
-  } else {
-    return -1;
+  if (a.D != 64 && a.D != 128) return -1;
+  const int mode = a.mode == 1 && a.noise == nullptr && a.tau == 1.0f ? 2 : a.mode;
+  switch (mode) {
+    case 0: return a.D == 128 ? launch_score_d<128, 0>(a, stream) : launch_score_d<64, 0>(a, stream);
+    case 1: return a.D == 128 ? launch_score_d<128, 1>(a, stream) : launch_score_d<64, 1>(a, stream);
+    default: return a.D == 128 ? launch_score_d<128, 2>(a, stream) : launch_score_d<64, 2>(a, stream);
   }
-  return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 }  // namespace tri
