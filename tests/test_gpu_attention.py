@@ -250,13 +250,16 @@ def test_keyformer_parity(dev, S, N, Hq, Hkv, D, P, causal, mode):
 
 
 # the score kernel's workgroups: one block of 64 keys each (64-key blocks x heads up to 256), two of them (up to twice
-# that, an odd number among them), two blocks of 128 keys beyond; odd numbers of query tiles, ragged ends, a prefix
+# that, an odd number among them), one block of 128 keys beyond, pairs of these for a single query tile; odd numbers of
+# query tiles, ragged ends, a prefix
 SCORE_CASES = [
     (500, 128, 32, 8, 128, 0, True),     # 8 blocks x 32 heads: 256
     (513, 128, 32, 8, 128, 0, True),     # 9 blocks, the middle one alone
     (65, 128, 32, 8, 64, 900, True),     # 16 blocks in pairs, two query tiles, the second with one row
     (200, 128, 32, 8, 128, 833, False),  # 17 blocks: 288 pairs of 64 keys are too many
     (129, 128, 40, 8, 64, 700, True),
+    (130, 128, 43, 1, 64, 700, True),    # heads no multiple of eight: 7 x 43
+    (40, 128, 64, 8, 128, 1570, True),   # 13 blocks x 64 heads, one query tile: pairs, the middle block alone
 ]
 
 

@@ -10,8 +10,9 @@
 // reduction at the very end.  Nothing of size [heads, S, S] ever reaches HBM.
 //
 // Under the causal mask key block b only meets queries >= its first key, so
-// the work per block falls linearly with b; every workgroup therefore takes
-// block b and block (n - 1 - b), which makes all workgroups equally long.
+// the work per block falls linearly with b: the longest blocks are dispatched
+// first.  (Pairs of blocks b and n - 1 - b, all equally long, remain where a
+// workgroup would have too little to do, see launch_score_d.)
 //
 // Where such workgroups leave CUs empty (up to 1024 keys x 32 heads) the kernel's time is one workgroup's chain of
 // tiles: there a workgroup owns 64 keys, its waves are two groups of keys times two query groups that take the tiles of
@@ -29,7 +30,7 @@ constexpr int kKeysPerWg = 128;  // (half of them with two query groups)
 constexpr int kScoreStages = 4;         // steps (a Q tile per query group) in LDS
 constexpr int kScoreMergeFloats = 64;   // sums a wave of the second query group hands over
 constexpr int kScoreRound = 256;        // workgroups that have a CU each
-constexpr int kScoreBlockTiles = 4;
+constexpr int kScoreBlockTiles = 4, kScorePairWorkgroups = 768;  // (launch_score_d; the latter per query tile)
 
 // s_waitcnt vmcnt(n) leaving the other counters unconstrained (gfx9 encoding)
 #define TRI_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | 0x0F70)
@@ -80,15 +81,16 @@ __device__ __forceinline__ void score_body(const ScoreArgs& a, half_t* lds) {
   const int l32 = lane & 31, g = lane >> 5;
   const int Ltot = a.P + a.S;
   const int nkb = (Ltot + KEYS - 1) / KEYS;
-  // Linear workgroup id -> (head, pair of key blocks).  Workgroups go to the eight XCDs round-robin by id; with a
+  // Linear workgroup id -> (head, key block or pair of them).  Workgroups go to the eight XCDs round-robin by id; with a
   // multiple of eight heads XCD x takes heads [x Hq / 8, (x + 1) Hq / 8), so that its L2 streams the Q rows of
   // those heads only (all workgroups of a head read the same Q).
   const int nbx = a.lone ? nkb : (nkb + 1) / 2;
   int h, bx;
   if (a.Hq % 8 == 0) {
     const int x = (int)blockIdx.x % 8, sidx = (int)blockIdx.x / 8;
-    h = x * (a.Hq / 8) + sidx / nbx;
-    bx = sidx % nbx;
+    const int hx = a.Hq / 8;
+    h = x * hx + (a.lone ? sidx % hx : sidx / nbx);
+    bx = a.lone ? sidx / hx : sidx % nbx;
   } else {
     h = (int)blockIdx.x / nbx;
     bx = (int)blockIdx.x % nbx;
@@ -356,28 +358,32 @@ static int launch_score_t(ScoreArgs a, bool lone, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-// One block a workgroup or two, of 128 keys or of 64 with two query groups: the shortest chain of those whose workgroups
-// have a CU each, a block's first loads and last sums taken for kScoreBlockTiles tiles.  Two blocks of 128 keys as the only
-// form -> this, whole calls of 32 heads on 8: RoCo, 130 tokens (one of 64, 96 workgroups) 39.1 -> 36.7 us, 512 (one of 64,
-// 256) 63.5 -> 57.7, 640 (one of 128, 160; two of 64: 70.2) 69.9 -> 64.8, 1000 (two of 64, 256) 89.6 -> 86.8, 64 against
-// 300 keys (one of 128, 96; one of 64: 33.6) 35.6 -> 32.0; KeyFormer 200 49.8 -> 43.5, 1024 100.4 -> 93.6, 300 against 600
-// 71.6 -> 63.5; 71 heads of 64, 100 against 200 keys 33.9 -> 30.4.
+// One block of 128 keys a workgroup, or, where workgroups have a CU each, one or two blocks of 64 with two query groups if
+// that chain is shorter, a block's first loads and last sums taken for kScoreBlockTiles tiles.  Pairs of 128-key blocks as
+// the only form -> this, whole calls of 32 heads on 8: RoCo, 130 tokens (one of 64, 96 workgroups) 39.1 -> 36.7 us, 512 (one
+// of 64, 256) 63.5 -> 57.7, 640 (one of 128, 160; two of 64: 70.2) 69.9 -> 64.8, 1000 (two of 64, 256) 89.6 -> 86.8, 64
+// against 300 keys (one of 128, 96; one of 64: 33.6) 35.6 -> 32.0; KeyFormer 200 49.8 -> 43.5, 1024 100.4 -> 93.6, 300 against
+// 600 71.6 -> 63.5; 71 heads of 64, 100 against 200 keys 33.9 -> 30.4.  Beyond a round, one block of 128: RoCo 1100 107.6 ->
+// 103.3, 2048 179.3 -> 177.8, 3000 309.6 -> 303.0, 4096 420.8 -> 422.7, KeyFormer 1280 136.0 -> 131.8, 2048 209.7 -> 206.5; but
+// pairs where a block meets few query tiles and there are many (one tile, 33 against 3000 keys, 768 blocks, 42.4 -> 41.4, 64
+// against 4000, 1024, 50.6 -> 51.1, 40 against 16000, 4032, 98.8 -> 102.7; two, 100 against 6000, 1536, 71.3 -> 70.5; three, 150
+// against 15000, 3808, 141.2 -> 142.9; five, 300 against 9000, 2336, 149.1 -> 145.1; seven, 71 heads, 400 against 15000,
+// 8520, 361.8 -> 363.5; eight, 512 against 16000, 4224, level).
 template <int D, int MODE>
 static int launch_score_d(const ScoreArgs& a, hipStream_t stream) {
-  int qg = 1, least = 1 << 30;
-  bool lone = false;
-  for (int g = 1; g <= 2; ++g) {
-    const int keys = kKeysPerWg / g, nkb = (a.P + a.S + keys - 1) / keys;
-    auto steps = [&](int kb) {  // of key block kb
-      const int q0 = a.causal ? kb * keys - a.P : 0;
-      const int tiles = (a.S - (q0 > 0 ? q0 / kQTile * kQTile : 0) + kQTile - 1) / kQTile;
-      return kScoreBlockTiles + (tiles + g - 1) / g;
-    };
-    const int one = steps(0), two = nkb > 1 ? one + steps(nkb - 1) : one;
-    if ((int64_t)nkb * a.Hq <= kScoreRound && one < least) { least = one; qg = g; lone = true; }
-    if ((int64_t)(nkb + 1) / 2 * a.Hq <= kScoreRound && two < least) { least = two; qg = g; lone = false; }
-  }
-  return qg == 2 ? launch_score_t<D, MODE, 2>(a, lone, stream) : launch_score_t<D, MODE, 1>(a, lone, stream);
+  auto blocks = [&](int g) { const int keys = kKeysPerWg / g; return (a.P + a.S + keys - 1) / keys; };
+  auto chain = [&](int g, int kb) {  // steps of key block kb
+    const int q0 = a.causal ? kb * (kKeysPerWg / g) - a.P : 0;
+    const int tiles = (a.S - (q0 > 0 ? q0 / kQTile * kQTile : 0) + kQTile - 1) / kQTile;
+    return kScoreBlockTiles + (tiles + g - 1) / g;
+  };
+  const int n1 = blocks(1), n2 = blocks(2);
+  const int64_t one = (int64_t)n1 * a.Hq, half = (int64_t)n2 * a.Hq;
+  const int whole = one <= kScoreRound ? chain(1, 0) : 1 << 30;
+  if (half <= kScoreRound && chain(2, 0) < whole) return launch_score_t<D, MODE, 2>(a, true, stream);
+  if (n2 > 1 && (int64_t)(n2 + 1) / 2 * a.Hq <= kScoreRound && chain(2, 0) + chain(2, n2 - 1) < whole)
+    return launch_score_t<D, MODE, 2>(a, false, stream);
+  return launch_score_t<D, MODE, 1>(a, one <= (int64_t)kScorePairWorkgroups * ((a.S + kQTile - 1) / kQTile), stream);
 }
 
 int launch_scores(const ScoreArgs& a, hipStream_t stream) {
