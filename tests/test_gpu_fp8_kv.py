@@ -76,6 +76,11 @@ CASES = [
     (200, 320, 5, 1, 64, 0, True),
     (16, 128, 4, 2, 128, 4200, True),    # long prefix: the looping key-split kernel converts the fp8 tiles itself
     (20, 128, 6, 1, 64, 3001, False),    # ... 120 stacked rows, ragged last tile
+    (33, 128, 4, 4, 128, 2100, True),    # ... chunks: 33 rows of a head, two waves a tile
+    (40, 128, 4, 2, 128, 9000, True),    # ... 80 rows, long runs: pairs of tiles
+    (200, 128, 2, 1, 64, 3001, True),    # ... four row blocks, the last one ragged
+    (130, 128, 4, 1, 128, 2500, False),
+    (33, 128, 2, 1, 64, 2014, True),     # ... one key short of the key-split kernel: through the 16-bit copy
 ]
 # models so wide that the projection runs in parts: their merge converts and appends the new rows
 PARTS = [

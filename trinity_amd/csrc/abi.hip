@@ -70,7 +70,7 @@ struct Scratch {
 inline int64_t align256(int64_t x) { return (x + 255) & ~(int64_t)255; }
 
 // Partial results of the key-split attention of a call of S tokens, for every run the key axis would be cut into, for the
-// fewest, or what the call cannot do without: up to 32 tokens the attention kernels (the only ones that read fp8 rows)
+// fewest, or what the call cannot do without: up to 32 tokens the attention kernels (for fp8 rows there are no others then)
 // always leave parts (kNoRunsAnyPrefix: a bound of that over all prefixes up to the call's).
 enum AttnParts { kAllRuns, kFewestRuns, kNoRuns, kNoRunsAnyPrefix };
 int64_t attn_parts_bytes(const tri_attn_params* p, int S, AttnParts runs) {

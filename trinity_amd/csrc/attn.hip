@@ -1212,6 +1212,11 @@ int64_t split_attn_workspace_bytes(int S, int Hq, int Hkv, int D, int Ltot, bool
   return (int64_t)Hq * (least ? fewest : nsplit) * S * (D + 4) * 4;
 }
 
+bool split_attn_takes(int S, int Hq, int Hkv, int D, int Ltot, int64_t ws_bytes) {
+  const int64_t least = split_attn_workspace_bytes(S, Hq, Hkv, D, Ltot, true);
+  return least > 0 && ws_bytes >= least;
+}
+
 static int launch_attn_split(const AttnArgs& a, hipStream_t stream) {
   const int Ltot = a.P + a.S;
   const int kf = a.lse_pert == nullptr ? 0 : ((a.noise == nullptr && a.tau == 1.0f) ? 2 : 1);

@@ -187,6 +187,7 @@ int launch_attention_few_combine(const AttnArgs& a, int nsplit, hipStream_t stre
 // workspace of launch_attention's long-prefix variant for a call (0 when it does not take it): for all the runs it would
 // cut the key axis into, or (least) for the fewest it works with - given less than the former it takes fewer runs
 int64_t split_attn_workspace_bytes(int S, int Hq, int Hkv, int D, int Ltot, bool least);
+bool split_attn_takes(int S, int Hq, int Hkv, int D, int Ltot, int64_t ws_bytes);  // the key-split kernel runs, with that workspace
 // From this many keys on, plain attention for few new tokens leaves the one-tile-per-wave kernel for one that
 // loops over its keys with the query heads of a KV head stacked along the query axis (launch_attention decides).
 // 16 tokens: at 1040 keys the two are level, at 2064 keys the looping kernel is 2-5 us ahead, at 32784 keys
