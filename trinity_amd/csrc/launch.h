@@ -239,7 +239,6 @@ struct ScoreArgs {
   half_t* out;
   int64_t ldo;
   float out_scale;
-  int lone;  // a workgroup takes one key block, not two (set by launch_scores)
 };
 int launch_scores(const ScoreArgs& a, hipStream_t stream);
 int launch_scores_few(const ScoreArgs& a, hipStream_t stream);  // S <= kFewMaxQueries; 1 = not applicable

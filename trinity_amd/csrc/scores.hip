@@ -63,7 +63,11 @@ __device__ __forceinline__ float half_wave_sum_dpp(float x) {
 // itself the compiler puts all MFMAs of a tile first, each waiting for its LDS read, and the arithmetic after.
 // The chain of (tile t + 1, first half) runs during step t, so a Q tile must be in LDS one step before its own:
 // four LDS stages, tiles loaded three steps ahead (tiles past the last one read as zero and are never used).
-template <int D, int MODE_, int QG>
+//
+// LONE: a workgroup takes one key block, not two.  (A template parameter: as a field of the arguments it left the loop's
+// instructions as they are and cost RoCo 13 % all the same - 10 heads of 128, 1500 tokens, the kernel alone, pairs 27.5 -> 31.0 us,
+// single blocks 21.6 -> 25.0; 71 heads of 64, 300 against 9000 keys, single blocks 71.5 -> 77.8; KeyFormer 31.1 -> 31.6.)
+template <int D, int MODE_, int QG, bool LONE>
 __device__ __forceinline__ void score_body(const ScoreArgs& a, half_t* lds) {
   constexpr int MODE = MODE_ == 0 ? 0 : 1;
   constexpr bool kf_fast = MODE_ == 2;  // seeded noise at temperature 1: exp(s + g) = exp(s) / (-ln u)
@@ -84,13 +88,13 @@ __device__ __forceinline__ void score_body(const ScoreArgs& a, half_t* lds) {
   // Linear workgroup id -> (head, key block or pair of them).  Workgroups go to the eight XCDs round-robin by id; with a
   // multiple of eight heads XCD x takes heads [x Hq / 8, (x + 1) Hq / 8), so that its L2 streams the Q rows of
   // those heads only (all workgroups of a head read the same Q).
-  const int nbx = a.lone ? nkb : (nkb + 1) / 2;
+  const int nbx = LONE ? nkb : (nkb + 1) / 2;
   int h, bx;
   if (a.Hq % 8 == 0) {
     const int x = (int)blockIdx.x % 8, sidx = (int)blockIdx.x / 8;
     const int hx = a.Hq / 8;
-    h = x * hx + (a.lone ? sidx % hx : sidx / nbx);
-    bx = a.lone ? sidx / hx : sidx % nbx;
+    h = x * hx + (LONE ? sidx % hx : sidx / nbx);
+    bx = LONE ? sidx / hx : sidx % nbx;
   } else {
     h = (int)blockIdx.x / nbx;
     bx = (int)blockIdx.x % nbx;
@@ -132,7 +136,7 @@ __device__ __forceinline__ void score_body(const ScoreArgs& a, half_t* lds) {
   for (int half = 0; half < 2; ++half) {
     // the two key blocks of this workgroup: b and n-1-b (the middle one only once)
     const int kb = half == 0 ? bx : nkb - 1 - bx;
-    if (half == 1 && (a.lone || kb <= bx)) break;
+    if (half == 1 && (LONE || kb <= bx)) break;
     const int kb0 = kb * KEYS;
     const int kw0 = kb0 + kgroup * 32;
 
@@ -341,20 +345,19 @@ __device__ __forceinline__ void score_body(const ScoreArgs& a, half_t* lds) {
 }
 
 // (body in a device function: see the note at attn_fwd_kernel)
-template <int D, int MODE, int QG>
+template <int D, int MODE, int QG, bool LONE>
 __global__ __launch_bounds__(256) void score_kernel(ScoreArgs a) {
   extern __shared__ __attribute__((aligned(16))) half_t lds[];
-  score_body<D, MODE, QG>(a, lds);
+  score_body<D, MODE, QG, LONE>(a, lds);
 }
 
-template <int D, int MODE, int QG>
-static int launch_score_t(ScoreArgs a, bool lone, hipStream_t stream) {
+template <int D, int MODE, int QG, bool LONE>
+static int launch_score_t(const ScoreArgs& a, hipStream_t stream) {
   constexpr int LDS = kScoreStages * QG * kQTile * D * 2 + (QG == 2 ? 2 * kScoreMergeFloats * 4 : 0);
-  constexpr auto kern = score_kernel<D, MODE, QG>;
+  constexpr auto kern = score_kernel<D, MODE, QG, LONE>;
   if (set_max_lds<kern, LDS>() != 0) return -1;
   const int nkb = (a.P + a.S + kKeysPerWg / QG - 1) / (kKeysPerWg / QG);
-  a.lone = lone;
-  hipLaunchKernelGGL(kern, dim3((lone ? nkb : (nkb + 1) / 2) * a.Hq), dim3(256), LDS, stream, a);
+  hipLaunchKernelGGL(kern, dim3((LONE ? nkb : (nkb + 1) / 2) * a.Hq), dim3(256), LDS, stream, a);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -380,10 +383,11 @@ static int launch_score_d(const ScoreArgs& a, hipStream_t stream) {
   const int n1 = blocks(1), n2 = blocks(2);
   const int64_t one = (int64_t)n1 * a.Hq, half = (int64_t)n2 * a.Hq;
   const int whole = one <= kScoreRound ? chain(1, 0) : 1 << 30;
-  if (half <= kScoreRound && chain(2, 0) < whole) return launch_score_t<D, MODE, 2>(a, true, stream);
+  if (half <= kScoreRound && chain(2, 0) < whole) return launch_score_t<D, MODE, 2, true>(a, stream);
   if (n2 > 1 && (int64_t)(n2 + 1) / 2 * a.Hq <= kScoreRound && chain(2, 0) + chain(2, n2 - 1) < whole)
-    return launch_score_t<D, MODE, 2>(a, false, stream);
-  return launch_score_t<D, MODE, 1>(a, one <= (int64_t)kScorePairWorkgroups * ((a.S + kQTile - 1) / kQTile), stream);
+    return launch_score_t<D, MODE, 2, false>(a, stream);
+  return one <= (int64_t)kScorePairWorkgroups * ((a.S + kQTile - 1) / kQTile) ? launch_score_t<D, MODE, 1, true>(a, stream)
+                                                                           : launch_score_t<D, MODE, 1, false>(a, stream);
 }
 
 int launch_scores(const ScoreArgs& a, hipStream_t stream) {
