@@ -87,7 +87,10 @@ __device__ __forceinline__ void score_body(const ScoreArgs& a, half_t* lds) {
   const int nkb = (Ltot + KEYS - 1) / KEYS;
   // Linear workgroup id -> (head, key block or pair of them).  Workgroups go to the eight XCDs round-robin by id; with a
   // multiple of eight heads XCD x takes heads [x Hq / 8, (x + 1) Hq / 8), so that its L2 streams the Q rows of
-  // those heads only (all workgroups of a head read the same Q).
+  // those heads only (all workgroups of a head read the same Q).  Other head counts: pairs head by head; single blocks by
+  // length, all heads' longest first (head by head the last heads' long blocks start last: whole calls, 71 heads of 64, RoCo 2048
+  // tokens 207 -> 188 us, 4096 548 -> 482, KeyFormer 1000 127 -> 111, 4096 904 -> 760; 20 of 128 on 4, KeyFormer 4096 441 -> 365; level
+  // behind long prefixes, where all blocks are as long).
   const int nbx = LONE ? nkb : (nkb + 1) / 2;
   int h, bx;
   if (a.Hq % 8 == 0) {
@@ -96,8 +99,8 @@ __device__ __forceinline__ void score_body(const ScoreArgs& a, half_t* lds) {
     h = x * hx + (LONE ? sidx % hx : sidx / nbx);
     bx = LONE ? sidx / hx : sidx % nbx;
   } else {
-    h = (int)blockIdx.x / nbx;
-    bx = (int)blockIdx.x % nbx;
+    h = LONE ? (int)blockIdx.x % a.Hq : (int)blockIdx.x / nbx;
+    bx = LONE ? (int)blockIdx.x / a.Hq : (int)blockIdx.x % nbx;
   }
   const int hk = h / (a.Hq / a.Hkv);
   // the wave's slot on its SIMD (HW_ID bits 3:0): the waves that share a SIMD differ in it
