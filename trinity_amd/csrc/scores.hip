@@ -30,7 +30,7 @@ constexpr int kKeysPerWg = 128;  // (half of them with two query groups)
 constexpr int kScoreStages = 4;         // steps (a Q tile per query group) in LDS
 constexpr int kScoreMergeFloats = 64;   // sums a wave of the second query group hands over
 constexpr int kScoreRound = 256;        // workgroups that have a CU each
-constexpr int kScoreBlockTiles = 4, kScorePairWorkgroups = 768;  // (launch_score_d; the latter per query tile)
+constexpr int kScoreBlockTiles = 4, kScoreHandTiles = 1, kScorePairWorkgroups = 768;  // (launch_score_d; the last per query tile)
 
 // s_waitcnt vmcnt(n) leaving the other counters unconstrained (gfx9 encoding)
 #define TRI_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | 0x0F70)
@@ -365,23 +365,25 @@ static int launch_score_t(const ScoreArgs& a, hipStream_t stream) {
 }
 
 // One block of 128 keys a workgroup, or, where workgroups have a CU each, one or two blocks of 64 with two query groups if
-// that chain is shorter, a block's first loads and last sums taken for kScoreBlockTiles tiles.  Pairs of 128-key blocks as
-// the only form -> this, whole calls of 32 heads on 8: RoCo, 130 tokens (one of 64, 96 workgroups) 39.1 -> 36.7 us, 512 (one
-// of 64, 256) 63.5 -> 57.7, 640 (one of 128, 160; two of 64: 70.2) 69.9 -> 64.8, 1000 (two of 64, 256) 89.6 -> 86.8, 64
-// against 300 keys (one of 128, 96; one of 64: 33.6) 35.6 -> 32.0; KeyFormer 200 49.8 -> 43.5, 1024 100.4 -> 93.6, 300 against
-// 600 71.6 -> 63.5; 71 heads of 64, 100 against 200 keys 33.9 -> 30.4.  Beyond a round, one block of 128: RoCo 1100 107.6 ->
-// 103.3, 2048 179.3 -> 177.8, 3000 309.6 -> 303.0, 4096 420.8 -> 422.7, KeyFormer 1280 136.0 -> 131.8, 2048 209.7 -> 206.5; but
-// pairs where a block meets few query tiles and there are many (one tile, 33 against 3000 keys, 768 blocks, 42.4 -> 41.4, 64
-// against 4000, 1024, 50.6 -> 51.1, 40 against 16000, 4032, 98.8 -> 102.7; two, 100 against 6000, 1536, 71.3 -> 70.5; three, 150
-// against 15000, 3808, 141.2 -> 142.9; five, 300 against 9000, 2336, 149.1 -> 145.1; seven, 71 heads, 400 against 15000,
-// 8520, 361.8 -> 363.5; eight, 512 against 16000, 4224, level).
+// that chain is shorter, a block's first loads and last sums taken for kScoreBlockTiles tiles and the hand-over between
+// two query groups for kScoreHandTiles.  (It counts: without it calls of 65 to 192 tokens took two groups, whole calls of 32
+// heads on 8, RoCo 65 tokens 33.7 -> 34.5 us, 192 45.6 -> 46.7, 8 heads, KeyFormer 192 42.1 -> 42.9.  Over 135 calls of 40 to 4000 tokens the
+// form taken is 0.3 % slower than the best on average, 0.8 without.)  Pairs of 128-key blocks as the only form -> this, whole
+// calls of 32 heads on 8: RoCo, 512 (one of 64, 256 workgroups) 71.9 -> 66.4, 700 (one of 128, 192) 93.9 -> 77.1, 1000
+// (two of 64, 256) 109.0 -> 98.5, 300 against 500 keys (one of 128, 224) 68.9 -> 62.7; KeyFormer 256 58.7 -> 54.5, 1000 121.2 ->
+// 106.5, 300 against 500 78.3 -> 70.7; 71 heads of 64, RoCo 100 against 100 keys 39.5 -> 35.5.  Beyond a round, one block of
+// 128: RoCo 1200 124.3 -> 117.4, 2048 189.2 -> 186.0, 3000 331.2 -> 321.8, 4096 433.3 -> 435.9, KeyFormer 1200 145.8 -> 136.4, 2048 224.2 ->
+// 222.1, 3000 416.8 -> 400.2; but pairs where a block meets few query tiles and there are many (one tile, 33 against 3000 keys,
+// 768 blocks, 42.4 -> 41.4, 64 against 4000, 1024, 50.6 -> 51.1, 40 against 16000, 4032, 98.8 -> 102.7; two, 100 against 6000, 1536, 71.3 ->
+// 70.5; three, 150 against 15000, 3808, 141.2 -> 142.9; five, 300 against 9000, 2336, 157.8 -> 152.9; seven, 71 heads, 400 against
+// 15000, 8520, 361.8 -> 363.5; eight, 512 against 16000, 4224, level).
 template <int D, int MODE>
 static int launch_score_d(const ScoreArgs& a, hipStream_t stream) {
   auto blocks = [&](int g) { const int keys = kKeysPerWg / g; return (a.P + a.S + keys - 1) / keys; };
   auto chain = [&](int g, int kb) {  // steps of key block kb
     const int q0 = a.causal ? kb * (kKeysPerWg / g) - a.P : 0;
     const int tiles = (a.S - (q0 > 0 ? q0 / kQTile * kQTile : 0) + kQTile - 1) / kQTile;
-    return kScoreBlockTiles + (tiles + g - 1) / g;
+    return kScoreBlockTiles + (tiles + g - 1) / g + (g - 1) * kScoreHandTiles;
   };
   const int n1 = blocks(1), n2 = blocks(2);
   const int64_t one = (int64_t)n1 * a.Hq, half = (int64_t)n2 * a.Hq;
