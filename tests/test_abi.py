@@ -52,6 +52,23 @@ def test_narrow_products_of_many_rows_run_in_parts(M, K, N):
     assert ext.gemm_workspace_bytes(M, K, N) % (M * N * 4) == 0
 
 
+class _RingPlan(ctypes.Structure):
+    _fields_ = [("tile", ctypes.c_int), ("parts", ctypes.c_int), ("us", ctypes.c_float)]
+
+
+@pytest.mark.parametrize("ncols,head", [(6144, 128), (6144, 1), (12288, 128), (4672, 64)])
+def test_projection_workspace_is_what_its_plan_uses(ncols, head):
+    """Scratch is asked for the parts that the projection then runs in, and for nothing else (the planner's own functions,
+    csrc/launch.h: no part of the C ABI)."""
+    room, plan = ext.lib()._ZN3tri19qkv_workspace_bytesEiiiib, ext.lib()._ZN3tri9ring_planEiiiiilf
+    room.restype, plan.restype = ctypes.c_int64, _RingPlan
+    K = 4544 if head == 64 else 4096
+    for S in (1, 16, 33, 100, 200, 333, *range(500, 1101, 12)):
+        ws = room(S, K, ncols, head, False)
+        parts = plan(S, K, ncols, head, 0, ctypes.c_int64(ws), ctypes.c_float(3.5)).parts
+        assert ws == (parts * S * ncols * 4 if parts > 1 else 0), "%d tokens: %d bytes for %d parts" % (S, ws, parts)
+
+
 def _h(*shape):
     return torch.zeros(*shape, dtype=torch.float16)
 

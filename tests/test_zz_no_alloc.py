@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from trinity_amd import ext
+from gpu_util import projection_parts
 from util import attn_inputs
 
 pytestmark = pytest.mark.gpu
@@ -141,7 +142,7 @@ def test_static_scratch_refuses_what_does_not_fit(dev):
 
 
 @pytest.mark.parametrize("S,Hq,Hkv,D,P,fp8", [
-    (700, 32, 8, 128, 4000, True),   # room for part of the projection's partial sums
+    (100, 32, 8, 128, 10400, True),  # room for fewer parts of the projection than it would run in
     (3, 32, 32, 128, 4000, True),    # ... and for the fewest runs of the key-split attention only
 ])
 def test_static_scratch_holds_calls_without_full_workspaces(dev, S, Hq, Hkv, D, P, fp8):
@@ -158,6 +159,10 @@ def test_static_scratch_holds_calls_without_full_workspaces(dev, S, Hq, Hkv, D, 
     p = ext.attn_params(Hq, Hkv, D, S, kv_prefix=P, causal=True, prenorm=S > 64, qknorm=S > 64, kv_fp8=fp8, k_scale=1.0,
                         v_scale=1.0)
     assert ext.qkv_scratch_bytes(p, N) > ext.STATIC_SCRATCH_BYTES
+    if S > 64:  # (the other row is short of room for attention's runs)
+        parts = projection_parts(N, S, Hq, Hkv, D, P, qknorm=True, kv_fp8=fp8, k_scale=1.0, v_scale=1.0)
+        missing = ext.qkv_scratch_bytes(p, N) - ext.STATIC_SCRATCH_BYTES
+        assert parts > 2 and missing < (parts - 1) * S * (Hq + 2 * Hkv) * D * 4
     want, got = (torch.zeros(S, Hq * D, dtype=torch.float16, device=dev) for _ in range(2))
     scratch = torch.empty(ext.qkv_scratch_bytes(p, N), dtype=torch.uint8, device=dev)
     ext.qkv_attention(x, None, wq, wk, wv, kc.clone(), vc.clone(), scratch, None, want, p)

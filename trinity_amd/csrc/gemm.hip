@@ -557,19 +557,8 @@ static int launch_qkv_d(const QkvProjArgs& a, hipStream_t stream) {
 // 0.3 faster to 0.7 slower for 16, 2.9 to 3.8 faster for 32.
 static float deferred_merge_us(int S) { return 1.2f + 0.12f * (float)S; }
 
-// Whole heads a tile (QKNorm), more than 512 tokens: room for the best plan in parts also where the best plan of all has
-// none but is ahead by no more than twice what the costs are off by (7 % rms), so that a buffer a caller lays out once does
-// not hinge on which of the two they put first (700 tokens, 6144 columns: 46.6 us in one part, 53.4 in two).
-constexpr float kQkvRoomMargin = 1.15f;
-constexpr int kQkvRoomMinRows = 512;
 int64_t qkv_workspace_bytes(int S, int K, int ncols, int unit, bool deferred) {
-  if (S > kRingMaxRows) return 0;
-  const float merge_us = deferred ? deferred_merge_us(S) : kRingMergeUs;
-  const int64_t best = plan_workspace_bytes(S, K, ncols, unit, 0, 2, merge_us);
-  if (best > 0 || unit == 1 || S <= kQkvRoomMinRows) return best;
-  const RingPlan any = ring_plan(S, K, ncols, unit, 0, INT64_MAX, merge_us);
-  const RingPlan parts = ring_plan(S, K, ncols, unit, 0, INT64_MAX, merge_us, 2);
-  return any.tile < 0 || parts.tile < 0 || parts.us > kQkvRoomMargin * any.us ? 0 : (int64_t)parts.ksplit * S * ncols * 4;
+  return S > kRingMaxRows ? 0 : plan_workspace_bytes(S, K, ncols, unit, 0, 2, deferred ? deferred_merge_us(S) : kRingMergeUs);
 }
 
 int launch_qkv_proj(const QkvProjArgs& a, hipStream_t stream, int* deferred_ksplit, bool* appended) {

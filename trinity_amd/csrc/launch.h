@@ -99,8 +99,7 @@ constexpr int kRingMaxRowsNarrow = 8192, kRingMaxColsNarrow = 1 << 16, kRingMinK
 // otherwise) and at least min_bn.  ws_bytes: fp32 workspace for partial results, ksplit * M * ncols * 4 bytes (1: none).
 // merge_us: what the merge of parts takes beside its bytes.
 constexpr float kRingMergeUs = 3.5f;
-// (least: the fewest parts)
-RingPlan ring_plan(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes, float merge_us = kRingMergeUs, int least = 1);
+RingPlan ring_plan(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes, float merge_us = kRingMergeUs);
 int launch_ring_gemm(const GemmArgs& a, const RingPlan& plan, hipStream_t stream);
 // few rows over K-contiguous weights in one part (strip.hip): what it should take (us; 1e30: not for it), and the launch
 float strip_us(const GemmArgs& a);

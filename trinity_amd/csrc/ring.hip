@@ -324,7 +324,7 @@ static const RingCost kRingCost[kRingTiles] = {
 constexpr float kRingStreamRate = 34e3f;
 constexpr int kRingStreamRows = 96, kRingStreamWorkgroups = 192;
 
-static RingPlan ring_plan_search(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes, float merge_us, int least) {
+static RingPlan ring_plan_search(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes, float merge_us) {
   RingPlan best = {-1, 1, 1e30f};
   const int KT = K / 64;
   const float wbytes = 2.0f * (float)K * (float)ncols, obytes = 4.0f * (float)M * (float)ncols;
@@ -342,7 +342,6 @@ static RingPlan ring_plan_search(int M, int K, int ncols, int unit, int min_bn, 
       const int ks = (KT + per - 1) / per;
       if (per == last_per || ks != s) continue;  // (no more parts than before)
       last_per = per;
-      if (ks < least) continue;
       const int wg = tiles * ks, share = (wg + 255) / 256;
       const float even = share == 1 ? 1.0f : sqrtf((float)wg / (256.0f * share));
       const float it = share == 1 ? alone : (alone > shared * share ? alone : shared * share);
@@ -368,17 +367,17 @@ static RingPlan ring_plan_search(int M, int K, int ncols, int unit, int min_bn, 
 
 // The search is a pure function of its arguments and takes 5 to 10 us, longer than a launch; each thread keeps the
 // answers it was last given.
-RingPlan ring_plan(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes, float merge_us, int least) {
+RingPlan ring_plan(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes, float merge_us) {
   if (M < 1 || K % 32 != 0 || K < 64 || ncols < 8) return RingPlan{-1, 1, 1e30f};
   if (M > kRingMaxRows && (M > kRingMaxRowsNarrow || ncols > kRingMaxColsNarrow || K < kRingMinKNarrow)) return RingPlan{-1, 1, 1e30f};
-  struct Entry { int M, K, ncols, unit, min_bn, least; int64_t ws_bytes; float merge_us; RingPlan plan; };
+  struct Entry { int M, K, ncols, unit, min_bn; int64_t ws_bytes; float merge_us; RingPlan plan; };
   static thread_local Entry memo[256] = {};
   uint64_t h = (uint64_t)M;
-  for (const uint64_t v : {(uint64_t)K, (uint64_t)ncols, (uint64_t)unit, (uint64_t)min_bn, (uint64_t)least, (uint64_t)ws_bytes, (uint64_t)(merge_us * 64.0f)}) h = (h ^ v) * 0x9E3779B97F4A7C15ull;
+  for (const uint64_t v : {(uint64_t)K, (uint64_t)ncols, (uint64_t)unit, (uint64_t)min_bn, (uint64_t)ws_bytes, (uint64_t)(merge_us * 64.0f)}) h = (h ^ v) * 0x9E3779B97F4A7C15ull;
   Entry& e = memo[h >> 56];
-  if (e.M != M || e.K != K || e.ncols != ncols || e.unit != unit || e.min_bn != min_bn || e.least != least || e.ws_bytes != ws_bytes ||
+  if (e.M != M || e.K != K || e.ncols != ncols || e.unit != unit || e.min_bn != min_bn || e.ws_bytes != ws_bytes ||
       e.merge_us != merge_us)
-    e = Entry{M, K, ncols, unit, min_bn, least, ws_bytes, merge_us, ring_plan_search(M, K, ncols, unit, min_bn, ws_bytes, merge_us, least)};
+    e = Entry{M, K, ncols, unit, min_bn, ws_bytes, merge_us, ring_plan_search(M, K, ncols, unit, min_bn, ws_bytes, merge_us)};
   return e.plan;
 }
 
