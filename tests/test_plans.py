@@ -1,0 +1,49 @@
+"""CPU: the plans that products are given (csrc/launch.h: gemm_plan, ring_plan) are among those measured fastest on the card.
+
+Each row lists the plans measured within 3 % of the fastest, as (rows, columns, parts) of a ring tile or LARGE for the
+large tiles; what such a product had been given before was 4 to 33 % behind."""
+import ctypes
+
+import pytest
+
+from trinity_amd import ext
+
+NONE, GELU, SWIGLU = 0, 1, 2
+LARGE = (256, 256, 1)
+# the ring kernels' tiles by number (csrc/ring.h: TRI_RING_TILES)
+TILES = [(32, 128), (64, 64), (64, 128), (96, 128), (128, 128), (128, 192), (128, 256), (160, 256), (192, 128), (192, 192),
+         (256, 128)]
+
+
+class Plan(ctypes.Structure):
+    _fields_ = [("tile", ctypes.c_int), ("parts", ctypes.c_int), ("us", ctypes.c_float)]
+
+
+def plan_of(M, K, N, epi=NONE, kcontig=False, workspace=1 << 62):
+    """(rows, columns, parts) of the tile that tri_matmul, tri_ffn_gelu or tri_gateup_swiglu run such a product on."""
+    plan = Plan()
+    takes = ext.lib()._ZN3tri9gemm_planEiiiiblRNS_8RingPlanE
+    takes.restype = ctypes.c_bool
+    if not takes(M, K, N, epi, ctypes.c_bool(kcontig), ctypes.c_int64(workspace), ctypes.byref(plan)):
+        return LARGE
+    return TILES[plan.tile] + (plan.parts,)
+
+
+@pytest.mark.parametrize("M,K,N,epi,fast", [
+    (96, 4096, 4096, NONE, [(64, 128, 4), (96, 128, 6)]),
+    (128, 4544, 4544, NONE, [(64, 128, 3)]),
+    (165, 4096, 4096, NONE, [(96, 128, 4)]),
+    (70, 4544, 18176, NONE, [(96, 128, 1), (128, 128, 1), (128, 256, 2)]),
+    (420, 4096, 4096, NONE, [(128, 128, 2)]),
+    (900, 4096, 14336, SWIGLU, [LARGE]),
+    (960, 4096, 14336, SWIGLU, [LARGE]),
+    (600, 4544, 18176, GELU, [(128, 192, 1)]),
+    (1200, 4544, 4544, NONE, [(192, 128, 1), (128, 192, 1)]),
+    (1300, 4096, 4096, NONE, [(192, 128, 1)]),
+    (1536, 8192, 4096, NONE, [(192, 128, 1)]),
+    (2500, 8192, 2048, NONE, [(192, 128, 1), (160, 256, 2), (128, 192, 1)]),
+    (8192, 4096, 1024, NONE, [LARGE]),
+    (8192, 14336, 1024, NONE, [LARGE]),
+])
+def test_plans_are_among_the_fastest_measured(M, K, N, epi, fast):
+    assert plan_of(M, K, N, epi) in fast

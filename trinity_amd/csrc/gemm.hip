@@ -394,14 +394,17 @@ static TilePlan best_plan(int M, int N, int& which) {
 // of 256 x 256 tiles (Llama-3-8B and Falcon-7B products, 256 to 1536 rows: within 12 %).
 static float plan_us(const TilePlan& p, int K) { return 6.0f + 0.0272f * (float)K * (float)p.cost; }
 
-// The ring kernels' plan for a product, if it beats a tile plan of big_us.  Beyond the rows that the costs were fitted
-// over, by three tenths: 14336 -> 1024, 2048 rows 162 -> 70 us (0.36 by the costs), 14336 -> 4096, 1200 rows 187 -> 142
-// (0.67), but 4096 rows of 4096 -> 1024 43.0 -> 45.8 (0.73), 3072 of 14336 -> 4096 310 -> 370 (0.79).
-constexpr float kRingMarginNarrow = 0.70f;
+// The ring kernels' plan for a product, if it beats a tile plan of big_us.  Beyond the rows that the costs were fitted over, by a
+// twentieth: over 195 products of 1101 to 6144 rows the choice is 1.0 % slower than the best plan on average, by a quarter 4.3 (2500
+// rows x [8192, 2048] 112 us on large tiles, 94 on the ring's, 1800 x [14336, 4096] 232 and 211).  Without a margin 0.8, but more products
+// slower than before by a few percent (13 in place of 10, 2635 x [14336, 4096] 316 -> 360).  Beyond 6144 rows by a quarter: over 15
+// products 2.4 %, 3.9 by a twentieth (8192 rows x [4096, 1024] 74.4 -> 88.3, x [14336, 1024] 239 -> 270).
+constexpr float kRingMarginNarrow = 0.95f, kRingMarginTall = 0.75f;
+constexpr int kRingTallRows = 6144;
 static bool ring_wins(float big_us, int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes, RingPlan& plan,
                       float merge_us = kRingMergeUs) {
   plan = ring_plan(M, K, ncols, unit, min_bn, ws_bytes, merge_us);
-  return plan.tile >= 0 && plan.us < (M <= kRingMaxRows ? big_us : kRingMarginNarrow * big_us);
+  return plan.tile >= 0 && plan.us < big_us * (M <= kRingMaxRows ? 1.0f : (M <= kRingTallRows ? kRingMarginNarrow : kRingMarginTall));
 }
 
 // plain and GELU epilogues on the direct-to-LDS path: pick the cheapest plan
@@ -481,13 +484,20 @@ static int launch_gemm_big(const GemmArgs& a, hipStream_t stream) {
   return -1;
 }
 
+// What the GELU adds to a plan of large tiles, 128 outputs a lane in one stretch (600 rows x [4544, 18176]: 118 us on 256 x 128 tiles
+// and on the ring's 128 x 192 without it, 148 and 126 with it).  The whole FFN, 1120 rows 405 -> 368 us, 1200 477 -> 431, 1800 666 -> 617.
+constexpr float kGeluBigCost = 1.2f;
+bool gemm_plan(int M, int K, int N, int epi, bool kcontig, int64_t ws_bytes, RingPlan& plan) {
+  const bool gated = epi == EPI_SWIGLU;
+  const float big_us = plan_us(big_plan(M, N, epi, kcontig), K) * (epi == EPI_GELU ? kGeluBigCost : 1.0f);
+  return ring_wins(big_us, M, K, gated ? 2 * N : N, 1, gated && !kcontig ? kGatedMinBn : 0, ws_bytes, plan);
+}
+
 int launch_gemm(const GemmArgs& a, hipStream_t stream) {
   if (a.M <= 0 || a.N <= 0) return 0;
   RingPlan plan;
-  const bool gated = a.epi == EPI_SWIGLU;
-  if (!(gated && a.M > kRingMaxRows) &&
-      (ring_wins(plan_us(big_plan(a.M, a.N, a.epi, a.w_kcontig != 0), a.K), a.M, a.K, gated ? 2 * a.N : a.N, 1,
-                 gated && !a.w_kcontig ? kGatedMinBn : 0, a.ws != nullptr ? a.ws_bytes : 0, plan) ||
+  if (!(a.epi == EPI_SWIGLU && a.M > kRingMaxRows) &&
+      (gemm_plan(a.M, a.K, a.N, a.epi, a.w_kcontig != 0, a.ws != nullptr ? a.ws_bytes : 0, plan) ||
        (plan.tile >= 0 && ring_gemm_in_place(a))))  // (the tile plans store while other tiles still read)
     return launch_ring_gemm(a, plan, stream);
   const int rc = launch_gemm_big(a, stream);
@@ -570,10 +580,8 @@ int launch_qkv_proj(const QkvProjArgs& a, hipStream_t stream, int* deferred_kspl
   int which;
   RingPlan plan;
   const TilePlan big = a.w_kcontig ? qkv_plan_kcontig(a.S, ncols) : qkv_plan(a.S, ncols, a.qknorm ? a.D : 0, which);
-  // (its weights are small enough to come from the Infinity Cache when the caller uses them again: the large tiles
-  // are then a tenth faster than over weights from HBM, the ring kernels hardly - 658 to 1000 rows, both within 2 %)
   if (a.S <= kRingMaxRows &&
-      ring_wins(0.9f * plan_us(big, a.K), a.S, a.K, ncols, a.qknorm ? a.D : 1, 0, a.ws != nullptr ? a.ws_bytes : 0, plan,
+      ring_wins(plan_us(big, a.K), a.S, a.K, ncols, a.qknorm ? a.D : 1, 0, a.ws != nullptr ? a.ws_bytes : 0, plan,
                 deferred_ksplit != nullptr ? deferred_merge_us(a.S) : kRingMergeUs))
     return launch_ring_qkv(a, plan, stream, deferred_ksplit, appended);
   return a.D == 128 ? launch_qkv_d<128>(a, stream) : launch_qkv_d<64>(a, stream);

@@ -101,6 +101,8 @@ constexpr int kRingMaxRowsNarrow = 8192, kRingMaxColsNarrow = 1 << 16, kRingMinK
 constexpr float kRingMergeUs = 3.5f;
 RingPlan ring_plan(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes, float merge_us = kRingMergeUs);
 int launch_ring_gemm(const GemmArgs& a, const RingPlan& plan, hipStream_t stream);
+// whether launch_gemm runs such a product by its ring plan (else by large tiles)
+bool gemm_plan(int M, int K, int N, int epi, bool kcontig, int64_t ws_bytes, RingPlan& plan);
 // few rows over K-contiguous weights in one part (strip.hip): what it should take (us; 1e30: not for it), and the launch
 float strip_us(const GemmArgs& a);
 int launch_strip(const GemmArgs& a, hipStream_t stream);

@@ -280,48 +280,55 @@ static int launch_epi(const GemmArgs& a, int tile, hipStream_t stream) {
   return -1;
 }
 
-// Cost of a plan in us.  Three times add up in part (as a 3/2-norm up to 32 rows, as a 4/3-norm above):
+// Cost of a plan in us.  Three times add up in part (as a 3/2-norm up to 32 rows, as a 2-norm above):
 //   memory    the weights once - less fast when the workgroups do not divide evenly over the CUs and some CUs have
 //             one more to stream - and what is written;
 //   compute   k tiles in a row on the busiest CU, by tile and by whether workgroups share a CU;
 //   loads     every byte that passes from L2 to LDS;
-// and per wave of workgroups 2 us of first loads and epilogue.  Parts cost a merge and their bytes.
+// and per wave of workgroups 2 us of first loads and epilogue.  Parts cost a merge and their bytes, and more (parts) per wave of
+// workgroups where the tile is large: its fp32 rows are stored by the waves that hold them alone.
 // Up to 32 rows: weights at 8 TB/s, loads at 37, fitted to 4100 timings on the card, 16 to 1024 rows, when the 32 x 128 tile had four
 // stages throughout; 4 % rms then, the plan it picks 1.3 % slower on average than the best plan of the family.  As that tile
 // runs now, ring_fourth_stage, the costs of plans on it are 7 % high, deviation 7, over 1170 row-major ones, 6 and 7 over
 // 980 K-contiguous ones, and 4 % low, deviation 9, over 190 with columns 8 or 16 KB apart.
-// Above: weights at 12 TB/s, loads at 62, fitted to 8800 timings of 600 products (33 to 1100 rows, K 1024 to 18176, 512 to 28672 columns,
-// plain and gated, both layouts, up to 16 parts; most out of HBM, 48 of Q/K/V projections out of the last-level cache): 7 % rms,
-// its choice, tile plans included, is 1.5 % slower than the best on average, at worst 19 % (800 rows x [4544, 4672], 52.8 / 44.4); over
-// the first 386 of them 1.3 %, where the constants of up to 32 rows throughout, without the tiles whose loads have waves of
-// their own, came to 2.9 %.
+// Above: the constants are those whose picks take least time, not those nearest to the times, and no rates of the chip - the
+// weights' 21 TB/s is what the other two times leave of them to be seen.  Chosen over 37700 timings of 1604 products (33 to 1100
+// rows, narrow outputs to 8192; K 1024 to 18176, 128 to 28672 columns, plain and gated, both layouts; among them the Q/K/V
+// projections and both FFN products inside whole calls).  The pick is 1.3 % slower on average than the best plan, the large
+// tiles' included, one in twenty by 7.5 % or more; constants nearest to the times, without the cost of parts by tile, had come to 2.7 %
+// and 14.5; over 220 products kept out of the choice 1.8 % for 2.7.  (us with these / with those: 128 rows x [4544, 4544] 23.4 ->
+// 21.2, 96 x [4096, 4096] 18.9 -> 17.5, 192 24.4 -> 21.9, 420 32.1 -> 30.7, 900 x [4096, 14336 x 2] 225 -> 211; the other way 230 x
+// [14336, 4096] 46.6 -> 49.0, 45 x [4544, 4544] 15.4 -> 16.2.)  Much of what is left is where the weights lie in memory: it moves
+// a product by a few percent from one allocation to the next, some with columns 8 KB apart by a fifth.
 struct RingCost {
   int bm, bn, per_cu;   // per_cu: workgroups that fit a CU's LDS
   float alone, shared;  // us per k tile of a workgroup with a CU to itself / of each of several
-  float few_alone, few_shared;  // the same in the fit for up to 32 rows (0: not for them)
+  float parts;          // us per wave of workgroups with parts
+  float few_alone, few_shared;  // alone and shared up to 32 rows (0: not for them)
 };
 #define TRI_RING_PER_CU(bm, bn, nst) ((160 * 1024) / (((bm) + (bn)) * 128 * (nst)))
 static const RingCost kRingCost[kRingTiles] = {
-    {32, 128, TRI_RING_PER_CU(32, 128, 3), 0.264f, 0.222f, 0.264f, 0.222f},
-    {64, 64, TRI_RING_PER_CU(64, 64, 5), 0.224f, 0.198f, 0.215f, 0.181f},
-    {64, 128, TRI_RING_PER_CU(64, 128, 3), 0.360f, 0.302f, 0.354f, 0.272f},
-    {96, 128, TRI_RING_PER_CU(96, 128, 5), 0.406f, 0.396f, 0.429f, 0.431f},
-    {128, 128, TRI_RING_PER_CU(128, 128, 5), 0.473f, 0.473f, 0.f, 0.f},
-    {128, 192, TRI_RING_PER_CU(128, 192, 3), 0.609f, 0.700f, 0.f, 0.f},
-    {128, 256, TRI_RING_PER_CU(128, 256, 3), 0.750f, 0.760f, 0.f, 0.f},
-    {160, 256, TRI_RING_PER_CU(160, 256, 3), 0.829f, 0.904f, 0.f, 0.f},
-    {192, 128, TRI_RING_PER_CU(192, 128, 3), 0.567f, 0.680f, 0.f, 0.f},
-    {192, 192, TRI_RING_PER_CU(192, 192, 3), 0.770f, 0.850f, 0.f, 0.f},
-    {256, 128, TRI_RING_PER_CU(256, 128, 3), 0.670f, 0.747f, 0.f, 0.f}};
+    {32, 128, TRI_RING_PER_CU(32, 128, 3), 0.f, 0.f, 0.f, 0.264f, 0.222f},
+    {64, 64, TRI_RING_PER_CU(64, 64, 5), 0.294f, 0.338f, -0.59f, 0.215f, 0.181f},
+    {64, 128, TRI_RING_PER_CU(64, 128, 3), 0.473f, 0.530f, -0.41f, 0.354f, 0.272f},
+    {96, 128, TRI_RING_PER_CU(96, 128, 5), 0.525f, 0.630f, 0.92f, 0.429f, 0.431f},
+    {128, 128, TRI_RING_PER_CU(128, 128, 5), 0.606f, 0.709f, 1.72f, 0.f, 0.f},
+    {128, 192, TRI_RING_PER_CU(128, 192, 3), 0.763f, 0.959f, 6.78f, 0.f, 0.f},
+    {128, 256, TRI_RING_PER_CU(128, 256, 3), 0.969f, 1.085f, 4.82f, 0.f, 0.f},
+    {160, 256, TRI_RING_PER_CU(160, 256, 3), 1.081f, 1.170f, 5.40f, 0.f, 0.f},
+    {192, 128, TRI_RING_PER_CU(192, 128, 3), 0.707f, 0.873f, 4.81f, 0.f, 0.f},
+    {192, 192, TRI_RING_PER_CU(192, 192, 3), 1.027f, 1.145f, 6.07f, 0.f, 0.f},
+    {256, 128, TRI_RING_PER_CU(256, 128, 3), 0.879f, 1.080f, 4.79f, 0.f, 0.f}};
 // A plan in one part on few workgroups: one streams no faster than about this many bytes of weights per us (16 rows x
 // [2048, 5632 x 2] as gate/up, 88 workgroups: 22.0 us, 16.0 in two parts; x [1024, 4096 x 2], 64: 12.0 and 10.1 in four; the
-// costs above, fitted where 200 and more workgroups share the memory's rate, say 14.9 and 7.8).  Up to 96 rows and 192
-// workgroups (75 rows x K-contiguous [4544, 18176], 142, 45.0 in three parts, 47.0 in one); beyond either the costs hold as they are (one row x K-contiguous [4096, 14336 x 2], 224 workgroups, would be
+// costs above, fitted where 200 and more workgroups share the memory's rate, say 14.9 and 7.8).  Up to 64 rows and 192
+// workgroups; beyond either the costs hold as they are (one row x K-contiguous [4096, 14336 x 2], 224 workgroups, would be
 // cut with the bound: the whole FFN 66.3 -> 72.4 us; 48 rows x [2048, 5632 x 2], 176, have to be cut: 22.2 -> 18.7).  What
 // the plan picked is slower than the best of the family on average, with this bound and without: gated products of 16 to
 // 100 rows, K of 512 to 8192, 2.1 % and 4.7; Q/K/V projections of 768- to 4544-wide models, up to 32 rows, 0.5 and 1.1;
 // plain products of such sizes 0.4 either way.
-constexpr float kRingStreamRate = 34e3f;
+// (Above 32 rows the bound holds up to 96 rows.)
+constexpr float kRingStreamRateFew = 34e3f, kRingStreamRate = 37.4e3f;
 constexpr int kRingStreamRows = 96, kRingStreamWorkgroups = 192;
 
 static RingPlan ring_plan_search(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes, float merge_us) {
@@ -346,7 +353,7 @@ static RingPlan ring_plan_search(int M, int K, int ncols, int unit, int min_bn, 
       const float even = share == 1 ? 1.0f : sqrtf((float)wg / (256.0f * share));
       const float it = share == 1 ? alone : (alone > shared * share ? alone : shared * share);
       float comp = per * it;
-      if (ks == 1 && wg <= kRingStreamWorkgroups && M <= kRingStreamRows) comp = fmaxf(comp, per * c.bn * 128.0f / kRingStreamRate);
+      if (ks == 1 && wg <= kRingStreamWorkgroups && M <= kRingStreamRows) comp = fmaxf(comp, per * c.bn * 128.0f / (few ? kRingStreamRateFew : kRingStreamRate));
       const float waves = (float)((share + c.per_cu - 1) / c.per_cu), loaded = (float)wg * per * (c.bm + c.bn) * 128.0f;
       const float written = ks > 1 ? ks * obytes : 0.5f * obytes;
       float us;
@@ -355,9 +362,9 @@ static RingPlan ring_plan_search(int M, int K, int ncols, int unit, int min_bn, 
         const float sum = cbrtf(mem * sqrtf(mem) + comp * sqrtf(comp) + loads * sqrtf(loads));
         us = 1.1f + 1.9f * waves + sum * sum + (ks > 1 ? merge_us + ks * obytes / 6e6f : 0.f);
       } else {
-        const float mem = wbytes / (12e6f * even) + written / 2.4e6f, loads = loaded / 62e6f;
-        const float sum = sqrtf(mem * cbrtf(mem) + comp * cbrtf(comp) + loads * cbrtf(loads));
-        us = 1.6f + 1.75f * waves + sum * sqrtf(sum) + (ks > 1 ? merge_us + 1.25f + ks * obytes / 10e6f : 0.f);
+        const float mem = wbytes / (21.3e6f * even) + written / 1.81e6f, loads = loaded / 50.4e6f;
+        us = 1.37f * waves + sqrtf(mem * mem + comp * comp + loads * loads) +
+             (ks > 1 ? merge_us + 1.79f + c.parts * waves + ks * obytes / 14.2e6f : 0.f);
       }
       if (us < best.us) { best.tile = tile; best.ksplit = ks; best.us = us; }
     }
