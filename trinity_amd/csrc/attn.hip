@@ -56,6 +56,7 @@ constexpr int kAttnStageRow = D + 8;  // halfs per row of an output tile staged 
 constexpr float kLazyMax = 8.0f;
 constexpr int kTwoWayMaxWorkgroups = 256, kTwoWayMinKeys = 640;  // when the eight-wave variant runs
 constexpr int kTwoWayRoundsPlain = 352, kTwoWayRoundsSeeded = 448;  // ... and how far beyond a round (launch_attention)
+constexpr int kTwoWayBlockShare = 16, kTwoWayLatePlain = 4, kTwoWayLateSeeded = 1;  // ... for so many query blocks a head
 constexpr int kEightGroupMinWorkgroups = 129, kEightGroupMaxWorkgroups = 256;  // (of 256 queries each)
 constexpr int kWideMinWorkgroups = 768;  // 64 queries per wave (head dimension 64) from this many workgroups on
 
@@ -1270,8 +1271,13 @@ int launch_attention(const AttnArgs& a, hipStream_t stream, int* merge_parts) {
   // 109.4, 1472 113.5 -> 113.3, 2048 142.9 -> 145.1, 2304 182 -> 189; seeded KeyFormer, 1408 161.6 -> 154.8, 1664 (416)
   // 180.5 -> 174.3, 2048 211.2 -> 210.2.  A cached prefix evens the blocks out: 1100 tokens behind 1100 keys level,
   // 1280 behind 3000 169.5 -> 176.4.  64-wide heads lose (71 heads, S = 768 57.8 -> 60.6).
+  // The workgroups beyond the round have to be few beside a head's query blocks: with short sequences and many heads the
+  // second round is as long as the first (plain, 32 heads x 9 blocks -1.9 %, 48 x 6 +0.6, 36 x 9 -0.9, 52 x 6 +2.4, 32 x 11 -0.8, 44 x 8
+  // +1.5; seeded, 28 x 12 -4.4, 56 x 6 +0.8, 32 x 13 -2.0, 52 x 8 +1.8, 36 x 12 level; 12 to 20 heads as long ones).
+  const int blocks = (a.S + 127) / 128, late = kf == 2 ? kTwoWayLateSeeded : kTwoWayLatePlain;
   const int rounds = kf == 2 ? kTwoWayRoundsSeeded : kTwoWayRoundsPlain;
-  const bool turns = a.D == 128 && a.causal && kf != 1 && 2 * a.P <= a.S && wgs <= rounds;
+  const bool turns = a.D == 128 && a.causal && kf != 1 && 2 * a.P <= a.S && wgs <= rounds &&
+                     wgs - kTwoWayMaxWorkgroups <= kTwoWayBlockShare * (blocks - late);
   const bool two = (wgs <= kTwoWayMaxWorkgroups || turns) && a.P + a.S >= kTwoWayMinKeys;
   // One round of four-wave workgroups under a causal mask: eight query groups per workgroup instead (128-wide
   // heads; with 64-wide heads it is level at best: 71 heads S = 768 17.2 -> 17.7 us, 32 heads S = 2048 36.3 -> 35.5)
