@@ -19,9 +19,9 @@ def rn():
     return lambda *s, std=1.0: torch.empty(*s, dtype=torch.float16, device="cuda:0").normal_(0.0, std, generator=g)
 
 
-def check(got, want, what):
+def check(got, want, what, rel=REL):
     torch.cuda.synchronize()
-    bad = (got.float() - want).abs() > REL * want.abs() + ABS
+    bad = (got.float() - want).abs() > rel * want.abs() + ABS
     assert torch.isfinite(got).all() and not bad.any(), "%s: %d of %d, first at %s" % (
         what, int(bad.sum()), bad.numel(), bad.nonzero()[:1].tolist())
 
@@ -46,16 +46,23 @@ def test_plain_and_residual(rn, M, K, N, kcontig, with_ws):
     check(out, x.float() @ w.float() + r.float(), "x.w + r")
 
 
-# Tiles whose loads have waves of their own - 128 x 192, 192 x 128, 192 x 192, 256 x 128 - in one part and in parts: a last row
-# block of one row and full ones, ragged columns, K = 16.5 and 64.5 k tiles (the last one begins half way back), one k tile
-# and two (fewer than the three stages that are requested ahead)
-@pytest.mark.parametrize("M,K,N", [
-    (193, 4128, 6144), (1000, 1056, 6144), (1000, 64, 6144), (150, 4128, 6136), (385, 1056, 9000), (384, 96, 9000),
-    (385, 4544, 4544), (700, 1056, 9000), (768, 64, 9000), (333, 18176, 4544), (576, 1056, 11264), (560, 128, 12000),
-])
+# Tiles whose loads have waves of their own, in one part and in parts (tests/test_plans.py holds the rows against the plans): one k
+# tile and two (fewer than the three stages that are requested ahead), K = 16.5, 64.5 and 109.5 k tiles (the last one
+# begins half way back), a last row block of one row and full ones, ragged columns
+LOADING_WAVES = [  # M, K, N, (rows, columns, parts)
+    (193, 64, 16424, (128, 192, 1)), (385, 96, 11264, (128, 192, 1)), (385, 1056, 11264, (128, 192, 1)),
+    (131, 64, 16424, (192, 128, 1)), (192, 128, 16584, (192, 128, 1)), (385, 1056, 9000, (192, 128, 1)),
+    (257, 128, 24000, (192, 192, 1)), (513, 1056, 14000, (192, 192, 1)), (257, 4128, 24000, (192, 192, 1)),
+    (385, 128, 14000, (256, 128, 1)), (512, 1056, 14000, (256, 128, 1)), (700, 1056, 9000, (256, 128, 1)),
+    (500, 7008, 6144, (128, 192, 2)), (333, 8192, 4544, (192, 128, 3)), (129, 14336, 3000, (192, 128, 10)),
+    (333, 18176, 4544, (192, 192, 5)), (500, 7008, 4544, (256, 128, 3)),
+]
+
+
+@pytest.mark.parametrize("M,K,N,plan", LOADING_WAVES)
 @pytest.mark.parametrize("kcontig", [False, True])
 @pytest.mark.parametrize("bf16", [False, True])
-def test_loading_waves(rn, M, K, N, kcontig, bf16):
+def test_loading_waves(rn, M, K, N, plan, kcontig, bf16):
     dt, tol = (torch.bfloat16, 2.0 ** -6) if bf16 else (torch.float16, REL)  # (bf16: two ulps of 2^-8)
     x = rn(M, K).to(dt)
     w = (rn(N, K, std=K ** -0.5).to(dt).t() if kcontig else rn(K, N, std=K ** -0.5).to(dt))
@@ -63,15 +70,21 @@ def test_loading_waves(rn, M, K, N, kcontig, bf16):
     for ws in (None, torch.empty(ext.gemm_workspace_bytes(M, K, N), dtype=torch.uint8, device="cuda:0")):
         out = torch.full((M, N), float("nan"), dtype=dt, device="cuda:0")
         ext.matmul(x, w, None, out, workspace=ws)
-        torch.cuda.synchronize()
-        assert not ((out.float() - want).abs() > tol * want.abs() + 1e-4).any()
+        check(out, want, "x.w", tol)
+
+
+LOADING_WAVES_GATED = [
+    (385, 96, 5632, (128, 192, 1)), (193, 4128, 8200, (128, 192, 1)), (131, 64, 8200, (192, 128, 1)),
+    (150, 1056, 14336, (192, 128, 1)), (257, 128, 11264, (192, 192, 1)), (300, 1056, 11264, (192, 192, 1)),
+    (193, 192, 14336, (256, 128, 1)), (700, 1056, 4544, (256, 128, 1)),
+]
 
 
 @pytest.mark.parametrize("M,K,F", [
     (1, 4096, 14336), (16, 96, 72), (48, 4096, 14336), (90, 4096, 14336), (130, 4096, 14336), (300, 4096, 14336),
     (100, 4544, 4544), (256, 4544, 4544), (500, 1024, 4000),
-    (150, 1056, 14336), (190, 4128, 3000), (1000, 96, 3064), (576, 1056, 5632),  # tiles whose loads have waves of their own
-])
+    (190, 4128, 3000), (1000, 96, 3064), (576, 1056, 5632),
+] + [row[:3] for row in LOADING_WAVES_GATED])
 @pytest.mark.parametrize("kcontig", [False, True])
 def test_gated_with_row_scale(rn, M, K, F, kcontig):
     x, rs = rn(M, K), torch.rand(M, device="cuda:0") + 0.5
@@ -112,11 +125,21 @@ def test_one_row_of_any_stride_in_place(rn, stride):
     check(t, want, "in place")
 
 
+LOADING_WAVES_QKV = [  # S, N, Hq, Hkv, D, (without, with QKNorm)
+    (577, 1056, 48, 48, 64, [(128, 192, 1)] * 2), (769, 64, 71, 1, 64, [(192, 128, 1)] * 2),
+    (1000, 1056, 71, 1, 64, [(192, 128, 1)] * 2), (900, 1056, 48, 48, 64, [(192, 192, 1)] * 2),
+    (700, 1056, 48, 48, 64, [(256, 128, 1)] * 2), (129, 4128, 48, 48, 64, [(192, 128, 3)] * 2),
+    (385, 96, 32, 32, 128, [(128, 192, 1), (256, 128, 1)]), (1000, 1056, 32, 8, 128, [(128, 192, 1), (256, 128, 1)]),
+    (650, 64, 32, 8, 128, [(192, 128, 1)] * 2), (333, 1056, 64, 64, 128, [(192, 192, 1), (192, 128, 1)]),
+    (577, 1056, 64, 8, 128, [(256, 128, 1)] * 2),
+]
+
+
 @pytest.mark.parametrize("S,N,Hq,Hkv,D", [
     (1, 64, 4, 4, 64), (33, 96, 5, 1, 128), (100, 4096, 32, 8, 128), (260, 4096, 32, 8, 128), (200, 4544, 71, 1, 64),
     (700, 128, 32, 8, 128), (1000, 128, 71, 1, 64), (1100, 160, 32, 4, 128),  # a tile across two weight matrices
-    (150, 4128, 32, 8, 128), (1000, 1056, 71, 1, 64), (1000, 1056, 32, 8, 128),  # loads in waves of their own
-])
+    (150, 4128, 32, 8, 128),
+] + [row[:5] for row in LOADING_WAVES_QKV])
 @pytest.mark.parametrize("qknorm", [False, True])
 @pytest.mark.parametrize("kcontig", [False, True])
 def test_qkv_projection(rn, S, N, Hq, Hkv, D, qknorm, kcontig):

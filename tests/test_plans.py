@@ -1,11 +1,10 @@
-"""CPU: the plans that products are given (csrc/launch.h: gemm_plan, ring_plan) are among those measured fastest on the card.
-
-Each row lists the plans measured within 3 % of the fastest, as (rows, columns, parts) of a ring tile or LARGE for the
-large tiles; what such a product had been given before was 4 to 33 % behind."""
+"""CPU: what the launchers choose (csrc/launch.h: gemm_plan and the others; no part of the C ABI) - that the plans products are
+given are among those measured fastest on the card, and that the GPU tests of a form of a kernel are given that form."""
 import ctypes
 
 import pytest
 
+import test_gpu_ring
 from trinity_amd import ext
 
 NONE, GELU, SWIGLU = 0, 1, 2
@@ -46,4 +45,37 @@ def plan_of(M, K, N, epi=NONE, kcontig=False, workspace=1 << 62):
     (8192, 14336, 1024, NONE, [LARGE]),
 ])
 def test_plans_are_among_the_fastest_measured(M, K, N, epi, fast):
+    """Plans measured within 3 % of the fastest, as (rows, columns, parts) of a ring tile or LARGE for the large tiles; what
+    such a product had been given before was 4 to 33 % behind."""
     assert plan_of(M, K, N, epi) in fast
+
+
+@pytest.mark.parametrize("row", test_gpu_ring.LOADING_WAVES)
+def test_loading_waves_are_given(row):
+    M, K, N, plan = row
+    room = ext.gemm_workspace_bytes(M, K, N)
+    for kcontig in (False, True):
+        for ws in (0, room) if plan[2] == 1 else (room,):
+            assert plan_of(M, K, N, kcontig=kcontig, workspace=ws) == plan
+
+
+@pytest.mark.parametrize("row", test_gpu_ring.LOADING_WAVES_GATED)
+def test_loading_waves_of_gated_products_are_given(row):
+    M, K, F, plan = row
+    for kcontig in (False, True):
+        for ws in (0, ext.gemm_workspace_bytes(M, K, 2 * F)):
+            assert plan_of(M, K, F, SWIGLU, kcontig, ws) == plan
+
+
+@pytest.mark.parametrize("row", test_gpu_ring.LOADING_WAVES_QKV)
+def test_loading_waves_of_projections_are_given(row):
+    S, N, Hq, Hkv, D, tiles = row
+    takes = ext.lib()._ZN3tri13qkv_ring_planEiiiiblbRNS_8RingPlanE
+    takes.restype = ctypes.c_bool
+    for qknorm, tile in zip((False, True), tiles):
+        for kcontig in (False, True):
+            p = ext.attn_params(Hq, Hkv, D, S, kv_prefix=5, qknorm=qknorm, rms_eps=1e-5)
+            plan = Plan()
+            assert takes(S, N, (Hq + 2 * Hkv) * D, D if qknorm else 0, ctypes.c_bool(kcontig),
+                         ctypes.c_int64(ext.qkv_scratch_bytes(p, N)), ctypes.c_bool(False), ctypes.byref(plan))
+            assert TILES[plan.tile] + (plan.parts,) == tile

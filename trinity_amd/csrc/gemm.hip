@@ -571,18 +571,22 @@ int64_t qkv_workspace_bytes(int S, int K, int ncols, int unit, bool deferred) {
   return S > kRingMaxRows ? 0 : plan_workspace_bytes(S, K, ncols, unit, 0, 2, deferred ? deferred_merge_us(S) : kRingMergeUs);
 }
 
+bool qkv_ring_plan(int S, int K, int ncols, int head, bool kcontig, int64_t ws_bytes, bool deferred, RingPlan& plan) {
+  int which;
+  const TilePlan big = kcontig ? qkv_plan_kcontig(S, ncols) : qkv_plan(S, ncols, head, which);
+  return S <= kRingMaxRows && ring_wins(plan_us(big, K), S, K, ncols, head > 0 ? head : 1, 0, ws_bytes, plan,
+                                        deferred ? deferred_merge_us(S) : kRingMergeUs);
+}
+
 int launch_qkv_proj(const QkvProjArgs& a, hipStream_t stream, int* deferred_ksplit, bool* appended) {
   if (deferred_ksplit != nullptr) *deferred_ksplit = 0;
   if (appended != nullptr) *appended = false;
   if (a.S <= 0) return 0;
   if (a.D != 64 && a.D != 128) return -1;
   const int ncols = (a.Hq + 2 * a.Hkv) * a.D;
-  int which;
   RingPlan plan;
-  const TilePlan big = a.w_kcontig ? qkv_plan_kcontig(a.S, ncols) : qkv_plan(a.S, ncols, a.qknorm ? a.D : 0, which);
-  if (a.S <= kRingMaxRows &&
-      ring_wins(plan_us(big, a.K), a.S, a.K, ncols, a.qknorm ? a.D : 1, 0, a.ws != nullptr ? a.ws_bytes : 0, plan,
-                deferred_ksplit != nullptr ? deferred_merge_us(a.S) : kRingMergeUs))
+  if (qkv_ring_plan(a.S, a.K, ncols, a.qknorm ? a.D : 0, a.w_kcontig != 0, a.ws != nullptr ? a.ws_bytes : 0,
+                    deferred_ksplit != nullptr, plan))
     return launch_ring_qkv(a, plan, stream, deferred_ksplit, appended);
   return a.D == 128 ? launch_qkv_d<128>(a, stream) : launch_qkv_d<64>(a, stream);
 }

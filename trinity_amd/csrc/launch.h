@@ -103,6 +103,8 @@ RingPlan ring_plan(int M, int K, int ncols, int unit, int min_bn, int64_t ws_byt
 int launch_ring_gemm(const GemmArgs& a, const RingPlan& plan, hipStream_t stream);
 // whether launch_gemm runs such a product by its ring plan (else by large tiles)
 bool gemm_plan(int M, int K, int N, int epi, bool kcontig, int64_t ws_bytes, RingPlan& plan);
+// ... and launch_qkv_proj a projection (head: QKNorm, tiles of whole heads of that width; 0: any)
+bool qkv_ring_plan(int S, int K, int ncols, int head, bool kcontig, int64_t ws_bytes, bool deferred, RingPlan& plan);
 // few rows over K-contiguous weights in one part (strip.hip): what it should take (us; 1e30: not for it), and the launch
 float strip_us(const GemmArgs& a);
 int launch_strip(const GemmArgs& a, hipStream_t stream);
