@@ -249,23 +249,31 @@ def test_keyformer_parity(dev, S, N, Hq, Hkv, D, P, causal, mode):
     assert torch.allclose(got["score"].sum(-1), torch.full((Hq,), float(S)), rtol=1e-3)
 
 
-# the score kernel's workgroups: one block of 64 keys each (64-key blocks x heads up to 256), two of them (up to twice
-# that, an odd number among them), one block of 128 keys beyond, pairs of these for a single query tile; odd numbers of
-# query tiles, ragged ends, a prefix
+# the score kernel's workgroups (tests/test_plans.py holds the rows against the launcher): one block of 64 keys, two of them,
+# one block of 128 keys within a round and beyond it, pairs of these; odd numbers of blocks, whose middle one has no partner,
+# and of query tiles, ragged ends, a prefix, head counts that are no multiple of eight
 SCORE_CASES = [
-    (500, 128, 32, 8, 128, 0, True),     # 8 blocks x 32 heads: 256
-    (513, 128, 32, 8, 128, 0, True),     # 9 blocks, the middle one alone
-    (65, 128, 32, 8, 64, 900, True),     # 16 blocks in pairs, two query tiles, the second with one row
-    (200, 128, 32, 8, 128, 833, False),  # 17 blocks: 288 pairs of 64 keys are too many
-    (129, 128, 40, 8, 64, 700, True),
-    (130, 128, 43, 1, 64, 700, True),    # heads no multiple of eight: 7 x 43
-    (40, 128, 64, 8, 128, 1570, True),   # 13 blocks x 64 heads, one query tile: pairs, the middle block alone
+    (500, 128, 32, 8, 128, 0, True, "half block"),
+    (300, 128, 43, 1, 64, 0, True, "half block"),
+    (500, 64, 17, 1, 128, 20, True, "half block"),         # nine blocks, a ragged last one
+    (1000, 64, 32, 8, 128, 0, True, "half block pair"),    # 16 blocks
+    (1060, 64, 24, 8, 128, 0, True, "half block pair"),    # 17, the middle one alone
+    (1060, 64, 28, 4, 64, 0, True, "half block pair"),     # ... plain order of the heads, 64-wide
+    (1000, 64, 32, 8, 64, 0, True, "half block pair"),
+    (513, 128, 32, 8, 128, 0, True, "block"),
+    (65, 128, 32, 8, 64, 900, True, "block"),              # two query tiles, the second with one row
+    (200, 128, 32, 8, 128, 833, False, "block"),
+    (130, 128, 43, 1, 64, 700, True, "block"),
+    (1030, 64, 32, 8, 64, 0, True, "block"),               # 288 workgroups
+    (700, 64, 43, 1, 128, 0, True, "block"),               # 258, heads by their blocks' length
+    (40, 128, 64, 8, 128, 1570, True, "block pair"),       # 13 blocks, the middle one alone
+    (40, 64, 71, 1, 64, 1500, True, "block pair"),         # 13, plain order of the heads
 ]
 
 
-@pytest.mark.parametrize("S,N,Hq,Hkv,D,P,causal", SCORE_CASES)
+@pytest.mark.parametrize("S,N,Hq,Hkv,D,P,causal,form", SCORE_CASES)
 @pytest.mark.parametrize("variant", ["roco", "seeded", "tensor"])
-def test_score_workgroups(dev, S, N, Hq, Hkv, D, P, causal, variant):
+def test_score_workgroups(dev, S, N, Hq, Hkv, D, P, causal, form, variant):
     t = attn_inputs(S, N, Hq, Hkv, D, P=P, w_std=0.06)
     scale = 1.0 / math.sqrt(D)
     kw = dict(n_q_heads=Hq, n_kv_heads=Hkv, head_dim=D, scale=scale, causal=causal, kv_prefix=P,

@@ -4,6 +4,7 @@ import ctypes
 
 import pytest
 
+import test_gpu_attention
 import test_gpu_ring
 from trinity_amd import ext
 
@@ -79,3 +80,10 @@ def test_loading_waves_of_projections_are_given(row):
             assert takes(S, N, (Hq + 2 * Hkv) * D, D if qknorm else 0, ctypes.c_bool(kcontig),
                          ctypes.c_int64(ext.qkv_scratch_bytes(p, N)), ctypes.c_bool(False), ctypes.byref(plan))
             assert TILES[plan.tile] + (plan.parts,) == tile
+
+
+@pytest.mark.parametrize("row", test_gpu_attention.SCORE_CASES)
+def test_score_cases_are_given_their_form(row):
+    S, _, Hq, _, _, P, causal, form = row
+    got = ext.lib()._ZN3tri10score_formEiiib(S, P, Hq, ctypes.c_bool(causal))
+    assert ["block", "block pair", "half block", "half block pair"][got] == form

@@ -244,6 +244,9 @@ struct ScoreArgs {
   float out_scale;
 };
 int launch_scores(const ScoreArgs& a, hipStream_t stream);
+// what a workgroup of launch_scores takes (more than kFewMaxQueries tokens): a block of 128 keys, two of them, a block of 64 keys, two
+enum ScoreForm { kScoreBlock, kScoreBlockPair, kScoreHalfBlock, kScoreHalfBlockPair };
+int score_form(int S, int P, int Hq, bool causal);
 int launch_scores_few(const ScoreArgs& a, hipStream_t stream);  // S <= kFewMaxQueries; 1 = not applicable
 
 }  // namespace tri

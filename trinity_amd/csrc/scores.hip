@@ -12,7 +12,7 @@
 // Under the causal mask key block b only meets queries >= its first key, so
 // the work per block falls linearly with b: the longest blocks are dispatched
 // first.  (Pairs of blocks b and n - 1 - b, all equally long, remain where a
-// workgroup would have too little to do, see launch_score_d.)
+// workgroup would have too little to do, see score_form.)
 //
 // Where such workgroups leave CUs empty (up to 1024 keys x 32 heads) the kernel's time is one workgroup's chain of
 // tiles: there a workgroup owns 64 keys, its waves are two groups of keys times two query groups that take the tiles of
@@ -30,7 +30,7 @@ constexpr int kKeysPerWg = 128;  // (half of them with two query groups)
 constexpr int kScoreStages = 4;         // steps (a Q tile per query group) in LDS
 constexpr int kScoreMergeFloats = 64;   // sums a wave of the second query group hands over
 constexpr int kScoreRound = 256;        // workgroups that have a CU each
-constexpr int kScoreBlockTiles = 4, kScoreHandTiles = 1, kScorePairWorkgroups = 768;  // (launch_score_d; the last per query tile)
+constexpr int kScoreBlockTiles = 4, kScoreHandTiles = 1, kScorePairWorkgroups = 768;  // (score_form; the last per query tile)
 
 // s_waitcnt vmcnt(n) leaving the other counters unconstrained (gfx9 encoding)
 #define TRI_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | 0x0F70)
@@ -377,22 +377,29 @@ static int launch_score_t(const ScoreArgs& a, hipStream_t stream) {
 // 768 blocks, 42.4 -> 41.4, 64 against 4000, 1024, 50.6 -> 51.1, 40 against 16000, 4032, 98.8 -> 102.7; two, 100 against 6000, 1536, 71.3 ->
 // 70.5; three, 150 against 15000, 3808, 141.2 -> 142.9; five, 300 against 9000, 2336, 157.8 -> 152.9; seven, 71 heads, 400 against
 // 15000, 8520, 361.8 -> 363.5; eight, 512 against 16000, 4224, level).
-template <int D, int MODE>
-static int launch_score_d(const ScoreArgs& a, hipStream_t stream) {
-  auto blocks = [&](int g) { const int keys = kKeysPerWg / g; return (a.P + a.S + keys - 1) / keys; };
+int score_form(int S, int P, int Hq, bool causal) {
+  auto blocks = [&](int g) { const int keys = kKeysPerWg / g; return (P + S + keys - 1) / keys; };
   auto chain = [&](int g, int kb) {  // steps of key block kb
-    const int q0 = a.causal ? kb * (kKeysPerWg / g) - a.P : 0;
-    const int tiles = (a.S - (q0 > 0 ? q0 / kQTile * kQTile : 0) + kQTile - 1) / kQTile;
+    const int q0 = causal ? kb * (kKeysPerWg / g) - P : 0;
+    const int tiles = (S - (q0 > 0 ? q0 / kQTile * kQTile : 0) + kQTile - 1) / kQTile;
     return kScoreBlockTiles + (tiles + g - 1) / g + (g - 1) * kScoreHandTiles;
   };
   const int n1 = blocks(1), n2 = blocks(2);
-  const int64_t one = (int64_t)n1 * a.Hq, half = (int64_t)n2 * a.Hq;
+  const int64_t one = (int64_t)n1 * Hq, half = (int64_t)n2 * Hq;
   const int whole = one <= kScoreRound ? chain(1, 0) : 1 << 30;
-  if (half <= kScoreRound && chain(2, 0) < whole) return launch_score_t<D, MODE, 2, true>(a, stream);
-  if (n2 > 1 && (int64_t)(n2 + 1) / 2 * a.Hq <= kScoreRound && chain(2, 0) + chain(2, n2 - 1) < whole)
-    return launch_score_t<D, MODE, 2, false>(a, stream);
-  return one <= (int64_t)kScorePairWorkgroups * ((a.S + kQTile - 1) / kQTile) ? launch_score_t<D, MODE, 1, true>(a, stream)
-                                                                           : launch_score_t<D, MODE, 1, false>(a, stream);
+  if (half <= kScoreRound && chain(2, 0) < whole) return kScoreHalfBlock;
+  if (n2 > 1 && (int64_t)(n2 + 1) / 2 * Hq <= kScoreRound && chain(2, 0) + chain(2, n2 - 1) < whole) return kScoreHalfBlockPair;
+  return one <= (int64_t)kScorePairWorkgroups * ((S + kQTile - 1) / kQTile) ? kScoreBlock : kScoreBlockPair;
+}
+
+template <int D, int MODE>
+static int launch_score_d(const ScoreArgs& a, hipStream_t stream) {
+  switch (score_form(a.S, a.P, a.Hq, a.causal != 0)) {
+    case kScoreHalfBlock: return launch_score_t<D, MODE, 2, true>(a, stream);
+    case kScoreHalfBlockPair: return launch_score_t<D, MODE, 2, false>(a, stream);
+    case kScoreBlock: return launch_score_t<D, MODE, 1, true>(a, stream);
+    default: return launch_score_t<D, MODE, 1, false>(a, stream);
+  }
 }
 
 int launch_scores(const ScoreArgs& a, hipStream_t stream) {
