@@ -77,10 +77,13 @@ CASES = [
     (16, 128, 4, 2, 128, 4200, True),    # long prefix: the looping key-split kernel converts the fp8 tiles itself
     (20, 128, 6, 1, 64, 3001, False),    # ... 120 stacked rows, ragged last tile
     (33, 128, 4, 4, 128, 2100, True),    # ... chunks: 33 rows of a head, two waves a tile
-    (40, 128, 4, 2, 128, 9000, True),    # ... 80 rows, long runs: pairs of tiles
+    (40, 128, 4, 2, 128, 9000, True),    # ... 80 rows, four waves on single tiles: 36 runs of up to four
     (200, 128, 2, 1, 64, 3001, True),    # ... four row blocks, the last one ragged
     (130, 128, 4, 1, 128, 2500, False),
     (33, 128, 2, 1, 64, 2014, True),     # ... one key short of the key-split kernel: through the 16-bit copy
+    (64, 64, 32, 8, 128, 7209, True),    # ... chunks in long runs: eight waves on pairs of tiles, two row blocks
+    (100, 64, 32, 8, 128, 3650, False),  # ... four row blocks, the last of 16 rows, a ragged last tile
+    (100, 64, 32, 8, 64, 3650, True),
 ]
 # models so wide that the projection runs in parts: their merge converts and appends the new rows
 PARTS = [

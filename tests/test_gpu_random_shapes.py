@@ -131,19 +131,35 @@ def test_prefill_workgroup_maps(dev, cfg):
     (1152, 128, 6, 3, 64, 0, False),     # no mask: nothing to fold, the blocks stay contiguous
     (650, 96, 8, 2, 64, 0, True),        # just past the key count from which eight waves run: 11 half blocks
     (768, 128, 4, 4, 128, 0, True),      # twelve half blocks, six steps
-    (1300, 128, 32, 8, 128, 0, True),    # eight query groups: 21 half blocks, the last workgroup holds one
-    (1100, 128, 32, 4, 128, 0, True),    # ... 18 half blocks (the last workgroup holds two)
-    (1216, 128, 24, 8, 128, 0, True),    # ... 19 half blocks (three)
-    (1200, 128, 32, 8, 128, 300, True),  # ... behind a cached prefix
-    (2048, 64, 32, 8, 128, 0, True),     # ... a full round of 256 workgroups (the upper end of the range)
+    (1300, 128, 32, 8, 128, 0, True),    # beyond a round: two key ways on whole blocks, 352 workgroups, a ragged last block
+    (1100, 128, 32, 4, 128, 0, True),    # ... 288 workgroups
+    (1216, 128, 24, 8, 128, 0, True),    # 240 workgroups: 19 half blocks by two key ways
+    (1200, 128, 32, 8, 128, 300, True),  # beyond a round behind a cached prefix
+    (2048, 64, 32, 8, 128, 0, True),     # eight query groups, a full round of 256 workgroups (the upper end of the range)
     (2048, 64, 32, 32, 64, 0, True),     # 64-wide heads keep the four-wave kernel at this size
 ])
 def test_prefill_folded_half_blocks(dev, cfg):
     """The eight-wave prefill kernels.  At most 256 workgroups and 640 keys or more: two key ways, and under a causal
-    mask a late and an early half block of 64 queries per workgroup instead of 128 consecutive queries.  Between
-    129 and 256 workgroups of 256 queries under a causal mask: eight query groups - two late and two early half
-    blocks - per workgroup."""
+    mask a late and an early half block of 64 queries per workgroup instead of 128 consecutive queries; somewhat
+    beyond, 128-wide heads, whole blocks.  Between 129 and 256 workgroups of 256 queries under a causal mask: eight
+    query groups - two late and two early half blocks - per workgroup."""
     _check_all_variants(dev, 500 + cfg[0], cfg)
+
+
+# calls beyond a round of 128-query workgroups that stay on eight query groups, plain and with seeded noise, by what the last
+# workgroup is left with (tests/test_plans.py holds them against the launcher): one, two and three half blocks
+EIGHT_GROUP_CASES = [
+    (830, 64, 56, 8, 128, 0, True),      # 13 half blocks, the last one ragged
+    (870, 64, 56, 8, 128, 0, True),      # 14
+    (1300, 64, 32, 8, 128, 700, True),   # 21, behind more than half as many cached keys
+    (1100, 64, 32, 4, 128, 600, True),   # 18
+    (700, 64, 44, 4, 128, 360, True),    # 11
+]
+
+
+@pytest.mark.parametrize("cfg", EIGHT_GROUP_CASES)
+def test_prefill_eight_query_groups(dev, cfg):
+    _check_all_variants(dev, 700 + cfg[0], cfg)
 
 
 @pytest.mark.parametrize("cfg", [

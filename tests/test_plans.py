@@ -5,9 +5,12 @@ import ctypes
 import pytest
 
 import test_gpu_attention
+import test_gpu_fp8_kv
+import test_gpu_random_shapes
 import test_gpu_ring
 from trinity_amd import ext
 
+EIGHT_GROUPS = 3  # (csrc/launch.h: PrefillForm)
 NONE, GELU, SWIGLU = 0, 1, 2
 LARGE = (256, 256, 1)
 # the ring kernels' tiles by number (csrc/ring.h: TRI_RING_TILES)
@@ -87,3 +90,17 @@ def test_score_cases_are_given_their_form(row):
     S, _, Hq, _, _, P, causal, form = row
     got = ext.lib()._ZN3tri10score_formEiiib(S, P, Hq, ctypes.c_bool(causal))
     assert ["block", "block pair", "half block", "half block pair"][got] == form
+
+
+@pytest.mark.parametrize("cfg", test_gpu_random_shapes.EIGHT_GROUP_CASES)
+def test_eight_query_groups_are_given(cfg):
+    S, _, Hq, _, D, P, causal = cfg
+    for kf in (0, 2):  # plain, KeyFormer with seeded noise
+        assert ext.lib()._ZN3tri12prefill_formEiiiibi(S, P, Hq, D, ctypes.c_bool(causal), kf) == EIGHT_GROUPS
+
+
+def test_fp8_chunks_meet_every_form():
+    """The key-split attention of more than 32 tokens over fp8 rows: each of its forms at each head width it is tested with."""
+    form = ext.lib()._ZN3tri15split_attn_formEiiiib
+    seen = {(D, form(S, Hq, Hkv, P + S, ctypes.c_bool(True))) for S, _, Hq, Hkv, D, P, _ in test_gpu_fp8_kv.CASES if S > 32}
+    assert seen >= {(128, f) for f in range(3)} | {(64, f) for f in (0, 2)}

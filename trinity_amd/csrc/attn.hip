@@ -55,7 +55,7 @@ constexpr int kAttnStageRow = D + 8;  // halfs per row of an output tile staged 
 // taken against the same reference value, so the result is unchanged.
 constexpr float kLazyMax = 8.0f;
 constexpr int kTwoWayMaxWorkgroups = 256, kTwoWayMinKeys = 640;  // when the eight-wave variant runs
-constexpr int kTwoWayRoundsPlain = 352, kTwoWayRoundsSeeded = 448;  // ... and how far beyond a round (launch_attention)
+constexpr int kTwoWayRoundsPlain = 352, kTwoWayRoundsSeeded = 448;  // ... and how far beyond a round (prefill_form)
 constexpr int kTwoWayBlockShare = 16, kTwoWayLatePlain = 4, kTwoWayLateSeeded = 1;  // ... for so many query blocks a head
 constexpr int kEightGroupMinWorkgroups = 129, kEightGroupMaxWorkgroups = 256;  // (of 256 queries each)
 constexpr int kWideMinWorkgroups = 768;  // 64 queries per wave (head dimension 64) from this many workgroups on
@@ -1159,25 +1159,31 @@ static int launch_attn_split_h(const AttnArgs& a, int nwg, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-template <int D, int KF, bool FP8>
-static int launch_attn_split_t(const AttnArgs& a, int nwg, hipStream_t stream) {
-  if constexpr (!FP8)
-    if (a.pj != nullptr) return launch_attn_split_h<D, KF, FP8, 2, 1, true>(a, nwg, stream);
+// how the waves of a workgroup share its rows and a run's tiles (runs of keys in nwg workgroups)
+static int split_form(int S, int group, int Ltot, bool fp8, int nwg, int runs) {
   // chunks: eight waves on two tiles at a time, half the runs and with them half the partial results (300 tokens against
   // 6000 keys 83.8 -> 77.7 us for the whole block, 48 against 6000 39.6 -> 35.7, 100 x 71 heads against 9000 51 -> 46)
-  if constexpr (!FP8)
-    if (a.S > kFewMaxQueries) return launch_attn_split_h<D, KF, FP8, 1, 2>(a, nwg, stream);
-  if ((a.Hq / a.Hkv) * a.S <= kSplitHalvesRows) return launch_attn_split_h<D, KF, FP8, 2, 1>(a, nwg, stream);
+  if (!fp8 && S > kFewMaxQueries) return kSplitPairs;
+  if (group * S <= kSplitHalvesRows) return kSplitHalves;
   // fp8 where a CU has one workgroup at most and a long run to walk: eight waves on pairs of tiles.  128-wide heads keep two tiles
   // on their way with them, one without; 64-wide heads two either way.  Both are ahead from seven tiles a run (whole calls at some
   // 4.5, 6 and 8 tiles a run: Llama-3-8B heads, 24 tokens 35.0 -> 35.8 us, 34.8 level, 36.9 -> 36.2, 32 tokens 37.1 -> 38.7, 37.6 -> 38.1,
   // 40.0 -> 39.6, 28 against 32000 keys, 16 tiles, 48.0 -> 45.1; 71 heads of 64 on one, 4 tokens 25.4 -> 26.0, 26.2 -> 26.0, 27.8 -> 27.2,
   // 16 tiles 34.0 -> 31.7, one token, 4, 6 and 8 tiles, 24.3 -> 24.4, 25.9 -> 25.6, 27.2 -> 26.4; 64 of 64 on 8, 16 tokens 29.1 -> 29.7,
   // 30.1 -> 30.6, 33.0 -> 32.4; 16-bit tiles, which do not pass through registers, 28 against 32000 keys 53.5 -> 54.9)
-  if constexpr (FP8)
-    if (nwg <= kSplitPairWorkgroups && (a.P + a.S) / kKeyTile >= kSplitPairTiles * a.split_runs)
-      return launch_attn_split_h<D, KF, FP8, 1, 2>(a, nwg, stream);
-  return launch_attn_split_h<D, KF, FP8, 1, 1>(a, nwg, stream);
+  if (fp8 && nwg <= kSplitPairWorkgroups && Ltot / kKeyTile >= kSplitPairTiles * runs) return kSplitPairs;
+  return kSplitFourWaves;
+}
+
+template <int D, int KF, bool FP8>
+static int launch_attn_split_t(const AttnArgs& a, int nwg, hipStream_t stream) {
+  if constexpr (!FP8)
+    if (a.pj != nullptr) return launch_attn_split_h<D, KF, FP8, 2, 1, true>(a, nwg, stream);
+  switch (split_form(a.S, a.Hq / a.Hkv, a.P + a.S, FP8, nwg, a.split_runs)) {
+    case kSplitPairs: return launch_attn_split_h<D, KF, FP8, 1, 2>(a, nwg, stream);
+    case kSplitHalves: return launch_attn_split_h<D, KF, FP8, 2, 1>(a, nwg, stream);
+    default: return launch_attn_split_h<D, KF, FP8, 1, 1>(a, nwg, stream);
+  }
 }
 
 // Number of runs for a call; false: the call is not of this kind, which takes at least kSplitMinKeys
@@ -1219,6 +1225,12 @@ bool split_attn_takes(int S, int Hq, int Hkv, int D, int Ltot, int64_t ws_bytes)
   return least > 0 && ws_bytes >= least;
 }
 
+int split_attn_form(int S, int Hq, int Hkv, int Ltot, bool fp8) {
+  int nsplit, fewest;
+  if (!split_plan(S, Hq, Hkv, Ltot, &nsplit, &fewest)) return -1;
+  return split_form(S, Hq / Hkv, Ltot, fp8, nsplit * ((((Hq / Hkv) * S + 127) / 128) * Hkv), nsplit);
+}
+
 static int launch_attn_split(const AttnArgs& a, hipStream_t stream) {
   const int Ltot = a.P + a.S;
   const int kf = a.lse_pert == nullptr ? 0 : ((a.noise == nullptr && a.tau == 1.0f) ? 2 : 1);
@@ -1247,6 +1259,38 @@ static int launch_attn_split(const AttnArgs& a, hipStream_t stream) {
   return launch_attention_few_combine(b, nsplit, stream);
 }
 
+int prefill_form(int S, int P, int Hq, int D, bool causal, int kf) {
+  // At most one workgroup per CU and a long key axis: eight waves per workgroup walk the keys two tiles at a
+  // time (Llama-3-8B, four-wave -> eight-wave kernel: S = 1024 26 -> 20.8 us, S = 768 20.0 -> 17.5 us, S = 512
+  // 14.4 -> 14.3 us, S = 256 9.6 -> 11.0 us).
+  const int64_t wgs = (int64_t)((S + 127) / 128) * Hq;
+  // Causal, 128-wide heads, somewhat more than a round: eight waves take whole query blocks, longest first, all of them
+  // busy to a block's end, where the eight query groups below leave a late wave alone on its SIMD.  Whole calls of 32
+  // heads on 8, eight groups -> this: plain, S = 1030 86.8 -> 83.4 us, 1152 89.8 -> 86.4, 1408 (352 workgroups) 112.9 ->
+  // 109.4, 1472 113.5 -> 113.3, 2048 142.9 -> 145.1, 2304 182 -> 189; seeded KeyFormer, 1408 161.6 -> 154.8, 1664 (416)
+  // 180.5 -> 174.3, 2048 211.2 -> 210.2.  A cached prefix evens the blocks out: 1100 tokens behind 1100 keys level,
+  // 1280 behind 3000 169.5 -> 176.4.  64-wide heads lose (71 heads, S = 768 57.8 -> 60.6).
+  // The workgroups beyond the round have to be few beside a head's query blocks: with short sequences and many heads the
+  // second round is as long as the first (plain, 32 heads x 9 blocks -1.9 %, 48 x 6 +0.6, 36 x 9 -0.9, 52 x 6 +2.4, 32 x 11 -0.8, 44 x 8
+  // +1.5; seeded, 28 x 12 -4.4, 56 x 6 +0.8, 32 x 13 -2.0, 52 x 8 +1.8, 36 x 12 level; 12 to 20 heads as long ones).
+  const int blocks = (S + 127) / 128, late = kf == 2 ? kTwoWayLateSeeded : kTwoWayLatePlain;
+  const int rounds = kf == 2 ? kTwoWayRoundsSeeded : kTwoWayRoundsPlain;
+  const bool turns = D == 128 && causal && kf != 1 && 2 * P <= S && wgs <= rounds &&
+                     wgs - kTwoWayMaxWorkgroups <= kTwoWayBlockShare * (blocks - late);
+  const bool two = (wgs <= kTwoWayMaxWorkgroups || turns) && P + S >= kTwoWayMinKeys;
+  // One round of four-wave workgroups under a causal mask: eight query groups per workgroup instead (128-wide
+  // heads; with 64-wide heads it is level at best: 71 heads S = 768 17.2 -> 17.7 us, 32 heads S = 2048 36.3 -> 35.5)
+  const int64_t wgs8 = (int64_t)((S + 255) / 256) * Hq;
+  const bool eight = causal && kf != 1 && !two && wgs8 >= kEightGroupMinWorkgroups && wgs8 <= kEightGroupMaxWorkgroups;
+  if (two) return turns && wgs > kTwoWayMaxWorkgroups ? kPrefillTwoWaysWhole : kPrefillTwoWays;
+  if (D == 128) return eight ? kPrefillEightGroups : kPrefillFourWaves;
+  // 64-wide heads leave registers for 64 queries per wave: half the LDS reads and K/V loads per flop.  It pays
+  // once the twice-as-large workgroups still fill the chip three times over (S = 3072 x 71 heads: 138.4 ->
+  // 133.7 us, S = 4096: 235 -> 224 us, S = 8192: 782 -> 718 us; S = 2048: 62.3 -> 67.5 us)
+  // (the general KeyFormer variant has no registers for it)
+  return kf != 1 && wgs8 >= kWideMinWorkgroups ? kPrefillWide : kPrefillFourWaves;
+}
+
 int launch_attention(const AttnArgs& a, hipStream_t stream, int* merge_parts) {
   if (merge_parts != nullptr) *merge_parts = 0;
   if (a.S <= 0) return 0;
@@ -1261,40 +1305,14 @@ int launch_attention(const AttnArgs& a, hipStream_t stream, int* merge_parts) {
   // (fp8 caches and projections in parts are read by the two variants above only)
   if (a.k == nullptr || a.v == nullptr || a.pj != nullptr) return -1;
   const int kf = a.lse_pert == nullptr ? 0 : ((a.noise == nullptr && a.tau == 1.0f) ? 2 : 1);
-  // At most one workgroup per CU and a long key axis: eight waves per workgroup walk the keys two tiles at a
-  // time (Llama-3-8B, four-wave -> eight-wave kernel: S = 1024 26 -> 20.8 us, S = 768 20.0 -> 17.5 us, S = 512
-  // 14.4 -> 14.3 us, S = 256 9.6 -> 11.0 us).
-  const int64_t wgs = (int64_t)((a.S + 127) / 128) * a.Hq;
-  // Causal, 128-wide heads, somewhat more than a round: eight waves take whole query blocks, longest first, all of them
-  // busy to a block's end, where the eight query groups below leave a late wave alone on its SIMD.  Whole calls of 32
-  // heads on 8, eight groups -> this: plain, S = 1030 86.8 -> 83.4 us, 1152 89.8 -> 86.4, 1408 (352 workgroups) 112.9 ->
-  // 109.4, 1472 113.5 -> 113.3, 2048 142.9 -> 145.1, 2304 182 -> 189; seeded KeyFormer, 1408 161.6 -> 154.8, 1664 (416)
-  // 180.5 -> 174.3, 2048 211.2 -> 210.2.  A cached prefix evens the blocks out: 1100 tokens behind 1100 keys level,
-  // 1280 behind 3000 169.5 -> 176.4.  64-wide heads lose (71 heads, S = 768 57.8 -> 60.6).
-  // The workgroups beyond the round have to be few beside a head's query blocks: with short sequences and many heads the
-  // second round is as long as the first (plain, 32 heads x 9 blocks -1.9 %, 48 x 6 +0.6, 36 x 9 -0.9, 52 x 6 +2.4, 32 x 11 -0.8, 44 x 8
-  // +1.5; seeded, 28 x 12 -4.4, 56 x 6 +0.8, 32 x 13 -2.0, 52 x 8 +1.8, 36 x 12 level; 12 to 20 heads as long ones).
-  const int blocks = (a.S + 127) / 128, late = kf == 2 ? kTwoWayLateSeeded : kTwoWayLatePlain;
-  const int rounds = kf == 2 ? kTwoWayRoundsSeeded : kTwoWayRoundsPlain;
-  const bool turns = a.D == 128 && a.causal && kf != 1 && 2 * a.P <= a.S && wgs <= rounds &&
-                     wgs - kTwoWayMaxWorkgroups <= kTwoWayBlockShare * (blocks - late);
-  const bool two = (wgs <= kTwoWayMaxWorkgroups || turns) && a.P + a.S >= kTwoWayMinKeys;
-  // One round of four-wave workgroups under a causal mask: eight query groups per workgroup instead (128-wide
-  // heads; with 64-wide heads it is level at best: 71 heads S = 768 17.2 -> 17.7 us, 32 heads S = 2048 36.3 -> 35.5)
-  const int64_t wgs8 = (int64_t)((a.S + 255) / 256) * a.Hq;
-  const bool eight = a.causal && kf != 1 && !two && wgs8 >= kEightGroupMinWorkgroups && wgs8 <= kEightGroupMaxWorkgroups;
+  const int form = prefill_form(a.S, a.P, a.Hq, a.D, a.causal != 0, kf);
+  const bool two = form == kPrefillTwoWays || form == kPrefillTwoWaysWhole;
   if (a.D == 128) {
-    if (eight) return kf == 0 ? launch_attn_t<128, 1, 0, 1, 2>(a, stream) : launch_attn_t<128, 1, 2, 1, 2>(a, stream);
+    if (form == kPrefillEightGroups) return kf == 0 ? launch_attn_t<128, 1, 0, 1, 2>(a, stream) : launch_attn_t<128, 1, 2, 1, 2>(a, stream);
     return two ? launch_attn_kf<128, 2>(a, kf, stream) : launch_attn_kf<128, 1>(a, kf, stream);
   }
   if (a.D == 64) {
-    // 64-wide heads leave registers for 64 queries per wave: half the LDS reads and K/V loads per flop.  It pays
-    // once the twice-as-large workgroups still fill the chip three times over (S = 3072 x 71 heads: 138.4 ->
-    // 133.7 us, S = 4096: 235 -> 224 us, S = 8192: 782 -> 718 us; S = 2048: 62.3 -> 67.5 us)
-    const int64_t wgs2 = (int64_t)((a.S + 255) / 256) * a.Hq;
-    // (the general KeyFormer variant has no registers for it)
-    if (kf != 1 && wgs2 >= kWideMinWorkgroups)
-      return kf == 0 ? launch_attn_t<64, 2, 0, 1>(a, stream) : launch_attn_t<64, 2, 2, 1>(a, stream);
+    if (form == kPrefillWide) return kf == 0 ? launch_attn_t<64, 2, 0, 1>(a, stream) : launch_attn_t<64, 2, 2, 1>(a, stream);
     return two ? launch_attn_kf<64, 2>(a, kf, stream) : launch_attn_kf<64, 1>(a, kf, stream);
   }
   return -1;

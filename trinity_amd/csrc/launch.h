@@ -190,7 +190,16 @@ int launch_attention_few_combine(const AttnArgs& a, int nsplit, hipStream_t stre
 // workspace of launch_attention's long-prefix variant for a call (0 when it does not take it): for all the runs it would
 // cut the key axis into, or (least) for the fewest it works with - given less than the former it takes fewer runs
 int64_t split_attn_workspace_bytes(int S, int Hq, int Hkv, int D, int Ltot, bool least);
+// the kernel of calls that neither the key-split nor the few-query kernels take: four waves on 32 queries each; eight waves on two
+// tiles of keys at a time, within a round of workgroups (causal: a late and an early half block of queries) or beyond it
+// (whole blocks); eight query groups; four waves on 64 queries each
+enum PrefillForm { kPrefillFourWaves, kPrefillTwoWays, kPrefillTwoWaysWhole, kPrefillEightGroups, kPrefillWide };
+int prefill_form(int S, int P, int Hq, int D, bool causal, int kf);  // (kf: 0 plain and RoCo, 1 KeyFormer, 2 with seeded noise)
 bool split_attn_takes(int S, int Hq, int Hkv, int D, int Ltot, int64_t ws_bytes);  // the key-split kernel runs, with that workspace
+// its form for a call with room for all runs (-1: not taken): four waves on 32 stacked rows each; two query groups whose waves take the
+// two halves of a tile; eight waves on two tiles at a time
+enum SplitForm { kSplitFourWaves, kSplitHalves, kSplitPairs };
+int split_attn_form(int S, int Hq, int Hkv, int Ltot, bool fp8);
 // From this many keys on, plain attention for few new tokens leaves the one-tile-per-wave kernel for one that
 // loops over its keys with the query heads of a KV head stacked along the query axis (launch_attention decides).
 // 16 tokens: at 1040 keys the two are level, at 2064 keys the looping kernel is 2-5 us ahead, at 32784 keys
