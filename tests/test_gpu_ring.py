@@ -125,6 +125,26 @@ def test_one_row_of_any_stride_in_place(rn, stride):
     check(t, want, "in place")
 
 
+# first products with GELU, whose hidden rows go through the epilogue of the same tiles, also beyond 1100 rows
+GELU_TILES = [
+    (385, 96, 11264, (128, 192, 1)), (257, 1056, 11264, (192, 128, 1)), (513, 96, 14016, (192, 192, 1)),
+    (700, 1056, 9024, (256, 128, 1)), (1120, 4544, 18176, (160, 256, 1)), (1500, 4544, 18176, (192, 192, 1)),
+]
+
+
+@pytest.mark.parametrize("M,K,N,plan", GELU_TILES)
+@pytest.mark.parametrize("kcontig", [False, True])
+def test_gelu_tiles(rn, M, K, N, plan, kcontig):
+    x = rn(M, K)
+    w = rn(N, K, std=K ** -0.5).t() if kcontig else rn(K, N, std=K ** -0.5)
+    w2 = rn(64, N, std=N ** -0.5).t() if kcontig else rn(N, 64, std=N ** -0.5)
+    want = torch.nn.functional.gelu(x.float() @ w.float())
+    for ws in (None, torch.empty(ext.ffn_workspace_bytes(M, K, N), dtype=torch.uint8, device="cuda:0")):
+        hidden = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda:0")
+        ext.ffn_gelu(x, w, w2, hidden, torch.empty(M, 64, dtype=torch.float16, device="cuda:0"), workspace=ws)
+        check(hidden, want, "gelu(x.w)")
+
+
 LOADING_WAVES_QKV = [  # S, N, Hq, Hkv, D, (without, with QKNorm)
     (577, 1056, 48, 48, 64, [(128, 192, 1)] * 2), (769, 64, 71, 1, 64, [(192, 128, 1)] * 2),
     (1000, 1056, 71, 1, 64, [(192, 128, 1)] * 2), (900, 1056, 48, 48, 64, [(192, 192, 1)] * 2),

@@ -71,6 +71,14 @@ def test_loading_waves_of_gated_products_are_given(row):
             assert plan_of(M, K, F, SWIGLU, kcontig, ws) == plan
 
 
+@pytest.mark.parametrize("row", test_gpu_ring.GELU_TILES)
+def test_gelu_tiles_are_given(row):
+    M, K, N, plan = row
+    for kcontig in (False, True):
+        for ws in (0, ext.ffn_workspace_bytes(M, K, N)):
+            assert plan_of(M, K, N, GELU, kcontig, ws) == plan
+
+
 @pytest.mark.parametrize("row", test_gpu_ring.LOADING_WAVES_QKV)
 def test_loading_waves_of_projections_are_given(row):
     S, N, Hq, Hkv, D, tiles = row
