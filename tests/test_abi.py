@@ -56,17 +56,17 @@ class _RingPlan(ctypes.Structure):
     _fields_ = [("tile", ctypes.c_int), ("parts", ctypes.c_int), ("us", ctypes.c_float)]
 
 
-@pytest.mark.parametrize("ncols,head", [(6144, 128), (6144, 1), (12288, 128), (4672, 64)])
+@pytest.mark.parametrize("ncols,head", [(6144, 128), (6144, 0), (12288, 128), (4672, 64)])
 def test_projection_workspace_is_what_its_plan_uses(ncols, head):
     """Scratch is asked for the parts that the projection then runs in, and for nothing else (the planner's own functions,
     csrc/launch.h: no part of the C ABI)."""
-    room, plan = ext.lib()._ZN3tri19qkv_workspace_bytesEiiiib, ext.lib()._ZN3tri9ring_planEiiiiilf
-    room.restype, plan.restype = ctypes.c_int64, _RingPlan
+    room, takes = ext.lib()._ZN3tri19qkv_workspace_bytesEiiiib, ext.lib()._ZN3tri13qkv_ring_planEiiiiblbRNS_8RingPlanE
+    room.restype = ctypes.c_int64
     K = 4544 if head == 64 else 4096
-    for S in (1, 16, 33, 100, 200, 333, *range(500, 1101, 12)):
-        ws = room(S, K, ncols, head, False)
-        parts = plan(S, K, ncols, head, 0, ctypes.c_int64(ws), ctypes.c_float(3.5)).parts
-        assert ws == (parts * S * ncols * 4 if parts > 1 else 0), "%d tokens: %d bytes for %d parts" % (S, ws, parts)
+    for S in (1, 16, 33, 100, 150, 200, 333, *range(500, 1101, 12)):
+        ws, plan = room(S, K, ncols, max(head, 1), False), _RingPlan()
+        takes(S, K, ncols, head, False, ctypes.c_int64(ws), False, ctypes.byref(plan))
+        assert ws == (plan.parts * S * ncols * 4 if plan.parts > 1 else 0), "%d tokens: %d bytes for %d parts" % (S, ws, plan.parts)
 
 
 def _h(*shape):

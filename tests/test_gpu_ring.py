@@ -145,13 +145,16 @@ def test_gelu_tiles(rn, M, K, N, plan, kcontig):
         check(hidden, want, "gelu(x.w)")
 
 
-LOADING_WAVES_QKV = [  # S, N, Hq, Hkv, D, (without, with QKNorm)
+QKV_TILES = [  # S, N, Hq, Hkv, D, (without, with QKNorm)
     (577, 1056, 48, 48, 64, [(128, 192, 1)] * 2), (769, 64, 71, 1, 64, [(192, 128, 1)] * 2),
     (1000, 1056, 71, 1, 64, [(192, 128, 1)] * 2), (900, 1056, 48, 48, 64, [(192, 192, 1)] * 2),
     (700, 1056, 48, 48, 64, [(256, 128, 1)] * 2), (129, 4128, 48, 48, 64, [(192, 128, 3)] * 2),
     (385, 96, 32, 32, 128, [(128, 192, 1), (256, 128, 1)]), (1000, 1056, 32, 8, 128, [(128, 192, 1), (256, 128, 1)]),
     (650, 64, 32, 8, 128, [(192, 128, 1)] * 2), (333, 1056, 64, 64, 128, [(192, 192, 1), (192, 128, 1)]),
     (577, 1056, 64, 8, 128, [(256, 128, 1)] * 2),
+    # one round of 32-row tiles: 240 workgroups, last row blocks of one row and full ones, columns that end in half a tile
+    (129, 96, 32, 8, 128, [(32, 128, 1)] * 2), (160, 4096, 32, 8, 128, [(32, 128, 1)] * 2),
+    (150, 2560, 95, 1, 64, [(32, 128, 1)] * 2), (289, 1056, 16, 4, 128, [(64, 64, 1), (32, 128, 1)]),
 ]
 
 
@@ -159,7 +162,7 @@ LOADING_WAVES_QKV = [  # S, N, Hq, Hkv, D, (without, with QKNorm)
     (1, 64, 4, 4, 64), (33, 96, 5, 1, 128), (100, 4096, 32, 8, 128), (260, 4096, 32, 8, 128), (200, 4544, 71, 1, 64),
     (700, 128, 32, 8, 128), (1000, 128, 71, 1, 64), (1100, 160, 32, 4, 128),  # a tile across two weight matrices
     (150, 4128, 32, 8, 128),
-] + [row[:5] for row in LOADING_WAVES_QKV])
+] + [row[:5] for row in QKV_TILES])
 @pytest.mark.parametrize("qknorm", [False, True])
 @pytest.mark.parametrize("kcontig", [False, True])
 def test_qkv_projection(rn, S, N, Hq, Hkv, D, qknorm, kcontig):

@@ -15,7 +15,7 @@ NONE, GELU, SWIGLU = 0, 1, 2
 LARGE = (256, 256, 1)
 # the ring kernels' tiles by number (csrc/ring.h: TRI_RING_TILES)
 TILES = [(32, 128), (64, 64), (64, 128), (96, 128), (128, 128), (128, 192), (128, 256), (160, 256), (192, 128), (192, 192),
-         (256, 128)]
+         (256, 128), (32, 128)]  # (the last for projections only: kRingTileFine)
 
 
 class Plan(ctypes.Structure):
@@ -79,8 +79,8 @@ def test_gelu_tiles_are_given(row):
             assert plan_of(M, K, N, GELU, kcontig, ws) == plan
 
 
-@pytest.mark.parametrize("row", test_gpu_ring.LOADING_WAVES_QKV)
-def test_loading_waves_of_projections_are_given(row):
+@pytest.mark.parametrize("row", test_gpu_ring.QKV_TILES)
+def test_projection_tiles_are_given(row):
     S, N, Hq, Hkv, D, tiles = row
     takes = ext.lib()._ZN3tri13qkv_ring_planEiiiiblbRNS_8RingPlanE
     takes.restype = ctypes.c_bool

@@ -401,9 +401,8 @@ static float plan_us(const TilePlan& p, int K) { return 6.0f + 0.0272f * (float)
 // products 2.4 %, 3.9 by a twentieth (8192 rows x [4096, 1024] 74.4 -> 88.3, x [14336, 1024] 239 -> 270).
 constexpr float kRingMarginNarrow = 0.95f, kRingMarginTall = 0.75f;
 constexpr int kRingTallRows = 6144;
-static bool ring_wins(float big_us, int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes, RingPlan& plan,
-                      float merge_us = kRingMergeUs) {
-  plan = ring_plan(M, K, ncols, unit, min_bn, ws_bytes, merge_us);
+static bool ring_wins(float big_us, int M, int K, int ncols, int min_bn, int64_t ws_bytes, RingPlan& plan) {
+  plan = ring_plan(M, K, ncols, 1, min_bn, ws_bytes);
   return plan.tile >= 0 && plan.us < big_us * (M <= kRingMaxRows ? 1.0f : (M <= kRingTallRows ? kRingMarginNarrow : kRingMarginTall));
 }
 
@@ -435,8 +434,8 @@ static TilePlan big_plan(int M, int N, int epi, bool kcontig) {
 constexpr int kGatedMinBn = 128;
 
 // workspace of the best plan, if it has at least `least` parts (0 otherwise)
-static int64_t plan_workspace_bytes(int M, int K, int ncols, int unit, int min_bn, int least, float merge_us = kRingMergeUs) {
-  const RingPlan plan = ring_plan(M, K, ncols, unit, min_bn, INT64_MAX, merge_us);
+static int64_t plan_workspace_bytes(int M, int K, int ncols, int min_bn, int least) {
+  const RingPlan plan = ring_plan(M, K, ncols, 1, min_bn, INT64_MAX);
   return plan.tile < 0 || plan.ksplit < least ? 0 : (int64_t)plan.ksplit * M * ncols * 4;
 }
 
@@ -448,14 +447,14 @@ int64_t gemm_workspace_bytes(int M, int K, int ncols) {
   if (M > kRingMaxRows) {  // (plain and GELU products only; the tile plan over K-contiguous weights is the dearer one)
     RingPlan plan;
     if (M > kRingMaxRowsNarrow || ncols > kRingMaxColsNarrow ||
-        !ring_wins(plan_us(big_plan(M, ncols, EPI_NONE, true), K), M, K, ncols, 1, 0, INT64_MAX, plan))
+        !ring_wins(plan_us(big_plan(M, ncols, EPI_NONE, true), K), M, K, ncols, 0, INT64_MAX, plan))
       return 0;
-    return plan_workspace_bytes(M, K, ncols, 1, 0, 2);
+    return plan_workspace_bytes(M, K, ncols, 0, 2);
   }
   const bool one_part = M <= kInPlaceRows || (M <= kInPlaceRowsSmall && 2 * (int64_t)K * ncols <= kInPlaceSmallBytes);
   const int least = one_part ? 1 : 2;
-  const int64_t any = plan_workspace_bytes(M, K, ncols, 1, 0, least);
-  const int64_t gated = plan_workspace_bytes(M, K, ncols, 1, kGatedMinBn, least);
+  const int64_t any = plan_workspace_bytes(M, K, ncols, 0, least);
+  const int64_t gated = plan_workspace_bytes(M, K, ncols, kGatedMinBn, least);
   return any > gated ? any : gated;
 }
 
@@ -490,7 +489,7 @@ constexpr float kGeluBigCost = 1.2f;
 bool gemm_plan(int M, int K, int N, int epi, bool kcontig, int64_t ws_bytes, RingPlan& plan) {
   const bool gated = epi == EPI_SWIGLU;
   const float big_us = plan_us(big_plan(M, N, epi, kcontig), K) * (epi == EPI_GELU ? kGeluBigCost : 1.0f);
-  return ring_wins(big_us, M, K, gated ? 2 * N : N, 1, gated && !kcontig ? kGatedMinBn : 0, ws_bytes, plan);
+  return ring_wins(big_us, M, K, gated ? 2 * N : N, gated && !kcontig ? kGatedMinBn : 0, ws_bytes, plan);
 }
 
 int launch_gemm(const GemmArgs& a, hipStream_t stream) {
@@ -567,15 +566,24 @@ static int launch_qkv_d(const QkvProjArgs& a, hipStream_t stream) {
 // 0.3 faster to 0.7 slower for 16, 2.9 to 3.8 faster for 32.
 static float deferred_merge_us(int S) { return 1.2f + 0.12f * (float)S; }
 
+static RingPlan qkv_ring(int S, int K, int ncols, int unit, int64_t ws_bytes, bool deferred) {
+  RingPlan plan = ring_plan(S, K, ncols, unit, 0, ws_bytes, deferred ? deferred_merge_us(S) : kRingMergeUs);
+  ring_fine_plan(S, K, ncols, plan);
+  return plan;
+}
+
 int64_t qkv_workspace_bytes(int S, int K, int ncols, int unit, bool deferred) {
-  return S > kRingMaxRows ? 0 : plan_workspace_bytes(S, K, ncols, unit, 0, 2, deferred ? deferred_merge_us(S) : kRingMergeUs);
+  if (S > kRingMaxRows) return 0;
+  const RingPlan plan = qkv_ring(S, K, ncols, unit, INT64_MAX, deferred);
+  return plan.tile < 0 || plan.ksplit < 2 ? 0 : (int64_t)plan.ksplit * S * ncols * 4;
 }
 
 bool qkv_ring_plan(int S, int K, int ncols, int head, bool kcontig, int64_t ws_bytes, bool deferred, RingPlan& plan) {
   int which;
   const TilePlan big = kcontig ? qkv_plan_kcontig(S, ncols) : qkv_plan(S, ncols, head, which);
-  return S <= kRingMaxRows && ring_wins(plan_us(big, K), S, K, ncols, head > 0 ? head : 1, 0, ws_bytes, plan,
-                                        deferred ? deferred_merge_us(S) : kRingMergeUs);
+  if (S > kRingMaxRows) return false;
+  plan = qkv_ring(S, K, ncols, head > 0 ? head : 1, ws_bytes, deferred);
+  return plan.tile >= 0 && plan.us < plan_us(big, K);
 }
 
 int launch_qkv_proj(const QkvProjArgs& a, hipStream_t stream, int* deferred_ksplit, bool* appended) {

@@ -100,6 +100,8 @@ constexpr int kRingMaxRowsNarrow = 8192, kRingMaxColsNarrow = 1 << 16, kRingMinK
 // merge_us: what the merge of parts takes beside its bytes.
 constexpr float kRingMergeUs = 3.5f;
 RingPlan ring_plan(int M, int K, int ncols, int unit, int min_bn, int64_t ws_bytes, float merge_us = kRingMergeUs);
+// a Q/K/V projection's ring plan gives way to 32-row tiles in one round where they are cheaper
+bool ring_fine_plan(int M, int K, int ncols, RingPlan& plan);
 int launch_ring_gemm(const GemmArgs& a, const RingPlan& plan, hipStream_t stream);
 // whether launch_gemm runs such a product by its ring plan (else by large tiles)
 bool gemm_plan(int M, int K, int N, int epi, bool kcontig, int64_t ws_bytes, RingPlan& plan);

@@ -97,6 +97,10 @@ constexpr int kRingTileOneBlock = 0;  // the non-temporal tile, for a single row
 // everywhere 2.3 and 0.4 %, four everywhere 0.7 and 1.5 %.  A column view whose first element is 128 bytes into a line of 256
 // changes nothing ([4096, 4096] three / four 11.6 / 11.9 with it, 11.8 / 12.0 without).
 using RingTileFour = RingTile<32, 128, 1, 4, 4, true>;
+// Q/K/V projections of more than 32 rows in one part and one round (ring_fine_plan): the only tile that takes whole 128-wide heads,
+// or 130 to 160 rows of 6144 columns, without parts, whose merge norms and scatters.
+using RingTileFine = RingTile<32, 128, 1, 4, 4>;
+constexpr int kRingTileFine = kRingTiles;
 // K-contiguous columns a power of two of 8 KB and more apart: the memory is slow there.
 inline bool ring_slow_columns(int64_t ld) { return ld >= 4096 && (ld & (ld - 1)) == 0; }
 // (ld: distances between rows or columns, several or-ed together; k_part: K of a workgroup)

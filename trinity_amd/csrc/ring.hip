@@ -260,7 +260,7 @@ static int launch_epi_t(const GemmArgs& a, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-constexpr int kRingTileNarrow = kRingTiles;  // (not planned by ring_plan: RingTileKContig)
+constexpr int kRingTileNarrow = kRingTileFine + 1;  // (not planned by ring_plan: RingTileKContig)
 
 template <int EPI>
 static int launch_epi(const GemmArgs& a, int tile, hipStream_t stream) {
@@ -370,6 +370,26 @@ static RingPlan ring_plan_search(int M, int K, int ncols, int unit, int min_bn, 
     }
   }
   return best;
+}
+
+// RingTileFine, for projections only (its cost chosen over 140 whole calls, with weights from memory and from the last-level
+// cache, 192 to 256 workgroups).  Whole calls, the best of the family without it -> this: 131 to 160 rows x [2560, 6144] 26.2 - 27.7 ->
+// 24.9 - 26.5 us, x [4096, 6144] 34.2 - 36.2 -> 35.0 - 36.9, but 29.0 -> 26.5 with the weights from the last-level cache; QKNorm of
+// 200 to 320 rows x [2048, 3072] 23.8 - 26.5 -> 20.0 - 23.3, 64 to 320 x [1024, 1536] 15.0 - 18.8 -> 13.2 - 17.6.  Not taken: QKNorm
+// of 35 to 64 x [4096, 12288] 34.5 -> 36.6, of 131 to 192 x [3072, 5120] 28.0 -> 30.1, of 99 to 128 x [4096, 6144] 30.6 -> 36.2; the
+// plain product of 150 x [4096, 6144], whose merge is cheaper, 26.4 -> 28.7.
+constexpr float kRingFineTile = 0.37f;  // us per k tile; the rest as in ring_plan_search
+bool ring_fine_plan(int M, int K, int ncols, RingPlan& plan) {
+  const int tiles = ((M + RingTileFine::BM - 1) / RingTileFine::BM) * ((ncols + RingTileFine::BN - 1) / RingTileFine::BN);
+  if (plan.tile < 0 || M <= kRingCost[kRingTileOneBlock].bm || M > kRingMaxRows || tiles > 256) return false;
+  const float mem = 2.0f * (float)K * (float)ncols / 21.3e6f + 2.0f * (float)M * (float)ncols / 1.81e6f;
+  const float per = (float)ring_kt_per_part(K, 1), loads = (float)tiles * per * (RingTileFine::BM + RingTileFine::BN) * 128.0f / 50.4e6f;
+  float comp = per * kRingFineTile;
+  if (tiles <= kRingStreamWorkgroups && M <= kRingStreamRows) comp = fmaxf(comp, per * RingTileFine::BN * 128.0f / kRingStreamRate);
+  const float us = 1.37f + sqrtf(mem * mem + comp * comp + loads * loads);
+  if (us >= plan.us) return false;
+  plan = RingPlan{kRingTileFine, 1, us};
+  return true;
 }
 
 // The search is a pure function of its arguments and takes 5 to 10 us, longer than a launch; each thread keeps the

@@ -133,6 +133,7 @@ template <int D>
 static int launch_qkv_tile(const QkvProjArgs& a, int tile, hipStream_t stream) {
   if (tile == kRingTileOneBlock && ring_fourth_stage(a.S, ((a.Hq + 2 * a.Hkv) * D + 127) / 128, a.ldwq | a.ldwk | a.ldwv, a.K, a.w_kcontig != 0, false))
     return a.w_kcontig ? launch_qkv_t<RingTileFour, D, true>(a, stream) : launch_qkv_t<RingTileFour, D, false>(a, stream);
+  if (tile == kRingTileFine) return a.w_kcontig ? launch_qkv_t<RingTileFine, D, true>(a, stream) : launch_qkv_t<RingTileFine, D, false>(a, stream);
   switch (tile) {
 #define TRI_RING_CASE(id, bm, bn, wm, wn, nst, nt, np)                                                    \
   case id:                                                                                        \
