@@ -211,10 +211,11 @@ int64_t tri_qkv_scratch_bytes(const tri_attn_params* p, int64_t n_model);
  *   With p->kv_fp8 the caches are TRI_FP8_E4M3 (required, also when P == 0), rows of a
  *   multiple of 16 bytes: the new rows are appended as fp8(k / k_scale), fp8(v / v_scale)
  *   (round to nearest even, saturating at +-448) and attention then reads every key,
- *   cached or new, from the fp8 rows - with at most 32 new tokens straight from the cache
- *   (half the bytes of a 16-bit cache), otherwise through a 16-bit copy in the scratch
- *   buffer; the scales are applied in fp32 (k_scale with the softmax scale, v_scale with
- *   the final normalisation).  No counterpart in the reference, whose caches are fp16;
+ *   cached or new, from the fp8 rows - without an lse straight from the cache (half the bytes
+ *   of a 16-bit one) for at most 32 new tokens and for chunks of more that leave most of the
+ *   chip idle otherwise, from 2048 keys on; in all other calls through a 16-bit copy in the
+ *   scratch buffer; the scales are applied in fp32 (k_scale with the softmax scale, v_scale
+ *   with the final normalisation).  No counterpart in the reference, whose caches are fp16;
  *   scratch: 1-D byte buffer (tri_qkv_scratch_bytes), 256-byte aligned; lse fp32 [Hq, S] or NULL;
  *   out [S, Hq*D]. */
 int tri_qkv_attention(const tri_tensor* x, const tri_tensor* norm_w, const tri_tensor* wq, const tri_tensor* wk,

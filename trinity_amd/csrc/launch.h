@@ -165,7 +165,7 @@ struct AttnArgs {
   float* ws;  // nullable: workspace of the few-query path (few_attn_workspace_bytes)
   int64_t ws_bytes;
   float out_scale;  // multiplies the normalised output (v_scale of an fp8 cache; 1 otherwise)
-  // fp8 (e4m3) caches read directly - few-query path only; k / v are then unused.  Strides in elements = bytes.
+  // fp8 (e4m3) caches read directly - by the few-query and key-split kernels, without log-sum-exps; k / v are then unused.  Strides in elements = bytes.
   const uint8_t *k8, *v8;
   int64_t k8_sh, k8_sr, v8_sh, v8_sr;
   // Few-query paths fused with the merge of a split-K projection (pj != nullptr): q and
